@@ -6,10 +6,11 @@
 //    products v_mfma_f32_32x32x16_bf16, three quarters of a fragment read for a product (the kernel for 33 to 256
 //    rows, a wave 32 columns wide and all the rows, reads more than one).  Four waves of 128 x 128, one a SIMD with
 //    256 accumulation registers, read half a fragment a product and were 2 % slower: with one wave a SIMD nobody
-//    multiplies while a wave waits for the barrier.  The products that do not give every CU a block of 256 rows
-//    have blocks of 128 rows by 256 columns, four waves of 64 x 128.
+//    multiplies while a wave waits for the barrier.  The products that do not give every CU such a block have blocks
+//    of 128 x 128, four waves of 64 x 64 (128 x 256 and 256 x 128 with four waves were never the best of 60 products
+//    of 300 to 2,048 rows, nor 128 x 128 with eight waves of 64 x 32).
 //  * A and W go from memory straight into LDS (global_load_lds_dwordx4), a stage of 32 columns of K at a time into a
-//    ring of five stages (all of LDS with blocks of 256 rows): a load is 16 rows of 64 bytes, whole halves of memory's
+//    ring of AHEAD + 3 stages: a load is 16 rows of 64 bytes, whole halves of memory's
 //    lines, and every wave sends its share of a stage's loads.  (W straight into registers, which a wave that owns
 //    its columns alone could do, is 64 cache accesses a load, one a lane, where these are 16: the cache then took
 //    longer than the products.)
@@ -27,7 +28,9 @@
 //    took a tenth of a block's time).  A pair of stages' loads go out one to two stages before the barrier that
 //    hands its first stage on (a ring
 //    of four stages with every load a stage later gave the same times: what the blocks wait for when every CU has
-//    one is not the latency of a load).
+//    one is not the latency of a load).  A block of 128 x 128 alone on its CU is another matter: a stage is 256 cycles
+//    of products, three of them are not a load's latency, and with the pairs six stages ahead (nine stages in LDS) 643
+//    rows of 4,096 x 1,024 take 12.4 us and not 14.1, 1,000 rows 12.6 and not 14.1; two blocks a CU need no more than two.
 //  * More rows than a block's are blocks of rows over the same W, which then comes from L2: the blocks of one XCD
 //    (every eighth of the grid) take a run of consecutive pieces of work, numbered in patches of 8 row blocks by 4
 //    column blocks, so that the 32 blocks that run together on an XCD read 12 different bands of A and W and not 33
@@ -49,26 +52,25 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define WIDE_STAGE 32                                      // columns of K a stage: rows of 64 bytes
-#define WIDE_TILE 256                                      // columns of C a block
-#define WIDE_RING 5                                        // stages in LDS: 160 KB with blocks of 256 rows, 120 with 128
 #define WIDE_ROW_BYTES (WIDE_STAGE * 2)
 #define WIDE_XCDS 8
+#define WIDE_HOST_US 24.0                                  // products of at most this time by wide_us are not the BLAS's
 
-// RT, CT: tiles of 32 rows and of 32 columns of a wave; WAVES: 8 (2 x 4 waves of RT = 4, CT = 2: blocks of 256 rows) or
-// 4 (2 x 2 waves of RT = 2, CT = 4: blocks of 128 rows).  OUT: bf16_t or float (the result; with splits of K float32
-// partial sums [split][M][N]).  GATED (one split): W holds gate and up rows in turns of 16, a tile of 32 columns is 16
+// RT, CT: tiles of 32 rows and of 32 columns of a wave; DOWN, ACROSS: the block's waves above each other and side by side;
+// AHEAD: stages (even) that a pair's loads go out ahead.  OUT: bf16_t or float (the result; with splits of K float32 partial sums [split][M][N]).  GATED (one split): W holds gate and up rows in turns of 16, a tile of 32 columns is 16
 // of each, and C [M, N / 2] gets silu(gate) * up (qil/model.py:71), both still in float32.
-template <typename OUT, int RT, int CT, int WAVES, bool GATED>
-__global__ void __launch_bounds__(WAVES * QIL_WAVE, 1)
+template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
+__global__ void __launch_bounds__(DOWN * ACROSS * QIL_WAVE, RT * CT <= 4 && AHEAD == 2 ? 2 : 1)
 gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M_all, int N, int K,
                       int stages, int col_blocks, int row_blocks, int splits, int patch_rows, int patch_cols) {
-  constexpr int ACROSS = WIDE_TILE / (32 * CT), DOWN = WAVES / ACROSS;     // the waves side by side, and above each other
-  constexpr int ROWS = 32 * RT * DOWN;                     // rows of C a block
-  constexpr int A_BYTES = ROWS * WIDE_ROW_BYTES, SLOT = A_BYTES + WIDE_TILE * WIDE_ROW_BYTES;
-  constexpr int A_LOADS = ROWS / 16 / WAVES, W_LOADS = WIDE_TILE / 16 / WAVES;
+  constexpr int WAVES = DOWN * ACROSS;
+  constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;            // rows and columns of C a block
+  constexpr int A_BYTES = ROWS * WIDE_ROW_BYTES, SLOT = A_BYTES + TILE * WIDE_ROW_BYTES;
+  constexpr int A_LOADS = ROWS / 16 / WAVES, W_LOADS = TILE / 16 / WAVES;
   constexpr int LOADS = A_LOADS + W_LOADS;                 // a wave's loads a stage: those of A, then those of W
-  constexpr int RING = WIDE_RING;
-  extern __shared__ __align__(1024) unsigned char ring[];  // a stage: the block's rows of A, then 256 of W, 64 bytes each
+  constexpr int RING = AHEAD + 3;
+  static_assert(LOADS % 2 == 0 && ROWS % (16 * WAVES) == 0 && TILE % (16 * WAVES) == 0, "whole loads, half of them in each half of a stage");
+  extern __shared__ __align__(1024) unsigned char ring[];  // a stage: the block's rows of A, then those of W, 64 bytes each
   const int lane = threadIdx.x & (QIL_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
   // The piece of work.  XCD x (blocks x, x + 8, ...) takes the pieces x * per .. (x + 1) * per - 1, and the pieces are
@@ -85,7 +87,7 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   const int column_block = (patch_at / patches_down) * patch_cols + within / patch_rows;
   if (split >= splits || row_block >= row_blocks || column_block >= col_blocks) return;
   const int row0 = row_block * ROWS, M = min(M_all - row0, ROWS);
-  const int n0 = column_block * WIDE_TILE;
+  const int n0 = column_block * TILE;
   const size_t k_begin = (size_t)split * stages * WIDE_STAGE;
   // the stage of K at which the block begins (even: a pair of stages stays the two halves of a line): its own for
   // every XCD and every row block of a patch
@@ -146,34 +148,39 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   auto part = [&](int ks, int i, int read_slot, int begin, int doubles, int pair_stage) __attribute__((always_inline)) {
     const int other = ks ^ 1;
     const unsigned char* at = ring + read_slot * SLOT + read_at[other];
-    const int first = doubles * i / RT, loads = 2 * (doubles * (i + 1) / RT - first);      // at most CT
-    const int w_first = CT * i / RT, w_reads = CT * (i + 1) / RT - w_first;                  // at most CT - 1
-    // a product, and before it one of the reads and one of the loads: the order is the one written here
+    const int first = doubles * i / RT, loads = 2 * (doubles * (i + 1) / RT - first);
+    const int w_first = CT * i / RT, w_reads = CT * (i + 1) / RT - w_first;
+    // a product, and before it one of the reads (two where a wave has one tile of columns) and its share of the loads:
+    // the order is the one written here
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
+      constexpr int BEHIND = CT == 1 ? 0 : 1;                // the reads of W begin behind the first product's of A
       if (j == 0) af[other][i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + a_rows + i * 2048));
-      if (j >= 1 && j <= w_reads)
-        wf[other][w_first + j - 1] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + w_rows + (w_first + j - 1) * 2048));
-      if (j < loads) {
-        const int stage = pair_stage + (j & 1);
-        load(begin + first + j / 2, min(stage, last), stage % RING);
+      if (j >= BEHIND && j - BEHIND < w_reads)
+        wf[other][w_first + j - BEHIND] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + w_rows + (w_first + j - BEHIND) * 2048));
+#pragma unroll
+      for (int l = loads <= CT ? j : loads * j / CT; l < (loads <= CT ? min(j + 1, loads) : loads * (j + 1) / CT); ++l) {
+        const int stage = pair_stage + (l & 1);
+        load(begin + first + l / 2, min(stage, last), stage % RING);
       }
       acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  // Stage s lies in place s % RING.  The loads of the stages a + 2 and a + 3 (a even) go out as HALF double loads in the
-  // second half of stage a - 1, behind the barrier that frees the place of stage a - 2, and HALF in the first half of
-  // stage a; the barrier in the middle of a stage waits for the next stage's loads, behind which come one load
-  // (the last of the odd stage of the same pair) or a whole pair's.  Loads past the last stage bring the last one
+  // Stage s lies in place s % RING.  The loads of the stages a + AHEAD and a + AHEAD + 1 (a even) go out as HALF double
+  // loads in the second half of stage a - 1, behind the barrier that frees the place of stage a - 2, and HALF in the first
+  // half of stage a; the barrier in the middle of a stage waits for the next stage's loads, behind which come one load
+  // (the last of the odd stage of the same pair) or none of that pair, and the pairs after it.  Loads past the last stage bring the last one
   // again, into a place nobody reads any more, so that these counts hold at every stage.
   constexpr int HALF = LOADS / 2;
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) load_both(i, 0);
+  for (int pair = 0; pair < AHEAD; pair += 2)
 #pragma unroll
-  for (int i = 0; i < HALF; ++i) load_both(i, 2);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(1 + 2 * HALF) : "memory");
+    for (int i = 0; i < LOADS; ++i) load_both(i, pair);
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) load_both(i, AHEAD);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(1 + LOADS * (AHEAD - 2) + 2 * HALF) : "memory");
 #pragma unroll
   for (int t = 0; t < RT; ++t)
     af[0][t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(ring + read_at[0] + a_rows + t * 2048));
@@ -184,8 +191,8 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
     __builtin_amdgcn_sched_barrier(0);
     // the even stage: its first 16 columns multiply while the fragments of the second are read ...
 #pragma unroll
-    for (int i = 0; i < RT; ++i) part(0, i, even % RING, HALF, HALF, even + 2);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * LOADS) : "memory");
+    for (int i = 0; i < RT; ++i) part(0, i, even % RING, HALF, HALF, even + AHEAD);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS * AHEAD) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     // ... and its second 16 columns while the first fragments of the odd stage are read (behind the last stage: what
     // nobody multiplies)
@@ -194,10 +201,10 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
     // the odd stage (the stages of a block are an even number)
 #pragma unroll
     for (int i = 0; i < RT; ++i) part(0, i, (even + 1) % RING, 0, 0, 0);
-    asm volatile("s_waitcnt vmcnt(1)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(1 + LOADS * (AHEAD - 2)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < RT; ++i) part(1, i, (even + 2) % RING, 0, HALF, even + 4);
+    for (int i = 0; i < RT; ++i) part(1, i, (even + 2) % RING, 0, HALF, even + AHEAD + 2);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the loads past the end, into LDS
 
@@ -253,47 +260,67 @@ static bool wide_takes(int M, int N, int K, int splits) {
   return pairs % splits == 0 && pairs / splits >= 2;
 }
 
-// Tiles of 32 rows of a wave (4 or 2: blocks of 256 or 128 rows): the one with the shorter time by this count, rounds
-// of the 256 CUs times a block's work (a block of 128 rows loads three quarters of what one of 256 does for half
-// the products).
-static int wide_row_tiles(int M, int N, int splits) {
-  double best = 0;
-  int tiles = 4;
-  for (int rt = 4; rt >= 2; rt -= 2) {
-    const long blocks = (long)((M + 64 * rt - 1) / (64 * rt)) * ((N + WIDE_TILE - 1) / WIDE_TILE) * splits;
-    const double cost = (double)((blocks + QIL_CUS - 1) / QIL_CUS) * rt * (rt == 2 ? 1.15 : 1.0);
-    if (rt == 4 || cost < best) { best = cost; tiles = rt; }
-  }
-  return tiles;
+// The shapes of a block: 256 x 256 of C, 128 x 128 with two blocks a CU, and 128 x 128 with the whole LDS as its ring
+// (one block a CU: what a CU has in flight is then the same as with two, for products that have no second block for it).
+enum { WIDE_256 = 0, WIDE_128 = 1, WIDE_128_DEEP = 2 };
+
+// A product's time by this count, us: a start and an end, rounds of blocks on the 256 CUs times a stage's time, which grows
+// with how many CUs work at once (memory, L2 and the clock are shared), and the partial sums out and in again at 5 TB/s.
+// Fitted to products of 300 to 2,048 rows at 0.6B, 8B and 2,048 x 6,144 sizes with cold weights, which it meets to 15 %.
+static double wide_us(int M, int N, int K, int splits, int shape) {
+  const int edge = shape == WIDE_256 ? 256 : 128, slots = QIL_CUS * (shape == WIDE_128 ? 2 : 1);
+  const long blocks = (long)((M + edge - 1) / edge) * ((N + edge - 1) / edge) * splits;
+  const long rounds = (blocks + slots - 1) / slots;
+  const double fill = (double)blocks / (rounds * slots);
+  const double stage = shape == WIDE_256 ? 0.45 + 0.45 * fill : shape == WIDE_128 ? 0.30 + 0.23 * fill : 0.26;
+  const double sums = splits > 1 ? 2.0 * splits * 4.0 * M * N / 5e6 : 0.0;
+  return (shape == WIDE_256 ? 6.0 : 4.5) + rounds * ((double)K / WIDE_STAGE / splits) * stage + sums;
 }
 
-template <typename OUT, int RT, int CT, int WAVES, bool GATED>
+template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
 static int wide_launch(const void* A, const void* W, void* C, int M, int N, int K, int splits, hipStream_t s) {
-  constexpr int ROWS = 32 * RT * (WAVES * 32 * CT / WIDE_TILE);
-  const size_t lds = (size_t)WIDE_RING * (ROWS + WIDE_TILE) * WIDE_ROW_BYTES;
-  auto kernel = gemm_bf16_wide_kernel<OUT, RT, CT, WAVES, GATED>;
+  constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;
+  const size_t lds = (size_t)(AHEAD + 3) * (ROWS + TILE) * WIDE_ROW_BYTES;
+  auto kernel = gemm_bf16_wide_kernel<OUT, RT, CT, DOWN, ACROSS, AHEAD, GATED>;
   static bool granted = false;                             // per instantiation
   if (!granted) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
     granted = true;
   }
-  const int col_blocks = (N + WIDE_TILE - 1) / WIDE_TILE, row_blocks = (M + ROWS - 1) / ROWS;
+  const int col_blocks = (N + TILE - 1) / TILE, row_blocks = (M + ROWS - 1) / ROWS;
   const int patch_rows = std::min(row_blocks, 8), patch_cols = std::min(col_blocks, std::max(1, QIL_CUS / WIDE_XCDS / patch_rows));
   const int patches = ((row_blocks + patch_rows - 1) / patch_rows) * ((col_blocks + patch_cols - 1) / patch_cols) * splits;
   const int blocks = (patches * patch_rows * patch_cols + WIDE_XCDS - 1) / WIDE_XCDS * WIDE_XCDS;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(WAVES * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N,
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(DOWN * ACROSS * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N,
                      K, K / WIDE_STAGE / splits, col_blocks, row_blocks, splits, patch_rows, patch_cols);
   QIL_RETURN_LAUNCH_STATUS();
 }
 
 template <bool GATED>
-static int wide_dispatch(const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s) {
-  if (wide_row_tiles(M, N, splits) == 4)
-    return out_dtype == QIL_F32 ? wide_launch<float, 4, 2, 8, GATED>(A, W, C, M, N, K, splits, s)
-                                : wide_launch<bf16_t, 4, 2, 8, GATED>(A, W, C, M, N, K, splits, s);
-  return out_dtype == QIL_F32 ? wide_launch<float, 2, 4, 4, GATED>(A, W, C, M, N, K, splits, s)
-                              : wide_launch<bf16_t, 2, 4, 4, GATED>(A, W, C, M, N, K, splits, s);
+static int wide_dispatch(int shape, const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s) {
+#define QIL_WIDE_CASE(SHAPE, RT, CT, DOWN, ACROSS, AHEAD)                                                             \
+  case SHAPE:                                                                                                         \
+    return out_dtype == QIL_F32 ? wide_launch<float, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, s) \
+                                : wide_launch<bf16_t, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, s)
+  switch (shape) {
+    QIL_WIDE_CASE(WIDE_256, 4, 2, 2, 4, 2);
+    QIL_WIDE_CASE(WIDE_128, 2, 2, 2, 2, 2);
+    QIL_WIDE_CASE(WIDE_128_DEEP, 2, 2, 2, 2, 6);
+  }
+#undef QIL_WIDE_CASE
+  return -1;
+}
+
+// The best shape at this number of splits.
+static int wide_shape(int M, int N, int K, int splits) {
+  double best = 1e30;
+  int shape = WIDE_256;
+  for (int one = WIDE_256; one <= WIDE_128_DEEP; ++one) {
+    const double us = wide_us(M, N, K, splits, one);
+    if (us < best) { best = us; shape = one; }
+  }
+  return shape;
 }
 
 extern "C" {
@@ -301,17 +328,45 @@ extern "C" {
 // 1 if qil_gemm_bf16_wide takes these sizes.
 int qil_gemm_bf16_wide_takes(int M, int N, int K, int splits) { return wide_takes(M, N, K, splits); }
 
+// Splits of K with which a product of more than 256 rows should run here rather than in the GPU BLAS (1: a result of
+// A's type; more, where `may_split` allows float32 partial sums and there are no more columns than K); 0: the BLAS.
+// What takes no more than WIDE_HOST_US by the count above stays here.  The GPU's times are level with the library's there (us
+// here against there at 643 rows, 0.6B sizes: q/k/v 12.4 / 11.9, attention output 10.3 / 10.7, down 12.1 / 13.9; 2,048 rows of
+// 2,048 x 2,048 21.0 / 21.6), but the host spends 21 us on a library product and 7 on one of ours, and steps of such
+// products wait for the host: prompts at 0.6B sizes, with the gated rule below, 530 rows 4.62 -> 2.69 ms, 1,000 rows
+// 4.59 -> 3.26, 1,400 rows 4.93 -> 4.23; 2,048 rows level.  Longer products are the library's inside a model even where this
+// kernel is ahead alone (4,096 x 12,288 in 4 splits, 643 rows: 78 us against 92 with cold operands, but 21 us a layer
+// behind in a prompt of 530 rows, whose norms then read the partial sums).
+int qil_gemm_bf16_wide_splits(int M, int N, int K, int may_split) {
+  int found = 0;
+  double best = WIDE_HOST_US;
+  for (int splits = 1; splits <= (may_split && K >= N ? 8 : 1); ++splits) {
+    if (!wide_takes(M, N, K, splits)) continue;
+    const double us = wide_us(M, N, K, splits, wide_shape(M, N, K, splits));
+    if (us <= best) { best = us; found = splits; }
+  }
+  return found;
+}
+
 // C = A[M, K] W[N, K]^T.  splits > 1: C float32 [splits][M][N] partial sums (out_dtype QIL_F32); splits == 1: C [M][N]
 // of out_dtype.
 int qil_gemm_bf16_wide(const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s) {
   if (M == 0 || N == 0) return 0;
   if (!wide_takes(M, N, K, splits) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) return -1;
   if ((splits > 1 && out_dtype != QIL_F32) || (out_dtype != QIL_F32 && out_dtype != QIL_BF16)) return -1;
-  return wide_dispatch<false>(A, W, C, M, N, K, out_dtype, splits, s);
+  return wide_dispatch<false>(wide_shape(M, N, K, splits), A, W, C, M, N, K, out_dtype, splits, s);
 }
 
 // 1 if qil_gemm_bf16_wide_gated takes these sizes: those of the product with 2 * inner columns in one split.
 int qil_gemm_bf16_wide_gated_takes(int M, int inner, int K) { return inner >= 16 && inner % 16 == 0 && wide_takes(M, 2 * inner, K, 1); }
+
+// 1 if a gated product of more than 256 rows should run here: by the same rule, and two kernels become one (643 rows of
+// 6,144 x 1,024 18.5 us against 18.9 and 4.4 for the activation; 2,048 rows 30.7 against 27.4 and 9.6, but a prompt of
+// 2,048 rows 4.89 ms against 4.78, of 5,000 13.1 against 12.8).
+int qil_gemm_bf16_wide_gated_wanted(int M, int inner, int K) {
+  return M > 256 && qil_gemm_bf16_wide_gated_takes(M, inner, K) &&
+         wide_us(M, 2 * inner, K, 1, wide_shape(M, 2 * inner, K, 1)) <= WIDE_HOST_US;
+}
 
 // out [M, inner] of out_dtype = silu(A gate^T) * (A up^T) for W [2 inner, K] with gate and up rows in turns of 16.
 int qil_gemm_bf16_wide_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, hipStream_t s) {
@@ -319,7 +374,7 @@ int qil_gemm_bf16_wide_gated(const void* A, const void* W, void* out, int M, int
   if (!qil_gemm_bf16_wide_gated_takes(M, inner, K) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16 ||
       (out_dtype != QIL_F32 && out_dtype != QIL_BF16))
     return -1;
-  return wide_dispatch<true>(A, W, out, M, 2 * inner, K, out_dtype, 1, s);
+  return wide_dispatch<true>(wide_shape(M, 2 * inner, K, 1), A, W, out, M, 2 * inner, K, out_dtype, 1, s);
 }
 
 }  // extern "C"

@@ -680,7 +680,17 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
         _check(lib.qil_gemm_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), n, o, k, _code(out_dtype), 1, 0, 0,
                                  _stream()), 'gemm_bf16')
         return out
-    if OWN_LARGE_PRODUCTS and out_dtype == x.dtype and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_takes(n, o, k, 1):
+    # beyond 256 rows: the products that the library is no faster at (the kernel's file says which)
+    splits = lib.qil_gemm_bf16_wide_splits(n, o, k, int(partials and bias is None)) \
+        if n > MID_GEMM_MOST_ROWS and out_dtype == x.dtype and not OWN_LARGE_PRODUCTS else 0
+    if splits:
+        out = torch.empty((splits, n, o), dtype=torch.float32 if splits > 1 else x.dtype, device=x.device)
+        _check(lib.qil_gemm_bf16_wide(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _code(out.dtype), splits, _stream()),
+               'gemm_bf16_wide')
+        if splits > 1:
+            return Partials(out)
+        out = out[0]
+    elif OWN_LARGE_PRODUCTS and out_dtype == x.dtype and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_takes(n, o, k, 1):
         out = torch.empty((n, o), dtype=x.dtype, device=x.device)
         _check(lib.qil_gemm_bf16_wide(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _code(out.dtype), 1, _stream()),
                'gemm_bf16_wide')
@@ -746,8 +756,9 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
         _check(lib.qil_gemm_bf16_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), 0, 0,
                                        int(interleaved), _stream()), 'gemm_bf16_gated')
         return out
-    if OWN_LARGE_PRODUCTS and x.dtype == torch.bfloat16 and interleaved and n >= WIDE_GEMM_FEWEST_ROWS and \
-            lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k):
+    if x.dtype == torch.bfloat16 and interleaved and \
+            ((OWN_LARGE_PRODUCTS and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k)) or
+             lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k)):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
         _check(lib.qil_gemm_bf16_wide_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
                'gemm_bf16_wide_gated')
