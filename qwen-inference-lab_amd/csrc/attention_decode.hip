@@ -23,6 +23,8 @@
 // slopes: slopes[h] * (position - key) is taken off head h's scaled score.
 //
 // Takes page_size % 8 == 0, d % 16 == 0, d <= 256, g <= 16; other sizes go to the row kernel.
+#include <algorithm>
+
 #include "common.h"
 #include "key_span.h"
 #include "qk_math.h"
@@ -30,6 +32,7 @@
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+#define PLAN_MOST_ROWS 128                                 // rows a plan may share the blocks out to
 #define DEC_MAX_WAVES 8                                    // waves of a block; each takes every waves-th 32-key step
 
 // FUSED: the queries do not come from memory but from the partial sums of the q/k/v product, with the
@@ -72,7 +75,7 @@ __device__ __forceinline__ uint4 shuffle4(uint4 v, int source) {
 }
 
 // WHOLE: d == DMAX (always so when FUSED).
-template <int DMAX, bool PAIRS, bool FUSED, bool WHOLE = FUSED>
+template <int DMAX, bool FUSED, bool WHOLE = FUSED>
 __global__ void __launch_bounds__(DEC_MAX_WAVES * QIL_WAVE)
 attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_cache,
                    const bf16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int table_stride,
@@ -80,12 +83,23 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
                    const int* __restrict__ row_index, float* __restrict__ part_acc, float* __restrict__ part_m,
                    float* __restrict__ part_l, bf16_t* __restrict__ out, int heads, int kv_heads, int d,
                    int page_size, int window, float scale, int P, int parts, float softcap,
-                   const float* __restrict__ sinks, const float* __restrict__ slopes, int keep) {
+                   const float* __restrict__ sinks, const float* __restrict__ slopes, int keep,
+                   const int* __restrict__ plan, int* __restrict__ part_keys) {
   constexpr int QFRAGS = DMAX / 32, DTILES = DMAX / 16;
+  constexpr int TG = DMAX / 8, HPP = QIL_WAVE / TG;          // lanes of a head (8 elements each), heads a wave
   if (WHOLE) d = DMAX;                                      // what the host has checked, known to the compiler: no
                                                             // condition on the head size stays in the loops
   extern __shared__ float lds[];
-  const int slot_row = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
+  int slot_row = blockIdx.x, part = blockIdx.z;
+  const int kvh = blockIdx.y;
+  if (plan) {                                               // the rows' parts one behind another (attn_plan_kernel)
+    const int job = plan[1 + blockIdx.x];
+    P = plan[0];
+    if (blockIdx.x == 0 && kvh == 0 && threadIdx.x == 0) *part_keys = P;       // for whoever merges the parts
+    if (job < 0) return;
+    slot_row = job >> 16;
+    part = job & 0xffff;
+  }
   const int row = row_index ? row_index[slot_row] : slot_row;
   const int g = heads / kv_heads;
   const int pos = positions[row], ctx = pos + 1;
@@ -106,7 +120,10 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
   // Q fragments: B operand, column r = head kvh * g + r (filled below, after the first loads are on their way)
   bf16x8 qb[QFRAGS];
   uint4 new_k = make_uint4(0, 0, 0, 0), new_v = make_uint4(0, 0, 0, 0);   // FUSED: chunk lane % (DMAX / 8) of the new key / value
-  bool owner = false;                                      // FUSED: this wave meets the row's own position
+  // FUSED: the block whose keys end with the row's own position makes the new key and value, its last wave does that;
+  // `owner` is the wave that meets the position among its steps
+  const bool new_here = FUSED && fused.writes && pos_place >= begin && pos_place < end;
+  const bool owner = new_here && wave == ((pos_place >> 5) - first_step) % waves;
 
   float m = -INFINITY, l = 0.f;
   f32x4 o[DTILES];
@@ -119,7 +136,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
     uint4 k[2][QFRAGS];
     uint4 v[DTILES];                                        // V^T[dim 16 t + r][keys 8 kb .. 8 kb + 7]: 16 bytes of one page row
   };
-  auto look_up = [&](int step, int (&page)[3]) {
+  auto look_up = [&](int step, int (&page)[3]) __attribute__((always_inline)) {
     const int k0 = span.key(step * 32);
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
@@ -128,7 +145,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
       page[jt] = table[min(k0 + 8 * (r >> 2) + 4 * jt + (r & 3), ctx - 1) / page_size];   // clamped: an invisible key's score is replaced
     page[2] = table[(min(k0 + 8 * kb, ctx - 1) & ~7) / page_size];
   };
-  auto request = [&](int step, const int (&page)[3], StepData& data) {
+  auto request = [&](int step, const int (&page)[3], StepData& data) __attribute__((always_inline)) {
     const int k0 = span.key(step * 32);
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt) {
@@ -146,7 +163,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
     for (int t = 0; t < DTILES; ++t)
       data.v[t] = t < dt ? once4(vbase + (size_t)(t * 16 + r) * page_size) : make_uint4(0, 0, 0, 0);
   };
-  auto attend = [&](int step, StepData& data) {
+  auto attend = [&](int step, StepData& data) __attribute__((always_inline)) {
     const int k0 = span.key(step * 32);
     if constexpr (FUSED) {
       if (owner && step == (pos_place >> 5)) {                   // the new key and value come from this wave's registers
@@ -239,53 +256,108 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
       }
     }
   };
-  auto make_queries = [&]() {
-    if constexpr (FUSED) {
-      constexpr int TG = DMAX / 8, HPP = QIL_WAVE / TG;      // lanes of a head (8 elements each), heads a pass
-      const int chunk = lane % TG, sub = lane / TG;
-      // the block's waves share the heads (HPP of them a wave and pass); the queries meet in LDS
-      uint4* shared_q = reinterpret_cast<uint4*>(lds);       // [g][TG] chunks; the end of the kernel uses the LDS again
-      for (int base = wave * HPP; base < g; base += waves * HPP) {
-        float x[8];
-        const int head = kvh * g + min(base + sub, g - 1);   // lanes past the group repeat its last head
-        load8_sum_wide(fused.qkv, (size_t)row * fused.row_elems + (size_t)head * DMAX + chunk * 8, fused.splits, fused.split_stride, x);
-        add_bias8(x, fused.bias, head * DMAX + chunk * 8);
-        norm_rope8<bf16_t>(x, chunk, TG, fused.q_weight, DMAX, fused.eps, fused.cos_table, fused.sin_table, pos, fused.rot,
-                           fused.rotate_first != 0);
-        if (fused.temp_every > 0) {
-          const float temperature = query_temperature(pos, fused.temp_coef, fused.temp_every);
+  // FUSED: a wave makes HPP of the group's queries, or (the last wave, in its first lane groups) the new key and value.
+  // Everything that takes is asked for ahead of the wave's keys and values, behind which it would wait otherwise: a
+  // wave's loads come back in order.  (With the pages looked up a step ahead: one row of 100 keys at 0.6B sizes 1,102 ->
+  // 1,068 us a step of 28 layers, eight of 2,000 1,501 -> 1,467; two steps' keys and values in flight a wave do not fit
+  // the registers, and blocks of four waves, three a CU, took 30 us where these take 19.)
+  const int chunk = lane % TG, sub = lane / TG;
+  const bool makes_q = FUSED && wave * HPP < g;            // wave-uniform, as the others
+  const bool makes_new = new_here && wave == waves - 1;
+  constexpr int AHEAD = 4;                                 // splits of the product whose sums are asked for at once
+  float4 sum_lo[AHEAD], sum_hi[AHEAD];
+  HeadFactors factors;
+  auto column = [&](bool query, int head) __attribute__((always_inline)) { return query ? (kvh * g + min(head, g - 1)) * DMAX + chunk * 8    // past the group: its last head
+                                                         : ((sub & 1 ? fused.v_head : heads) + kvh) * DMAX + chunk * 8; };
+  auto ask = [&](bool query, int head) __attribute__((always_inline)) {
+    const float* from = fused.qkv + (size_t)row * fused.row_elems + column(query, head);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] *= temperature;
+    for (int u = 0; u < AHEAD; ++u) {
+      const float* p = from + (size_t)min(u, fused.splits - 1) * fused.split_stride;
+      sum_lo[u] = *reinterpret_cast<const float4*>(p);
+      sum_hi[u] = *reinterpret_cast<const float4*>(p + 4);
+    }
+    const float* weight = query ? fused.q_weight : fused.k_weight;
+    if (weight) load_eight(weight + chunk * 8, factors.w);
+    if (fused.cos_table && fused.rot > 0) load_turns(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
+  };
+  auto answer = [&](bool query, int head, float (&x)[8], float (&plain)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = 0.f;
+    for (int s0 = 0; s0 < fused.splits; s0 += AHEAD) {
+      if (s0) {
+        const float* from = fused.qkv + (size_t)row * fused.row_elems + column(query, head);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+          const float* p = from + (size_t)min(s0 + u, fused.splits - 1) * fused.split_stride;
+          sum_lo[u] = *reinterpret_cast<const float4*>(p);
+          sum_hi[u] = *reinterpret_cast<const float4*>(p + 4);
         }
-        if (base + sub < g) shared_q[(base + sub) * TG + chunk] = pack8(x);
       }
-      owner = fused.writes && pos_place >= begin && pos_place < end && wave == ((pos_place >> 5) - first_step) % waves;
-      if (owner) {                                           // wave-uniform
-        float x[8];
-        load8_sum_wide(fused.qkv, (size_t)row * fused.row_elems + (size_t)(heads + kvh) * DMAX + chunk * 8, fused.splits, fused.split_stride, x);
-        add_bias8(x, fused.bias, (heads + kvh) * DMAX + chunk * 8);
-        norm_rope8<bf16_t>(x, chunk, TG, fused.k_weight, DMAX, fused.eps, fused.cos_table, fused.sin_table, pos, fused.rot,
-                           fused.rotate_first != 0);
-        new_k = pack8(x);
-        load8_sum_wide(fused.qkv, (size_t)row * fused.row_elems + (size_t)(fused.v_head + kvh) * DMAX + chunk * 8, fused.splits,
-                       fused.split_stride, x);
-        add_bias8(x, fused.bias, (fused.v_head + kvh) * DMAX + chunk * 8);
-        new_v = pack8(x);
-        if (sub == 0) {                                      // into the pages (qil/cache.py:79-82)
-          const size_t page = table[pos / page_size];
-          const int offset = pos % page_size;
-          bf16_t* k_row = const_cast<bf16_t*>(k_cache) + ((page * kv_heads + kvh) * page_size + offset) * (size_t)DMAX;
-          *reinterpret_cast<uint4*>(k_row + chunk * 8) = new_k;
-          bf16_t* column = const_cast<bf16_t*>(v_cache) + ((page * kv_heads + kvh) * (size_t)DMAX + chunk * 8) * page_size + offset;
-          const uint32_t words[4] = {new_v.x, new_v.y, new_v.z, new_v.w};
 #pragma unroll
-          for (int e = 0; e < 8; ++e) column[(size_t)e * page_size] = (bf16_t)(words[e >> 1] >> ((e & 1) * 16));
+      for (int u = 0; u < AHEAD; ++u)
+        if (s0 + u < fused.splits) {
+          x[0] += sum_lo[u].x; x[1] += sum_lo[u].y; x[2] += sum_lo[u].z; x[3] += sum_lo[u].w;
+          x[4] += sum_hi[u].x; x[5] += sum_hi[u].y; x[6] += sum_hi[u].z; x[7] += sum_hi[u].w;
+        }
+    }
+    add_bias8(x, fused.bias, column(query, head));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) plain[e] = x[e];
+    norm_rope8<bf16_t>(x, chunk, TG, factors, fused.q_weight != nullptr, DMAX, fused.eps, fused.cos_table && fused.rot > 0,
+                       fused.rot, fused.rotate_first != 0);
+  };
+  auto make_queries = [&]() __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      uint4* shared_q = reinterpret_cast<uint4*>(lds);       // [g][TG] chunks; the end of the kernel uses the LDS again
+      uint4* shared_new = shared_q + g * TG;                 // the new key, then the new value
+      if (makes_q || makes_new) {
+        bool query = makes_q;
+        for (int base = wave * HPP;;) {                      // once, unless the group is large for the block's waves
+          float x[8], plain[8];
+          answer(query, base + sub, x, plain);
+          if (query) {
+            if (fused.temp_every > 0) {
+              const float temperature = query_temperature(pos, fused.temp_coef, fused.temp_every);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) x[e] *= temperature;
+            }
+            if (base + sub < g) shared_q[(base + sub) * TG + chunk] = pack8(x);
+          } else {
+            const bool value = sub & 1;
+            const uint4 made = value ? pack8(plain) : pack8(x);
+            if (sub < 2) {                                   // into the pages (qil/cache.py:79-82), and for this row's own step
+              shared_new[sub * TG + chunk] = made;
+              const size_t page = table[pos / page_size];
+              const int offset = pos % page_size;
+              if (!value) {
+                bf16_t* k_row = const_cast<bf16_t*>(k_cache) + ((page * kv_heads + kvh) * page_size + offset) * (size_t)DMAX;
+                *reinterpret_cast<uint4*>(k_row + chunk * 8) = made;
+              } else {
+                bf16_t* column = const_cast<bf16_t*>(v_cache) + ((page * kv_heads + kvh) * (size_t)DMAX + chunk * 8) * page_size + offset;
+                const uint32_t words[4] = {made.x, made.y, made.z, made.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) column[(size_t)e * page_size] = (bf16_t)(words[e >> 1] >> ((e & 1) * 16));
+              }
+            }
+          }
+          if (!query) break;
+          base += waves * HPP;
+          if (base >= g) {
+            if (!makes_new) break;
+            query = false;
+          }
+          ask(query, base + sub);
         }
       }
       __syncthreads();
 #pragma unroll
       for (int ks = 0; ks < QFRAGS; ++ks)                    // fragment ks of head r = chunk 4 ks + kb of that head
         qb[ks] = __builtin_bit_cast(bf16x8, r < g ? shared_q[r * TG + 4 * ks + kb] : make_uint4(0, 0, 0, 0));
+      if (owner) {
+        new_k = shared_new[chunk];
+        new_v = shared_new[TG + chunk];
+      }
       __syncthreads();                                       // the LDS is free again
     } else {
 #pragma unroll
@@ -297,47 +369,30 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
       }
     }
   };
-  // The loads of a wave's first step (or pair of steps) go out before its queries are made, so that the
-  // two waits overlap; later steps are loaded when the step before is done.
-  if (PAIRS) {
-    // Two of the wave's steps at a time: both steps' table entries, then both steps' K and V, then the
-    // arithmetic; a wave waits for memory twice per pair instead of twice per step.  (Twice the
-    // registers: for launches that leave a CU's register file to one block.)
-    int step = first_step + wave;
-    int page_a[3], page_b[3];
-    StepData a, b;
-    auto load_pair = [&]() {
-      look_up(step, page_a);
-      if (step + waves <= last_step) look_up(step + waves, page_b);
-      request(step, page_a, a);
-      if (step + waves <= last_step) request(step + waves, page_b, b);
-    };
-    if (step <= last_step) load_pair();
-    make_queries();
-    while (step <= last_step) {
-      attend(step, a);
-      if (step + waves <= last_step) attend(step + waves, b);
-      step += 2 * waves;
-      if (step <= last_step) load_pair();
-    }
-  } else {
-    int step = first_step + wave;
-    int page[3];
-    StepData data;
-    if (step <= last_step) {
-      look_up(step, page);
-      request(step, page, data);
-    }
-    make_queries();
-    while (step <= last_step) {
-      attend(step, data);
-      step += waves;
-      if (step <= last_step) {
-        look_up(step, page);
-        request(step, page, data);
-      }
-    }
+  if constexpr (FUSED) {
+    if (makes_q || makes_new) ask(makes_q, wave * HPP + sub);
   }
+  // The loads of a wave's first step go out before its queries are made, so that the two waits overlap, and the table's
+  // entries are looked up a step ahead of the loads that need them.
+  constexpr bool EARLY = FUSED;
+  int step = first_step + wave;
+  int page[3];
+  StepData here;
+  if (step <= last_step) {
+    look_up(step, page);
+    request(step, page, here);
+    if (EARLY) look_up(step + waves, page);                  // (clamped: any entry will do where there is no such step)
+  }
+  make_queries();
+  if (step <= last_step)
+    for (;;) {
+      attend(step, here);
+      step += waves;
+      if (step > last_step) break;
+      if (!EARLY) look_up(step, page);
+      request(step, page, here);
+      if (EARLY) look_up(step + waves, page);
+    }
 
   // ---- the waves' (m, l, O) meet in LDS: [wave][head < g][d + 2]
   l += __shfl_xor(l, 16, QIL_WAVE);
@@ -376,6 +431,64 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
   }
 }
 
+// How the keys of rows of different lengths are shared out: parts of one size for all rows, the smallest multiple of 32 keys
+// (at least `fewest`) that leaves no more than `blocks` parts in all.  plan[0]: the keys of a part; plan[1 + j]: the j-th
+// part, row << 16 | part, the rows one behind another, or -1.  One wave, a row a lane and turn; once a step, for all layers.
+__global__ void __launch_bounds__(QIL_WAVE)
+attn_plan_kernel(const int* __restrict__ positions, const int* __restrict__ row_index, int rows, int blocks, int fewest,
+                 int* __restrict__ plan) {
+  const int lane = threadIdx.x;
+  constexpr int MOST = PLAN_MOST_ROWS / QIL_WAVE;
+  int steps[MOST], total = 0;                              // steps of 32 keys
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int r = i * QIL_WAVE + lane;
+    steps[i] = r < rows ? (positions[row_index ? row_index[r] : r] + 32) / 32 : 0;
+    total += steps[i];
+  }
+  auto sum = [](int v) {
+    for (int o = QIL_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, QIL_WAVE);
+    return v;
+  };
+  total = sum(total);
+  // parts(L) = sum over the rows of ceil(steps / L) falls with L; at the longest row's length it is the number of rows
+  int low = max(fewest / 32, (total + blocks - 1) / blocks), high = max(low, total);
+  while (low < high) {
+    const int middle = (low + high) / 2;
+    int parts = 0;
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) parts += (steps[i] + middle - 1) / middle;
+    if (sum(parts) <= blocks) high = middle;
+    else low = middle + 1;
+  }
+  if (lane == 0) plan[0] = low * 32;
+  int at = 0;
+  for (int i = 0; i < MOST; ++i) {
+    const int parts = (steps[i] + low - 1) / low;
+    int before = parts;                                    // the parts of the rows up to this lane's
+    for (int o = 1; o < QIL_WAVE; o *= 2) {
+      const int other = __shfl_up(before, o, QIL_WAVE);
+      if (lane >= o) before += other;
+    }
+    for (int p = 0; p < parts; ++p) plan[1 + at + before - parts + p] = ((i * QIL_WAVE + lane) << 16) | p;
+    at += __shfl(before, QIL_WAVE - 1, QIL_WAVE);
+  }
+  for (int j = at + lane; j < blocks; j += QIL_WAVE) plan[1 + j] = -1;
+}
+
+// plan: int32 [1 + blocks].  rows <= blocks (a part a row fits) and at most PLAN_MOST_ROWS.
+extern "C" int qil_attn_plan(const int* positions, const int* row_index, int rows, int blocks, int fewest, int* plan, hipStream_t s) {
+  if (rows < 1 || rows > blocks || rows > PLAN_MOST_ROWS || blocks > 32768 || fewest < 32 || fewest % 32) return -1;
+  hipLaunchKernelGGL(attn_plan_kernel, dim3(1), dim3(QIL_WAVE), 0, s, positions, row_index, rows, blocks, fewest, plan);
+  QIL_RETURN_LAUNCH_STATUS();
+}
+
+// A plan counts whole contexts and needs a workspace; the workspace's rows then hold `parts` parts each, as many as the
+// longest row can have.
+static bool plan_fits(const int* plan, int blocks, int rows, int parts, int window, const void* workspace) {
+  return !plan || (blocks >= rows && rows <= PLAN_MOST_ROWS && parts > 1 && window == 0 && workspace);
+}
+
 // 1 if the matrix-core decode kernel takes these sizes.
 extern "C" int qil_attn_decode_takes(int heads, int kv_heads, int d, int page_size) {
   if (heads % kv_heads || d % 16 || d < 16 || d > 256 || page_size % 8) return 0;
@@ -385,47 +498,41 @@ extern "C" int qil_attn_decode_takes(int heads, int kv_heads, int d, int page_si
 
 // Partial results in the layout of the row kernel (acc [rows, heads, parts, d], then m, then l);
 // the caller runs the row kernel's merge when parts > 1.  P must be a multiple of 32; a block has
-// `waves` waves (at most 8), best one or two 32-key steps of P for each.  pairs != 0: a wave loads two of
-// its steps at a time (twice the registers; for launches of at most one block a CU).  sinks: null, or float32 [heads]:
+// `waves` waves (at most 8), best one or two 32-key steps of P for each.  sinks: null, or float32 [heads]:
 // exp(sink) joins a head's divisor (here when parts == 1, else in the merge).  slopes: null, or float32 [heads]; keep > 0
-// (with a window): the kept first keys, and P and parts count places.
+// (with a window): the kept first keys, and P and parts count places.  plan: null, or what qil_attn_plan made for these
+// rows and `blocks` (no window): blocks take its parts, P is not used, and the keys of a part are left as an int32 behind
+// the partial results (four floats more of workspace) for whoever merges them.
 extern "C" int qil_attn_decode(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                                const int* block_tables, int table_stride, const int* row_seq, const int* positions,
                                const int* row_index, void* workspace, void* out, int rows, int heads, int kv_heads,
-                               int d, int page_size, int window, float scale, int P, int parts, int waves,
-                               int pairs, float softcap, const float* sinks, const float* slopes, int keep,
-                               hipStream_t s) {
+                               int d, int page_size, int window, float scale, int P, int parts, int waves, float softcap, const float* sinks, const float* slopes, int keep,
+                               const int* plan, int blocks, hipStream_t s) {
   if (rows == 0) return 0;
-  if (!qil_attn_decode_takes(heads, kv_heads, d, page_size) || P % 32 || P < 32 || parts < 1 || parts > 65535 ||
-      kv_heads > 65535 || waves < 1 || waves > DEC_MAX_WAVES || keep < 0 || (keep > 0 && window <= 0))
+  if (!qil_attn_decode_takes(heads, kv_heads, d, page_size) || (!plan && (P % 32 || P < 32)) || parts < 1 || parts > 65535 ||
+      kv_heads > 65535 || waves < 1 || waves > DEC_MAX_WAVES || keep < 0 || (keep > 0 && window <= 0) ||
+      !plan_fits(plan, blocks, rows, parts, window, workspace))
     return -1;
   const int g = heads / kv_heads;
   float* acc = (float*)workspace;
   float* m = acc ? acc + (size_t)rows * heads * parts * d : nullptr;
   float* l = m ? m + (size_t)rows * heads * parts : nullptr;
   const size_t lds = (size_t)waves * g * (d + 2) * sizeof(float);
-  dim3 grid(rows, kv_heads, parts);
+  const dim3 grid = plan ? dim3(blocks, kv_heads) : dim3(rows, kv_heads, parts);
+  int* part_keys = plan ? reinterpret_cast<int*>(l + (size_t)rows * heads * parts) : nullptr;
   const FusedQKV none = {};
-#define QIL_DEC_LAUNCH(DMAX, PAIRS, FUSED, FIELDS)                                                                  \
-  hipLaunchKernelGGL((attn_decode_kernel<DMAX, PAIRS, FUSED>), grid, dim3(waves * QIL_WAVE), lds, s, FIELDS,         \
+#define QIL_DEC_LAUNCH(DMAX, FUSED, WHOLE, FIELDS)                                                                 \
+  hipLaunchKernelGGL((attn_decode_kernel<DMAX, FUSED, WHOLE>), grid, dim3(waves * QIL_WAVE), lds, s, FIELDS,        \
                      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,       \
                      table_stride, row_seq, positions, row_index, acc, m, l, (bf16_t*)out, heads, kv_heads, d,        \
-                     page_size, window, scale, P, parts, softcap, sinks, slopes, keep)
-#define QIL_DEC_WHOLE(DMAX, PAIRS)                                                                                  \
-  hipLaunchKernelGGL((attn_decode_kernel<DMAX, PAIRS, false, true>), grid, dim3(waves * QIL_WAVE), lds, s, none,     \
-                     (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,       \
-                     table_stride, row_seq, positions, row_index, acc, m, l, (bf16_t*)out, heads, kv_heads, d,        \
-                     page_size, window, scale, P, parts, softcap, sinks, slopes, keep)
-#define QIL_DEC_CASE(DMAX)                                                                                          \
-  if (d == DMAX && pairs) QIL_DEC_WHOLE(DMAX, true);                                                                \
-  else if (d == DMAX) QIL_DEC_WHOLE(DMAX, false);                                                                   \
-  else if (pairs) QIL_DEC_LAUNCH(DMAX, true, false, none);                                                          \
+                     page_size, window, scale, P, parts, softcap, sinks, slopes, keep, plan, part_keys)
+#define QIL_DEC_CASE(DMAX)                                \
+  if (d == DMAX) QIL_DEC_LAUNCH(DMAX, false, true, none); \
   else QIL_DEC_LAUNCH(DMAX, false, false, none)
   if (d <= 64) QIL_DEC_CASE(64);
   else if (d <= 128) QIL_DEC_CASE(128);
   else QIL_DEC_CASE(256);
 #undef QIL_DEC_CASE
-#undef QIL_DEC_WHOLE
   QIL_RETURN_LAUNCH_STATUS();
 }
 
@@ -452,13 +559,14 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
                                      void* k_cache, void* v_cache, const int* block_tables, int table_stride,
                                      const int* row_seq, const int* positions, void* workspace, void* out, int rows,
                                      int heads, int kv_heads, int d, int page_size, int window, float scale, int P,
-                                     int parts, int waves, int pairs, int rotate_first, float softcap,
+                                     int parts, int waves, int rotate_first, float softcap,
                                      int has_kv, int extra_columns, const float* bias, float temp_coef, int temp_every,
-                                     const float* sinks, int shared_kv, const float* slopes, int keep, hipStream_t s) {
+                                     const float* sinks, int shared_kv, const float* slopes, int keep,
+                                     const int* plan, int blocks, hipStream_t s) {
   if (rows == 0) return 0;
-  if (keep < 0 || (keep > 0 && window <= 0) || (shared_kv && !has_kv)) return -1;
+  if (keep < 0 || (keep > 0 && window <= 0) || (shared_kv && !has_kv) || !plan_fits(plan, blocks, rows, parts, window, workspace)) return -1;
   if (extra_columns < 0 || temp_every < 0 || (writes && !has_kv) || ((uintptr_t)bias % 16) || extra_columns % 8) return -1;
-  if (!qil_attn_decode_fused_takes(heads, kv_heads, d, page_size, cos_table ? rot : 0) || P % 32 || P < 32 ||
+  if (!qil_attn_decode_fused_takes(heads, kv_heads, d, page_size, cos_table ? rot : 0) || (!plan && (P % 32 || P < 32)) ||
       parts < 1 || parts > 65535 || kv_heads > 65535 || waves < 1 || waves > DEC_MAX_WAVES || splits < 1 ||
       (q_weight == nullptr) != (k_weight == nullptr) || (sin_table != nullptr && cos_table == nullptr) ||
       (((uintptr_t)qkv | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)cos_table | (uintptr_t)sin_table |
@@ -468,8 +576,9 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   float* acc = (float*)workspace;
   float* m = acc ? acc + (size_t)rows * heads * parts * d : nullptr;
   float* l = m ? m + (size_t)rows * heads * parts : nullptr;
-  const size_t lds = (size_t)waves * g * (d + 2) * sizeof(float);
-  dim3 grid(rows, kv_heads, parts);
+  const size_t lds = std::max((size_t)waves * g * (d + 2) * sizeof(float), (size_t)(g + 2) * d * sizeof(bf16_t));
+  const dim3 grid = plan ? dim3(blocks, kv_heads) : dim3(rows, kv_heads, parts);
+  int* part_keys = plan ? reinterpret_cast<int*>(l + (size_t)rows * heads * parts) : nullptr;
   FusedQKV fused;
   fused.qkv = qkv;
   fused.row_elems = (heads + (has_kv ? (shared_kv ? 1 : 2) * kv_heads : 0)) * d + extra_columns;
@@ -484,12 +593,8 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
-#define QIL_DEC_CASE(DMAX)                                                                                          \
-  if (pairs) QIL_DEC_LAUNCH(DMAX, true, true, fused);                                                               \
-  else QIL_DEC_LAUNCH(DMAX, false, true, fused)
-  if (d == 64) QIL_DEC_CASE(64);
-  else QIL_DEC_CASE(128);
-#undef QIL_DEC_CASE
+  if (d == 64) QIL_DEC_LAUNCH(64, true, true, fused);
+  else QIL_DEC_LAUNCH(128, true, true, fused);
 #undef QIL_DEC_LAUNCH
   QIL_RETURN_LAUNCH_STATUS();
 }

@@ -23,6 +23,7 @@
 // lane; a wave handles 64 / TG tokens at a time.
 #include "common.h"
 #include "key_span.h"
+#include "merge_parts.h"
 #include "operand.h"
 
 #define ATT_THREADS 256
@@ -247,7 +248,8 @@ attn_rows_merge_kernel(const float* __restrict__ part_acc, const float* __restri
                        const float* __restrict__ part_l, const int* __restrict__ positions,
                        const int* __restrict__ row_index, T* __restrict__ out, int heads, int d,
                        int window, int P, int parts, int tg, const float* __restrict__ sinks, int keep, Operand gate,
-                       int gate_row) {
+                       int gate_row, const int* __restrict__ part_keys) {
+  if (part_keys) P = *part_keys;
   const int slot_row = blockIdx.x;
   const int head = blockIdx.y * (QIL_WAVE / tg) + threadIdx.x / tg, e = (threadIdx.x % tg) * 4;
   const bool head_there = head < heads;                    // the same for the tg lanes of a head; all of them take part in the maximum
@@ -350,7 +352,7 @@ static int launch_rows(const void* q, int q_stride, const void* k_cache, const v
   dim3 merge_grid;
   merge_shape(rows, heads, d, &tg, &merge_grid);
   hipLaunchKernelGGL(attn_rows_merge_kernel<T>, merge_grid, dim3(QIL_WAVE), 0, s, part_acc, part_m, part_l, positions,
-                     row_index, (T*)out, heads, d, window, P, parts, tg, sinks, keep, Operand{}, 0);
+                     row_index, (T*)out, heads, d, window, P, parts, tg, sinks, keep, Operand{}, 0, nullptr);
   return (int)hipGetLastError();
 }
 
@@ -413,7 +415,8 @@ int qil_attn_rows_unmerged(const void* q, int q_stride, const void* k_cache, con
                              acc, m, l, nullptr, rows, heads, kv_heads, d, page_size, window, scale, softcap, P, parts, s, false);
 }
 
-// Merge of partial results written by a partial kernel (this file's or the matrix-core decode kernel's).
+// Merge of partial results written by a partial kernel (this file's or the matrix-core decode kernel's; P 0: parts of the
+// latter's plan).
 // sinks: null, or float32 [heads]: exp(sink) joins every head's divisor once.  keep: the kept first keys (key_span.h).
 // gate: null, or an operand of rows of gate_row elements (total_rows of them, split stride their product) whose first
 // heads * d columns are the logits of an output gate: a row's result is multiplied by their sigmoids before it is rounded.
@@ -428,17 +431,18 @@ int qil_attn_merge(const void* workspace, const int* positions, const int* row_i
   const float* acc = (const float*)workspace;
   const float* m = acc + (size_t)rows * heads * parts * d;
   const float* l = m + (size_t)rows * heads * parts;
-  if (d % 4 || d > 256) return -1;
+  if (d % 4 || d > 256 || P < 0) return -1;
+  const int* part_keys = planned_keys(l, (size_t)rows * heads * parts, P);
   int tg;
   dim3 grid;
   merge_shape(rows, heads, d, &tg, &grid);
   const dim3 block(QIL_WAVE);
   if (dtype == QIL_F32)
     hipLaunchKernelGGL(attn_rows_merge_kernel<float>, grid, block, 0, s, acc, m, l, positions, row_index, (float*)out,
-                       heads, d, window, P, parts, tg, sinks, keep, operand, gate_row);
+                       heads, d, window, P, parts, tg, sinks, keep, operand, gate_row, part_keys);
   else
     hipLaunchKernelGGL(attn_rows_merge_kernel<bf16_t>, grid, block, 0, s, acc, m, l, positions, row_index, (bf16_t*)out,
-                       heads, d, window, P, parts, tg, sinks, keep, operand, gate_row);
+                       heads, d, window, P, parts, tg, sinks, keep, operand, gate_row, part_keys);
   QIL_RETURN_LAUNCH_STATUS();
 }
 

@@ -911,7 +911,7 @@ extern "C" int qil_gemm_bf16_unmerged_takes(int M, int N, int heads, int d, int 
 extern "C" int qil_gemm_bf16_unmerged(const void* workspace, const int* positions, const void* W, void* C, int M, int N,
                                       int heads, int d, int window, int P, int parts, int splits, hipStream_t s) {
   if (M == 0 || N == 0) return 0;
-  if (!qil_gemm_bf16_unmerged_takes(M, N, heads, d, splits) || parts < 1 || P < 1 || ((uintptr_t)W % 16) ||
+  if (!qil_gemm_bf16_unmerged_takes(M, N, heads, d, splits) || parts < 1 || P < 0 || ((uintptr_t)W % 16) ||
       ((uintptr_t)workspace % 16))
     return -1;
   UnmergedA u;
@@ -920,6 +920,7 @@ extern "C" int qil_gemm_bf16_unmerged(const void* workspace, const int* position
   u.l = u.m + (size_t)M * heads * parts;
   u.positions = positions;
   u.heads = heads; u.d = d; u.parts = parts; u.P = P; u.window = window;
+  u.part_keys = planned_keys(u.l, (size_t)M * heads * parts, P);
   const int status = launch_lines<float, 1>(nullptr, (const bf16_t*)W, (float*)C, M, N, heads * d, splits, s, u);
   if (status) return status;
   QIL_RETURN_LAUNCH_STATUS();

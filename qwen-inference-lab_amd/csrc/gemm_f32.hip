@@ -562,7 +562,7 @@ extern "C" int qil_gemm_f32_unmerged_takes(int M, int N, int heads, int d, int s
 extern "C" int qil_gemm_f32_unmerged(const void* workspace, const int* positions, const void* W, float* C, int M, int N,
                                      int heads, int d, int window, int P, int parts, int splits, hipStream_t s) {
   if (M == 0 || N == 0) return 0;
-  if (!qil_gemm_f32_unmerged_takes(M, N, heads, d, splits) || parts < 1 || P < 1 ||
+  if (!qil_gemm_f32_unmerged_takes(M, N, heads, d, splits) || parts < 1 || P < 0 ||
       (((uintptr_t)workspace | (uintptr_t)W) % 16))
     return -1;
   UnmergedA u;
@@ -571,6 +571,7 @@ extern "C" int qil_gemm_f32_unmerged(const void* workspace, const int* positions
   u.l = u.m + (size_t)M * heads * parts;
   u.positions = positions;
   u.heads = heads; u.d = d; u.parts = parts; u.P = P; u.window = window;
+  u.part_keys = planned_keys(u.l, (size_t)M * heads * parts, P);
   return launch_f32_lines<1>(nullptr, u, GatedA(), (const float*)W, C, M, N, heads * d, splits, s);
 }
 

@@ -12,7 +12,12 @@ struct UnmergedA {
   const float* l;
   const int* positions;                                    // [M]: a row's context is its position + 1
   int heads, d, parts, P, window;
+  const int* part_keys;                                    // null, or where the keys of a part stand (P is not used then)
 };
+// P == 0 in a launch: the keys of a part stand behind the partial results (attention_decode.hip's plan).
+__host__ __device__ inline const int* planned_keys(const float* l, size_t cells, int P) {
+  return P ? nullptr : reinterpret_cast<const int*>(l + cells);
+}
 
 // E (4 or 8) merged values of row m starting at column k (all of one head: d % E == 0), float32.
 // AT_ONCE: parts whose loads are in flight together (E * AT_ONCE registers).
@@ -21,7 +26,8 @@ __device__ __forceinline__ void merged_values(const UnmergedA& u, int m, int k, 
   const int head = k / u.d, e = k - head * u.d;
   const int ctx = u.positions[m] + 1;
   const int lo = u.window > 0 ? max(0, ctx - u.window) : 0;
-  const int first = lo / u.P, last = (ctx - 1) / u.P;
+  const int P = u.part_keys ? *u.part_keys : u.P;
+  const int first = lo / P, last = (ctx - 1) / P;
   const size_t cell0 = ((size_t)m * u.heads + head) * u.parts;
   auto load = [&](const float* p, float (&to)[E]) {
     if constexpr (E == 8) {

@@ -75,42 +75,59 @@ __device__ __forceinline__ void store8(bf16_t* p, const float* v) {
 // its cosine and its sine are made here in float32 (no table bounds the positions).
 // rotate_first: the rotation comes before the norm (a design that norms what it has rotated).
 // (qil/model.py:15-23, 42-46, 52-55)
+// What eight elements of a head are normed and turned with: the norm's weights, and the cosines and sines of their pairs
+// (chunks in the rotated part).  Loading them is apart from using them, for a kernel that asks for all it needs first.
+struct HeadFactors {
+  float w[8], c[8], sn[8];
+};
+__device__ __forceinline__ void load_eight(const float* p, float (&to)[8]) {
+  const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 4);
+  to[0] = lo.x; to[1] = lo.y; to[2] = lo.z; to[3] = lo.w; to[4] = hi.x; to[5] = hi.y; to[6] = hi.z; to[7] = hi.w;
+}
+__device__ __forceinline__ void load_turns(HeadFactors& f, int chunk, const float* __restrict__ cos_table,
+                                           const float* __restrict__ sin_table, int position, int rot) {
+  const int half_chunks = rot >> 4;                   // chunks in half of the rotated width (a power of two)
+  if (chunk < 2 * half_chunks) {
+    const int pair = chunk < half_chunks ? chunk : chunk - half_chunks;
+    if (sin_table) {
+      const size_t at = (size_t)position * (rot >> 1) + pair * 8;
+      load_eight(cos_table + at, f.c);
+      load_eight(sin_table + at, f.sn);
+    } else {
+      const float* freq = cos_table + pair * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sincosf((float)position * freq[e], &f.sn[e], &f.c[e]);
+    }
+  }
+}
 template <typename T>
-__device__ __forceinline__ void head_norm8(float (&x)[8], int chunk, int TG, const float* __restrict__ weight, int d, float eps) {
+__device__ __forceinline__ void head_norm8(float (&x)[8], int TG, const HeadFactors& f, int d, float eps) {
   float sum = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) sum += x[e] * x[e];
   for (int o = TG >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, QIL_WAVE);
   const float rstd = rsqrtf(sum / (float)d + eps);
-  const float4 w0 = *reinterpret_cast<const float4*>(weight + chunk * 8);
-  const float4 w1 = *reinterpret_cast<const float4*>(weight + chunk * 8 + 4);
-  const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = round_to<T>(x[e] * rstd) * w[e];
+  for (int e = 0; e < 8; ++e) x[e] = round_to<T>(x[e] * rstd) * f.w[e];
 }
-__device__ __forceinline__ void rotate8(float (&x)[8], int chunk, const float* __restrict__ cos_table,
-                                        const float* __restrict__ sin_table, int position, int rot) {
-  const int half_chunks = rot >> 4;                   // chunks in half of the rotated width (a power of two)
+__device__ __forceinline__ void rotate8(float (&x)[8], int chunk, const HeadFactors& f, int rot) {
+  const int half_chunks = rot >> 4;
   float other[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) other[e] = __shfl_xor(x[e], half_chunks, QIL_WAVE);
   if (chunk < 2 * half_chunks) {
     const bool first = chunk < half_chunks;
-    float c[8], sn[8];
-    if (sin_table) {
-      const size_t at = (size_t)position * (rot >> 1) + (first ? chunk : chunk - half_chunks) * 8;
-      const float4 c0 = *reinterpret_cast<const float4*>(cos_table + at), c1 = *reinterpret_cast<const float4*>(cos_table + at + 4);
-      const float4 s0 = *reinterpret_cast<const float4*>(sin_table + at), s1 = *reinterpret_cast<const float4*>(sin_table + at + 4);
-      c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-      sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
-    } else {
-      const float* freq = cos_table + (first ? chunk : chunk - half_chunks) * 8;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sincosf((float)position * freq[e], &sn[e], &c[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = first ? x[e] * c[e] - other[e] * sn[e] : other[e] * sn[e] + x[e] * c[e];
+    for (int e = 0; e < 8; ++e)                         // (which product is rounded alone is written out: the same in every kernel)
+      x[e] = fmaf(x[e], f.c[e], first ? -(other[e] * f.sn[e]) : other[e] * f.sn[e]);
   }
+}
+template <typename T>
+__device__ __forceinline__ void norm_rope8(float (&x)[8], int chunk, int TG, const HeadFactors& f, bool norms, int d, float eps,
+                                           bool rotates, int rot, bool rotate_first) {
+  if (rotates && rotate_first) rotate8(x, chunk, f, rot);
+  if (norms) head_norm8<T>(x, TG, f, d, eps);
+  if (rotates && !rotate_first) rotate8(x, chunk, f, rot);
 }
 template <typename T>
 __device__ __forceinline__ void norm_rope8(float (&x)[8], int chunk, int TG, const float* __restrict__ weight, int d,
@@ -118,7 +135,8 @@ __device__ __forceinline__ void norm_rope8(float (&x)[8], int chunk, int TG, con
                                            const float* __restrict__ sin_table, int position, int rot,
                                            bool rotate_first = false) {
   const bool rotates = cos_table && rot > 0;
-  if (rotates && rotate_first) rotate8(x, chunk, cos_table, sin_table, position, rot);
-  if (weight) head_norm8<T>(x, chunk, TG, weight, d, eps);
-  if (rotates && !rotate_first) rotate8(x, chunk, cos_table, sin_table, position, rot);
+  HeadFactors f;
+  if (weight) load_eight(weight + chunk * 8, f.w);
+  if (rotates) load_turns(f, chunk, cos_table, sin_table, position, rot);
+  norm_rope8<T>(x, chunk, TG, f, weight != nullptr, d, eps, rotates, rot, rotate_first);
 }

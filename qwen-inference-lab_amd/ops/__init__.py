@@ -48,10 +48,6 @@ DECODE_MAX_PART = 8192
 FUSED_DECODE_MOST_ROWS = 32
 # Rows up to which the row kernel leaves its parts unmerged when the caller allows (the product after it merges them).
 UNMERGED_ROWS_MOST = 16
-# Launches of at most this many blocks (one a CU) let a wave load two of its steps at a time.
-DECODE_PAIRS_BLOCKS = 256
-# ... in the kernel that makes its queries itself only up to this head size (it needs the registers for them).
-FUSED_PAIRS_MOST_DIM = 64
 
 
 # A product of few rows may add its result into the residual stream itself (``add_to``), and the product after it may
@@ -921,6 +917,45 @@ def _decode_parts(rows, kv_heads, max_context):
     return part, max(1, -(-max_context // part))
 
 
+# Fewest keys of a planned part: a step of 32 for each of a block's eight waves.
+PLAN_MIN_PART = 256
+# Rows that a plan is made for at most, and blocks that it shares out (all kv heads together: one a CU; two or three a CU
+# with half the keys each are slower, a block's start and end are some 6 us).
+PLAN_MOST_ROWS, PLAN_BLOCKS = 128, 256
+# Fewest keys (rows times the longest context) of a planned step: below, the plan's own 3 us are more than idle CUs cost
+# (a step of 450 us with two such layers lost 1 %); six rows of 4,096 to 16,384 keys at 12 layers of 8B sizes 2.09 -> 1.80 ms,
+# sixteen of 1,000 to 4,000 1.85 -> 1.79.
+PLAN_FEWEST_KEYS = 32768
+
+
+def _decode_shares(rows, kv_heads, places, window, positions, row_index, plans):
+    """(keys a part, parts, blocks a kv head, plan) of the matrix-core decode kernel.
+
+    With the step's ``plans`` and no window the parts are cut on the GPU from the rows' own lengths (``qil_attn_plan``): one
+    size for all rows, the smallest that gives at most a block a CU.  Cut by the longest context alone (``_decode_parts``),
+    rows of different lengths leave CUs idle."""
+    blocks = PLAN_BLOCKS // kv_heads
+    parts = min(blocks, -(-places // PLAN_MIN_PART))
+    if plans is None or window or rows < 2 or rows * places < PLAN_FEWEST_KEYS or rows * 2 > blocks or rows > PLAN_MOST_ROWS or \
+            parts < 2:
+        part, parts = _decode_parts(rows, kv_heads, places)
+        return part, parts, rows * parts, None
+    blocks = min(blocks, rows * parts)
+    key = (rows, blocks, row_index is None)
+    if key not in plans:
+        plan = torch.empty(1 + blocks, dtype=torch.int32, device=positions.device)
+        _check(library.load().qil_attn_plan(_ptr(positions), _ptr(row_index), rows, blocks, PLAN_MIN_PART, _ptr(plan), _stream()),
+               'attn_plan')
+        plans[key] = plan
+    return 0, parts, blocks, plans[key]
+
+
+def _parts_workspace(rows, heads, head_dim, parts, plan, device):
+    """float32 memory for the parts' results (and the size of a planned part behind them), or None."""
+    floats = library.load().qil_attn_rows_workspace(rows, heads, head_dim, parts) // 4
+    return torch.empty(floats + (4 if plan is not None else 0), dtype=torch.float32, device=device) if floats else None
+
+
 def decode_attention_takes(qkv, *, heads, kv_heads, head_dim, page_size, rotation, dtype):
     """Whether ``decode_attention`` takes the step: a float32 ``Partials`` q/k/v product, bfloat16 caches, sizes of
     the fused kernel."""
@@ -935,7 +970,7 @@ def decode_attention_takes(qkv, *, heads, kv_heads, head_dim, page_size, rotatio
 def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps, rotation, positions, writes, k_cache,
                      v_cache, page_size, block_tables, row_seq, max_context, scale, window, unmerged=False,
                      rotate_first=False, softcap=None, has_kv=True, extra_columns=0, bias=None, q_temperature=None, sinks=None,
-                     values_are_keys=False, slopes=None, keep_first=0, gate=None):
+                     values_are_keys=False, slopes=None, keep_first=0, gate=None, plans=None):
     """``qk_norm_rope_store`` and ``paged_attention`` in one kernel for a step whose rows are all alone in their
     sequences: queries, the new key and the new value are made from the partial sums ``qkv`` inside the
     attention kernel (bit for bit what the two kernels make), the new key and value are written into the
@@ -944,7 +979,8 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     ``extra_columns``, ``bias``, ``q_temperature`` as in ``qk_norm_rope_store``, ``sinks`` as in ``paged_attention``
     (a step with sinks comes back merged); ``values_are_keys`` as in ``qk_norm_rope_store``, ``slopes`` and
     ``keep_first`` as in ``paged_attention``.  ``gate`` [N, heads * d] (a tensor, Partials or Columns): the result is
-    multiplied by its sigmoid (before the rounding, where parts are merged), and comes back merged.  Returns what ``paged_attention`` returns."""
+    multiplied by its sigmoid (before the rounding, where parts are merged), and comes back merged.  ``plans`` as in
+    ``paged_attention``.  Returns what ``paged_attention`` returns."""
     n = qkv.shape[0]
     dtype = torch.bfloat16
     stored = kv_heads if has_kv else 0
@@ -974,17 +1010,15 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     lib = library.load()
     out = torch.empty((n, heads * head_dim), dtype=dtype, device=k_cache.device)
     window_arg = int(window or 0)
-    part, parts = _decode_parts(n, kv_heads, _places(max_context, window, keep))
-    nbytes = lib.qil_attn_rows_workspace(n, heads, head_dim, parts)
-    workspace = torch.empty(nbytes // 4, dtype=torch.float32, device=out.device) if nbytes else None
+    part, parts, blocks, plan = _decode_shares(n, kv_heads, _places(max_context, window, keep), window_arg, positions, None, plans)
+    workspace = _parts_workspace(n, heads, head_dim, parts, plan, out.device)
     _check(lib.qil_attn_decode_fused(pointer, splits, _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(cos),
                                      _ptr(sin), rot, int(bool(writes)), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
                                      block_tables.shape[1], _ptr(row_seq), _ptr(positions), _ptr(workspace), _ptr(out),
                                      n, heads, kv_heads, head_dim, page_size, window_arg, float(scale), part, parts,
-                                     DECODE_WAVES, int(n * kv_heads * parts <= DECODE_PAIRS_BLOCKS and head_dim <= FUSED_PAIRS_MOST_DIM),
-                                     int(bool(rotate_first)), float(softcap or 0.0), int(bool(has_kv)), row - own,
+                                     DECODE_WAVES, int(bool(rotate_first)), float(softcap or 0.0), int(bool(has_kv)), row - own,
                                      _ptr(bias), float(coef), int(every), _ptr(sinks), int(bool(values_are_keys)),
-                                     _ptr(slopes), keep, _stream()), 'attn_decode_fused')
+                                     _ptr(slopes), keep, _ptr(plan), blocks, _stream()), 'attn_decode_fused')
     if parts > 1:
         if sinks is not None or keep or gate is not None:
             # the merge adds the sinks' term and multiplies by the gate; its parts count places
@@ -1025,7 +1059,7 @@ def tile_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, pag
 
 def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size, block_tables, row_seq, positions,
                     cu_seqlens, seq_starts, single_rows, n_seqs, max_query, max_context, scale, window,
-                    unmerged=False, tile_seqs=None, softcap=None, sinks=None, slopes=None, keep_first=0):
+                    unmerged=False, tile_seqs=None, softcap=None, sinks=None, slopes=None, keep_first=0, plans=None):
     """Attention of every row of the step over its request's cached keys.
 
     ``q`` [N, heads * head_dim] (head h at columns [h d, (h + 1) d)).  Row n belongs to sequence ``row_seq[n]`` (a row of ``block_tables``) and sees keys j with
@@ -1047,6 +1081,8 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
     ``keep_first``: with a window, the first so many keys stay visible: row n sees j <= positions[n] with
     j > positions[n] - window or j < keep_first.  Both run on the kernels that take sinks; with kept keys the parts of a
     row's keys leave out the whole steps between the two ranges, and a portion's keys stay in one part.
+    ``plans``: a dict of the step's own, shared by its layers, in which the matrix-core decode kernel's plan of how the
+    keys are shared out among its blocks is kept (made from the positions on the GPU by the step's first layer).
     """
     cap = float(softcap or 0.0)
     if sinks is not None:
@@ -1127,16 +1163,13 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
         window_arg = int(window or 0)
         places = _places(max_context, window, keep)
         if qkv.dtype == torch.bfloat16 and lib.qil_attn_decode_takes(heads, kv_heads, head_dim, page_size):
-            # matrix-core kernel; split the context until the chip has about four blocks per CU
-            part, parts = _decode_parts(rows, kv_heads, places)
-            nbytes = lib.qil_attn_rows_workspace(rows, heads, head_dim, parts)
-            workspace = torch.empty(nbytes // 4, dtype=torch.float32, device=qkv.device) if nbytes else None
+            part, parts, blocks, plan = _decode_shares(rows, kv_heads, places, window_arg, positions, single_rows, plans)
+            workspace = _parts_workspace(rows, heads, head_dim, parts, plan, qkv.device)
             _check(lib.qil_attn_decode(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
                                        block_tables.shape[1], _ptr(row_seq), _ptr(positions), _ptr(single_rows),
                                        _ptr(workspace), _ptr(out), rows, heads, kv_heads, head_dim, page_size,
-                                       window_arg, float(scale), part, parts, DECODE_WAVES,
-                                       int(rows * kv_heads * parts <= DECODE_PAIRS_BLOCKS and head_dim <= 128), cap,
-                                       _ptr(sinks), _ptr(slopes), keep, _stream()), 'attn_decode')
+                                       window_arg, float(scale), part, parts, DECODE_WAVES, cap,
+                                       _ptr(sinks), _ptr(slopes), keep, _ptr(plan), blocks, _stream()), 'attn_decode')
             if unmerged and parts > 1 and single_rows is None:
                 return Unmerged(workspace, positions, out, heads=heads, head_dim=head_dim, window=window_arg,
                                 part=part, parts=parts)

@@ -230,19 +230,20 @@ class Attention(Mixer):
             attended = ops.decode_attention(
                 qkv, rotation=rotation, positions=ctx.positions, writes=cache.writes, k_cache=cache.k, v_cache=cache.v,
                 page_size=cache.page_size, block_tables=cache.block_tables, row_seq=ctx.row_seq,
-                max_context=ctx.max_context, scale=self.scale, window=self.window, unmerged=True,
+                max_context=ctx.max_context, scale=self.scale, window=self.window, unmerged=True, plans=ctx.plans,
                 rotate_first=self.norm_after_rotation, softcap=self.softcap, **sizes, **norms)
             return ops.linear(attended, p['o_proj.weight'], p.get('o_proj.bias'), partials=True)
         q = ops.qk_norm_rope_store(
             qkv, rotation=rotation, positions=ctx.positions, slots=cache.slots if cache.writes else None,
             k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size, dtype=self.dtype, norm_dim=self.head_dim,
             rotate_first=self.norm_after_rotation, **sizes, **norms)
+        planned = dict(plans=ctx.plans) if q.is_cuda else {}
         attended = ops.paged_attention(
             q, k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size,
             block_tables=cache.block_tables, row_seq=ctx.row_seq, positions=ctx.positions,
             cu_seqlens=ctx.cu_seqlens, seq_starts=ctx.seq_starts, single_rows=ctx.single_rows, n_seqs=ctx.n_seqs,
             max_query=ctx.max_query, max_context=ctx.max_context, tile_seqs=ctx.tile_seqs,
-            scale=self.scale, window=self.window, unmerged=True, softcap=self.softcap, **sizes)
+            scale=self.scale, window=self.window, unmerged=True, softcap=self.softcap, **planned, **sizes)
         return ops.linear(attended, p['o_proj.weight'], p.get('o_proj.bias'), partials=True)
 
     def _forward_extended(self, qkv, rotation, norms, sizes, ctx, cache):
@@ -263,7 +264,7 @@ class Attention(Mixer):
             attended = ops.decode_attention(
                 qkv, rotation=rotation, positions=ctx.positions, writes=cache.writes, k_cache=cache.k, v_cache=cache.v,
                 page_size=cache.page_size, block_tables=cache.block_tables, row_seq=ctx.row_seq,
-                max_context=ctx.max_context, unmerged=False, rotate_first=self.norm_after_rotation, has_kv=self.own_kv,
+                max_context=ctx.max_context, unmerged=False, rotate_first=self.norm_after_rotation, has_kv=self.own_kv, plans=ctx.plans,
                 extra_columns=gate_columns, bias=self.b_qkv_own, q_temperature=self.q_temperature,
                 values_are_keys=self.values_are_keys,
                 gate=ops.columns(qkv, own, gate_columns) if self.gate else None, **masks, **sizes, **norms)
@@ -277,11 +278,12 @@ class Attention(Mixer):
         else:
             q = ops.qk_norm_rope_store(qkv, norm_dim=self.head_dim, rotate_first=self.norm_after_rotation,
                                        q_temperature=self.q_temperature, bias=self.b_qkv_own, **store)
+        planned = dict(plans=ctx.plans) if q.is_cuda else {}
         attended = ops.paged_attention(
             q, k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size,
             block_tables=cache.block_tables, row_seq=ctx.row_seq, positions=ctx.positions,
             cu_seqlens=ctx.cu_seqlens, seq_starts=ctx.seq_starts, single_rows=ctx.single_rows, n_seqs=ctx.n_seqs,
-            max_query=ctx.max_query, max_context=ctx.max_context, tile_seqs=ctx.tile_seqs, unmerged=False, **masks, **sizes)
+            max_query=ctx.max_query, max_context=ctx.max_context, tile_seqs=ctx.tile_seqs, unmerged=False, **planned, **masks, **sizes)
         if self.gate:
             attended = ops.sigmoid_gate(attended, qkv, offset=own)
         return ops.linear(attended, p['o_proj.weight'], p.get('o_proj.bias'), partials=True)

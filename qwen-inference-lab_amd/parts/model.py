@@ -115,6 +115,7 @@ class CausalLM:
         Rows are selected before the final norm; with no wanted row neither the
         norm nor the head runs (qil/model.py:130-134).
         """
+        ctx.plans = {}                              # made by each run (a graph's warm-up shares its context with the capture)
         if self.keeps_embedding:
             stream, embedded = self.embedding.forward_step_kept(ctx)
         else:
