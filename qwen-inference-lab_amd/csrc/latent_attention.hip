@@ -29,7 +29,13 @@ __global__ void latent_prepare_kernel(const TD* __restrict__ x, int splits, size
                                       const float* __restrict__ wc, const float* __restrict__ freq,
                                       const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ cq_out,
                                       T* __restrict__ latent, T* __restrict__ rope, float* __restrict__ gate_out, int q_rank,
-                                      int rank, int rot, int gates, float eps, int held, int x_row) {
+                                      int rank, int rot, int gates, float eps, int held, int x_row, int rows,
+                                      T* __restrict__ c_rows, T* __restrict__ rope_rows) {
+  if ((int)blockIdx.x >= rows) {                      // a row that fills the copies up
+    for (int i = threadIdx.x; i < rank; i += blockDim.x) st(c_rows + (size_t)blockIdx.x * rank + i, 0.f);
+    for (int i = threadIdx.x; i < rot; i += blockDim.x) st(rope_rows + (size_t)blockIdx.x * rot + i, 0.f);
+    return;
+  }
   extern __shared__ float sums[];                     // [q_rank + rank + rot + gates] when `held`: the row, its partial sums added
   __shared__ float scratch[16];
   const int n = blockIdx.x, total = q_rank + rank + rot + gates;
@@ -50,7 +56,11 @@ __global__ void latent_prepare_kernel(const TD* __restrict__ x, int splits, size
     gate_out[(size_t)n * gates + i] = 1.f / (1.f + expf(-value(q_rank + rank + rot + i)));
   if (!slots) return;
   const size_t slot = (size_t)slots[n];
-  for (int i = threadIdx.x; i < rank; i += blockDim.x) st(latent + slot * rank + i, value(q_rank + i) * rc * wc[i]);
+  for (int i = threadIdx.x; i < rank; i += blockDim.x) {
+    const float c = value(q_rank + i) * rc * wc[i];
+    st(latent + slot * rank + i, c);
+    if (c_rows) st(c_rows + (size_t)n * rank + i, c);
+  }
   const int half = rot / 2;
   const float p = (float)positions[n];
   for (int i = threadIdx.x; i < half; i += blockDim.x) {
@@ -58,8 +68,13 @@ __global__ void latent_prepare_kernel(const TD* __restrict__ x, int splits, size
     const float v = value(q_rank + rank + half + i);
     float sn, cs;
     sincosf(p * freq[i], &sn, &cs);
-    st(rope + slot * rot + i, u * cs - v * sn);
-    st(rope + slot * rot + half + i, v * cs + u * sn);
+    const float first = u * cs - v * sn, second = v * cs + u * sn;
+    st(rope + slot * rot + i, first);
+    st(rope + slot * rot + half + i, second);
+    if (rope_rows) {
+      st(rope_rows + (size_t)n * rot + i, first);
+      st(rope_rows + (size_t)n * rot + half + i, second);
+    }
   }
 }
 
@@ -311,11 +326,15 @@ static void latent_plan(int heads, int rank, int rot, int* group, int* kt, size_
 
 extern "C" {
 
-// x: rows of x_row elements (split stride n * x_row), the first q_rank + rank + rot + gates of them meant.
+// x: rows of x_row elements (split stride n * x_row), the first q_rank + rank + rot + gates of them meant.  c_rows, rope_rows:
+// null, or copies of what goes into the caches, a row of the step a row ([padded, rank] and [padded, rot], zeros from row n on).
 int qil_latent_prepare(const void* x, int x_dtype, int splits, int x_row, const float* wq, const float* wc, const float* freq,
                        const int* positions, const int* slots, void* cq_out, void* latent, void* rope, float* gate_out,
-                       int n, int q_rank, int rank, int rot, int gates, float eps, int dtype, hipStream_t s) {
+                       int n, int q_rank, int rank, int rot, int gates, float eps, int dtype, void* c_rows, void* rope_rows,
+                       int padded, hipStream_t s) {
   if (n == 0) return 0;
+  if ((c_rows == nullptr) != (rope_rows == nullptr) || (c_rows && (!slots || padded < n))) return -1;
+  const int blocks = c_rows ? padded : n;
   if (q_rank < 1 || rank < 1 || rot < 2 || rot % 2 || splits < 1 || (x_dtype == QIL_BF16 && splits != 1) || gates < 0 ||
       (gates > 0 && !gate_out) || x_row < q_rank + rank + rot + gates)
     return -1;
@@ -326,8 +345,8 @@ int qil_latent_prepare(const void* x, int x_dtype, int splits, int x_row, const 
   // more threads, not more turns
   const int total = q_rank + rank + rot + gates, threads = n > 64 ? 256 : total >= 2048 ? 1024 : total >= 1024 ? 512 : 256;
 #define QIL_LP(TD, T)                                                                                               \
-  hipLaunchKernelGGL((latent_prepare_kernel<TD, T>), dim3(n), dim3(threads), held ? row_bytes : 0, s, (const TD*)x, splits, \
-                     stride, wq, wc, freq, positions, slots, (T*)cq_out, (T*)latent, (T*)rope, gate_out, q_rank, rank, rot, gates, eps, held, x_row)
+  hipLaunchKernelGGL((latent_prepare_kernel<TD, T>), dim3(blocks), dim3(threads), held ? row_bytes : 0, s, (const TD*)x, splits, \
+                     stride, wq, wc, freq, positions, slots, (T*)cq_out, (T*)latent, (T*)rope, gate_out, q_rank, rank, rot, gates, eps, held, x_row, n, (T*)c_rows, (T*)rope_rows)
   if (dtype == QIL_F32) {
     if (x_dtype != QIL_F32) return -1;
     QIL_LP(float, float);

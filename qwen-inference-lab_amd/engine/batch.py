@@ -41,6 +41,7 @@ class StepContext:
     requests: list = field(default_factory=list)
     previous_tokens: torch.Tensor = None   # [N] the token before each row's in its sequence (-1: none), for embeddings
                                            # that ask for it (``needs_previous_tokens``)
+    fresh: bool = False            # every sequence of the step begins with it, and the step is not described for a graph
     plans: dict = field(default_factory=dict)    # how the step's attention kernels share out their keys, kept from its first layer on
     tile_seqs: int = None          # sequences 0 .. tile_seqs - 1 are those of two or more rows; None: any may be
 

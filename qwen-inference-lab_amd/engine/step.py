@@ -181,7 +181,9 @@ class ModelRunner:
     def prepare(self, entries):
         """Pages, then the batch description on the device.  Does not touch the cache contents."""
         entries, pieces, facts = self._describe(entries)
-        return entries, self._context(entries, pieces, facts, torch.from_numpy(pieces.flat()).to(self.model.device))
+        ctx = self._context(entries, pieces, facts, torch.from_numpy(pieces.flat()).to(self.model.device))
+        ctx.fresh = not any(facts['starts'])
+        return entries, ctx
 
     @torch.inference_mode()
     def step(self, entries):

@@ -1365,11 +1365,12 @@ def short_conv(x, weight, *, state, cu_seqlens, seq_starts, seq_slots, row_seq, 
 # ---------------------------------------------------------------------------------------------------------------
 # Attention over a cached latent
 def latent_prepare(down, *, q_rank, rank, rot, q_weight, c_weight, eps, frequencies, positions, slots, latent, rope,
-                   dtype, gates=0):
+                   dtype, gates=0, copies=None):
     """From the stacked down products ``down`` [N, q_rank + rank + rot (+ gates)] (tensor of ``dtype``, Partials or Columns):
     the RMS-normed query latent [N, q_rank] (returned); the RMS-normed key/value latent and the rotated shared key
     part go into the caches ``latent`` [.., rank] / ``rope`` [.., rot] at ``slots`` (None: nothing is stored).  With
-    ``gates`` more columns the result is (query latent, float32 [N, gates] of their sigmoids)."""
+    ``gates`` more columns the result is (query latent, float32 [N, gates] of their sigmoids).  ``copies``: a pair
+    [M, rank], [M, rot] of ``dtype`` (M >= N) that gets what is stored too, row by row, and zeros from row N on."""
     n = down.shape[0]
     pointer, code, splits, row = _row_operand(down, 'down', n, q_rank + rank + rot + gates, (dtype, torch.float32))
     _require(q_weight, 'q_weight', torch.float32, (q_rank,))
@@ -1382,13 +1383,57 @@ def latent_prepare(down, *, q_rank, rank, rot, q_weight, c_weight, eps, frequenc
         _require(rope, 'rope', dtype)
         if latent.shape[-1] != rank or rope.shape[-1] != rot or latent.shape[:-1] != rope.shape[:-1]:
             raise ValueError('latent_prepare: caches must be [.., rank] and [.., rot] over the same slots')
+    c_rows, rope_rows, padded = None, None, 0
+    if copies is not None:
+        c_rows, rope_rows = copies
+        padded = c_rows.shape[0]
+        _require(c_rows, 'copies', dtype, (padded, rank))
+        _require(rope_rows, 'copies', dtype, (padded, rot))
     out = torch.empty((n, q_rank), dtype=dtype, device=down.device)
     gate = torch.empty((n, gates), dtype=torch.float32, device=down.device) if gates else None
     _check(library.load().qil_latent_prepare(pointer, code, splits, row, _ptr(q_weight), _ptr(c_weight), _ptr(frequencies),
                                              _ptr(positions), _ptr(slots), _ptr(out), _ptr(latent), _ptr(rope), _ptr(gate),
-                                             n, q_rank, rank, rot, gates, float(eps), _code(dtype), _stream()),
+                                             n, q_rank, rank, rot, gates, float(eps), _code(dtype), _ptr(c_rows),
+                                             _ptr(rope_rows), padded, _stream()),
            'latent_prepare')
     return (out, gate) if gates else out
+
+
+# Rows from which a step of whole prompts runs its latent attention over expanded keys and values (more than a captured step
+# has: which sequences begin with a step is known on the host only).
+EXPAND_FEWEST_ROWS = 513
+
+
+def expands_latents(rows, *, dim, rot, vdim, dtype):
+    """Whether ``latent_expanded`` should serve a step of ``rows`` rows whose sequences all begin with it."""
+    return rows >= EXPAND_FEWEST_ROWS and dtype == torch.bfloat16 and bool(library.load().qil_latent_expanded_takes(dim, rot, vdim))
+
+
+def expanded_rows(rows):
+    """Rows of the arrays that ``latent_expanded`` reads: up to the next whole tile of keys."""
+    return -(-rows // 64) * 64
+
+
+def latent_expanded(q, k, kr, vt, *, heads, cu_seqlens, frequencies, sink, gate, scale, n_seqs, max_query):
+    """Attention of sequences that begin with the step, over the step's own rows: ``q`` [N, heads * 192] (a head's 128
+    unrotated elements, then 64 not yet turned), ``k`` [M, heads * 128], ``kr`` [M, 64] (turned, every head's), ``vt`` [heads * 128, M]
+    (M = ``expanded_rows(N)``), all bfloat16.  ``sink`` and ``gate`` as in ``latent_attention``.  -> bfloat16 [N, heads * 128]."""
+    n, padded = q.shape[0], k.shape[0]
+    _require(q, 'q', torch.bfloat16, (n, heads * 192))
+    _require(k, 'k', torch.bfloat16, (expanded_rows(n), heads * 128))
+    _require(kr, 'kr', torch.bfloat16, (padded, 64))
+    _require(vt, 'vt', torch.bfloat16, (heads * 128, padded))
+    _require(cu_seqlens, 'cu_seqlens', torch.int32, (n_seqs + 1,))
+    _require(frequencies, 'frequencies', torch.float32, (32,))
+    if sink is not None:
+        _require(sink, 'sink', torch.float32, (heads,))
+    if gate is not None:
+        _require(gate, 'gate', torch.float32, (n, heads))
+    out = torch.empty((n, heads * 128), dtype=torch.bfloat16, device=q.device)
+    _check(library.load().qil_latent_expanded(_ptr(q), _ptr(k), _ptr(kr), _ptr(vt), padded, _ptr(cu_seqlens), _ptr(frequencies),
+                                              _ptr(sink), _ptr(gate), _ptr(out), n_seqs, max_query, heads, float(scale),
+                                              _stream()), 'latent_expanded')
+    return out
 
 
 HEAD_PRODUCT_BLAS_ROWS = 256     # rows from which a bfloat16 product per head goes to the GPU BLAS in one batch

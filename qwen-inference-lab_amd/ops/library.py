@@ -295,7 +295,10 @@ def _declare(lib):
     lib.qil_gemm_bf16_wide_gated.argtypes = [p, p, p, i, i, i, i, p]
     lib.qil_add_norm.argtypes = [p, p, i, i, i, f, p, p, p, p, i, i, f, i, i, i, p]
     lib.qil_gated_act.argtypes = [p, i, i, i, p, i, i, i, i, i, f, f, p]
-    lib.qil_latent_prepare.argtypes = [p, i, i, i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, f, i, p]
+    lib.qil_latent_prepare.argtypes = [p, i, i, i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, f, i, p, p, i, p]
+    lib.qil_latent_expanded_takes.argtypes = [i, i, i]
+    lib.qil_latent_expanded_takes.restype = i
+    lib.qil_latent_expanded.argtypes = [p, p, p, p, i, p, p, p, p, p, i, i, i, f, p]
     lib.qil_head_product.argtypes = [p, i, i, i, p, i, p, i, i, i, i, i, i, i, p, i, i, i, p]
     lib.qil_gated_heads.argtypes = [p, p, i, i, i, p, i, i, i, p]
     lib.qil_gated_heads.restype = i

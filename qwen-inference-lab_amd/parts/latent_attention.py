@@ -99,6 +99,7 @@ class LatentAttention(Mixer):
         p['down.weight'] = self.w_down
         # W_uk as [heads, dim, kv_rank] is the layout the query's product reads (a pure view); W_uv per head transposed
         self.k_up = p['k_up.weight'].view(self.heads, self.dim, self.kv_rank)
+        self.v_rows = p['v_up.weight']                  # as stored: whole prompts expand their values with it
         p['v_up.weight'] = p['v_up.weight'].view(self.heads, self.vdim, self.kv_rank).transpose(1, 2).contiguous()
         self.position.frequencies()                     # made here, not in a step that may be captured
 
@@ -107,13 +108,26 @@ class LatentAttention(Mixer):
         frequencies = self.position.frequencies()
         down = ops.linear(h, self.w_down, None, partials=True)
         own = down if self.gate != 'element' else ops.columns(down, 0, self.own_rows)
+        # whole prompts: their rows are all the keys there are, and attention over expanded keys and values costs a third
+        expands = ctx.fresh and cache.writes and self.window is None and self.gate != 'element' and down.device.type == 'cuda' and \
+            ops.expands_latents(h.shape[0], dim=self.dim, rot=self.rot_dim, vdim=self.vdim, dtype=self.dtype)
+        copies = {}
+        if expands:
+            padded = ops.expanded_rows(h.shape[0])
+            c, kr = (torch.empty((padded, size), dtype=self.dtype, device=down.device) for size in (self.kv_rank, self.rot_dim))
+            copies = dict(copies=(c, kr))
         cq = ops.latent_prepare(own, q_rank=self.q_rank, rank=self.kv_rank, rot=self.rot_dim, q_weight=p['q_norm.weight'],
                                 c_weight=p['kv_norm.weight'], eps=self.eps, frequencies=frequencies,
                                 positions=ctx.positions, slots=cache.slots if cache.writes else None,
                                 latent=cache.tensors['latent'], rope=cache.tensors['rope'], dtype=self.dtype,
-                                gates=self.heads if self.gate == 'head' else 0)
+                                gates=self.heads if self.gate == 'head' else 0, **copies)
         cq, gate = cq if self.gate == 'head' else (cq, None)
         q = ops.linear(cq, p['q_up.weight'], None)
+        if expands:
+            values = ops.latent_expanded(q, ops.linear(c, p['k_up.weight']), kr, ops.linear(self.v_rows, c), heads=self.heads,
+                                         cu_seqlens=ctx.cu_seqlens, frequencies=frequencies, sink=p.get('sink'), gate=gate,
+                                         scale=self.scale, n_seqs=ctx.n_seqs, max_query=ctx.max_query)
+            return ops.linear(values, p['o_proj.weight'], None, partials=True)
         q = ops.latent_query(q, self.k_up, heads=self.heads, dim=self.dim, rot=self.rot_dim, rank=self.kv_rank,
                              frequencies=frequencies, positions=ctx.positions)
         mixed = ops.latent_attention(q, latent=cache.tensors['latent'], rope=cache.tensors['rope'],
