@@ -1,0 +1,46 @@
+"""Kernels of steps with few rows: norms with the row in registers, products whose result has to be whole, small gated ones."""
+import pytest
+import torch
+
+import kernel_refs as refs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def ops():
+    from qil_amd import ops
+    ops.library.load()
+    return ops
+
+
+def rand(*shape, dtype=torch.float32, scale=1.0, seed=0):
+    g = torch.Generator().manual_seed(seed + sum(shape))
+    return (torch.randn(*shape, generator=g) * scale).to(dtype).cuda()
+
+
+# a width at each edge of the register shapes, one that no thread fills, one beyond them and one that is no multiple of four
+@pytest.mark.parametrize('width', [4, 256, 260, 1024, 2044, 2048, 4096, 8192, 8196, 1002])
+@pytest.mark.parametrize('centre', [True, False])
+@pytest.mark.parametrize('kind', ['none', 'bfloat16', 'partials', 'float32'])
+def test_norms_with_the_row_in_registers(ops, width, centre, kind):
+    """Against the reference in float64: sums of `width` float32 terms are off by about 2^-24 sqrt(width) of the row's size, the
+    result is rounded once.  The stream's sum is the same float32 sum, split by split, to one rounding of the scaled delta."""
+    n, dtype = 3, torch.float32 if kind == 'float32' else torch.bfloat16
+    stream = rand(n, width, scale=2.0) + 5.0                 # a mean to be removed
+    weight, bias = 1 + 0.2 * rand(width, seed=2), rand(width, seed=3)
+    delta = {'none': None, 'bfloat16': rand(n, width, dtype=torch.bfloat16, seed=4), 'float32': rand(n, width, seed=4),
+             'partials': ops.Partials(rand(5, n, width, seed=5))}[kind]
+    value = 0.0 if delta is None else (delta.tensor.double().sum(0) if kind == 'partials' else delta.double())
+    total = stream.double() + 0.5 * value
+    centred = total - total.mean(-1, keepdim=True) if centre else total
+    want = centred / torch.sqrt(centred.square().mean(-1, keepdim=True) + 1e-5) * weight.double() + bias.double()
+    rows = torch.tensor([2, 0], dtype=torch.int32).cuda()
+    close = dict(atol=2e-5, rtol=2e-5) if dtype == torch.float32 else dict(atol=2e-4, rtol=2.0 ** -8)
+    before = stream.clone()
+    some = ops.rows_norm(stream, delta, rows, weight, 1e-5, dtype, centre=centre, delta_scale=0.5, bias=bias)
+    assert torch.equal(stream, before)
+    got = ops.add_norm(stream, delta, weight, 1e-5, dtype, centre=centre, delta_scale=0.5, bias=bias)
+    torch.testing.assert_close(got.double(), want, **close)
+    assert torch.equal(some, got[rows.long()])
+    torch.testing.assert_close(stream.double(), total, atol=1e-5, rtol=2.0 ** -22)
