@@ -9,6 +9,7 @@
 // W and A both travel in whole cache lines (4 rows x 256 bytes a load), three stages of 128 columns ahead in
 // registers, through buffers of the wave's own in LDS that turn them into matrix-core fragments (see the whole-line
 // kernel in gemm_bf16.hip); A comes from L2.  K may be any length (the down product of a gated feed-forward).
+// The same kernel makes the products whose bfloat16 result has to be whole (no consumer of partial sums behind them).
 // Takes N a multiple of 16, K a multiple of 128 ksplit with at least 3 stages a wave, 16-byte aligned operands.
 #include <algorithm>
 
@@ -22,11 +23,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define ADD_DEPTH 3                                        // stages in flight per wave
 #define ADD_LDS_LIMIT (160 * 1024)
 
-// AROWS: rows of A kept (8 or 16).
-template <int AROWS>
+// AROWS: rows of A kept (8 or 16).  INTO: the result goes into the stream; else out [M, N] of bfloat16 gets it (squares null).
+template <int AROWS, bool INTO>
 __global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE, AROWS == 8 ? 4 : 3)
 gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ stream,
-                     float* __restrict__ squares, int M, int N, int K, int ksplit) {
+                     bf16_t* __restrict__ out, float* __restrict__ squares, int M, int N, int K, int ksplit) {
   extern __shared__ __align__(16) bf16_t lds[];            // per wave: 4 KB for W, AROWS x 256 bytes for A
   constexpr int ALOADS = AROWS / 4, PER_WAVE = (16 + AROWS) * 128;
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
@@ -112,6 +113,10 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
     for (int i = 0; i < 4; ++i) {
       const int m = 4 * kb + i;
       float value = 0.f;
+      if (!INTO) {
+        if (m < M && stores) out[(size_t)m * N + n0 + r] = f32_to_bf16(total[i]);
+        continue;
+      }
       if (m < M && stores) {
         float* cell = stream + (size_t)m * N + n0 + r;
         value = *cell + total[i];
@@ -168,9 +173,10 @@ int qil_gemm_bf16_add_takes(int M, int N, int K) {
   return add_plan(M, N, K, &groups, &ksplit);
 }
 
-// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [N / 16][M] that gets the rows' sums of squares
-// of the new stream in pieces of 16 columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set them).
-int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* squares, int M, int N, int K, int groups,
+}  // extern "C"
+
+template <bool INTO>
+static int add_launch(const void* A, const void* W, float* stream, void* out, float* squares, int M, int N, int K, int groups,
                       int ksplit, hipStream_t s) {
   if (M == 0 || N == 0) return 0;
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)stream) % 16) return -1;
@@ -183,12 +189,35 @@ int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* square
   const size_t lds = add_lds_bytes(M, groups * ksplit);
   dim3 grid((N / 16 + groups - 1) / groups), block(groups * ksplit * QIL_WAVE);
   if (M <= 8)
-    hipLaunchKernelGGL(gemm_bf16_add_kernel<8>, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, stream, squares, M,
-                       N, K, ksplit);
+    hipLaunchKernelGGL((gemm_bf16_add_kernel<8, INTO>), grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, stream,
+                       (bf16_t*)out, squares, M, N, K, ksplit);
   else
-    hipLaunchKernelGGL(gemm_bf16_add_kernel<16>, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, stream, squares,
-                       M, N, K, ksplit);
+    hipLaunchKernelGGL((gemm_bf16_add_kernel<16, INTO>), grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, stream,
+                       (bf16_t*)out, squares, M, N, K, ksplit);
   QIL_RETURN_LAUNCH_STATUS();
+}
+
+extern "C" {
+
+// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [N / 16][M] that gets the rows' sums of squares
+// of the new stream in pieces of 16 columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set them).
+int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* squares, int M, int N, int K, int groups,
+                      int ksplit, hipStream_t s) {
+  return add_launch<true>(A, W, stream, nullptr, squares, M, N, K, groups, ksplit, s);
+}
+
+// 1 if a product of up to 16 rows whose result has to be whole and of bfloat16 should run here (qil_gemm_bf16_whole): where
+// the whole-line kernel (gemm_bf16.hip), which can split K only into partial sums, is a block of 128 columns on each of few
+// CUs.  us there and here, 8 rows: 3,072 x 1,536 10.0 / 6.1, 6,144 x 2,048 13.2 / 7.9, 12,288 x 2,048 16.5 / 10.9, 16,384 x
+// 2,048 16.7 / 13.4, 32,768 x 2,048 22.9 / 23.2, 4,096 x 4,096 22.3 / 8.7, 2,048 x 6,144 70 / 10.7, 1,536 x 512 5.0 / 6.1.
+int qil_gemm_bf16_whole_takes(int M, int N, int K) {
+  int groups, ksplit;
+  return N <= 16384 && K >= 1024 && add_plan(M, N, K, &groups, &ksplit);
+}
+
+// out bfloat16 [M, N] = A[M, K] W[N, K]^T, K split over a block's waves.
+int qil_gemm_bf16_whole(const void* A, const void* W, void* out, int M, int N, int K, hipStream_t s) {
+  return add_launch<false>(A, W, nullptr, out, nullptr, M, N, K, 0, 0, s);
 }
 
 }  // extern "C"

@@ -671,6 +671,10 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
             _check(lib.qil_gemm_bf16(_ptr(x), _ptr(weight), None, _ptr(out), n, o, k, 0, splits, 0, 0, _stream()),
                    'gemm_bf16')
             return Partials(out)
+    if streams and n <= STREAM_GEMM_MAX_ROWS and bias is None and out_dtype == x.dtype and lib.qil_gemm_bf16_whole_takes(n, o, k):
+        out = torch.empty((n, o), dtype=x.dtype, device=x.device)
+        _check(lib.qil_gemm_bf16_whole(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _stream()), 'gemm_bf16_whole')
+        return out
     if out_dtype == torch.float32 or streams:
         out = torch.empty((n, o), dtype=out_dtype, device=x.device)
         _check(lib.qil_gemm_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), n, o, k, _code(out_dtype), 1, 0, 0,

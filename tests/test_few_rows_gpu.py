@@ -44,3 +44,15 @@ def test_norms_with_the_row_in_registers(ops, width, centre, kind):
     torch.testing.assert_close(got.double(), want, **close)
     assert torch.equal(some, got[rows.long()])
     torch.testing.assert_close(stream.double(), total, atol=1e-5, rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize('m', [1, 8, 9, 16])
+@pytest.mark.parametrize('n,k', [(16, 1024), (3072, 1536), (2064, 6144), (16384, 1152)])
+def test_whole_products_of_few_rows(ops, m, n, k):
+    """One rounding of a float32 sum of k terms of size one (3e-6 of the largest covers 6,144 of them)."""
+    assert ops.library.load().qil_gemm_bf16_whole_takes(m, n, k)
+    x, w = rand(m, k, dtype=torch.bfloat16), rand(n, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5)
+    want = x.double() @ w.double().t()
+    got = ops.linear(x, w)
+    assert got.dtype == torch.bfloat16
+    torch.testing.assert_close(got.double(), want, atol=3e-6 * want.abs().max().item(), rtol=2.0 ** -8)
