@@ -717,6 +717,15 @@ static bool gated_plan(const void* A, const void* W, int M, int inner, int K, in
   for (int c = 8; c >= 1 && !ks; c /= 2)
     if (K % (128 * c) == 0 && K / (128 * c) >= (c == 1 || (long)(inner / 16) * c <= 8 * QIL_CUS ? 2 : 16)) ks = c;
   if (!ks) return false;
+  // Pairs that are fewer than the CUs: a CU each, and waves that have four stages where K is long enough (3,072 x 1,024: 192
+  // blocks of two waves instead of 96 of eight, a step of 28 layers 1,056 -> 1,024 us for one row, 1,443 -> 1,415 for eight).
+  if (inner / 16 <= QIL_CUS && gated_lds(M, K, 8) <= 156 * 1024) {
+    *pairs = 1;
+    *ksplit = 1;
+    for (int c = 2; c <= 8; c *= 2)
+      if (K % (128 * c) == 0 && K / (128 * c) >= 4) *ksplit = c;
+    return K / (128 * *ksplit) >= 2;
+  }
   // Pairs a block: what a CU has to do in all (its blocks one after the other, as many at a time as LDS and
   // the 12 wave slots allow) over how well its waves keep memory busy (8 or more do).  Ties go to more pairs.
   const int all_pairs = inner / 16;

@@ -56,3 +56,14 @@ def test_whole_products_of_few_rows(ops, m, n, k):
     got = ops.linear(x, w)
     assert got.dtype == torch.bfloat16
     torch.testing.assert_close(got.double(), want, atol=3e-6 * want.abs().max().item(), rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize('m', [1, 8, 16])
+@pytest.mark.parametrize('inner,k', [(3072, 1024), (16, 256), (4096, 4096), (4096, 384), (48, 640)])
+def test_small_gated_products(ops, m, inner, k):
+    """Fewer pairs of tiles than CUs: a block each.  As above, through silu(gate) * up."""
+    x, w = rand(m, k, dtype=torch.bfloat16), rand(2 * inner, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5)
+    y = x.double() @ w.double().t()
+    want = torch.nn.functional.silu(y[:, :inner]) * y[:, inner:]
+    got = ops.gated_linear(x, ops.interleave_gate_up(w[:inner].contiguous(), w[inner:].contiguous()), interleaved=True)
+    torch.testing.assert_close(got.double(), want, atol=3e-5 * want.abs().max().item(), rtol=2.0 ** -8)
