@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import kernel_refs as refs
+from test_kernels_gpu import build_cache
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,22 @@ def test_small_gated_products(ops, m, inner, k):
     want = torch.nn.functional.silu(y[:, :inner]) * y[:, inner:]
     got = ops.gated_linear(x, ops.interleave_gate_up(w[:inner].contiguous(), w[inner:].contiguous()), interleaved=True)
     torch.testing.assert_close(got.double(), want, atol=3e-5 * want.abs().max().item(), rtol=2.0 ** -8)
+
+
+# every way the waves share a head's elements: one run of 32 for four waves, two, three (a wave idles), four, more than four;
+# every head tile; a part of one key, parts that end inside a run of keys, and keys behind a window
+@pytest.mark.parametrize('d', [8, 32, 64, 96, 128, 136, 256])
+@pytest.mark.parametrize('heads,kv_heads', [(2, 2), (4, 2), (6, 2), (16, 2)])
+def test_rows_attention_shares_out_the_values(ops, monkeypatch, d, heads, kv_heads):
+    """Float32 rows against float64: weights and values of size one over 600 keys, sums off by a few 1e-6."""
+    lengths, page_size = [1, 17, 256, 600], 16
+    k_cache, v_cache, table, _ = build_cache(lengths, page_size, kv_heads, d, torch.float32)
+    positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32).cuda()
+    q = rand(len(lengths), heads * d, seed=5)
+    for window in (None, 40):
+        step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=page_size, block_tables=table, scale=d ** -0.5,
+                    row_seq=torch.arange(len(lengths), dtype=torch.int32).cuda(), positions=positions, max_context=max(lengths),
+                    window=window, cu_seqlens=None, seq_starts=None, single_rows=None, n_seqs=len(lengths), max_query=1)
+        got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+        want = refs.paged_attention(q.double(), k_cache=k_cache.double(), v_cache=v_cache.double(), accumulate=torch.float64, **step)
+        torch.testing.assert_close(got.double(), want.double(), atol=1e-5, rtol=1e-5)
