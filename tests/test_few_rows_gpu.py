@@ -87,3 +87,17 @@ def test_rows_attention_shares_out_the_values(ops, monkeypatch, d, heads, kv_hea
         got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
         want = refs.paged_attention(q.double(), k_cache=k_cache.double(), v_cache=v_cache.double(), accumulate=torch.float64, **step)
         torch.testing.assert_close(got.double(), want.double(), atol=1e-5, rtol=1e-5)
+
+
+# widths the four-element kernel takes and does not, a gate that starts between its loads, an input that is not aligned
+@pytest.mark.parametrize('columns,offset,width,shift', [(1024, 4, 1028, 0), (4, 0, 4, 0), (1024, 2, 1028, 0), (30, 4, 64, 0), (64, 4, 70, 0),
+                                                        (64, 4, 68, 1)])
+@pytest.mark.parametrize('kind', ['bfloat16', 'partials', 'float32'])
+def test_gate_of_four_elements(ops, columns, offset, width, shift, kind):
+    """The sigmoid to a few float32 roundings, then one rounding of the product."""
+    n, dtype = 5, torch.float32 if kind == 'float32' else torch.bfloat16
+    x = rand(n * columns + shift, dtype=dtype)[shift:].view(n, columns)
+    source = ops.Partials(rand(3, n, width, seed=1)) if kind == 'partials' else rand(n, width, dtype=dtype, seed=1)
+    logits = (source.tensor.double().sum(0) if kind == 'partials' else source.double())[:, offset:offset + columns]
+    got = ops.sigmoid_gate(x, source, offset=offset)
+    torch.testing.assert_close(got.double(), x.double() * torch.sigmoid(logits), atol=1e-6, rtol=2e-6 if kind == 'float32' else 2.0 ** -8)
