@@ -107,6 +107,50 @@ template <int V> __device__ __forceinline__ void store_floats(bf16_t* p, const f
   for (int e = 0; e < V; e += 4) st4(p + e, make_float4(v[e], v[e + 1], v[e + 2], v[e + 3]));
 }
 
+// Outputs r = from .. upto - 1 of a sequence whose first row is row0 (V channels from c on): the factors' products in
+// tap order, inputs before the step's rows from the state.
+template <typename TI, typename T, int V>
+__device__ __forceinline__ void conv_outputs(const TI* __restrict__ x, int splits, size_t split_stride, int x_columns,
+                                             const float* __restrict__ w, const float* b, const float* held, int start, int row0,
+                                             int from, int upto, T* __restrict__ out, int c, int channels, int taps, int act) {
+  const int keep = taps - 1;
+  for (int r = from; r < upto; ++r) {
+    float acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = b[e];
+    for (int j = 0; j < taps; ++j) {
+      const int source = r - keep + j;
+      float in[V], f[V];
+      if (source >= 0) conv_in<TI, V>::load(x, (size_t)(row0 + source) * x_columns + c, splits, split_stride, in);
+      else if (held && start + source >= 0) load_floats<V>(held + (size_t)(keep + source) * channels + c, in);
+      else continue;
+      load_floats<V>(w + (size_t)j * channels + c, f);
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc[e] += f[e] * in[e];
+    }
+    if (act) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc[e] = silu_f(acc[e]);
+    }
+    store_floats<V>(out + (size_t)(row0 + r) * channels + c, acc);
+  }
+}
+
+// The state after the step's rows: the sequence's last taps - 1 inputs (by the thread that has read the state before).
+template <typename TI, int V>
+__device__ __forceinline__ void conv_keep(const TI* __restrict__ x, int splits, size_t split_stride, int x_columns, float* held,
+                                          int start, int row0, int rows, int c, int channels, int keep) {
+  for (int k = 0; k < keep; ++k) {
+    const int source = rows - keep + k;
+    float in[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) in[e] = 0.f;
+    if (source >= 0) conv_in<TI, V>::load(x, (size_t)(row0 + source) * x_columns + c, splits, split_stride, in);
+    else if (start + source >= 0) load_floats<V>(held + (size_t)(k + rows) * channels + c, in);
+    store_floats<V>(held + (size_t)k * channels + c, in);
+  }
+}
+
 template <typename TI, typename T, int V>
 __global__ void channel_conv_vec_kernel(const TI* __restrict__ x, int splits, size_t split_stride, int x_columns,
                                         const float* __restrict__ w, const float* __restrict__ bias, float* state,
@@ -129,40 +173,77 @@ __global__ void channel_conv_vec_kernel(const TI* __restrict__ x, int splits, si
   if (t > 0 && t < keep) return;                       // computed with the sequence's first row
   const int rows = cu_seqlens[s + 1] - row0, start = seq_starts[s];
   float* held = state ? state + (size_t)seq_slots[s] * keep * channels : nullptr;
-  const int upto = t == 0 ? min(rows, max(keep, 1)) : t + 1;
   float b[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) b[e] = 0.f;
   if (bias) load_floats<V>(bias + c, b);
-  for (int r = t; r < upto; ++r) {
-    float acc[V];
+  conv_outputs<TI, T, V>(x, splits, split_stride, x_columns, w, b, held, start, row0, t,
+                         t == 0 ? min(rows, max(keep, 1)) : t + 1, out, c, channels, taps, act);
+  if (t == 0 && held) conv_keep<TI, V>(x, splits, split_stride, x_columns, held, start, row0, rows, c, channels, keep);
+}
+
+// Long sequences of bfloat16 rows: CONV_ROWS consecutive rows a thread (8 channels), whose inputs and the TAPS - 1 before
+// them are asked for at once and read once; so are the factors.  A thread of the kernel above reads TAPS rows and 32
+// bytes of factors a tap for 16 bytes of results.  A sequence's first rows, which need its state, are computed as above
+// by the thread that meets the first of them.  2,048 rows of 6,144 channels, silu, 27.8 -> 21.4 us: the vector instructions of
+// the silu's exponential and quotient are what is left (looking a run of rows' sequence up once instead of row by row
+// changed nothing).
+#define CONV_ROWS 8
+template <int TAPS>
+__global__ void __launch_bounds__(128)
+channel_conv_rows_kernel(const bf16_t* __restrict__ x, int x_columns, const float* __restrict__ w, const float* __restrict__ bias,
+                         float* state, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_starts,
+                         const int* __restrict__ seq_slots, const int* __restrict__ row_seq, bf16_t* __restrict__ out, int n,
+                         int channels, int act, int pass_from, int passed, bf16_t* __restrict__ passed_out) {
+  constexpr int V = 8, KEEP = TAPS - 1;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V, n0 = blockIdx.x * CONV_ROWS;
+  uint4 in[KEEP + CONV_ROWS];                          // the rows n0 - KEEP .. n0 + CONV_ROWS - 1
+  if (c >= channels) {
+    const int i = c - channels;
+    if (i < passed) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] = b[e];
-    for (int j = 0; j < taps; ++j) {
-      const int source = r - keep + j;
-      float in[V], f[V];
-      if (source >= 0) conv_in<TI, V>::load(x, (size_t)(row0 + source) * x_columns + c, splits, split_stride, in);
-      else if (held && start + source >= 0) load_floats<V>(held + (size_t)(keep + source) * channels + c, in);
-      else continue;
-      load_floats<V>(w + (size_t)j * channels + c, f);
+      for (int k = 0; k < CONV_ROWS; ++k)
+        in[k] = *reinterpret_cast<const uint4*>(x + (size_t)min(n0 + k, n - 1) * x_columns + pass_from + i);
 #pragma unroll
-      for (int e = 0; e < V; ++e) acc[e] += f[e] * in[e];
+      for (int k = 0; k < CONV_ROWS; ++k)
+        if (n0 + k < n) *reinterpret_cast<uint4*>(passed_out + (size_t)(n0 + k) * passed + i) = in[k];
     }
-    if (act) {
-#pragma unroll
-      for (int e = 0; e < V; ++e) acc[e] = silu_f(acc[e]);
-    }
-    store_floats<V>(out + (size_t)(row0 + r) * channels + c, acc);
+    return;
   }
-  if (t == 0 && held) {
-    for (int k = 0; k < keep; ++k) {
-      const int source = rows - keep + k;
-      float in[V];
 #pragma unroll
-      for (int e = 0; e < V; ++e) in[e] = 0.f;
-      if (source >= 0) conv_in<TI, V>::load(x, (size_t)(row0 + source) * x_columns + c, splits, split_stride, in);
-      else if (start + source >= 0) load_floats<V>(held + (size_t)(k + rows) * channels + c, in);
-      store_floats<V>(held + (size_t)k * channels + c, in);
+  for (int k = 0; k < KEEP + CONV_ROWS; ++k)
+    in[k] = *reinterpret_cast<const uint4*>(x + (size_t)min(max(n0 - KEEP + k, 0), n - 1) * x_columns + c);
+  float f[TAPS][V], b[V];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) load_floats<V>(w + (size_t)j * channels + c, f[j]);
+#pragma unroll
+  for (int e = 0; e < V; ++e) b[e] = 0.f;
+  if (bias) load_floats<V>(bias + c, b);
+#pragma unroll
+  for (int k = 0; k < CONV_ROWS; ++k) {
+    const int row = n0 + k;
+    if (row >= n) return;
+    const int s = row_seq[row], row0 = cu_seqlens[s], t = row - row0;
+    if (t >= KEEP) {                                   // every input is a row of this sequence
+      float acc[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc[e] = b[e];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        const uint32_t q[4] = {in[k + j].x, in[k + j].y, in[k + j].z, in[k + j].w};
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] += f[j][e] * __uint_as_float(e % 2 ? q[e / 2] & 0xffff0000u : q[e / 2] << 16);
+      }
+      if (act) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] = silu_f(acc[e]);
+      }
+      store_floats<V>(out + (size_t)row * channels + c, acc);
+    } else if (t == 0) {
+      const int rows = cu_seqlens[s + 1] - row0, start = seq_starts[s];
+      float* held = state + (size_t)seq_slots[s] * KEEP * channels;
+      conv_outputs<bf16_t, bf16_t, V>(x, 1, 0, x_columns, w, b, held, start, row0, 0, min(rows, KEEP), out, c, channels, TAPS, act);
+      conv_keep<bf16_t, V>(x, 1, 0, x_columns, held, start, row0, rows, c, channels, KEEP);
     }
   }
 }
@@ -376,13 +457,13 @@ int qil_selective_scan_takes(int channels, int states, int taps) {
 }
 
 // x: [n, x_columns] (x_code QIL_F32 with x_splits partial sums, or QIL_BF16), its first `channels` columns are the
-// convolution's input; w float32 [taps, channels]; bias float32 [channels] or null; state float32 [slots][taps - 1]
+// convolution's input; n_seqs: the step's sequences; w float32 [taps, channels]; bias float32 [channels] or null; state float32 [slots][taps - 1]
 // [channels] (null only for one tap); out [n, channels] of out_dtype; act: 0 none, 1 silu.  passed > 0: the columns
 // [pass_from, pass_from + passed) go to passed_out [n, passed] of out_dtype.
 int qil_channel_conv(const void* x, int x_code, int x_splits, int x_columns, const float* w, const float* bias, float* state,
                      const int* cu_seqlens, const int* seq_starts, const int* seq_slots, const int* row_seq, void* out,
-                     int out_dtype, int n, int channels, int taps, int act, int pass_from, int passed, void* passed_out,
-                     hipStream_t s) {
+                     int out_dtype, int n, int n_seqs, int channels, int taps, int act, int pass_from, int passed,
+                     void* passed_out, hipStream_t s) {
   if (n == 0) return 0;
   if (passed < 0 || (passed && (!passed_out || pass_from < 0 || pass_from + passed > x_columns))) return -1;
   if (channels < 1 || channels > x_columns || taps < 1 || (taps > 1 && !state) || x_splits < 1 ||
@@ -393,6 +474,13 @@ int qil_channel_conv(const void* x, int x_code, int x_splits, int x_columns, con
       !(x_code == QIL_BF16 && out_dtype == QIL_F32)) {
     const int lanes = (channels + passed) / V;
     const int threads = lanes >= 128 ? 128 : (lanes + 63) / 64 * 64;
+    // enough rows that a thread can have several, in sequences long enough that few of them need the state
+    if (x_code == QIL_BF16 && taps == 4 && n > 512 && n / 32 >= n_seqs) {
+      hipLaunchKernelGGL(channel_conv_rows_kernel<4>, dim3((n + CONV_ROWS - 1) / CONV_ROWS, (lanes + threads - 1) / threads),
+                         dim3(threads), 0, s, (const bf16_t*)x, x_columns, w, bias, state, cu_seqlens, seq_starts, seq_slots,
+                         row_seq, (bf16_t*)out, n, channels, act, pass_from, passed, (bf16_t*)passed_out);
+      QIL_RETURN_LAUNCH_STATUS();
+    }
     const dim3 grid(n, (lanes + threads - 1) / threads);
     const size_t stride = (size_t)n * x_columns;
     if (x_code == QIL_BF16)

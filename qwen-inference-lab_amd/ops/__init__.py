@@ -1889,7 +1889,7 @@ def channel_conv(x, weight, bias, *, columns, state, cu_seqlens, seq_starts, seq
     through = torch.empty((n, passed), dtype=out_dtype, device=weight.device) if passed else None
     _check(library.load().qil_channel_conv(pointer, code, splits, width, _ptr(weight), _ptr(bias),
                                            _ptr(state) if taps > 1 else None, _ptr(cu_seqlens), _ptr(seq_starts),
-                                           _ptr(seq_slots), _ptr(row_seq), _ptr(out), _code(out_dtype), n, columns, taps,
+                                           _ptr(seq_slots), _ptr(row_seq), _ptr(out), _code(out_dtype), n, n_seqs, columns, taps,
                                            CONV_ACTIVATIONS[activation], int(pass_from), int(passed), _ptr(through), _stream()),
            'channel_conv')
     return (out, through) if passed else out

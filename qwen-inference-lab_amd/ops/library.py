@@ -346,7 +346,7 @@ def _declare(lib):
     lib.qil_scaled_sum.argtypes = [p, i, i, p, i, i, f, f, p, i, i, p]
     lib.qil_sigmoid_gate.argtypes = [p, p, i, i, i, i, p, i, i, i, p]
     lib.qil_soft_cap.argtypes = [p, f, z, p]
-    lib.qil_channel_conv.argtypes = [p, i, i, i, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, p, p]
+    lib.qil_channel_conv.argtypes = [p, i, i, i, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i, p, p]
     lib.qil_selective_scan_takes.argtypes = [i, i, i]
     lib.qil_selective_scan.argtypes = [p, p, i, i, p, p, p, i, i, p, p, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, p]
     lib.qil_selective_scan_workspace.argtypes = [i, i, i, i]

@@ -1,4 +1,5 @@
-"""Kernels of steps with few rows: norms with the row in registers, products whose result has to be whole, small gated ones."""
+"""Kernels of steps with few rows (norms with the row in registers, products whose result has to be whole, small gated ones, the
+row attention's values), the gate of four elements a thread and the convolution of long sequences."""
 import pytest
 import torch
 
@@ -101,3 +102,31 @@ def test_gate_of_four_elements(ops, columns, offset, width, shift, kind):
     logits = (source.tensor.double().sum(0) if kind == 'partials' else source.double())[:, offset:offset + columns]
     got = ops.sigmoid_gate(x, source, offset=offset)
     torch.testing.assert_close(got.double(), x.double() * torch.sigmoid(logits), atol=1e-6, rtol=2e-6 if kind == 'float32' else 2.0 ** -8)
+
+
+# rows whose last group is not whole; sequences that start at the edge of a group, inside one, next to each other, with fewer
+# rows than the state holds, that begin or continue (from a state shorter than three inputs too); passed columns or none
+@pytest.mark.parametrize('counts,starts', [([513], [0]), ([301, 8, 1, 2, 3, 250], [0, 5, 1, 0, 2, 7]), ([520, 505], [2, 0]),
+                                           ([256, 2, 256], [9, 1, 0])])
+@pytest.mark.parametrize('channels,passed', [(1024, 64), (1032, 0), (8, 8)])
+def test_convolution_of_long_sequences(ops, counts, starts, channels, passed):
+    """Against the reference in float32: four products of size one and a silu, then one rounding; the state is the inputs."""
+    n, width, n_seqs = sum(counts), channels + passed + 8, len(counts)
+    x = rand(n, width, dtype=torch.bfloat16)
+    weight, bias = rand(4, channels, seed=1), rand(channels, seed=2)
+    state = rand(8, 3, channels, seed=3)
+    for s, start in enumerate(starts):                        # what lies before a sequence's first position is never read
+        state[s + 1, :max(3 - start, 0)] = float('nan')
+    step = dict(cu_seqlens=torch.tensor([0] + counts).cumsum(0).to(torch.int32), seq_starts=torch.tensor(starts, dtype=torch.int32),
+                seq_slots=torch.arange(1, n_seqs + 1, dtype=torch.int32),
+                row_seq=torch.arange(n_seqs, dtype=torch.int32).repeat_interleave(torch.tensor(counts)))
+    sizes = dict(columns=channels, n_seqs=n_seqs, activation='silu', out_dtype=torch.bfloat16, pass_from=channels + 8 if passed else 0,
+                 passed=passed)
+    state_c = state.cpu()
+    want = refs.channel_conv(x.cpu(), weight.cpu(), bias.cpu(), state=state_c, **step, **sizes)
+    got = ops.channel_conv(x, weight, bias, state=state, **{k: v.cuda() for k, v in step.items()}, **sizes)
+    if passed:
+        assert torch.equal(got[1].cpu(), want[1])
+        got, want = got[0], want[0]
+    torch.testing.assert_close(got.cpu().float(), want.float(), atol=2e-6, rtol=2.0 ** -7)
+    assert torch.equal(state.cpu().nan_to_num(7.0), state_c.nan_to_num(7.0))
