@@ -341,16 +341,18 @@ __global__ void gated_group_norm_kernel(const float* __restrict__ o, const T* __
     float a[V], b[V], g[V];
     const size_t at = (size_t)n * gridDim.y * size + j;
     if constexpr (V == 4) {
-      const float4 a4 = ld4(o + at), b4 = ld4(u + (size_t)n * u_row + j), g4 = operand_at4(z, (size_t)n * z_row + j);
+      const AskedOperand asked = operand_ask4(z, (size_t)n * z_row + j);
+      const float4 a4 = ld4(o + at), b4 = ld4(u + (size_t)n * u_row + j), g4 = operand_take4(z, (size_t)n * z_row + j, asked);
       a[0] = a4.x; a[1] = a4.y; a[2] = a4.z; a[3] = a4.w;
       b[0] = b4.x; b[1] = b4.y; b[2] = b4.z; b[3] = b4.w;
       g[0] = g4.x; g[1] = g4.y; g[2] = g4.z; g[3] = g4.w;
     } else {
       a[0] = o[at]; b[0] = ld(u + (size_t)n * u_row + j); g[0] = operand_at(z, (size_t)n * z_row + j);
     }
+    const int head = j / vdim, last = (head + 1) * vdim;               // (neighbours lie in one head or the next ones)
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-      const float v = (a[e] + skip[(j + e) / vdim] * b[e]) * (g[e] / (1.f + expf(-g[e])));
+      const float v = (a[e] + skip[j + e < last ? head : (j + e) / vdim] * b[e]) * (g[e] / (1.f + expf(-g[e])));
       held[i + e] = v;
       squares += v * v;
     }
