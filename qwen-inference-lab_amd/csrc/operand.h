@@ -39,16 +39,18 @@ __device__ __forceinline__ float4 operand_at4(const Operand& x, size_t index) {
   return v;
 }
 
-// operand_at4 in two halves: the load of the array (or of the first split), and what becomes of it.  A kernel with several
-// operands asks for all of them before it takes the first: operand_at4 waits for its own load inside its branch
-// (2,048 rows: the residual join with its gates 25.0 -> 22.8 us, the gated group norm 24.8 -> 22.4).
+// operand_at4 in two halves: the load of a plain array, and what becomes of it, for a kernel that asks for its operands
+// before it takes the first (operand_at4 waits for its own load inside its branch): the gated group norm, 2,048 rows
+// 24.8 -> 22.9 us.  Partial sums are not asked for: their loop has four splits in flight.  The residual join, which has
+// five operands, gained 2 us at 2,048 rows only where it asked for partial sums too, and then took 8.8 us instead of 7.7
+// for 12 rows (twelve splits: a turn of the loop more).
 struct AskedOperand { uint32_t bits[4]; };
 __device__ __forceinline__ AskedOperand operand_ask4(const Operand& x, size_t index) {
-  AskedOperand asked;
+  AskedOperand asked{};
   if (x.code == QIL_BF16) {
     const uint2 q = *reinterpret_cast<const uint2*>(reinterpret_cast<const bf16_t*>(x.data) + index);
-    asked.bits[0] = q.x; asked.bits[1] = q.y; asked.bits[2] = 0; asked.bits[3] = 0;
-  } else {
+    asked.bits[0] = q.x; asked.bits[1] = q.y;
+  } else if (x.splits == 1) {
     const uint4 q = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(x.data) + index);
     asked.bits[0] = q.x; asked.bits[1] = q.y; asked.bits[2] = q.z; asked.bits[3] = q.w;
   }
@@ -58,16 +60,8 @@ __device__ __forceinline__ float4 operand_take4(const Operand& x, size_t index, 
   if (x.code == QIL_BF16)
     return make_float4(__uint_as_float(asked.bits[0] << 16), __uint_as_float(asked.bits[0] & 0xffff0000u),
                        __uint_as_float(asked.bits[1] << 16), __uint_as_float(asked.bits[1] & 0xffff0000u));
-  const float* base = reinterpret_cast<const float*>(x.data) + index;
-  float4 v = make_float4(0.f + __uint_as_float(asked.bits[0]), 0.f + __uint_as_float(asked.bits[1]),
-                         0.f + __uint_as_float(asked.bits[2]), 0.f + __uint_as_float(asked.bits[3]));
-  for (int s0 = 1; s0 < x.splits; s0 += 4) {
-    float4 part[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      part[k] = s0 + k < x.splits ? ld4(base + (size_t)(s0 + k) * x.stride) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { v.x += part[k].x; v.y += part[k].y; v.z += part[k].z; v.w += part[k].w; }
-  }
-  return v;
+  if (x.splits == 1)
+    return make_float4(__uint_as_float(asked.bits[0]), __uint_as_float(asked.bits[1]), __uint_as_float(asked.bits[2]),
+                       __uint_as_float(asked.bits[3]));
+  return operand_at4(x, index);
 }

@@ -21,12 +21,9 @@ struct JoinInputs {
   const float* step;
 };
 
-template <int V> __device__ __forceinline__ void join_ask(const Operand& x, size_t at, AskedOperand& asked) {
-  if constexpr (V == 4) asked = operand_ask4(x, at);
-}
-template <int V> __device__ __forceinline__ void join_load(const Operand& x, size_t at, const AskedOperand& asked, float* v) {
+template <int V> __device__ __forceinline__ void join_load(const Operand& x, size_t at, float* v) {
   if constexpr (V == 4) {
-    const float4 q = operand_take4(x, at, asked);
+    const float4 q = operand_at4(x, at);
     v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
   } else {
     v[0] = operand_at(x, at);
@@ -52,41 +49,35 @@ __global__ void residual_join_kernel(float* __restrict__ stream, JoinInputs in, 
   float squares = 0.f;
   for (int i = threadIdx.x * V; i < width; i += blockDim.x * V) {
     float v[V], t[V], u[V];
-    AskedOperand a{}, b{}, f{}, g1{}, g2{};                // all asked for before the first is taken
-    if (in.a.data) join_ask<V>(in.a, r * in.a_row + i, a);
-    if (in.b.data) join_ask<V>(in.b, r * in.b_row + i, b);
-    if (in.f.data) join_ask<V>(in.f, r * in.f_row + i, f);
-    if (in.gates.data) join_ask<V>(in.gates, r * in.g_row + i, g1);
-    if (in.gates.data && in.f.data) join_ask<V>(in.gates, r * in.g_row + width + i, g2);
     join_floats<V>(x + i, v);
     if (in.a.data) {
-      join_load<V>(in.a, r * in.a_row + i, a, t);
+      join_load<V>(in.a, r * in.a_row + i, t);
 #pragma unroll
       for (int e = 0; e < V; ++e) t[e] *= in.a_scale;
       if (in.b.data) {
-        join_load<V>(in.b, r * in.b_row + i, b, u);
+        join_load<V>(in.b, r * in.b_row + i, u);
 #pragma unroll
         for (int e = 0; e < V; ++e) t[e] += in.b_scale * u[e];
       }
       if (in.gates.data) {
-        float bias[V];
-        join_load<V>(in.gates, r * in.g_row + i, g1, u);
-        join_floats<V>(in.bias + i, bias);
+        float b[V];
+        join_load<V>(in.gates, r * in.g_row + i, u);
+        join_floats<V>(in.bias + i, b);
 #pragma unroll
-        for (int e = 0; e < V; ++e) t[e] = t[e] / (1.f + expf(-(u[e] + bias[e])));
+        for (int e = 0; e < V; ++e) t[e] = t[e] / (1.f + expf(-(u[e] + b[e])));
       }
       if (in.f.data) {
-        float fed[V];
-        join_load<V>(in.f, r * in.f_row + i, f, fed);
+        float f[V];
+        join_load<V>(in.f, r * in.f_row + i, f);
         if (in.gates.data) {
-          float bias[V];
-          join_load<V>(in.gates, r * in.g_row + width + i, g2, u);
-          join_floats<V>(in.bias + width + i, bias);
+          float b[V];
+          join_load<V>(in.gates, r * in.g_row + width + i, u);
+          join_floats<V>(in.bias + width + i, b);
 #pragma unroll
-          for (int e = 0; e < V; ++e) fed[e] = fed[e] / (1.f + expf(-(u[e] + bias[e])));
+          for (int e = 0; e < V; ++e) f[e] = f[e] / (1.f + expf(-(u[e] + b[e])));
         }
 #pragma unroll
-        for (int e = 0; e < V; ++e) t[e] += fed[e];
+        for (int e = 0; e < V; ++e) t[e] += f[e];
       }
 #pragma unroll
       for (int e = 0; e < V; ++e) v[e] += t[e];
