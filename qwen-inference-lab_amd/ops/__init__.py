@@ -3,7 +3,7 @@
 Each function checks what its kernel assumes (shapes, types, contiguity, sizes it
 takes), then launches the hand-written HIP kernel on torch's current stream.
 Nothing here computes on the host or through a library, with one exception:
-bfloat16 matrix products with many rows and a bfloat16 result go to the GPU BLAS
+long bfloat16 matrix products with many rows and a bfloat16 result go to the GPU BLAS
 library, where the reference uses one too (nn.Linear, qil/model.py:32-40).  An
 op refuses sizes its kernel does not take with ``UnsupportedShape``; if the
 kernel library cannot be built or loaded every op raises.
