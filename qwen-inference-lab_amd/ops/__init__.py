@@ -363,6 +363,12 @@ def _ptr(tensor):
     return None if tensor is None else tensor.data_ptr()
 
 
+def _whole_pieces(*tensors):
+    """Whether the tensors begin at multiples of 16 bytes: what a kernel that reads 16 bytes at a time needs (a contiguous
+    view may begin anywhere)."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _check(status, name):
     if status:
         raise RuntimeError(f'{name}: HIP kernel launch failed (status {status})'
@@ -671,7 +677,8 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
             _check(lib.qil_gemm_bf16(_ptr(x), _ptr(weight), None, _ptr(out), n, o, k, 0, splits, 0, 0, _stream()),
                    'gemm_bf16')
             return Partials(out)
-    if streams and n <= STREAM_GEMM_MAX_ROWS and bias is None and out_dtype == x.dtype and lib.qil_gemm_bf16_whole_takes(n, o, k):
+    if streams and n <= STREAM_GEMM_MAX_ROWS and bias is None and out_dtype == x.dtype and \
+            lib.qil_gemm_bf16_whole_takes(n, o, k) and _whole_pieces(x, weight):
         out = torch.empty((n, o), dtype=x.dtype, device=x.device)
         _check(lib.qil_gemm_bf16_whole(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _stream()), 'gemm_bf16_whole')
         return out
@@ -682,7 +689,7 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
         return out
     # beyond 256 rows: the products that the library is no faster at (the kernel's file says which)
     splits = lib.qil_gemm_bf16_wide_splits(n, o, k, int(partials and bias is None)) \
-        if n > MID_GEMM_MOST_ROWS and out_dtype == x.dtype and not OWN_LARGE_PRODUCTS else 0
+        if n > MID_GEMM_MOST_ROWS and out_dtype == x.dtype and not OWN_LARGE_PRODUCTS and _whole_pieces(x, weight) else 0
     if splits:
         out = torch.empty((splits, n, o), dtype=torch.float32 if splits > 1 else x.dtype, device=x.device)
         _check(lib.qil_gemm_bf16_wide(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _code(out.dtype), splits, _stream()),
@@ -758,7 +765,7 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
         return out
     if x.dtype == torch.bfloat16 and interleaved and \
             ((OWN_LARGE_PRODUCTS and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k)) or
-             lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k)):
+             (lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k) and _whole_pieces(x, weight))):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
         _check(lib.qil_gemm_bf16_wide_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
                'gemm_bf16_wide_gated')

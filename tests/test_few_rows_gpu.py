@@ -130,3 +130,30 @@ def test_convolution_of_long_sequences(ops, counts, starts, channels, passed):
         got, want = got[0], want[0]
     torch.testing.assert_close(got.cpu().float(), want.float(), atol=2e-6, rtol=2.0 ** -7)
     assert torch.equal(state.cpu().nan_to_num(7.0), state_c.nan_to_num(7.0))
+
+
+# eight rows: K split over a block's waves where the operands lie on 16 bytes; 600: a block kernel of this library's
+@pytest.mark.parametrize('m', [8, 600])
+@pytest.mark.parametrize('shifted', ['x', 'weight', 'both'])
+def test_products_of_views_at_odd_offsets(ops, m, shifted):
+    """Contiguous views that begin between two multiples of 16 bytes are taken as they always were: whole results, and the
+    gated product of many rows, against float64.  (One rounding of the sums; through the gate the products' own rounding to
+    bfloat16 too, 2^-8 of values up to the largest sum.)"""
+    n, k = 2048, 1024
+    lib = ops.library.load()
+    assert lib.qil_gemm_bf16_whole_takes(8, n, k) and lib.qil_gemm_bf16_wide_splits(600, n, k, 0) and \
+        lib.qil_gemm_bf16_wide_gated_wanted(600, n // 2, k)
+    view = lambda rows, columns, name, **kw: rand(rows * columns + 8, dtype=torch.bfloat16, **kw)[
+        1 if shifted in (name, 'both') else 0:][:rows * columns].view(rows, columns)
+    x, w = view(m, k, 'x'), view(n, k, 'weight', seed=1, scale=k ** -0.5)
+    assert (x.data_ptr() | w.data_ptr()) % 16
+    want = x.double() @ w.double().t()
+    got = ops.linear(x, w)
+    assert isinstance(got, torch.Tensor) and got.dtype == torch.bfloat16
+    torch.testing.assert_close(got.double(), want, atol=3e-6 * want.abs().max().item(), rtol=2.0 ** -8)
+    if m > 16:
+        at = torch.arange(n).view(-1, 2, 16)                 # gate and up rows in turns of 16
+        gate, up = want[:, at[:, 0].reshape(-1).cuda()], want[:, at[:, 1].reshape(-1).cuda()]
+        gated = ops.gated_linear(x, w, interleaved=True)
+        torch.testing.assert_close(gated.double(), torch.nn.functional.silu(gate) * up,
+                                   atol=2.0 ** -7 * want.abs().max().item(), rtol=2.0 ** -6)
