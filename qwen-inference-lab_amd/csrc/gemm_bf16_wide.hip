@@ -54,6 +54,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define WIDE_STAGE 32                                      // columns of K a stage: rows of 64 bytes
 #define WIDE_ROW_BYTES (WIDE_STAGE * 2)
 #define WIDE_XCDS 8
+#define WIDE_SPLIT_COLUMNS 1024                            // fewest columns of a product of many rows that is left as partial sums
 #define WIDE_HOST_US 24.0                                  // products of at most this time by wide_us are not the BLAS's
 
 // RT, CT: tiles of 32 rows and of 32 columns of a wave; DOWN, ACROSS: the block's waves above each other and side by side;
@@ -329,7 +330,10 @@ extern "C" {
 int qil_gemm_bf16_wide_takes(int M, int N, int K, int splits) { return wide_takes(M, N, K, splits); }
 
 // Splits of K with which a product of more than 256 rows should run here rather than in the GPU BLAS (1: a result of
-// A's type; more, where `may_split` allows float32 partial sums and there are no more columns than K); 0: the BLAS.
+// A's type; more, where `may_split` allows float32 partial sums and there are no more columns than K, but 1,024 or more);
+// 0: the BLAS.  Fewer columns are not a stream's but factors that their consumer reads again and again (the 32 columns of a
+// state-space scan's B and C: left as partial sums of 4,096 rows of K, the scan's two passes over 2,048 rows took 96 and
+// 54 us, with a bfloat16 result 51 and 40).
 // What takes no more than WIDE_HOST_US by the count above stays here.  The GPU's times are level with the library's there (us
 // here against there at 643 rows, 0.6B sizes: q/k/v 12.4 / 11.9, attention output 10.3 / 10.7, down 12.1 / 13.9; 2,048 rows of
 // 2,048 x 2,048 21.0 / 21.6), but the host spends 21 us on a library product and 7 on one of ours, and steps of such
@@ -340,7 +344,7 @@ int qil_gemm_bf16_wide_takes(int M, int N, int K, int splits) { return wide_take
 int qil_gemm_bf16_wide_splits(int M, int N, int K, int may_split) {
   int found = 0;
   double best = WIDE_HOST_US;
-  for (int splits = 1; splits <= (may_split && K >= N ? 8 : 1); ++splits) {
+  for (int splits = 1; splits <= (may_split && K >= N && N >= WIDE_SPLIT_COLUMNS ? 8 : 1); ++splits) {
     if (!wide_takes(M, N, K, splits)) continue;
     const double us = wide_us(M, N, K, splits, wide_shape(M, N, K, splits));
     if (us <= best) { best = us; found = splits; }

@@ -99,3 +99,12 @@ def test_general_tile_kernel_cuts_the_keys_of_few_row_tiles(lib):
             if parts > 1:
                 assert part.value % 64 == 0 and part.value >= 128 and parts <= 32
                 assert part.value * parts >= context > part.value * (parts - 1)
+
+
+def test_narrow_products_of_many_rows_are_whole(lib):
+    """Partial sums only of what a norm or a join reads once: not of factors that a scan reads again and again."""
+    for rows in (513, 700, 2048):
+        for columns in (32, 64, 288, 992):
+            assert lib.qil_gemm_bf16_wide_splits(rows, columns, 4096, 1) in (0, 1)
+        assert lib.qil_gemm_bf16_wide_splits(rows, 32, 1024, 1) == lib.qil_gemm_bf16_wide_splits(rows, 32, 1024, 0)
+    assert lib.qil_gemm_bf16_wide_splits(700, 1024, 3072, 1) > 1
