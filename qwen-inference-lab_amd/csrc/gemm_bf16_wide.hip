@@ -265,13 +265,34 @@ static bool wide_takes(int M, int N, int K, int splits) {
 // (one block a CU: what a CU has in flight is then the same as with two, for products that have no second block for it).
 enum { WIDE_256 = 0, WIDE_128 = 1, WIDE_128_DEEP = 2 };
 
-// A product's time by this count, us: a start and an end, rounds of blocks on the 256 CUs times a stage's time, which grows
+// How a product's pieces of work lie in its grid (the kernel's first lines): patches of row and column blocks, places
+// without a piece at the patches' edges among them, and a run of as many places for each XCD.
+struct WideGrid {
+  int row_blocks, col_blocks, patch_rows, patch_cols, blocks;
+};
+static WideGrid wide_grid(int M, int N, int rows, int tile, int splits) {
+  WideGrid g;
+  g.row_blocks = (M + rows - 1) / rows;
+  g.col_blocks = (N + tile - 1) / tile;
+  g.patch_rows = std::min(g.row_blocks, 8);
+  g.patch_cols = std::min(g.col_blocks, std::max(1, QIL_CUS / WIDE_XCDS / g.patch_rows));
+  const int patches = ((g.row_blocks + g.patch_rows - 1) / g.patch_rows) * ((g.col_blocks + g.patch_cols - 1) / g.patch_cols) * splits;
+  g.blocks = (patches * g.patch_rows * g.patch_cols + WIDE_XCDS - 1) / WIDE_XCDS * WIDE_XCDS;
+  return g;
+}
+
+// A product's time by this count, us: a start and an end, rounds of blocks on the CUs times a stage's time, which grows
 // with how many CUs work at once (memory, L2 and the clock are shared), and the partial sums out and in again at 5 TB/s.
 // Fitted to products of 300 to 2,048 rows at 0.6B, 8B and 2,048 x 6,144 sizes with cold weights, which it meets to 15 %.
 static double wide_us(int M, int N, int K, int splits, int shape) {
   const int edge = shape == WIDE_256 ? 256 : 128, slots = QIL_CUS * (shape == WIDE_128 ? 2 : 1);
-  const long blocks = (long)((M + edge - 1) / edge) * ((N + edge - 1) / edge) * splits;
-  const long rounds = (blocks + slots - 1) / slots;
+  const WideGrid grid = wide_grid(M, N, edge, edge, splits);
+  const long blocks = (long)grid.row_blocks * grid.col_blocks * splits;
+  // One block a CU: the rounds of the XCD with the most pieces.  The first XCDs' places all hold one, and where the last
+  // patches are nearly empty those are more than an eighth of the pieces (257 rows of 10,304 columns: 243 blocks, but 34
+  // on XCDs of 32 CUs, 37 us where one round of K = 2,048 is 21).  Two a CU: what is left over runs alone, twice as fast.
+  const long most = shape == WIDE_128 ? 0 : std::min<long>(blocks, grid.blocks / WIDE_XCDS);
+  const long rounds = std::max((blocks + slots - 1) / slots, (most + slots / WIDE_XCDS - 1) / (slots / WIDE_XCDS));
   const double fill = (double)blocks / (rounds * slots);
   const double stage = shape == WIDE_256 ? 0.45 + 0.45 * fill : shape == WIDE_128 ? 0.30 + 0.23 * fill : 0.26;
   const double sums = splits > 1 ? 2.0 * splits * 4.0 * M * N / 5e6 : 0.0;
@@ -289,12 +310,9 @@ static int wide_launch(const void* A, const void* W, void* C, int M, int N, int 
     if (e != hipSuccess) return (int)e;
     granted = true;
   }
-  const int col_blocks = (N + TILE - 1) / TILE, row_blocks = (M + ROWS - 1) / ROWS;
-  const int patch_rows = std::min(row_blocks, 8), patch_cols = std::min(col_blocks, std::max(1, QIL_CUS / WIDE_XCDS / patch_rows));
-  const int patches = ((row_blocks + patch_rows - 1) / patch_rows) * ((col_blocks + patch_cols - 1) / patch_cols) * splits;
-  const int blocks = (patches * patch_rows * patch_cols + WIDE_XCDS - 1) / WIDE_XCDS * WIDE_XCDS;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(DOWN * ACROSS * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N,
-                     K, K / WIDE_STAGE / splits, col_blocks, row_blocks, splits, patch_rows, patch_cols);
+  const WideGrid g = wide_grid(M, N, ROWS, TILE, splits);
+  hipLaunchKernelGGL(kernel, dim3(g.blocks), dim3(DOWN * ACROSS * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N,
+                     K, K / WIDE_STAGE / splits, g.col_blocks, g.row_blocks, splits, g.patch_rows, g.patch_cols);
   QIL_RETURN_LAUNCH_STATUS();
 }
 

@@ -108,3 +108,11 @@ def test_narrow_products_of_many_rows_are_whole(lib):
             assert lib.qil_gemm_bf16_wide_splits(rows, columns, 4096, 1) in (0, 1)
         assert lib.qil_gemm_bf16_wide_splits(rows, 32, 1024, 1) == lib.qil_gemm_bf16_wide_splits(rows, 32, 1024, 0)
     assert lib.qil_gemm_bf16_wide_splits(700, 1024, 3072, 1) > 1
+
+
+def test_a_products_rounds_are_those_of_the_fullest_xcd(lib):
+    """243 blocks of 128 x 128 whose last patch of columns is nearly empty: 34 of them on XCDs of 32 CUs, two rounds.
+    Where the patches are whole (48 bands of columns) every XCD has 30."""
+    assert lib.qil_gemm_bf16_wide_splits(640, 6528, 1024, 0) == 1            # (short enough for two rounds)
+    assert lib.qil_gemm_bf16_wide_splits(257, 10304, 2048, 0) == 0
+    assert lib.qil_gemm_bf16_wide_splits(600, 6400, 2048, 0) == 0 and lib.qil_gemm_bf16_wide_splits(600, 6144, 2048, 0) == 1
