@@ -55,7 +55,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define WIDE_ROW_BYTES (WIDE_STAGE * 2)
 #define WIDE_XCDS 8
 #define WIDE_SPLIT_COLUMNS 1024                            // fewest columns of a product of many rows that is left as partial sums
-#define WIDE_HOST_US 24.0                                  // products of at most this time by wide_us are not the BLAS's
+#define WIDE_HOST_US 24.0                                  // products of at most this time by wide_us are not the BLAS's ...
+#define WIDE_GRAPH_ROWS 512                                // ... but up to so many rows, which a graph may replay,
+#define WIDE_LEVEL_US 3.0                                  // only those within so much of its time on the GPU
 
 // RT, CT: tiles of 32 rows and of 32 columns of a wave; DOWN, ACROSS: the block's waves above each other and side by side;
 // AHEAD: stages (even) that a pair's loads go out ahead.  OUT: bf16_t or float (the result; with splits of K float32 partial sums [split][M][N]).  GATED (one split): W holds gate and up rows in turns of 16, a tile of 32 columns is 16
@@ -299,6 +301,17 @@ static double wide_us(int M, int N, int K, int splits, int shape) {
   return (shape == WIDE_256 ? 6.0 : 4.5) + rounds * ((double)K / WIDE_STAGE / splits) * stage + sums;
 }
 
+// The GPU BLAS's time for a product of up to 512 rows, us (fitted to 257 to 512 rows of 19 products from 512 x 4,096 to
+// 12,288 x 2,048 with cold weights, which it meets to 24 %, 9 % on average), and the activation's behind it.
+static double blas_us(int M, int N, int K, bool gated) {
+  return 5.5 + 1.25e-9 * (2.0 * M * N * K) + 1.1 * K / 1024.0 + (gated ? 2.0 : 0.0);
+}
+
+// Whether a product of this time by the count above should not be the BLAS's.
+static bool wide_wanted(int M, int N, int K, double us, bool gated) {
+  return us <= WIDE_HOST_US && (M > WIDE_GRAPH_ROWS || us <= blas_us(M, N, K, gated) + WIDE_LEVEL_US);
+}
+
 template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
 static int wide_launch(const void* A, const void* W, void* C, int M, int N, int K, int splits, hipStream_t s) {
   constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;
@@ -348,24 +361,35 @@ extern "C" {
 int qil_gemm_bf16_wide_takes(int M, int N, int K, int splits) { return wide_takes(M, N, K, splits); }
 
 // Splits of K with which a product of more than 256 rows should run here rather than in the GPU BLAS (1: a result of
-// A's type; more, where `may_split` allows float32 partial sums and there are no more columns than K, but 1,024 or more);
-// 0: the BLAS.  Fewer columns are not a stream's but factors that their consumer reads again and again (the 32 columns of a
-// state-space scan's B and C: left as partial sums of 4,096 rows of K, the scan's two passes over 2,048 rows took 96 and
-// 54 us, with a bfloat16 result 51 and 40).
-// What takes no more than WIDE_HOST_US by the count above stays here.  The GPU's times are level with the library's there (us
-// here against there at 643 rows, 0.6B sizes: q/k/v 12.4 / 11.9, attention output 10.3 / 10.7, down 12.1 / 13.9; 2,048 rows of
-// 2,048 x 2,048 21.0 / 21.6), but the host spends 21 us on a library product and 7 on one of ours, and steps of such
-// products wait for the host: prompts at 0.6B sizes, with the gated rule below, 530 rows 4.62 -> 2.69 ms, 1,000 rows
-// 4.59 -> 3.26, 1,400 rows 4.93 -> 4.23; 2,048 rows level.  Longer products are the library's inside a model even where this
-// kernel is ahead alone (4,096 x 12,288 in 4 splits, 643 rows: 78 us against 92 with cold operands, but 21 us a layer
-// behind in a prompt of 530 rows, whose norms then read the partial sums).
+// A's type; more, where `may_split` allows float32 partial sums, from 513 rows and 1,024 columns on, where there are no more
+// columns than K); 0: the BLAS.  Fewer columns are not a stream's but factors that their consumer reads again and again (the 32
+// columns of a state-space scan's B and C: left as partial sums of 4,096 rows of K, the scan's two passes over 2,048 rows took
+// 96 and 54 us, with a bfloat16 result 51 and 40).
+//
+// Beyond 512 rows, where steps are launched kernel by kernel, what takes no more than WIDE_HOST_US by the count above stays
+// here: the host spends 21 us on a library product and 7 on one of ours, and steps of such products wait for the host
+// (prompts at 0.6B sizes, with the gated rule below, 530 rows 4.62 -> 2.69 ms, 1,000 rows 4.59 -> 3.26, 1,400 rows 4.93 ->
+// 4.23; at 8B and 2,048-wide sizes level).  On the GPU that costs nothing to 8 us a product (us here against there, 513 / 1,000
+// rows: 4,096 x 1,024 12.5 / 13.8 against 13.3 / 13.7, 3,072 x 1,536 15.5 / 17.7 against 13.1 / 17.9, 2,048 x 2,048 18.6 / 19.5
+// against 12.7 / 15.5, 1,024 x 2,048 18.5 / 18.7 against 10.7 / 11.3; 2,048 rows of 2,048 x 2,048 21.0 against 21.6).
+//
+// Up to 512 rows a graph may replay the step, where the host's time is nothing, and a step and its replay have to run the
+// same kernels: there only products within WIDE_LEVEL_US of the library's time by its count (300 / 400 / 512 rows: 8,192 x
+// 1,024 12.4 / 13.4 / 14.5 against 13.7 / 14.3 / 14.6, 4,096 x 1,024 11.9 / 12.0 / 12.1 against 10.2 / 10.7 / 10.8 and the
+// library at 300; 5,120 x 2,048 19.8 / 22.5 against 21.3 / 23.2 at 400 / 512; the library's are 2,048 x 2,048 with 18.4 against 11.3, 1,024 x 1,024 with 11.2 against 8.7, 3,072 x 1,536 with 15.6
+// against 13.3, 5,120 x 2,048 with 19.9 against 16.4 at 300), and no partial sums (with the norm behind them 2,048 x 2,048
+// 19.3 against 15.1 at 400 rows, 1,024 x 1,024 13.2 against 12.3).
+//
+// Longer products are the library's inside a model even where this kernel is ahead alone (4,096 x 12,288 in 4 splits, 643
+// rows: 78 us against 92 with cold operands, but 21 us a layer behind in a prompt of 530 rows, whose norms then read the
+// partial sums).
 int qil_gemm_bf16_wide_splits(int M, int N, int K, int may_split) {
   int found = 0;
-  double best = WIDE_HOST_US;
-  for (int splits = 1; splits <= (may_split && K >= N && N >= WIDE_SPLIT_COLUMNS ? 8 : 1); ++splits) {
+  double best = 1e30;
+  for (int splits = 1; splits <= (may_split && M > WIDE_GRAPH_ROWS && K >= N && N >= WIDE_SPLIT_COLUMNS ? 8 : 1); ++splits) {
     if (!wide_takes(M, N, K, splits)) continue;
     const double us = wide_us(M, N, K, splits, wide_shape(M, N, K, splits));
-    if (us <= best) { best = us; found = splits; }
+    if (us <= best && wide_wanted(M, N, K, us, false)) { best = us; found = splits; }
   }
   return found;
 }
@@ -384,10 +408,11 @@ int qil_gemm_bf16_wide_gated_takes(int M, int inner, int K) { return inner >= 16
 
 // 1 if a gated product of more than 256 rows should run here: by the same rule, and two kernels become one (643 rows of
 // 6,144 x 1,024 18.5 us against 18.9 and 4.4 for the activation; 2,048 rows 30.7 against 27.4 and 9.6, but a prompt of
-// 2,048 rows 4.89 ms against 4.78, of 5,000 13.1 against 12.8).
+// 2,048 rows 4.89 ms against 4.78, of 5,000 13.1 against 12.8; up to 512 rows inner 3,072 x 1,024 13.2 against 19.0 with the
+// activation, 4,096 x 1,024 14.4 against 20.2, and the library's 1,024 x 2,048 with 19.6 against 13.9).
 int qil_gemm_bf16_wide_gated_wanted(int M, int inner, int K) {
   return M > 256 && qil_gemm_bf16_wide_gated_takes(M, inner, K) &&
-         wide_us(M, 2 * inner, K, 1, wide_shape(M, 2 * inner, K, 1)) <= WIDE_HOST_US;
+         wide_wanted(M, 2 * inner, K, wide_us(M, 2 * inner, K, 1, wide_shape(M, 2 * inner, K, 1)), true);
 }
 
 // out [M, inner] of out_dtype = silu(A gate^T) * (A up^T) for W [2 inner, K] with gate and up rows in turns of 16.

@@ -116,3 +116,15 @@ def test_a_products_rounds_are_those_of_the_fullest_xcd(lib):
     assert lib.qil_gemm_bf16_wide_splits(640, 6528, 1024, 0) == 1            # (short enough for two rounds)
     assert lib.qil_gemm_bf16_wide_splits(257, 10304, 2048, 0) == 0
     assert lib.qil_gemm_bf16_wide_splits(600, 6400, 2048, 0) == 0 and lib.qil_gemm_bf16_wide_splits(600, 6144, 2048, 0) == 1
+
+
+def test_products_of_steps_that_a_graph_may_replay(lib):
+    """Up to 512 rows only products that are level with the library's on the GPU: not few blocks with a long K, and no
+    partial sums.  From 513 rows on the host's time for a library product counts too."""
+    for rows in (257, 300, 400, 512):
+        for columns, k in ((2048, 2048), (1024, 2048), (1024, 1024), (3072, 1536), (2112, 2048)):
+            assert lib.qil_gemm_bf16_wide_splits(rows, columns, k, 1) == 0
+        assert lib.qil_gemm_bf16_wide_splits(rows, 8192, 1024, 1) == 1
+        assert lib.qil_gemm_bf16_wide_gated_wanted(rows, 3072, 1024) and not lib.qil_gemm_bf16_wide_gated_wanted(rows, 1024, 2048)
+    assert lib.qil_gemm_bf16_wide_splits(513, 2048, 2048, 0) == 1 and lib.qil_gemm_bf16_wide_splits(513, 1024, 1024, 1) > 1
+    assert lib.qil_gemm_bf16_wide_gated_wanted(513, 1024, 2048)
