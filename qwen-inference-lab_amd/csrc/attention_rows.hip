@@ -51,16 +51,18 @@ __device__ __forceinline__ float group_sum(float v, int log2) {
   return v;
 }
 
-template <typename T, int GT>
-__global__ void __launch_bounds__(ATT_THREADS)
+// GT: heads taken together.  RUNS: runs of 16 keys whose values a wave asks for at once (2 or 4).  KEYS: the waves share out
+// the values' keys and each takes all elements; else the elements, `share` (1 or 2) waves a run of 32 of them.
+template <typename T, int GT, int RUNS, bool KEYS>
+__global__ void __launch_bounds__(ATT_THREADS, GT <= 4 ? 4 : 2)
 attn_rows_partial_kernel(const T* __restrict__ q, int q_stride, const T* __restrict__ k_cache,
                          const T* __restrict__ v_cache, const int* __restrict__ block_tables, int table_stride,
                          const int* __restrict__ row_seq, const int* __restrict__ positions,
                          const int* __restrict__ row_index, float* __restrict__ part_acc,
                          float* __restrict__ part_m, float* __restrict__ part_l,
                          T* __restrict__ out, int heads, int kv_heads, int d, int page_size, int window,
-                         float scale, float softcap, int P, int parts, int tg_log2, const float* __restrict__ sinks,
-                         const float* __restrict__ slopes, int keep) {
+                         float scale, float softcap, int P, int parts, int tg_log2, int share,
+                         const float* __restrict__ sinks, const float* __restrict__ slopes, int keep) {
   extern __shared__ float lds[];
   const int slot_row = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;   // slot_row indexes the workspace
   const int row = row_index ? row_index[slot_row] : slot_row;             // row of the step's batch
@@ -169,12 +171,12 @@ attn_rows_partial_kernel(const T* __restrict__ q, int q_stride, const T* __restr
     // of a page side by side, so here a wave's lanes are 16 consecutive keys x 4 chunks of 8 elements (a load
     // instruction then reads whole 64-byte runs of 16 keys, not 16 bytes of 4 keys): 32 of the head's elements.  The
     // waves share out the elements, and where those are fewer than 32 a wave the keys too, so that a wave waits for
-    // memory once for four of its runs of keys (with the keys shared out and all elements one wave's, as it was, it
-    // waited once for every 32 elements: 14.9 -> 12.8 us at four rows of 512 float32 keys, 16 heads of 128 in 8 groups).
+    // memory once for RUNS of its runs of keys (with the keys shared out and all elements one wave's it waits once for
+    // every 32 elements: 14.9 -> 12.8 us at four rows of 512 float32 keys, 16 heads of 128 in 8 groups).
     const int v_key = lane & 15, v_e0 = (lane >> 4) * 8;
-    const int chunks = (d + 31) / 32, share = chunks >= ATT_WAVES ? 1 : ATT_WAVES / chunks;      // waves on one run of elements
-    const int turn = wave % share;
-    for (int c0 = wave / share * 32; c0 < d; c0 += ATT_WAVES / share * 32) {
+    if (KEYS) share = ATT_WAVES;
+    const int turn = wave & (share - 1), across = KEYS ? 1 : share == 1 ? ATT_WAVES : ATT_WAVES / 2;
+    for (int c0 = KEYS ? 0 : (share == 1 ? wave : wave / 2) * 32; c0 < d; c0 += across * 32) {
       const int ve = c0 + v_e0;
       const bool v_live = ve < d;
       float acc[GT][8];
@@ -182,12 +184,11 @@ attn_rows_partial_kernel(const T* __restrict__ q, int q_stride, const T* __restr
       for (int h = 0; h < GT; ++h)
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
-      constexpr int AT_ONCE = GT < 8 ? 4 : 2;                   // (eight heads' sums and four runs take 240 registers)
       const int v_stride = share * 16;
-      for (int t0 = turn * 16 + v_key; t0 < count; t0 += AT_ONCE * v_stride) {      // runs of keys at a time, their loads first
-        float vv[AT_ONCE][8];
+      for (int t0 = turn * 16 + v_key; t0 < count; t0 += RUNS * v_stride) {      // runs of keys at a time, their loads first
+        float vv[RUNS][8];
 #pragma unroll
-        for (int u = 0; u < AT_ONCE; ++u) {
+        for (int u = 0; u < RUNS; ++u) {
           const int j = span.key(begin + min(t0 + u * v_stride, count - 1));
           const size_t page = table[j / page_size];
           const T* column = v_cache + ((page * kv_heads + kvh) * (size_t)d + ve) * page_size + (j % page_size);
@@ -196,7 +197,7 @@ attn_rows_partial_kernel(const T* __restrict__ q, int q_stride, const T* __restr
           for (int e = 0; e < 8; ++e) vv[u][e] = seen ? ld(column + (size_t)e * page_size) : 0.f;
         }
 #pragma unroll
-        for (int u = 0; u < AT_ONCE; ++u) {
+        for (int u = 0; u < RUNS; ++u) {
           const int t = t0 + u * v_stride;
           if (t < count) {
 #pragma unroll
@@ -338,16 +339,27 @@ static int launch_rows(const void* q, int q_stride, const void* k_cache, const v
   const int tg_log2 = next_pow2_log2((d + 7) / 8);
   const size_t lds = rows_lds_floats(gt, P, d) * sizeof(float);
   dim3 grid(rows, kv_heads, parts);
-#define QIL_ROWS_CASE(GT)                                                                                          \
-  hipLaunchKernelGGL((attn_rows_partial_kernel<T, GT>), grid, dim3(ATT_THREADS), lds, s, (const T*)q, q_stride,    \
+  // Which of the values' elements and keys are shared out.  Heads of up to 32 elements have nothing but keys to share; those
+  // of 3, 5, 6 or 7 runs of elements leave waves without one in the last turn, and parts long enough to be bound by the
+  // keys' bytes and not by the wait for them share out the keys alone (64 rows of 2,000 keys, 10 heads of 160 in 2, 194 us
+  // by elements, 180 by keys; 12 of 80 in 4, 100 and 96).
+  const int chunks = (d + 31) / 32, share = chunks == 2 ? 2 : 1;
+  const bool keys = chunks == 1 || (chunks > 2 && chunks % 4 && P >= 256);
+  // Four runs of values at once where a wave of the longest part has more than two.  With four heads and more they would take
+  // over 128 registers, three blocks a CU instead of four, and a second round of the usual 1,024 blocks (64 rows of 2,000
+  // keys, 32 heads of 128 in 8 groups, 276 us with four and 225 with two; 16 of 64 in 4, 93 and 66).  With one run or two a
+  // wave the others only repeat the last key (one row of 300 keys, 16 heads of 64 in 16 groups, 10.3 and 9.5).
+  const bool four = !keys && gt < 4 && P > 2 * 16 * share;
+#define QIL_ROWS_CASE(GT, RUNS, KEYS)                                                                               \
+  hipLaunchKernelGGL((attn_rows_partial_kernel<T, GT, RUNS, KEYS>), grid, dim3(ATT_THREADS), lds, s, (const T*)q, q_stride,    \
                      (const T*)k_cache, (const T*)v_cache, block_tables, table_stride, row_seq, positions,         \
                      row_index, part_acc, part_m, part_l, (T*)out, heads, kv_heads, d, page_size, window, scale, softcap, P, parts,    \
-                     tg_log2, sinks, slopes, keep)
+                     tg_log2, share, sinks, slopes, keep)
   switch (gt) {
-    case 1: QIL_ROWS_CASE(1); break;
-    case 2: QIL_ROWS_CASE(2); break;
-    case 4: QIL_ROWS_CASE(4); break;
-    default: QIL_ROWS_CASE(8); break;
+    case 1: if (four) QIL_ROWS_CASE(1, 4, false); else if (keys) QIL_ROWS_CASE(1, 2, true); else QIL_ROWS_CASE(1, 2, false); break;
+    case 2: if (four) QIL_ROWS_CASE(2, 4, false); else if (keys) QIL_ROWS_CASE(2, 2, true); else QIL_ROWS_CASE(2, 2, false); break;
+    case 4: if (keys) QIL_ROWS_CASE(4, 2, true); else QIL_ROWS_CASE(4, 2, false); break;
+    default: if (keys) QIL_ROWS_CASE(8, 2, true); else QIL_ROWS_CASE(8, 2, false); break;
   }
 #undef QIL_ROWS_CASE
   int status = (int)hipGetLastError();

@@ -90,6 +90,24 @@ def test_rows_attention_shares_out_the_values(ops, monkeypatch, d, heads, kv_hea
         torch.testing.assert_close(got.double(), want.double(), atol=1e-5, rtol=1e-5)
 
 
+# long parts, whose head sizes decide whether the waves share out elements or keys, and how many runs of keys they ask for
+@pytest.mark.parametrize('d', [32, 64, 80, 128, 160, 192])
+@pytest.mark.parametrize('heads,kv_heads', [(2, 2), (4, 2), (8, 2), (16, 2)])
+def test_rows_attention_with_long_parts(ops, monkeypatch, d, heads, kv_heads):
+    """Parts of 512 keys, one of a key and one that is not whole.  Float32 rows against float64 as above, over 1,300 keys."""
+    monkeypatch.setattr(ops, 'ATTENTION_PART', 512)
+    lengths, page_size = [1, 513, 1300, 512], 16
+    k_cache, v_cache, table, _ = build_cache(lengths, page_size, kv_heads, d, torch.float32)
+    positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32).cuda()
+    q = rand(len(lengths), heads * d, seed=6)
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=page_size, block_tables=table, scale=d ** -0.5,
+                row_seq=torch.arange(len(lengths), dtype=torch.int32).cuda(), positions=positions, max_context=max(lengths),
+                window=None, cu_seqlens=None, seq_starts=None, single_rows=None, n_seqs=len(lengths), max_query=1)
+    got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    want = refs.paged_attention(q.double(), k_cache=k_cache.double(), v_cache=v_cache.double(), accumulate=torch.float64, **step)
+    torch.testing.assert_close(got.double(), want.double(), atol=1e-5, rtol=1e-5)
+
+
 # widths the four-element kernel takes and does not, a gate that starts between its loads, an input that is not aligned
 @pytest.mark.parametrize('columns,offset,width,shift', [(1024, 4, 1028, 0), (4, 0, 4, 0), (1024, 2, 1028, 0), (30, 4, 64, 0), (64, 4, 70, 0),
                                                         (64, 4, 68, 1)])
