@@ -185,9 +185,11 @@ __global__ void channel_conv_vec_kernel(const TI* __restrict__ x, int splits, si
 // Long sequences of bfloat16 rows: CONV_ROWS consecutive rows a thread (8 channels), whose inputs and the TAPS - 1 before
 // them are asked for at once and read once; so are the factors.  A thread of the kernel above reads TAPS rows and 32
 // bytes of factors a tap for 16 bytes of results.  A sequence's first rows, which need its state, are computed as above
-// by the thread that meets the first of them.  2,048 rows of 6,144 channels, silu, 27.8 -> 21.4 us: the vector instructions of
-// the silu's exponential and quotient are what is left (looking a run of rows' sequence up once instead of row by row
-// changed nothing).
+// in blocks of the sequence's own behind those of the rows: in the rows' blocks, by the thread that met the first of them,
+// short sequences were a chain of states in a few threads (1,024 rows and 31 sequences of one, 6,144 channels: 23.5 us, 18.8
+// in the kernel above, 12.8 so; at 2,048 channels 19.1, 9.4 and 10.6).  2,048 rows of 6,144 channels, silu, 26.9 -> 22.8 us,
+// 513 rows 11.2 -> 11.0: the vector instructions of the silu's exponential and quotient are what is left (looking a run of
+// rows' sequence up once instead of row by row changed nothing).
 #define CONV_ROWS 8
 template <int TAPS>
 __global__ void __launch_bounds__(128)
@@ -197,6 +199,18 @@ channel_conv_rows_kernel(const bf16_t* __restrict__ x, int x_columns, const floa
                          int channels, int act, int pass_from, int passed, bf16_t* __restrict__ passed_out) {
   constexpr int V = 8, KEEP = TAPS - 1;
   const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V, n0 = blockIdx.x * CONV_ROWS;
+  if (n0 >= n) {                                       // behind the rows' blocks: a sequence's first rows and its state
+    const int s = blockIdx.x - (n + CONV_ROWS - 1) / CONV_ROWS, row0 = cu_seqlens[s], rows = cu_seqlens[s + 1] - row0, start = seq_starts[s];
+    if (c >= channels || rows < 1) return;
+    float b[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) b[e] = 0.f;
+    if (bias) load_floats<V>(bias + c, b);
+    float* held = state + (size_t)seq_slots[s] * KEEP * channels;
+    conv_outputs<bf16_t, bf16_t, V>(x, 1, 0, x_columns, w, b, held, start, row0, 0, min(rows, KEEP), out, c, channels, TAPS, act);
+    conv_keep<bf16_t, V>(x, 1, 0, x_columns, held, start, row0, rows, c, channels, KEEP);
+    return;
+  }
   uint4 in[KEEP + CONV_ROWS];                          // the rows n0 - KEEP .. n0 + CONV_ROWS - 1
   if (c >= channels) {
     const int i = c - channels;
@@ -239,11 +253,6 @@ channel_conv_rows_kernel(const bf16_t* __restrict__ x, int x_columns, const floa
         for (int e = 0; e < V; ++e) acc[e] = silu_f(acc[e]);
       }
       store_floats<V>(out + (size_t)row * channels + c, acc);
-    } else if (t == 0) {
-      const int rows = cu_seqlens[s + 1] - row0, start = seq_starts[s];
-      float* held = state + (size_t)seq_slots[s] * KEEP * channels;
-      conv_outputs<bf16_t, bf16_t, V>(x, 1, 0, x_columns, w, b, held, start, row0, 0, min(rows, KEEP), out, c, channels, TAPS, act);
-      conv_keep<bf16_t, V>(x, 1, 0, x_columns, held, start, row0, rows, c, channels, KEEP);
     }
   }
 }
@@ -476,7 +485,7 @@ int qil_channel_conv(const void* x, int x_code, int x_splits, int x_columns, con
     const int threads = lanes >= 128 ? 128 : (lanes + 63) / 64 * 64;
     // enough rows that a thread can have several, in sequences long enough that few of them need the state
     if (x_code == QIL_BF16 && taps == 4 && n > 512 && n / 32 >= n_seqs) {
-      hipLaunchKernelGGL(channel_conv_rows_kernel<4>, dim3((n + CONV_ROWS - 1) / CONV_ROWS, (lanes + threads - 1) / threads),
+      hipLaunchKernelGGL(channel_conv_rows_kernel<4>, dim3((n + CONV_ROWS - 1) / CONV_ROWS + n_seqs, (lanes + threads - 1) / threads),
                          dim3(threads), 0, s, (const bf16_t*)x, x_columns, w, bias, state, cu_seqlens, seq_starts, seq_slots,
                          row_seq, (bf16_t*)out, n, channels, act, pass_from, passed, (bf16_t*)passed_out);
       QIL_RETURN_LAUNCH_STATUS();
