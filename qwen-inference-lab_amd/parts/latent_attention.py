@@ -15,8 +15,9 @@ class LatentAttention(Mixer):
                          that has no key and no value; it only enlarges the denominator)
         out_i          = W_o concat_h(W_uv,h sum_j p(h, i, j) c_j)
 
-    Keys and values are never expanded: the query is multiplied by W_uk,h^T once (``ops.latent_query``), the
-    attention kernel works on the cached rows themselves, and W_uv,h is applied to the weighted sum of latents.
+    Behind cached rows keys and values are not expanded: the query is multiplied by W_uk,h^T once (``ops.latent_query``),
+    the attention kernel works on the cached rows themselves, and W_uv,h is applied to the weighted sum of latents.  Steps
+    of whole prompts that ``ops.expands_latents`` takes multiply their own latents out instead (``ops.latent_expanded``).
     ``position``: a ``RotaryFrequencies`` over ``rot_dim`` elements.
     ``window`` w: row i sees the keys j with 0 <= i - j < w only, and the cache gives pages back that no later row
     sees (None: every key j <= i).
@@ -99,9 +100,14 @@ class LatentAttention(Mixer):
         p['down.weight'] = self.w_down
         # W_uk as [heads, dim, kv_rank] is the layout the query's product reads (a pure view); W_uv per head transposed
         self.k_up = p['k_up.weight'].view(self.heads, self.dim, self.kv_rank)
-        self.v_rows = p['v_up.weight']                  # as stored: whole prompts expand their values with it
+        # W_uv as stored too, where whole prompts may expand their values with it: a second copy that no other layer keeps
+        self.v_rows = p['v_up.weight'] if self._may_expand(p['v_up.weight'].device) else None
         p['v_up.weight'] = p['v_up.weight'].view(self.heads, self.vdim, self.kv_rank).transpose(1, 2).contiguous()
         self.position.frequencies()                     # made here, not in a step that may be captured
+
+    def _may_expand(self, device):
+        return self.window is None and self.gate != 'element' and device.type == 'cuda' and \
+            ops.expands_latents(ops.EXPAND_FEWEST_ROWS, dim=self.dim, rot=self.rot_dim, vdim=self.vdim, dtype=self.dtype)
 
     def forward(self, h, ctx, cache):
         p = self.p
@@ -109,7 +115,7 @@ class LatentAttention(Mixer):
         down = ops.linear(h, self.w_down, None, partials=True)
         own = down if self.gate != 'element' else ops.columns(down, 0, self.own_rows)
         # whole prompts: their rows are all the keys there are, and attention over expanded keys and values costs a third
-        expands = ctx.fresh and cache.writes and self.window is None and self.gate != 'element' and down.device.type == 'cuda' and \
+        expands = self.v_rows is not None and ctx.fresh and cache.writes and \
             ops.expands_latents(h.shape[0], dim=self.dim, rot=self.rot_dim, vdim=self.vdim, dtype=self.dtype)
         copies = {}
         if expands:

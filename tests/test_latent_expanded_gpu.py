@@ -87,3 +87,16 @@ def test_the_engine_takes_whole_prompts_to_it(ops, monkeypatch):
     assert all(torch.equal(used(a)[:411], used(b)[:411]) for a, b in zip(caches, plain_caches))
     for a, b in ((first, plain_first), (second, plain_second)):
         assert (a - b).norm() < 0.02 * b.norm()
+
+
+@pytest.mark.parametrize('change,kept', [({}, True), (dict(gate='head'), True), (dict(dtype=torch.float32), False), (dict(window=64), False),
+                                         (dict(gate='element'), False), (dict(dim=64), False), (dict(rot_dim=32), False), (dict(vdim=64), False)])
+def test_only_layers_that_may_expand_keep_the_value_weight_twice(ops, change, kept):
+    from qil_amd.parts.latent_attention import LatentAttention
+    from qil_amd.parts.rotary import RotaryFrequencies
+    sizes = dict(width=256, heads=4, dim=128, rot_dim=64, vdim=128, kv_rank=128, q_rank=96, scale=192 ** -0.5, eps=1e-5,
+                 dtype=torch.bfloat16) | change
+    layer = LatentAttention(position=RotaryFrequencies(rot_dim=sizes['rot_dim'], base=10000.0, device='cuda'), **sizes)
+    layer.p = {name: torch.zeros(spec.shape, dtype=sizes['dtype'], device='cuda') for name, spec in layer.param_specs().items()}
+    layer.finalize()
+    assert (layer.v_rows is not None) == kept
