@@ -210,9 +210,14 @@ int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* square
 // the whole-line kernel (gemm_bf16.hip), which can split K only into partial sums, is a block of 128 columns on each of few
 // CUs.  us there and here, 8 rows: 3,072 x 1,536 10.0 / 6.1, 6,144 x 2,048 13.2 / 7.9, 12,288 x 2,048 16.5 / 10.9, 16,384 x
 // 2,048 16.7 / 13.4, 32,768 x 2,048 22.9 / 23.2, 4,096 x 4,096 22.3 / 8.7, 2,048 x 6,144 70 / 10.7, 1,536 x 512 5.0 / 6.1.
+// A K of an odd number of stages cannot be split over waves, and with no more groups of columns than CUs the plan then has
+// fewer waves than that kernel's: 4,096 x 1,152 8.1 / 10.1, 1,024 x 3,200 17.6 / 22.4, 16 rows of 2,048 x 6,272 36.6 / 52.4;
+// with more groups it is ahead (4,112 x 1,152 8.1 / 4.8), and so for up to 8 rows where K is too long for the whole-line
+// kernel (1,024 x 4,480 50.7 / 30.5).
 int qil_gemm_bf16_whole_takes(int M, int N, int K) {
   int groups, ksplit;
-  return N <= 16384 && K >= 1024 && add_plan(M, N, K, &groups, &ksplit);
+  if (N > 16384 || K < 1024 || !add_plan(M, N, K, &groups, &ksplit)) return 0;
+  return ksplit > 1 || N > 16 * QIL_CUS || (M <= 8 && K > 4224);
 }
 
 // out bfloat16 [M, N] = A[M, K] W[N, K]^T, K split over a block's waves.

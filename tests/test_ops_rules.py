@@ -128,3 +128,15 @@ def test_products_of_steps_that_a_graph_may_replay(lib):
         assert lib.qil_gemm_bf16_wide_gated_wanted(rows, 3072, 1024) and not lib.qil_gemm_bf16_wide_gated_wanted(rows, 1024, 2048)
     assert lib.qil_gemm_bf16_wide_splits(513, 2048, 2048, 0) == 1 and lib.qil_gemm_bf16_wide_splits(513, 1024, 1024, 1) > 1
     assert lib.qil_gemm_bf16_wide_gated_wanted(513, 1024, 2048)
+
+
+def test_whole_products_of_few_rows_that_cannot_split_k(lib):
+    """A K of an odd number of stages of 128 runs with K split over the waves only where the columns alone fill the chip, or
+    where the other kernel does not take it (up to 8 rows and more than 33 stages)."""
+    for rows in (1, 8, 16):
+        for columns in (32, 1024, 4096):
+            for k in (1152, 1408, 3200, 4224):
+                assert not lib.qil_gemm_bf16_whole_takes(rows, columns, k)
+            assert lib.qil_gemm_bf16_whole_takes(rows, columns, 1280) and lib.qil_gemm_bf16_whole_takes(rows, columns, 2304)
+            assert lib.qil_gemm_bf16_whole_takes(rows, columns, 4480) == (rows <= 8)
+        assert lib.qil_gemm_bf16_whole_takes(rows, 4112, 1152) and lib.qil_gemm_bf16_whole_takes(rows, 12288, 4480)
