@@ -74,8 +74,8 @@ __device__ __forceinline__ uint4 shuffle4(uint4 v, int source) {
                     __shfl(v.w, source, QIL_WAVE));
 }
 
-// WHOLE: d == DMAX (always so when FUSED).
-template <int DMAX, bool FUSED, bool WHOLE = FUSED>
+// WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
+template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false>
 __global__ void __launch_bounds__(DEC_MAX_WAVES * QIL_WAVE)
 attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_cache,
                    const bf16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int table_stride,
@@ -376,23 +376,43 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
   // entries are looked up a step ahead of the loads that need them.
   constexpr bool EARLY = FUSED;
   int step = first_step + wave;
-  int page[3];
-  StepData here;
-  if (step <= last_step) {
-    look_up(step, page);
-    request(step, page, here);
-    if (EARLY) look_up(step + waves, page);                  // (clamped: any entry will do where there is no such step)
-  }
-  make_queries();
-  if (step <= last_step)
-    for (;;) {
-      attend(step, here);
-      step += waves;
-      if (step > last_step) break;
-      if (!EARLY) look_up(step, page);
-      request(step, page, here);
-      if (EARLY) look_up(step + waves, page);
+  if constexpr (PAIRS) {
+    // both steps' table entries, then both steps' keys and values, then the arithmetic
+    int page_a[3], page_b[3];
+    StepData a, b;
+    auto load_pair = [&]() __attribute__((always_inline)) {
+      look_up(step, page_a);
+      if (step + waves <= last_step) look_up(step + waves, page_b);
+      request(step, page_a, a);
+      if (step + waves <= last_step) request(step + waves, page_b, b);
+    };
+    if (step <= last_step) load_pair();
+    make_queries();
+    while (step <= last_step) {
+      attend(step, a);
+      if (step + waves <= last_step) attend(step + waves, b);
+      step += 2 * waves;
+      if (step <= last_step) load_pair();
     }
+  } else {
+    int page[3];
+    StepData here;
+    if (step <= last_step) {
+      look_up(step, page);
+      request(step, page, here);
+      if (EARLY) look_up(step + waves, page);                // (clamped: any entry will do where there is no such step)
+    }
+    make_queries();
+    if (step <= last_step)
+      for (;;) {
+        attend(step, here);
+        step += waves;
+        if (step > last_step) break;
+        if (!EARLY) look_up(step, page);
+        request(step, page, here);
+        if (EARLY) look_up(step + waves, page);
+      }
+  }
 
   // ---- the waves' (m, l, O) meet in LDS: [wave][head < g][d + 2]
   l += __shfl_xor(l, 16, QIL_WAVE);
@@ -521,18 +541,26 @@ extern "C" int qil_attn_decode(const void* q, int q_stride, const void* k_cache,
   const dim3 grid = plan ? dim3(blocks, kv_heads) : dim3(rows, kv_heads, parts);
   int* part_keys = plan ? reinterpret_cast<int*>(l + (size_t)rows * heads * parts) : nullptr;
   const FusedQKV none = {};
-#define QIL_DEC_LAUNCH(DMAX, FUSED, WHOLE, FIELDS)                                                                 \
-  hipLaunchKernelGGL((attn_decode_kernel<DMAX, FUSED, WHOLE>), grid, dim3(waves * QIL_WAVE), lds, s, FIELDS,        \
+  // Two of a wave's steps in flight (twice the registers) in launches of at most a block a CU: heads of fewer than 128 elements
+  // that do not fill their fragments wherever a wave has a second step, heads of 64 from four steps a wave on.  us with one
+  // step / with two: 64 rows of 300 keys, 8 heads of 96 in 4, 12.0 / 10.9, 32 rows of 2,000 keys, 8 heads of 32, 26.5 / 23.4,
+  // 16 heads of 64 in 8 groups 30.8 / 29.2, but 16 rows of 1,000 keys 12.9 / 13.4; heads of 128 48.6 / 53.
+  const bool pairs = (plan ? (long)blocks : (long)rows * parts) * kv_heads <= QIL_CUS && d < 128 &&
+                     (plan || (d == 64 ? P >= 128 * waves : P > 32 * waves));
+#define QIL_DEC_LAUNCH(DMAX, FUSED, WHOLE, PAIRS, FIELDS)                                                          \
+  hipLaunchKernelGGL((attn_decode_kernel<DMAX, FUSED, WHOLE, PAIRS>), grid, dim3(waves * QIL_WAVE), lds, s, FIELDS,        \
                      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,       \
                      table_stride, row_seq, positions, row_index, acc, m, l, (bf16_t*)out, heads, kv_heads, d,        \
                      page_size, window, scale, P, parts, softcap, sinks, slopes, keep, plan, part_keys)
-#define QIL_DEC_CASE(DMAX)                                \
-  if (d == DMAX) QIL_DEC_LAUNCH(DMAX, false, true, none); \
-  else QIL_DEC_LAUNCH(DMAX, false, false, none)
-  if (d <= 64) QIL_DEC_CASE(64);
-  else if (d <= 128) QIL_DEC_CASE(128);
-  else QIL_DEC_CASE(256);
-#undef QIL_DEC_CASE
+  if (d == 64 && pairs) QIL_DEC_LAUNCH(64, false, true, true, none);
+  else if (d == 64) QIL_DEC_LAUNCH(64, false, true, false, none);
+  else if (d < 64 && pairs) QIL_DEC_LAUNCH(64, false, false, true, none);
+  else if (d < 64) QIL_DEC_LAUNCH(64, false, false, false, none);
+  else if (d == 128) QIL_DEC_LAUNCH(128, false, true, false, none);
+  else if (d < 128 && pairs) QIL_DEC_LAUNCH(128, false, false, true, none);
+  else if (d < 128) QIL_DEC_LAUNCH(128, false, false, false, none);
+  else if (d == 256) QIL_DEC_LAUNCH(256, false, true, false, none);
+  else QIL_DEC_LAUNCH(256, false, false, false, none);
   QIL_RETURN_LAUNCH_STATUS();
 }
 
@@ -593,8 +621,8 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
-  if (d == 64) QIL_DEC_LAUNCH(64, true, true, fused);
-  else QIL_DEC_LAUNCH(128, true, true, fused);
+  if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused);
+  else QIL_DEC_LAUNCH(128, true, true, false, fused);
 #undef QIL_DEC_LAUNCH
   QIL_RETURN_LAUNCH_STATUS();
 }

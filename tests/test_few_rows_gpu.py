@@ -175,3 +175,22 @@ def test_products_of_views_at_odd_offsets(ops, m, shifted):
         gated = ops.gated_linear(x, w, interleaved=True)
         torch.testing.assert_close(gated.double(), torch.nn.functional.silu(gate) * up,
                                    atol=2.0 ** -7 * want.abs().max().item(), rtol=2.0 ** -6)
+
+
+@pytest.mark.parametrize('d,heads,kv_heads', [(32, 8, 8), (48, 8, 4), (64, 16, 8), (80, 16, 4), (96, 8, 4)])
+@pytest.mark.parametrize('lengths,window', [([320], None), ([2049, 1, 33, 545, 1024, 1056, 1300, 2017] * 2, None), ([700, 289, 5, 2000] * 6, 256)])
+def test_decode_attention_with_two_steps_in_flight(ops, d, heads, kv_heads, lengths, window):
+    """Launches of at most a block a CU whose waves have several steps of 32 keys, an even and an odd number of them, none for
+    some waves: against the float32 reference, one rounding to bfloat16 and its neighbour (2^-7), values of size one."""
+    lengths = lengths * (256 // kv_heads) if len(lengths) == 1 else lengths
+    dtype, rows, page_size = torch.bfloat16, len(lengths), 16
+    k_cache, v_cache, table, _ = build_cache(lengths, page_size, kv_heads, d, dtype)
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, k_cache=k_cache, v_cache=v_cache, page_size=page_size, block_tables=table,
+                row_seq=torch.arange(rows, dtype=torch.int32).cuda(), positions=torch.tensor([n - 1 for n in lengths], dtype=torch.int32).cuda(),
+                cu_seqlens=None, seq_starts=None, single_rows=None, n_seqs=rows, max_query=1, max_context=max(lengths), scale=d ** -0.5,
+                window=window)
+    part, parts = ops._decode_parts(rows, kv_heads, ops._places(max(lengths), window, 0))
+    assert rows * kv_heads * parts <= 256 and part > 32 * ops.DECODE_WAVES
+    q = rand(rows, heads * d, dtype=dtype, seed=5)
+    got = ops.paged_attention(q, **step)
+    torch.testing.assert_close(got.float(), refs.paged_attention(q, **step).float(), atol=2.0 ** -8, rtol=2.0 ** -7)
