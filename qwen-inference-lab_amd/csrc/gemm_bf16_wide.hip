@@ -73,6 +73,7 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   constexpr int LOADS = A_LOADS + W_LOADS;                 // a wave's loads a stage: those of A, then those of W
   constexpr int RING = AHEAD + 3;
   static_assert(LOADS % 2 == 0 && ROWS % (16 * WAVES) == 0 && TILE % (16 * WAVES) == 0, "whole loads, half of them in each half of a stage");
+  static_assert(CT >= 2 && LOADS % 2 == 0 && 2 * ((LOADS / 2 + RT - 1) / RT) <= CT, "a load and a read a product at most");
   extern __shared__ __align__(1024) unsigned char ring[];  // a stage: the block's rows of A, then those of W, 64 bytes each
   const int lane = threadIdx.x & (QIL_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
@@ -152,19 +153,16 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
     const int other = ks ^ 1;
     const unsigned char* at = ring + read_slot * SLOT + read_at[other];
     const int first = doubles * i / RT, loads = 2 * (doubles * (i + 1) / RT - first);
-    const int w_first = CT * i / RT, w_reads = CT * (i + 1) / RT - w_first;
-    // a product, and before it one of the reads (two where a wave has one tile of columns) and its share of the loads:
-    // the order is the one written here
+    const int w_first = CT * i / RT, w_reads = CT * (i + 1) / RT - w_first;      // at most CT loads, at most CT - 1 reads of W
+    // a product, and before it one of the reads and one of the loads: the order is the one written here
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
-      constexpr int BEHIND = CT == 1 ? 0 : 1;                // the reads of W begin behind the first product's of A
       if (j == 0) af[other][i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + a_rows + i * 2048));
-      if (j >= BEHIND && j - BEHIND < w_reads)
-        wf[other][w_first + j - BEHIND] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + w_rows + (w_first + j - BEHIND) * 2048));
-#pragma unroll
-      for (int l = loads <= CT ? j : loads * j / CT; l < (loads <= CT ? min(j + 1, loads) : loads * (j + 1) / CT); ++l) {
-        const int stage = pair_stage + (l & 1);
-        load(begin + first + l / 2, min(stage, last), stage % RING);
+      if (j >= 1 && j <= w_reads)
+        wf[other][w_first + j - 1] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(at + w_rows + (w_first + j - 1) * 2048));
+      if (j < loads) {
+        const int stage = pair_stage + (j & 1);
+        load(begin + first + j / 2, min(stage, last), stage % RING);
       }
       acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
@@ -359,6 +357,9 @@ extern "C" {
 
 // 1 if qil_gemm_bf16_wide takes these sizes.
 int qil_gemm_bf16_wide_takes(int M, int N, int K, int splits) { return wide_takes(M, N, K, splits); }
+
+// The block's shape there (0: 256 x 256, 1: 128 x 128, 2: 128 x 128 with the long ring); a gated product has 2 * inner columns.
+int qil_gemm_bf16_wide_shape(int M, int N, int K, int splits) { return wide_takes(M, N, K, splits) ? wide_shape(M, N, K, splits) : -1; }
 
 // Splits of K with which a product of more than 256 rows should run here rather than in the GPU BLAS (1: a result of
 // A's type; more, where `may_split` allows float32 partial sums, from 513 rows and 1,024 columns on, where there are no more

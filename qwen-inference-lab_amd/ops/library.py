@@ -288,6 +288,8 @@ def _declare(lib):
     lib.qil_gemm_bf16_mid_gated.argtypes = [p, p, p, i, i, i, i, p]
     lib.qil_gemm_bf16_wide_takes.argtypes = [i, i, i, i]
     lib.qil_gemm_bf16_wide_takes.restype = i
+    lib.qil_gemm_bf16_wide_shape.argtypes = [i, i, i, i]
+    lib.qil_gemm_bf16_wide_shape.restype = i
     lib.qil_gemm_bf16_wide_splits.argtypes = [i, i, i, i]
     lib.qil_gemm_bf16_wide_splits.restype = i
     lib.qil_gemm_bf16_wide_gated_wanted.argtypes = [i, i, i]

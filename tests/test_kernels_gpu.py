@@ -489,8 +489,8 @@ def test_large_products_without_the_gpu_blas(ops, monkeypatch, m, n, k, bias):
 @pytest.mark.parametrize('m,n,k', [(2048, 4096, 4096), (2048, 6144, 1024), (300, 96, 192), (257, 1056, 448), (1000, 4128, 1024),
                                    (33, 64, 128), (513, 160, 448), (129, 288, 320), (1, 32, 128)])
 def test_products_in_blocks_of_256_columns(ops, m, n, k):
-    """The kernel for products of many rows alone, through its C interface: blocks of 256 and of 128 rows (the first two
-    sizes: one of each), rows, columns and stages that fill no block, tile or ring; bfloat16 and float32 results
+    """The kernel for products of many rows alone, through its C interface: blocks of 128 x 128 (with two splits of the
+    first size of 256 x 256), rows, columns and stages that fill no block, tile or ring; bfloat16 and float32 results
     against float64; partial sums of 2 splits of K, which add up to the float32 result; the same bits every time."""
     lib = ops.library.load()
     x = rand(m, k, dtype=torch.bfloat16)
@@ -526,7 +526,7 @@ def test_products_in_blocks_of_256_columns(ops, m, n, k):
 def test_gated_products_in_blocks_of_256_columns(ops, monkeypatch, m, inner, k, dtype):
     """The same kernel with the gate's epilogue (gate and up rows in turns of 16, silu(gate) * up written once), alone
     and through ``gated_linear`` under ``OWN_LARGE_PRODUCTS``, where neither torch.mm nor the activation kernel runs;
-    both block shapes, results in bfloat16 and float32, against float64."""
+    blocks of 128 x 128, results in bfloat16 and float32, against float64."""
     lib = ops.library.load()
     x = rand(m, k, dtype=torch.bfloat16)
     stacked = rand(2 * inner, k, dtype=torch.bfloat16, seed=1, scale=2.0 * k ** -0.5)
