@@ -363,12 +363,6 @@ def _ptr(tensor):
     return None if tensor is None else tensor.data_ptr()
 
 
-def _whole_pieces(*tensors):
-    """Whether the tensors begin at multiples of 16 bytes: what a kernel that reads 16 bytes at a time needs (a contiguous
-    view may begin anywhere)."""
-    return all(t.data_ptr() % 16 == 0 for t in tensors)
-
-
 def _check(status, name):
     if status:
         raise RuntimeError(f'{name}: HIP kernel launch failed (status {status})'
@@ -677,10 +671,13 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
             _check(lib.qil_gemm_bf16(_ptr(x), _ptr(weight), None, _ptr(out), n, o, k, 0, splits, 0, 0, _stream()),
                    'gemm_bf16')
             return Partials(out)
-    if streams and n <= STREAM_GEMM_MAX_ROWS and bias is None and out_dtype == x.dtype and \
-            lib.qil_gemm_bf16_whole_takes(n, o, k) and _whole_pieces(x, weight):
+    # kernels that read 16 bytes at a time need operands at such addresses (a contiguous view may begin anywhere)
+    at_x, at_weight = x.data_ptr(), weight.data_ptr()
+    whole_pieces = not (at_x | at_weight) & 15
+    if streams and n <= STREAM_GEMM_MAX_ROWS and bias is None and out_dtype == x.dtype and whole_pieces and \
+            lib.qil_gemm_bf16_whole_takes(n, o, k):
         out = torch.empty((n, o), dtype=x.dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_whole(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _stream()), 'gemm_bf16_whole')
+        _check(lib.qil_gemm_bf16_whole(at_x, at_weight, _ptr(out), n, o, k, _stream()), 'gemm_bf16_whole')
         return out
     if out_dtype == torch.float32 or streams:
         out = torch.empty((n, o), dtype=out_dtype, device=x.device)
@@ -689,10 +686,10 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
         return out
     # beyond 256 rows: the products that the library is no faster at (the kernel's file says which)
     splits = lib.qil_gemm_bf16_wide_splits(n, o, k, int(partials and bias is None)) \
-        if n > MID_GEMM_MOST_ROWS and out_dtype == x.dtype and not OWN_LARGE_PRODUCTS and _whole_pieces(x, weight) else 0
+        if n > MID_GEMM_MOST_ROWS and out_dtype == x.dtype and not OWN_LARGE_PRODUCTS and whole_pieces else 0
     if splits:
         out = torch.empty((splits, n, o), dtype=torch.float32 if splits > 1 else x.dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_wide(_ptr(x), _ptr(weight), _ptr(out), n, o, k, _code(out.dtype), splits, _stream()),
+        _check(lib.qil_gemm_bf16_wide(at_x, at_weight, _ptr(out), n, o, k, _code(out.dtype), splits, _stream()),
                'gemm_bf16_wide')
         if splits > 1:
             return Partials(out)
@@ -763,11 +760,12 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
         _check(lib.qil_gemm_bf16_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), 0, 0,
                                        int(interleaved), _stream()), 'gemm_bf16_gated')
         return out
+    at_x, at_weight = x.data_ptr(), weight.data_ptr()
     if x.dtype == torch.bfloat16 and interleaved and \
             ((OWN_LARGE_PRODUCTS and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k)) or
-             (lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k) and _whole_pieces(x, weight))):
+             (not (at_x | at_weight) & 15 and lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k))):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_wide_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
+        _check(lib.qil_gemm_bf16_wide_gated(at_x, at_weight, _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
                'gemm_bf16_wide_gated')
         return out
     sums = linear(x, weight, None, partials=True)
