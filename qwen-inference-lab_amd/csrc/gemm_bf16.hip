@@ -718,13 +718,15 @@ static bool gated_plan(const void* A, const void* W, int M, int inner, int K, in
     if (K % (128 * c) == 0 && K / (128 * c) >= (c == 1 || (long)(inner / 16) * c <= 8 * QIL_CUS ? 2 : 16)) ks = c;
   if (!ks) return false;
   // Pairs that are fewer than the CUs: a CU each, and waves that have four stages where K is long enough (3,072 x 1,024: 192
-  // blocks of two waves instead of 96 of eight, a step of 28 layers 1,056 -> 1,024 us for one row, 1,443 -> 1,415 for eight).
+  // blocks of two waves instead of 96 of eight, part of 1,098 -> 1,053 us for a step of 28 layers and one row; 8 rows of 4,096 x
+  // 768 7.8 -> 6.2 us, 3,072 x 768 7.6 -> 6.0).  With many stages both shapes fill the CUs alike, also where the products are
+  // large enough for the count below: 4,096 x 6,144 20.8 us (21.1 by that count), 4,096 x 7,168 23.6 (24.1).
   if (inner / 16 <= QIL_CUS && gated_lds(M, K, 8) <= 156 * 1024) {
     *pairs = 1;
     *ksplit = 1;
     for (int c = 2; c <= 8; c *= 2)
       if (K % (128 * c) == 0 && K / (128 * c) >= 4) *ksplit = c;
-    return K / (128 * *ksplit) >= 2;
+    return true;
   }
   // Pairs a block: what a CU has to do in all (its blocks one after the other, as many at a time as LDS and
   // the 12 wave slots allow) over how well its waves keep memory busy (8 or more do).  Ties go to more pairs.
