@@ -48,9 +48,9 @@ __global__ void add_norm_kernel(float* __restrict__ stream, const TD* __restrict
   }
 }
 
-// The same with the row in registers (width % 4 == 0, at most 4 * J * THREADS, 16-byte aligned operands): 16-byte accesses,
-// all of them asked for before the first is used, one pass over memory where the kernel above makes three of 4 bytes a
-// lane.  Bound by memory with many rows and by the waits for it with few (3,044 rows of 2,048 in bfloat16
+// The same with the row in registers (width % 4 == 0, at most 4 * J * THREADS, 16-byte aligned operands): 16-byte accesses
+// and one pass over memory where the kernel above makes three of 4 bytes a lane; what is added waits for its own loads, partial
+// sums four at a time (operand_at4).  Bound by memory with many rows and by the waits for it with few (3,044 rows of 2,048 in bfloat16
 // 27 -> 17 us, 8 rows with four partial sums 9.5 -> 4.1).
 template <typename TD, typename T, int CENTRE, int THREADS, int J>
 __global__ void __launch_bounds__(THREADS)

@@ -725,8 +725,8 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
     before the up rows, or (``interleaved``) both in turns of 16 rows, which the kernels read faster.
 
     One kernel when a fused kernel takes the sizes (bfloat16; up to 16 rows, or up to 256 rows of an interleaved
-    matrix large enough to fill the chip, or from 512 rows on under ``OWN_LARGE_PRODUCTS``); otherwise the product
-    followed by ``silu_mul``.  Both add in float32.
+    matrix large enough to fill the chip, or more rows of one whose product is short (``qil_gemm_bf16_wide_gated_wanted``),
+    or from 512 rows on under ``OWN_LARGE_PRODUCTS``); otherwise the product followed by ``silu_mul``.  Both add in float32.
     ``lazy``: a few float32 rows may come back as ``Gated`` (the product's partial sums) for ``linear`` to finish."""
     if isinstance(x, Normed):
         x = x.materialize()
@@ -929,7 +929,10 @@ def _decode_parts(rows, kv_heads, max_context):
 # Fewest keys of a planned part: a step of 32 for each of a block's eight waves.
 PLAN_MIN_PART = 256
 # Rows that a plan is made for at most, and blocks that it shares out (all kv heads together: one a CU; two or three a CU
-# with half the keys each are slower, a block's start and end are some 6 us).
+# with half the keys each are slower, a block's start and end are some 6 us).  A plan is made where a row has two blocks: with
+# more rows rows of one length lose by it (8 kv heads, us of a layer cut by the longest row and planned: 17 rows of 2,000 keys
+# 37.8 / 41.4, 24 41.6 / 44.0, 32 45.6 / 48.2, 12 and 16 rows level), though rows of different lengths would gain up to 28 of
+# them (1,000 to 4,000 keys: 17 rows 63.9 / 43.8, 24 66.9 / 67.7, 32 72.5 / 75.0; 100 to 8,000: 24 rows 124 / 105, 32 130 / 135).
 PLAN_MOST_ROWS, PLAN_BLOCKS = 128, 256
 # Fewest keys (rows times the longest context) of a planned step: below, the plan's own 3 us are more than idle CUs cost
 # (a step of 450 us with two such layers lost 1 %); six rows of 4,096 to 16,384 keys at 12 layers of 8B sizes 2.09 -> 1.80 ms,
