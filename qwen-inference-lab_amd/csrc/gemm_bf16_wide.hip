@@ -370,7 +370,7 @@ int qil_gemm_bf16_wide_shape(int M, int N, int K, int splits) { return wide_take
 // Beyond 512 rows, where steps are launched kernel by kernel, what takes no more than WIDE_HOST_US by the count above stays
 // here: the host spends 21 us on a library product and 7 on one of ours, and steps of such products wait for the host
 // (prompts at 0.6B sizes, with the gated rule below, 530 rows 4.62 -> 2.69 ms, 1,000 rows 4.59 -> 3.26, 1,400 rows 4.93 ->
-// 4.23; at 8B and 2,048-wide sizes level).  On the GPU that costs nothing to 8 us a product (us here against there, 513 / 1,000
+// 4.23, 2,048 rows, which the host does not hold up any more, 4.98 -> 5.04; at 8B and 2,048-wide sizes level).  On the GPU that costs nothing to 8 us a product (us here against there, 513 / 1,000
 // rows: 4,096 x 1,024 12.5 / 13.8 against 13.3 / 13.7, 3,072 x 1,536 15.5 / 17.7 against 13.1 / 17.9, 2,048 x 2,048 18.6 / 19.5
 // against 12.7 / 15.5, 1,024 x 2,048 18.5 / 18.7 against 10.7 / 11.3; 2,048 rows of 2,048 x 2,048 21.0 against 21.6).
 //
@@ -408,7 +408,7 @@ int qil_gemm_bf16_wide(const void* A, const void* W, void* C, int M, int N, int 
 int qil_gemm_bf16_wide_gated_takes(int M, int inner, int K) { return inner >= 16 && inner % 16 == 0 && wide_takes(M, 2 * inner, K, 1); }
 
 // 1 if a gated product of more than 256 rows should run here: by the same rule, and two kernels become one (643 rows of
-// 6,144 x 1,024 18.5 us against 18.9 and 4.4 for the activation; 2,048 rows 30.7 against 27.4 and 9.6, but a prompt of
+// 6,144 x 1,024 18.5 us, inside a prompt 22, against 18.9 and 4.4 for the activation; 2,048 rows 30.7 against 27.4 and 9.6, but a prompt of
 // 2,048 rows 4.89 ms against 4.78, of 5,000 13.1 against 12.8; up to 512 rows inner 3,072 x 1,024 13.2 against 19.0 with the
 // activation, 4,096 x 1,024 14.4 against 20.2, and the library's 1,024 x 2,048 with 19.6 against 13.9).
 int qil_gemm_bf16_wide_gated_wanted(int M, int inner, int K) {
