@@ -86,30 +86,6 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
   const int low = window > 0 ? pos - window + 1 : 0;        // the column's oldest visible key (<= 0: from the start)
   const size_t gcol = (size_t)grow * heads + head;
 
-  bf16x8 qb[QF];
-  {
-    const float* qrow = q + gcol * d;
-    const bool wide = d % 4 == 0;                           // rows start on 16 bytes: two 16-byte reads a fragment
-#pragma unroll
-    for (int f = 0; f < QF; ++f) {
-      float x[8];
-      const int dim0 = 32 * f + 8 * kb;
-      if (wide && valid && f < qf && dim0 + 8 <= d) {
-        const float4 a = *reinterpret_cast<const float4*>(qrow + dim0), b = *reinterpret_cast<const float4*>(qrow + dim0 + 4);
-        x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = (valid && f < qf && dim0 + e < d) ? qrow[dim0 + e] : 0.f;
-      }
-      qb[f] = __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]),
-                                                    pack_bf16(x[6], x[7])));
-    }
-  }
-  float m = -INFINITY, l = 0.f;
-  if (parts == 1 && sink && valid) {                       // the sink: maximum s_h, sum 1 (held once a column), result 0
-    m = sink[head];
-    l = kb == 0 ? 1.f : 0.f;
-  }
   f32x4 o[VTW];
 #pragma unroll
   for (int t = 0; t < VTW; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -124,30 +100,92 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
   constexpr int NU = (QF * 4 + CSTEP - 1) / CSTEP;
   const int chunks = dp / 8, jp = tid % (LM_KEYS / 2), c0 = tid / (LM_KEYS / 2);
   uint4 ahead[NU][2];
-  int place[2];                                             // the cache slots of keys 2 jp, 2 jp + 1 of a step; -1: none
+  int place[2];                                             // the cache slots of keys 2 jp, 2 jp + 1 of a step
+  // Keys behind the block's last one stand in as that last key (their scores are masked), so that neither the look-ups
+  // nor the rows' loads are under a condition; dims behind the row (other sizes than the template's) are read from its
+  // start and made zero.
   auto lookup = [&](int j0) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const int key = j0 + 2 * jp + e;
-      place[e] = key < end ? table[key / page_size] * page_size + key % page_size : -1;
+      const int key = min(j0 + 2 * jp + e, end - 1);
+      place[e] = table[key / page_size] * page_size + key % page_size;
     }
   };
   auto fetch = [&]() {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-      const int chunk = c0 + CSTEP * u, dim = chunk * 8;
+      const int chunk = c0 + CSTEP * u, dim = chunk * 8, from = dim < d ? dim : 0;
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (chunk < chunks && place[e] >= 0 && dim < d)
-          v = dim < rank ? *reinterpret_cast<const uint4*>(latent + (size_t)place[e] * rank + dim)
-                         : *reinterpret_cast<const uint4*>(rope + (size_t)place[e] * rot + (dim - rank));
-        ahead[u][e] = v;
+        const bf16_t* row = from < rank ? latent + (size_t)place[e] * rank + from : rope + (size_t)place[e] * rot + (from - rank);
+        ahead[u][e] = *reinterpret_cast<const uint4*>(row);
       }
+    }
+    if constexpr (!EXACT) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+        if ((c0 + CSTEP * u) * 8 >= d) ahead[u][0] = ahead[u][1] = make_uint4(0, 0, 0, 0);
     }
   };
   lookup(begin);
-  fetch();
+  // The queries, eight dims a fragment (rank and rot are multiples of 8, so a fragment lies inside the row or behind it),
+  // asked for behind the first keys' places and ahead of the keys, none of them under a condition: columns without a row
+  // read their block's first one, fragments behind the row its first dims, and a mask makes both zero.  Under conditions
+  // every fragment's two loads waited for those before them, 18 round trips to memory one after the other (8 rows of
+  // 2,048 keys: 20.3 us; now 13.2).  Where all waves hold the same columns they bring a quarter each and exchange them in
+  // the keys' place in LDS, which leaves the registers to the keys in flight.
+  bf16x8 qb[QF];
+  if constexpr (SPLIT) {
+    constexpr int NQ = QF / 2;                              // 16 columns of 32 QF dims, four a thread and turn
+    const int quads = dp / 4;
+    const float* rows_q = q + ((size_t)(seq_row0 + r0) * heads + h0) * d;      // the columns' rows lie side by side
+    float4 x[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      const int item = tid + LM_THREADS * u, c = item / quads, dim = 4 * (item - c * quads);
+      x[u] = *reinterpret_cast<const float4*>(rows_q + (c < heads_here && dim < d ? c * d + dim : 0));
+    }
+    fetch();
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      const int item = tid + LM_THREADS * u, c = item / quads, dim = 4 * (item - c * quads);
+      const uint32_t mask = c < heads_here && dim < d ? ~0u : 0u;
+      if (EXACT || c < 16)
+        *reinterpret_cast<uint2*>(ks + c * krow + dim) =
+            make_uint2(pack_bf16(x[u].x, x[u].y) & mask, pack_bf16(x[u].z, x[u].w) & mask);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < QF; ++f)
+      qb[f] = *reinterpret_cast<const bf16x8*>(ks + r * krow + (EXACT || f < qf ? 32 * f : 0) + 8 * kb);
+  } else {
+    const float* qrow = q + gcol * d;
+    constexpr int G = QF % 6 == 0 ? 6 : 4;                  // fragments in flight: all of them would spill
+#pragma unroll
+    for (int f0 = 0; f0 < QF; f0 += G) {
+      float4 x[G][2];
+#pragma unroll
+      for (int f = 0; f < G; ++f) {
+        const float* src = qrow + (EXACT || 32 * (f0 + f) + 8 * kb < d ? 32 * (f0 + f) + 8 * kb : 0);
+        x[f][0] = *reinterpret_cast<const float4*>(src);
+        x[f][1] = *reinterpret_cast<const float4*>(src + 4);
+      }
+#pragma unroll
+      for (int f = 0; f < G; ++f) {
+        const uint32_t mask = valid && (EXACT || 32 * (f0 + f) + 8 * kb < d) ? ~0u : 0u;
+        const float4 a = x[f][0], b = x[f][1];
+        qb[f0 + f] = __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(a.x, a.y) & mask, pack_bf16(a.z, a.w) & mask,
+                                                           pack_bf16(b.x, b.y) & mask, pack_bf16(b.z, b.w) & mask));
+        asm volatile("" : "+v"(qb[f0 + f]));                // made here, ahead of the next loads
+      }
+    }
+    fetch();
+  }
+  float m = -INFINITY, l = 0.f;
+  if (parts == 1 && sink && valid) {                       // the sink: maximum s_h, sum 1 (held once a column), result 0
+    m = sink[head];
+    l = kb == 0 ? 1.f : 0.f;
+  }
   lookup(begin + LM_KEYS);
   for (int j0 = begin; j0 < end; j0 += LM_KEYS) {
     __syncthreads();                                        // the last step's reads are done
@@ -279,19 +317,34 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
 }
 
 // out[column] = sum_p w_p acc_p / (sum_p w_p l_p + exp(sink - M)), w_p = exp(m_p - M), M the largest of the parts'
-// references and the sink, over the parts that the row's position reaches.  One block per (row, head); the parts'
-// weights are made once, side by side, and kept in LDS (`parts` floats of dynamic LDS), so that the sums below wait
-// for no value that another read has to bring first.
-__global__ void latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_m,
-                                    const float* __restrict__ part_l, const int* __restrict__ positions,
-                                    const float* __restrict__ sink, const float* __restrict__ gate,
-                                    float* __restrict__ out, int heads, int rank, int P, int parts, int window) {
-  extern __shared__ float weight[];
+// references and the sink, over the parts that the row's position reaches.  One block per (row, head): a thread holds four
+// neighbouring elements of every Gth part (G = threads / (rank / 4)) and asks for the first LMM_AHEAD of them before the
+// parts' weights are made, none under a condition (a place behind the last part reads that part with weight zero); the G
+// groups' sums meet in LDS.  Dynamic LDS: [parts] weights, then 4 floats a thread.
+// What bounds it is its waits: with one element and four parts in flight a thread, 8 rows of 16 heads of 33 parts of 512
+// elements (8.7 MB) took 9.6 us; now 5.5.
+#define LMM_AHEAD 8
+__global__ void __launch_bounds__(512)
+latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_m, const float* __restrict__ part_l,
+                    const int* __restrict__ positions, const float* __restrict__ sink, const float* __restrict__ gate,
+                    float* __restrict__ out, int heads, int rank, int P, int parts, int window) {
+  extern __shared__ __align__(16) float merge_lds[];
   __shared__ float scratch[16];
   const int n = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
+  float4* sums = reinterpret_cast<float4*>(merge_lds);      // [groups][rank / 4]
+  float* weight = merge_lds + 4 * nt;
   const size_t column = (size_t)n * heads + h;
-  const int reached = min(parts, positions[n] / P + 1);
-  const int from = window > 0 ? max(0, positions[n] - window + 1) / P : 0;     // the part of the row's oldest visible key
+  const int position = positions[n];
+  const int reached = min(parts, position / P + 1);
+  const int from = window > 0 ? max(0, position - window + 1) / P : 0;     // the part of the row's oldest visible key
+  const int quads = rank / 4, groups = nt / quads, group = tid / quads, quad = tid - group * quads;
+  const float* acc_p = part_acc + column * parts * rank + 4 * quad;
+  float4 ahead[LMM_AHEAD];
+  auto fetch = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < LMM_AHEAD; ++u) ahead[u] = ld4(acc_p + (size_t)min(p0 + groups * u, reached - 1) * rank);
+  };
+  fetch(from + group);
   const float floor_ = sink ? sink[h] : -INFINITY;
   float top = floor_;
   for (int p = from + tid; p < reached; p += nt) {
@@ -308,12 +361,24 @@ __global__ void latent_merge_kernel(const float* __restrict__ part_acc, const fl
   }
   below = block_sum(below, scratch);                        // its barriers also publish the weights
   const float inv = (gate ? gate[column] : 1.f) / below;
-  const float* acc_p = part_acc + column * parts * rank;
-  for (int c = tid; c < rank; c += nt) {
-    float acc = 0.f;
-#pragma unroll 4
-    for (int p = from; p < reached; ++p) acc += weight[p] * acc_p[(size_t)p * rank + c];
-    out[column * rank + c] = acc * inv;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int p0 = from + group; p0 < reached; p0 += groups * LMM_AHEAD) {
+    if (p0 != from + group) fetch(p0);
+#pragma unroll
+    for (int u = 0; u < LMM_AHEAD; ++u) {
+      const int p = p0 + groups * u;
+      const float w = p < reached ? weight[p] : 0.f;
+      acc.x += w * ahead[u].x; acc.y += w * ahead[u].y; acc.z += w * ahead[u].z; acc.w += w * ahead[u].w;
+    }
+  }
+  if (group < groups) sums[tid] = acc;
+  __syncthreads();
+  if (tid < quads) {
+    for (int g = 1; g < groups; ++g) {
+      const float4 v = sums[g * quads + tid];
+      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+    }
+    st4(out + column * rank + 4 * tid, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
   }
 }
 
@@ -405,9 +470,13 @@ int qil_latent_mfma(const float* q, const void* latent, const void* rope, const 
 #undef QIL_LM
 #undef QIL_LM_ARGS
   if (status) return status;
-  if (parts > 1)
-    hipLaunchKernelGGL(latent_merge_kernel, dim3(n_rows, heads), dim3(rank >= 256 ? 256 : 64), parts * sizeof(float), s, part_acc, part_m,
-                       part_l, positions, sink, gate, out, heads, rank, P, parts, window);
+  if (parts > 1) {
+    // parts in turns of as many threads as hold them all in LMM_AHEAD loads each, as far as 512 threads go
+    const int want = rank / 4 * ((parts + LMM_AHEAD - 1) / LMM_AHEAD);
+    const int threads = want >= 512 ? 512 : want <= 128 ? 128 : (want + 63) / 64 * 64;
+    hipLaunchKernelGGL(latent_merge_kernel, dim3(n_rows, heads), dim3(threads), (parts + 4 * threads) * sizeof(float), s,
+                       part_acc, part_m, part_l, positions, sink, gate, out, heads, rank, P, parts, window);
+  }
   QIL_RETURN_LAUNCH_STATUS();
 }
 
