@@ -79,6 +79,48 @@ __global__ void latent_prepare_kernel(const TD* __restrict__ x, int splits, size
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// Element i and i + half of a vector turned by `position`.
+template <typename TX>
+__device__ __forceinline__ void turn_tail(const TX* __restrict__ src, float* __restrict__ dst, int i, int half, float freq,
+                                          float position) {
+  const float u = ld(src + i), v = ld(src + half + i);
+  float sn, cs;
+  sincosf(position * freq, &sn, &cs);
+  dst[i] = u * cs - v * sn;
+  dst[half + i] = v * cs + u * sn;
+}
+
+// What the product per head turns beside its own work: `rot` elements of every head's input from `offset` on (0: none).
+struct RotatedTail {
+  const float* freq;
+  const int* positions;
+  int offset, rot;
+};
+
+// Eight elements in flight as they lie in memory.
+template <typename T> struct Eight;
+template <> struct Eight<bf16_t> {
+  uint4 raw;
+  __device__ __forceinline__ void load(const bf16_t* p) { raw = *reinterpret_cast<const uint4*>(p); }
+  __device__ __forceinline__ void get(float* out) const {
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out[2 * i] = __uint_as_float(w[i] << 16);
+      out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+  }
+};
+template <> struct Eight<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) { a = ld4(p); b = ld4(p + 4); }
+  __device__ __forceinline__ void get(float* out) const {
+    out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
+    out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
+  }
+};
+
+// ---------------------------------------------------------------------------------------------------------------
 // A product per head: out[n, h, o] = sum_k W[h, k, o] x[n, h, k]   (W "k-major": the outputs of one k side by side).
 // With a gate (an operand of rows of g_row elements) the result is multiplied by sigmoid(gate[n, h * o_dim + o]).
 // x: row stride x_row, head stride x_head (elements); out likewise.  A block takes ROWS rows of one head and 256
@@ -113,60 +155,102 @@ __global__ void head_product_kernel(const TX* __restrict__ x, int x_row, int x_h
     }
 }
 
-// The same product for few rows (decoding): the weights of a head are then read by too few blocks for the chip, so a
-// block takes 8 rows, OT * 8 outputs (OT = 8, or 4 where that still leaves few blocks) and splits k 256 / OT ways: a
-// thread reads 8 consecutive outputs of every (256 / OT)th k (16 bytes of bfloat16), and the partial sums meet by
-// shuffles in a wave and through LDS between the four waves.  Takes o_dim % 8 == 0 and w aligned to 8 elements.
+// The same product for few rows: the weights of a head are then read by too few blocks for the chip, so a block takes 8
+// rows and OT * 8 outputs and splits k 256 / OT ways: a thread reads 8 consecutive outputs of every (256 / OT)th k (16 bytes
+// of bfloat16).  Takes o_dim % 8 == 0 and w aligned to 8 elements.
+// What bounds it is the chain of its waits, so the first HP_AHEAD weights of a thread and all of its part of x are asked
+// for before anything is waited for, none under a condition (rows behind the last one read the last one: what they give is
+// not written), and the partial sums of a wave meet by exchanging halves (a step leaves half as many sums a lane: 60
+// shuffles for 64 sums over 16 lanes, 256 if every lane kept them all), then through LDS between the four waves.
+// 8 rows of 16 heads: 512 x 128 a head 13.8 us -> 6.6, 128 x 512 and the turned parts (a kernel of their own
+// before) 8.8 + 3.9 -> 6.0; up to 255 rows it beats the plain kernel above, whose reads of W wait one by one (64 rows 32.9 and
+// 11.9 us, here 7.8 and 7.7; 255 rows 34.3 and 22.8, here 12.8 and 20.2), and from 256 rows on bfloat16 is the GPU BLAS's.
+// With `tail` the last blocks of grid.z turn the heads' rotated parts (see rotate_tail_kernel) instead.
+#define HP_AHEAD 8
+#define HP_FEW_ROWS 255
 template <typename TX, typename TW, typename TO, int OT>
 __global__ void __launch_bounds__(256)
 head_product_few_kernel(const TX* __restrict__ x, int x_row, int x_head, const TW* __restrict__ w, TO* __restrict__ out,
-                        int out_row, int out_head, int n_rows, int k_dim, int o_dim, Operand gate, int g_row) {
+                        int out_row, int out_head, int n_rows, int k_dim, int o_dim, Operand gate, int g_row, int x_wide,
+                        RotatedTail tail) {
   constexpr int OB = OT * 8, KG = 256 / OT;           // outputs a block, k groups
-  extern __shared__ float xs[];                       // [8][k_dim], then [4 waves][8 rows][OB outputs]
-  float* sums = xs + 8 * k_dim;
+  extern __shared__ __align__(16) float xs[];         // [8][k_dim], then [4 waves][8 rows][OB outputs]
   const int row0 = blockIdx.x * 8, h = blockIdx.y, tid = threadIdx.x, to = tid % OT, kg = tid / OT;
-  const int o0 = blockIdx.z * OB + to * 8;
+  const int rows = min(8, n_rows - row0);
+  if constexpr (sizeof(TO) == 4) {
+    if (blockIdx.z * OB >= o_dim) {                   // turns the tails of this head's rows
+      const int half = tail.rot / 2;
+      for (int idx = tid; idx < rows * half; idx += 256) {
+        const int r = idx / half, i = idx - r * half;
+        turn_tail(x + (size_t)(row0 + r) * x_row + (size_t)h * x_head + tail.offset,
+                  out + (size_t)(row0 + r) * out_row + (size_t)h * out_head + o_dim, i, half, tail.freq[i],
+                  (float)tail.positions[row0 + r]);
+      }
+      return;
+    }
+  }
+  float* sums = xs + 8 * k_dim;
+  const int o0 = min((int)blockIdx.z * OB + to * 8, o_dim - 8);
+  const TW* wh = w + (size_t)h * k_dim * o_dim + o0;
+  Eight<TW> ahead[HP_AHEAD];
+#pragma unroll
+  for (int i = 0; i < HP_AHEAD; ++i) ahead[i].load(wh + (size_t)min(kg + KG * i, k_dim - 1) * o_dim);
+  // x into LDS: 32 threads a row
+  const int xr = tid >> 5, x_lane = tid & 31;
+  const TX* from = x + (size_t)min(row0 + xr, n_rows - 1) * x_row + (size_t)h * x_head;
+  if (x_wide) {
 #pragma unroll 4
-  for (int idx = tid; idx < 8 * k_dim; idx += 256) {
-    const int r = idx / k_dim, k = idx - r * k_dim;
-    xs[idx] = row0 + r < n_rows ? ld(x + (size_t)(row0 + r) * x_row + (size_t)h * x_head + k) : 0.f;
+    for (int k = 4 * x_lane; k < k_dim; k += 128) st4(xs + xr * k_dim + k, ld4(from + k));
+  } else {
+#pragma unroll 4
+    for (int k = x_lane; k < k_dim; k += 32) xs[xr * k_dim + k] = ld(from + k);
   }
   __syncthreads();
-  float acc[8][8] = {};
-  if (o0 < o_dim) {
-    const TW* wh = w + (size_t)h * k_dim * o_dim + o0;
-#pragma unroll 4                                      // four weight reads on their way at a time
-    for (int k = kg; k < k_dim; k += KG) {
+  float acc[64] = {};                                  // [row][output]
+  for (int k0 = 0; k0 < k_dim; k0 += KG * HP_AHEAD) {
+    if (k0 > 0)
+#pragma unroll
+      for (int i = 0; i < HP_AHEAD; ++i) ahead[i].load(wh + (size_t)min(k0 + kg + KG * i, k_dim - 1) * o_dim);
+#pragma unroll
+    for (int i = 0; i < HP_AHEAD; ++i) {
+      const int k = k0 + kg + KG * i;
+      if (k0 + KG * i >= k_dim) break;                 // the same for all threads
       float wv[8];
-      ld8(wh + (size_t)k * o_dim, wv);
+      ahead[i].get(wv);
+      if (k < k_dim) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const float xv = xs[r * k_dim + k];
+        for (int r = 0; r < 8; ++r) {
+          const float xv = xs[r * k_dim + k];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[r][j] += xv * wv[j];
+          for (int j = 0; j < 8; ++j) acc[r * 8 + j] += xv * wv[j];
+        }
       }
     }
   }
+  // the wave's 64 / OT lanes of a `to`: a step hands half of the sums over, lane bit set: the upper half stays
+  const int lane = tid & 63;
+  int first = 0;                                       // of the 64 sums: the first of those that this lane still holds
 #pragma unroll
-  for (int r = 0; r < 8; ++r)
+  for (int step = OT, held = 64; step < QIL_WAVE; step *= 2, held /= 2) {
+    const bool upper = lane & step;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = acc[r][j];
-#pragma unroll
-      for (int step = OT; step < QIL_WAVE; step *= 2) v += __shfl_xor(v, step, QIL_WAVE);
-      acc[r][j] = v;
+    for (int i = 0; i < held / 2; ++i) {
+      const float give = upper ? acc[i] : acc[i + held / 2], keep = upper ? acc[i + held / 2] : acc[i];
+      acc[i] = keep + __shfl_xor(give, step, QIL_WAVE);
     }
+    if (upper) first += held / 2;
+  }
+  constexpr int LEFT = 64 * OT / QIL_WAVE;
   const int wave = tid >> 6;
-  if ((tid & 63) < OT) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sums[(wave * 8 + r) * OB + to * 8 + j] = acc[r][j];
+  for (int i = 0; i < LEFT; ++i) {
+    const int sum = first + i;
+    sums[(wave * 8 + (sum >> 3)) * OB + to * 8 + (sum & 7)] = acc[i];
   }
   __syncthreads();
   for (int idx = tid; idx < 8 * OB; idx += 256) {
     const int r = idx / OB, j = idx % OB, o = blockIdx.z * OB + j;
-    if (row0 + r < n_rows && o < o_dim) {
+    if (r < rows && o < o_dim) {
       float v = sums[r * OB + j] + sums[(8 + r) * OB + j] + sums[(16 + r) * OB + j] + sums[(24 + r) * OB + j];
       if (gate.data) v /= 1.f + expf(-operand_at(gate, (size_t)(row0 + r) * g_row + (size_t)h * o_dim + o));
       st(out + (size_t)(row0 + r) * out_row + (size_t)h * out_head + o, v);
@@ -200,16 +284,9 @@ __global__ void rotate_tail_kernel(const TX* __restrict__ q, int q_row, int q_he
                                    const int* __restrict__ positions, float* __restrict__ out, int out_row, int out_head,
                                    int out_offset, int rot) {
   const int n = blockIdx.x, h = blockIdx.y, half = rot / 2;
-  const float p = (float)positions[n];
   const TX* src = q + (size_t)n * q_row + (size_t)h * q_head + offset;
   float* dst = out + (size_t)n * out_row + (size_t)h * out_head + out_offset;
-  for (int i = threadIdx.x; i < half; i += blockDim.x) {
-    const float u = ld(src + i), v = ld(src + half + i);
-    float sn, cs;
-    sincosf(p * freq[i], &sn, &cs);
-    dst[i] = u * cs - v * sn;
-    dst[half + i] = v * cs + u * sn;
-  }
+  for (int i = threadIdx.x; i < half; i += blockDim.x) turn_tail(src, dst, i, half, freq[i], (float)positions[n]);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -361,11 +438,17 @@ int qil_latent_prepare(const void* x, int x_dtype, int splits, int x_row, const 
 
 // out[n, h, o] = sum_k w[h, k, o] x[n, h, k]; x_dtype / w_dtype / out_dtype element codes; strides in elements.
 // Combinations: all float32; x bfloat16, w bfloat16, out float32; x float32, w bfloat16, out bfloat16.
+// tail_rot > 0 (out float32): the tail_rot elements of every head's input from tail_offset on are turned by the row's position
+// and follow the o_dim results of the head in out.
 int qil_head_product(const void* x, int x_dtype, int x_row, int x_head, const void* w, int w_dtype, void* out,
                      int out_dtype, int out_row, int out_head, int n, int heads, int k_dim, int o_dim, const void* gate,
-                     int gate_code, int gate_splits, int gate_row, hipStream_t s) {
+                     int gate_code, int gate_splits, int gate_row, const float* tail_freq, const int* positions, int tail_offset,
+                     int tail_rot, hipStream_t s) {
   if (n == 0 || heads == 0 || o_dim == 0) return 0;
   if (k_dim < 1 || (gate && (gate_splits < 1 || (gate_code == QIL_BF16 && gate_splits != 1) || gate_row < heads * o_dim)))
+    return -1;
+  if (tail_rot < 0 || tail_rot % 2 || (tail_rot > 0 && (out_dtype != QIL_F32 || !tail_freq || !positions || tail_offset < 0 ||
+                                                        tail_offset + tail_rot > x_head || o_dim + tail_rot > out_head)))
     return -1;
   const Operand g{gate, gate_code, gate_splits, (size_t)n * gate_row};
   const int rows = 8;
@@ -373,22 +456,33 @@ int qil_head_product(const void* x, int x_dtype, int x_row, int x_head, const vo
   if (lds > 64 * 1024) return -1;
   const int threads = o_dim >= 256 ? 256 : (o_dim + 63) / 64 * 64;
   dim3 grid((n + rows - 1) / rows, heads, (o_dim + threads - 1) / threads);
-  const size_t w_bytes = w_dtype == QIL_F32 ? 4 : 2;
-  const bool few = n <= 32 && o_dim % 8 == 0 && (size_t)w % (8 * w_bytes) == 0 && lds + 4 * 8 * 64 * sizeof(float) <= 64 * 1024;
-  const dim3 grid_few((n + 7) / 8, heads, (o_dim + 63) / 64);
+  const size_t w_bytes = w_dtype == QIL_F32 ? 4 : 2, x_bytes = x_dtype == QIL_F32 ? 4 : 2;
+  const bool few = n <= HP_FEW_ROWS && o_dim % 8 == 0 && (size_t)w % (8 * w_bytes) == 0 &&
+                   lds + 4 * 8 * 64 * sizeof(float) <= 64 * 1024;
+  const int wide = k_dim % 4 == 0 && x_row % 4 == 0 && x_head % 4 == 0 && (size_t)x % (4 * x_bytes) == 0;
+  const RotatedTail tail{tail_freq, positions, tail_offset, tail_rot};
+  const int more = tail_rot > 0 ? 1 : 0;
+  dim3 grid_few((n + 7) / 8, heads, (o_dim + 63) / 64);
   const bool narrow = grid_few.x * grid_few.y * grid_few.z < 128;      // few blocks: 32 outputs a block, k split 64 ways
-  const dim3 grid_narrow((n + 7) / 8, heads, (o_dim + 31) / 32);
+  dim3 grid_narrow((n + 7) / 8, heads, (o_dim + 31) / 32);
+  grid_few.z += more;
+  grid_narrow.z += more;
 #define QIL_HP(TX, TW, TO)                                                                                            \
   do {                                                                                                                  \
     if (few && narrow)                                                                                                  \
       hipLaunchKernelGGL((head_product_few_kernel<TX, TW, TO, 4>), grid_narrow, dim3(256), lds + 4 * 8 * 32 * sizeof(float), s, \
-                         (const TX*)x, x_row, x_head, (const TW*)w, (TO*)out, out_row, out_head, n, k_dim, o_dim, g, gate_row);       \
+                         (const TX*)x, x_row, x_head, (const TW*)w, (TO*)out, out_row, out_head, n, k_dim, o_dim, g, gate_row,        \
+                         wide, tail);                                                                                   \
     else if (few)                                                                                                       \
       hipLaunchKernelGGL((head_product_few_kernel<TX, TW, TO, 8>), grid_few, dim3(256), lds + 4 * 8 * 64 * sizeof(float), s, \
-                         (const TX*)x, x_row, x_head, (const TW*)w, (TO*)out, out_row, out_head, n, k_dim, o_dim, g, gate_row);       \
+                         (const TX*)x, x_row, x_head, (const TW*)w, (TO*)out, out_row, out_head, n, k_dim, o_dim, g, gate_row,        \
+                         wide, tail);                                                                                   \
     else                                                                                                                \
       hipLaunchKernelGGL((head_product_kernel<TX, TW, TO, 8>), grid, dim3(threads), lds, s, (const TX*)x, x_row, x_head, \
                          (const TW*)w, (TO*)out, out_row, out_head, n, k_dim, o_dim, g, gate_row);                                    \
+    if (!few && more)                                                                                                   \
+      hipLaunchKernelGGL(rotate_tail_kernel<TX>, dim3(n, heads), dim3(64), 0, s, (const TX*)x, x_row, x_head, tail_offset, \
+                         tail_freq, positions, (float*)out, out_row, out_head, o_dim, tail_rot);                        \
   } while (0)
   if (x_dtype == QIL_F32 && w_dtype == QIL_F32 && out_dtype == QIL_F32) QIL_HP(float, float, float);
   else if (x_dtype == QIL_BF16 && w_dtype == QIL_BF16 && out_dtype == QIL_F32) QIL_HP(bf16_t, bf16_t, float);

@@ -1483,7 +1483,7 @@ def head_product(x, weight, *, heads, out_dtype, out=None, out_columns=None, gat
         return out
     _check(library.load().qil_head_product(_ptr(x), _code(x.dtype), x.shape[1], x.shape[1] // heads, _ptr(weight),
                                            _code(weight.dtype), _ptr(out), _code(out_dtype), heads * out_columns,
-                                           out_columns, n, heads, k, o, *gate_operand, _stream()), 'head_product')
+                                           out_columns, n, heads, k, o, *gate_operand, None, None, 0, 0, _stream()), 'head_product')
     return out
 
 
@@ -1497,10 +1497,16 @@ def latent_query(q, k_up, *, heads, dim, rot, rank, frequencies, positions):
     _require(frequencies, 'frequencies', torch.float32, (rot // 2,))
     _require(positions, 'positions', torch.int32, (n,))
     out = torch.empty((n, heads * (rank + rot)), dtype=torch.float32, device=q.device)
-    head_product(q, k_up, heads=heads, out_dtype=torch.float32, out=out, out_columns=rank + rot)
-    _check(library.load().qil_rotate_tail(_ptr(q), _code(q.dtype), heads * (dim + rot), dim + rot, dim, _ptr(frequencies),
-                                          _ptr(positions), _ptr(out), heads * (rank + rot), rank + rot, rank, n, heads,
-                                          rot, _stream()), 'rotate_tail')
+    if n >= HEAD_PRODUCT_BLAS_ROWS and q.dtype == torch.bfloat16:
+        head_product(q, k_up, heads=heads, out_dtype=torch.float32, out=out, out_columns=rank + rot)
+        _check(library.load().qil_rotate_tail(_ptr(q), _code(q.dtype), heads * (dim + rot), dim + rot, dim, _ptr(frequencies),
+                                              _ptr(positions), _ptr(out), heads * (rank + rot), rank + rot, rank, n, heads,
+                                              rot, _stream()), 'rotate_tail')
+        return out
+    _check(library.load().qil_head_product(_ptr(q), _code(q.dtype), heads * (dim + rot), dim + rot, _ptr(k_up), _code(k_up.dtype),
+                                           _ptr(out), _code(out.dtype), heads * (rank + rot), rank + rot, n, heads, dim, rank,
+                                           None, 0, 1, 0, _ptr(frequencies), _ptr(positions), dim, rot, _stream()),
+           'latent_query')
     return out
 
 

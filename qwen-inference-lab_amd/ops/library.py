@@ -304,7 +304,7 @@ def _declare(lib):
     lib.qil_latent_expanded_takes.argtypes = [i, i, i]
     lib.qil_latent_expanded_takes.restype = i
     lib.qil_latent_expanded.argtypes = [p, p, p, p, i, p, p, p, p, p, i, i, i, f, p]
-    lib.qil_head_product.argtypes = [p, i, i, i, p, i, p, i, i, i, i, i, i, i, p, i, i, i, p]
+    lib.qil_head_product.argtypes = [p, i, i, i, p, i, p, i, i, i, i, i, i, i, p, i, i, i, p, p, i, i, p]
     lib.qil_gated_heads.argtypes = [p, p, i, i, i, p, i, i, i, p]
     lib.qil_gated_heads.restype = i
     lib.qil_rotate_tail.argtypes = [p, i, i, i, i, p, p, p, i, i, i, i, i, i, p]
