@@ -78,6 +78,81 @@ __global__ void latent_prepare_kernel(const TD* __restrict__ x, int splits, size
   }
 }
 
+// The same with the row in registers: the q_rank + rank normalised elements in quads, at most J a thread, both sums of squares
+// in one reduction, the rotated part and the gates by the block's last threads while the others wait for their quads.  All
+// sizes and x_row are multiples of 4, all arrays aligned to a quad.
+// What bounds it is the chain of its waits: scalar reads of the row, a turn through LDS and two reductions took 9.8 us for 8
+// rows of 1,536 + 512 + 64 columns in four splits, 17.0 us for 3,044 plain rows (29 MB); now 5.3 and 9.3.
+template <typename TD, typename T, int J>
+__global__ void __launch_bounds__(512)
+latent_prepare_vec_kernel(Operand x, const float* __restrict__ wq, const float* __restrict__ wc, const float* __restrict__ freq,
+                          const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ cq_out,
+                          T* __restrict__ latent, T* __restrict__ rope, float* __restrict__ gate_out, int q_rank, int rank, int rot,
+                          int gates, float eps, int x_row, int rows, T* __restrict__ c_rows, T* __restrict__ rope_rows) {
+  const int n = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+  if (n >= rows) {                                    // a row that fills the copies up
+    for (int i = 4 * tid; i < rank; i += 4 * nt) st4(c_rows + (size_t)n * rank + i, make_float4(0.f, 0.f, 0.f, 0.f));
+    for (int i = 4 * tid; i < rot; i += 4 * nt) st4(rope_rows + (size_t)n * rot + i, make_float4(0.f, 0.f, 0.f, 0.f));
+    return;
+  }
+  __shared__ float scratch[2][8];
+  const size_t at = (size_t)n * x_row;
+  const int normed = q_rank + rank;
+  const size_t slot = slots ? (size_t)slots[n] : 0;
+  const int position = positions[n];
+  float4 v[J], w[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int i = min(4 * (tid + nt * j), normed - 4);      // (no load under a condition: it would be waited for there)
+    w[j] = ld4(i < q_rank ? wq + i : wc + (i - q_rank));
+    if constexpr (sizeof(TD) == 2) v[j] = ld4(reinterpret_cast<const bf16_t*>(x.data) + at + i);
+    else v[j] = operand_at4(x, at + i);
+  }
+  const int last = nt - 1 - tid, half = rot / 2;
+  for (int i = last; i < gates; i += nt) gate_out[(size_t)n * gates + i] = 1.f / (1.f + expf(-operand_at(x, at + normed + rot + i)));
+  if (slots)
+    for (int i = last; i < half; i += nt) {
+      const float u = operand_at(x, at + normed + i), t = operand_at(x, at + normed + half + i);
+      float sn, cs;
+      sincosf((float)position * freq[i], &sn, &cs);
+      const float first = u * cs - t * sn, second = t * cs + u * sn;
+      st(rope + slot * rot + i, first);
+      st(rope + slot * rot + half + i, second);
+      if (rope_rows) {
+        st(rope_rows + (size_t)n * rot + i, first);
+        st(rope_rows + (size_t)n * rot + half + i, second);
+      }
+    }
+  float sq = 0.f, sc = 0.f;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const float squares = v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    const int i = 4 * (tid + nt * j);
+    sq += i < q_rank ? squares : 0.f;
+    sc += i >= q_rank && i < normed ? squares : 0.f;
+  }
+  sq = wave_sum(sq);
+  sc = wave_sum(sc);
+  if ((tid & 63) == 0) scratch[0][tid >> 6] = sq, scratch[1][tid >> 6] = sc;
+  __syncthreads();
+  sq = sc = 0.f;
+  for (int wave = 0; wave < nt / QIL_WAVE; ++wave) sq += scratch[0][wave], sc += scratch[1][wave];
+  const float rq = 1.f / sqrtf(sq / (float)q_rank + eps), rc = 1.f / sqrtf(sc / (float)rank + eps);
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int i = 4 * (tid + nt * j);
+    if (i >= normed) continue;
+    const float f = i < q_rank ? rq : rc;
+    const float4 y = make_float4(v[j].x * f * w[j].x, v[j].y * f * w[j].y, v[j].z * f * w[j].z, v[j].w * f * w[j].w);
+    if (i < q_rank) {
+      st4(cq_out + (size_t)n * q_rank + i, y);
+    } else if (slots) {
+      st4(latent + slot * rank + (i - q_rank), y);
+      if (c_rows) st4(c_rows + (size_t)n * rank + (i - q_rank), y);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // Element i and i + half of a vector turned by `position`.
 template <typename TX>
@@ -415,6 +490,36 @@ int qil_latent_prepare(const void* x, int x_dtype, int splits, int x_row, const 
   if (q_rank < 1 || rank < 1 || rot < 2 || rot % 2 || splits < 1 || (x_dtype == QIL_BF16 && splits != 1) || gates < 0 ||
       (gates > 0 && !gate_out) || x_row < q_rank + rank + rot + gates)
     return -1;
+  // the row in registers where quads fit every array: few rows a quad a thread as far as 512 threads go, many rows (enough
+  // blocks to hide a row's waits) 256 threads
+  const size_t quad = dtype == QIL_F32 ? 16 : 8, x_quad = x_dtype == QIL_F32 ? 16 : 8;
+  const bool quads = q_rank % 4 == 0 && rank % 4 == 0 && rot % 4 == 0 && x_row % 4 == 0 && (size_t)x % x_quad == 0 &&
+                     ((size_t)wq | (size_t)wc) % 16 == 0 &&
+                     ((size_t)cq_out | (size_t)latent | (size_t)rope | (size_t)c_rows | (size_t)rope_rows) % quad == 0;
+  const int items = (q_rank + rank) / 4, wide = n > 64 || items <= 256 ? 256 : 512, turns = (items + wide - 1) / wide;
+  if (quads && turns <= 4) {
+    const Operand operand{x, x_dtype, splits, (size_t)n * x_row};
+#define QIL_LPV(TD, T, J)                                                                                              \
+  hipLaunchKernelGGL((latent_prepare_vec_kernel<TD, T, J>), dim3(blocks), dim3(wide), 0, s, operand, wq, wc, freq, positions, slots, \
+                     (T*)cq_out, (T*)latent, (T*)rope, gate_out, q_rank, rank, rot, gates, eps, x_row, n, (T*)c_rows, (T*)rope_rows)
+#define QIL_LPJ(TD, T)                                                                                                 \
+  do {                                                                                                                  \
+    if (turns == 1) QIL_LPV(TD, T, 1);                                                                                  \
+    else if (turns == 2) QIL_LPV(TD, T, 2);                                                                             \
+    else QIL_LPV(TD, T, 4);                                                                                             \
+  } while (0)
+    if (dtype == QIL_F32) {
+      if (x_dtype != QIL_F32) return -1;
+      QIL_LPJ(float, float);
+    } else if (x_dtype == QIL_F32) {
+      QIL_LPJ(float, bf16_t);
+    } else {
+      QIL_LPJ(bf16_t, bf16_t);
+    }
+#undef QIL_LPJ
+#undef QIL_LPV
+    QIL_RETURN_LAUNCH_STATUS();
+  }
   const size_t stride = (size_t)n * x_row;
   const size_t row_bytes = (size_t)(q_rank + rank + rot + gates) * sizeof(float);
   const int held = row_bytes <= 48 * 1024;            // the row's sums fit in LDS
