@@ -15,7 +15,8 @@
 //   carry    block after block, S_out = exp(m_in - M_end) S_in + exp(max e - M_end) U, element by element; every block's
 //            S_in replaces its U, the last S_out goes to the state slot;
 //   outputs  per block: [q scaled by its carry weight | masked weighted q k^T] x [S_in ; v], tiled 64 tokens x 64 columns.
-// The tiled products run on the vector units in float32 (4 x 4 outputs a thread, operands staged in LDS).
+// The tiled products are float32: on the matrix cores for DECAY and MLSTM at the sizes scan_mfma_takes names, otherwise on
+// the vector units (4 x 4 outputs a thread, operands staged in LDS).
 //
 // QIL_SCAN_CHANNEL (every row i of S decays by a factor of its own, a_t[i] = exp(logsigmoid(z_t[i]) / tau)): with
 // G_t[i] the sum of the block's log2 decays of row i up to token t (one more kernel, `decays`, walks them),
@@ -55,6 +56,18 @@ __device__ __forceinline__ GateLane gate_lane(const float* __restrict__ gates, c
   g.sum = sum;
   g.lead = live ? (double)in - sum : -INFINITY;
   return g;
+}
+
+// d^n for n of 0 to 127 by squaring, in float64 (a dozen multiplications, each good to 2^-53: the float32 it is rounded to
+// is pow's, which costs a wave 1.5 us).
+__device__ __forceinline__ float decay_power(double d, int n) {
+  double power = 1.0;
+#pragma unroll
+  for (int bit = 0; bit < 7; ++bit) {
+    if (n >> bit & 1) power *= d;
+    d *= d;
+  }
+  return (float)power;
 }
 
 // STEP, lane t: F_t and the step size d_t of token t (0 past the block's end).
@@ -102,27 +115,83 @@ scan_decays_kernel(const float* __restrict__ z, float tau, const int* __restrict
   }
 }
 
+// One block a row.  A thread owns one pair of rotated elements (or one that passes through) of a head and meets it in every
+// head's query and key, so that its sine and cosine are made once a row and not once an element: 3,044 rows of 2 x 8 heads
+// of 128 elements 22.8 -> 12.4 us (37 MB).  blockDim.x is a multiple of the units a head has, dim - rot / 2.
 template <typename T>
-__global__ void scan_rotate_kernel(const T* __restrict__ proj, int proj_row, int q_off, int k_off,
-                                   const float* __restrict__ freq, int rot, float q_scale, float k_scale,
-                                   const int* __restrict__ cu_seqlens, const int* __restrict__ seq_starts, int n_seqs,
-                                   float* __restrict__ qk, int heads, int dim) {
-  const int row = blockIdx.x;
-  int seq = 0;
-  while (seq + 1 < n_seqs && cu_seqlens[seq + 1] <= row) ++seq;
-  const float position = (float)(seq_starts[seq] + row - cu_seqlens[seq]);
-  const int half = rot / 2, hd = heads * dim;
-  for (int idx = threadIdx.x; idx < 2 * hd; idx += blockDim.x) {
-    const int which = idx / hd, e = idx - which * hd, i = e % dim;
-    const T* x = proj + (size_t)row * proj_row + (which ? k_off : q_off) + e;
-    float value = ld(x);
-    if (i < rot) {
-      float sn, cs;
-      sincosf(position * freq[i < half ? i : i - half], &sn, &cs);
-      value = i < half ? value * cs - ld(x + half) * sn : value * cs + ld(x - half) * sn;
-    }
-    qk[(size_t)row * 2 * hd + idx] = value * (which ? k_scale : q_scale);
+__global__ void __launch_bounds__(256)
+scan_rotate_kernel(const T* __restrict__ proj, int proj_row, int q_off, int k_off, const float* __restrict__ freq, int rot,
+                   float q_scale, float k_scale, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_starts,
+                   int n_seqs, float* __restrict__ qk, int heads, int dim) {
+  const int row = blockIdx.x, half = rot / 2, units = dim - half, hd = heads * dim;
+  const int unit = threadIdx.x % units, step = blockDim.x / units;
+  const int i = unit < half ? unit : unit + half;
+  float sn = 0.f, cs = 1.f;
+  if (unit < half) {
+    int seq = 0;
+    while (seq + 1 < n_seqs && cu_seqlens[seq + 1] <= row) ++seq;
+    const float position = (float)(seq_starts[seq] + row - cu_seqlens[seq]);
+    sincosf(position * freq[unit], &sn, &cs);
   }
+  const T* x = proj + (size_t)row * proj_row;
+  float* to = qk + (size_t)row * 2 * hd;
+#pragma unroll 4
+  for (int place = threadIdx.x / units; place < 2 * heads; place += step) {
+    const bool key = place >= heads;
+    const int e = (key ? place - heads : place) * dim + i;
+    const T* src = x + (key ? k_off : q_off) + e;
+    const float scale = key ? k_scale : q_scale, first = ld(src);
+    float* out = to + (key ? hd : 0) + e;
+    if (unit < half) {
+      const float second = ld(src + half);
+      out[0] = (first * cs - second * sn) * scale;
+      out[half] = (second * cs + first * sn) * scale;
+    } else {
+      out[0] = first * scale;
+    }
+  }
+}
+
+// Lane s of a wave: what the key and value of token s of block c are worth in the block's sum; the lane of the first token
+// of the grid's first z also leaves what the carry needs of the block's gates.
+template <int MODE>
+__device__ __forceinline__ float sums_weight(const float* __restrict__ gates, const float* __restrict__ gate_bias, float cap,
+                                             const float* __restrict__ decay, const float* __restrict__ state,
+                                             size_t slot_stride, const int* __restrict__ seq_starts,
+                                             const int* __restrict__ seq_slots, double* __restrict__ info,
+                                             float* __restrict__ carried, int heads, int dim, int vdim,
+                                             const StepInput& steps, int seq, int h, int c, int r0, int lc, size_t at,
+                                             bool writes, int lane) {
+  const bool live = lane < lc;
+  float weight;
+  if (MODE == QIL_SCAN_MLSTM) {
+    const GateLane g = gate_lane(gates, gate_bias, cap, r0 + (live ? lane : 0), h, heads, live, lane);
+    double top = g.lead;
+#pragma unroll
+    for (int d = QIL_WAVE / 2; d > 0; d >>= 1) top = fmax(top, __shfl_xor(top, d, QIL_WAVE));
+    weight = live ? expf((float)(g.lead - top)) : 0.f;
+    const double total = __shfl(g.sum, lc - 1, QIL_WAVE);
+    if (writes && lane == 0) {
+      info[at * 2] = top;
+      info[at * 2 + 1] = total;
+      if (c == 0) {                                            // the maximum the sequence brings: read before carry writes
+        const int tiles = (vdim + SCAN_TOP_TILE - 1) / SCAN_TOP_TILE;
+        const float* s_top = state + (size_t)seq_slots[seq] * slot_stride + (size_t)heads * dim * vdim +
+                             (size_t)heads * dim + (size_t)h * (tiles + 1);
+        carried[at] = seq_starts[seq] == 0 ? 0.f : *s_top;
+      }
+    }
+  } else if (MODE == QIL_SCAN_STEP) {
+    const StepLane g = step_lane(steps, gate_bias, decay[h], r0 + (live ? lane : 0), h, live, lane);
+    const double total = __shfl(g.sum, lc - 1, QIL_WAVE);
+    weight = live ? expf((float)(total - g.sum)) * g.step : 0.f;
+    if (writes && lane == 0) info[at * 2] = total;
+  } else if (MODE == QIL_SCAN_CHANNEL) {
+    weight = live ? 1.f : 0.f;                                 // (the rows' own weights follow below)
+  } else {
+    weight = live ? decay_power((double)decay[h], lc - 1 - lane) : 0.f;
+  }
+  return weight;
 }
 
 // grid (blocks of the longest sequence, sequences x heads, dim tiles x vdim tiles)
@@ -144,38 +213,9 @@ scan_sums_kernel(const T* __restrict__ proj, int proj_row, int v_off, const floa
   if (c * SCAN_BLOCK >= len) return;
   const int r0 = row0 + c * SCAN_BLOCK, lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
   const size_t at = (size_t)block_place(row0, seq, c) * heads + h;
-  if (tid < QIL_WAVE) {
-    const bool live = tid < lc;
-    float weight;
-    if (MODE == QIL_SCAN_MLSTM) {
-      const GateLane g = gate_lane(gates, gate_bias, cap, r0 + (live ? tid : 0), h, heads, live, tid);
-      double top = g.lead;
-#pragma unroll
-      for (int d = QIL_WAVE / 2; d > 0; d >>= 1) top = fmax(top, __shfl_xor(top, d, QIL_WAVE));
-      weight = live ? expf((float)(g.lead - top)) : 0.f;
-      const double total = __shfl(g.sum, lc - 1, QIL_WAVE);
-      if (blockIdx.z == 0 && tid == 0) {
-        info[at * 2] = top;
-        info[at * 2 + 1] = total;
-        if (c == 0) {                                            // the maximum the sequence brings: read before carry writes
-          const int tiles = (vdim + SCAN_TOP_TILE - 1) / SCAN_TOP_TILE;
-          const float* s_top = state + (size_t)seq_slots[seq] * slot_stride + (size_t)heads * dim * vdim +
-                               (size_t)heads * dim + (size_t)h * (tiles + 1);
-          carried[at] = seq_starts[seq] == 0 ? 0.f : *s_top;
-        }
-      }
-    } else if (MODE == QIL_SCAN_STEP) {
-      const StepLane g = step_lane(steps, gate_bias, decay[h], r0 + (live ? tid : 0), h, live, tid);
-      const double total = __shfl(g.sum, lc - 1, QIL_WAVE);
-      weight = live ? expf((float)(total - g.sum)) * g.step : 0.f;
-      if (blockIdx.z == 0 && tid == 0) info[at * 2] = total;
-    } else if (MODE == QIL_SCAN_CHANNEL) {
-      weight = live ? 1.f : 0.f;                                 // (the rows' own weights follow below)
-    } else {
-      weight = live ? (float)pow((double)decay[h], (double)(lc - 1 - tid)) : 0.f;
-    }
-    w[tid] = weight;
-  }
+  if (tid < QIL_WAVE)
+    w[tid] = sums_weight<MODE>(gates, gate_bias, cap, decay, state, slot_stride, seq_starts, seq_slots, info, carried, heads,
+                               dim, vdim, steps, seq, h, c, r0, lc, at, blockIdx.z == 0, tid);
   __syncthreads();
   const size_t hd = (size_t)heads * dim;
   const int group = MODE == QIL_SCAN_STEP ? h / (heads / steps.groups) : h;
@@ -218,53 +258,101 @@ scan_sums_kernel(const T* __restrict__ proj, int proj_row, int v_off, const floa
   }
 }
 
-// grid (sequences, heads, elements of a head's state / 256): one thread an element of S (or of n), block after block.
-template <int MODE>
+// grid (sequences, heads, elements of a head's state / 256 V): a thread takes V neighbouring elements of S (or of n) block
+// after block.  Four where they are aligned and lie in one row of S (V == 4: dim and vdim multiples of 4): 28 blocks of
+// 8 heads of 128 x 256 26.8 -> 18.0 us (102 MB).
+#define CARRY_AHEAD 8
+template <int MODE, int V>
 __global__ void __launch_bounds__(256)
 scan_carry_kernel(float* __restrict__ sums, float* __restrict__ norm_sums, const double* __restrict__ info,
                   float* __restrict__ carried, const float* __restrict__ decay, float* __restrict__ state,
                   size_t slot_stride, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_starts,
                   const int* __restrict__ seq_slots, int heads, int dim, int vdim, const float* __restrict__ gsum) {
-  const int seq = blockIdx.x, h = blockIdx.y, e = blockIdx.z * blockDim.x + threadIdx.x;
+  typedef float Piece __attribute__((ext_vector_type(V)));
+  const int seq = blockIdx.x, h = blockIdx.y, e = (blockIdx.z * blockDim.x + threadIdx.x) * V;
   const int mat = dim * vdim, total = mat + (MODE == QIL_SCAN_MLSTM ? dim : 0);
   const int row0 = cu_seqlens[seq], len = cu_seqlens[seq + 1] - row0;
   if (len <= 0 || e >= total) return;
   const bool fresh = seq_starts[seq] == 0;
   const int tiles = (vdim + SCAN_TOP_TILE - 1) / SCAN_TOP_TILE;
   float* slot = state + (size_t)seq_slots[seq] * slot_stride;
-  float* mine = e < mat ? slot + (size_t)h * mat + e : slot + (size_t)heads * mat + (size_t)h * dim + (e - mat);
+  Piece* mine = reinterpret_cast<Piece*>(e < mat ? slot + (size_t)h * mat + e : slot + (size_t)heads * mat + (size_t)h * dim + (e - mat));
   float* s_top = slot + (size_t)heads * mat + (size_t)heads * dim + (size_t)h * (tiles + 1);
-  float value = fresh ? 0.f : *mine;
   const int blocks = (len + SCAN_BLOCK - 1) / SCAN_BLOCK;
-  const size_t first = (size_t)block_place(row0, seq, 0) * heads + h;
+  const size_t first = (size_t)block_place(row0, seq, 0) * heads + h, width = e < mat ? mat : dim;
+  float* mine_sums = (e < mat ? sums + e : norm_sums + (e - mat)) + first * width;
+  const size_t stride = (size_t)heads * width;
+  Piece value = fresh ? Piece(0.f) : *mine;
   float top = MODE == QIL_SCAN_MLSTM ? carried[first] : 0.f;
   const double rate = MODE == QIL_SCAN_DECAY ? (double)decay[h] : 0.0;
-  const float keep_whole = MODE == QIL_SCAN_DECAY ? (float)pow(rate, (double)SCAN_BLOCK) : 0.f;   // a whole block's decay
-  for (int c = 0; c < blocks; ++c) {
-    const size_t at = first + (size_t)c * heads;
-    float* u = e < mat ? sums + at * mat + e : norm_sums + at * dim + (e - mat);
-    float keep, take = 1.f;
-    if (MODE == QIL_SCAN_MLSTM) {
-      const double local = info[at * 2], end = fmax((double)top, local);
-      keep = expf((float)((double)top - end));
-      take = expf((float)(local - end));
-      if (e == 0) carried[at] = top;
-      top = (float)(info[at * 2 + 1] + end);
-    } else if (MODE == QIL_SCAN_STEP) {
-      keep = expf((float)info[at * 2]);
-    } else if (MODE == QIL_SCAN_CHANNEL) {
-      const int last = row0 + min((c + 1) * SCAN_BLOCK, len) - 1;       // the block's last token
-      keep = __builtin_amdgcn_exp2f(gsum[(size_t)last * heads * dim + (size_t)h * dim + e / vdim]);
-    } else {
-      const int lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
-      keep = lc == SCAN_BLOCK ? keep_whole : (float)pow(rate, (double)lc);
+  const float keep_whole = MODE == QIL_SCAN_DECAY ? decay_power(rate, SCAN_BLOCK) : 0.f;   // a whole block's decay
+  // eight blocks' sums are asked for before the first is taken: loads behind a store to the same array wait for nothing
+  for (int c0 = 0; c0 < blocks; c0 += CARRY_AHEAD) {
+    Piece add[CARRY_AHEAD];
+#pragma unroll
+    for (int u = 0; u < CARRY_AHEAD; ++u)
+      add[u] = *reinterpret_cast<const Piece*>(mine_sums + (size_t)min(c0 + u, blocks - 1) * stride);
+#pragma unroll
+    for (int u = 0; u < CARRY_AHEAD; ++u) {
+      const int c = c0 + u;
+      if (c >= blocks) break;
+      const size_t at = first + (size_t)c * heads;
+      float keep, take = 1.f;
+      if (MODE == QIL_SCAN_MLSTM) {
+        const double local = info[at * 2], end = fmax((double)top, local);
+        keep = expf((float)((double)top - end));
+        take = expf((float)(local - end));
+        if (e == 0) carried[at] = top;
+        top = (float)(info[at * 2 + 1] + end);
+      } else if (MODE == QIL_SCAN_STEP) {
+        keep = expf((float)info[at * 2]);
+      } else if (MODE == QIL_SCAN_CHANNEL) {
+        const int last = row0 + min((c + 1) * SCAN_BLOCK, len) - 1;     // the block's last token
+        keep = __builtin_amdgcn_exp2f(gsum[(size_t)last * heads * dim + (size_t)h * dim + e / vdim]);
+      } else {
+        const int lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
+        keep = lc == SCAN_BLOCK ? keep_whole : decay_power(rate, lc);
+      }
+      *reinterpret_cast<Piece*>(mine_sums + (size_t)c * stride) = value;
+      value = keep * value + take * add[u];
     }
-    const float add = *u;
-    *u = value;
-    value = keep * value + take * add;
   }
   *mine = value;
-  if (MODE == QIL_SCAN_MLSTM && e <= tiles) s_top[e] = top;
+  if (MODE == QIL_SCAN_MLSTM)
+    for (int x = e; x < e + V && x <= tiles; ++x) s_top[x] = top;
+}
+
+// Lane t of a wave: what token t of the block weighs keys before it and the state brought in with.
+template <int MODE>
+__device__ __forceinline__ void outputs_weights(const float* __restrict__ gates, const float* __restrict__ gate_bias, float cap,
+                                                const float* __restrict__ decay, const float* __restrict__ carried,
+                                                const StepInput& steps, int h, int heads, int r0, int lc, size_t at, int lane,
+                                                float* cw, float* em, float* pw, double* lead, double* tops) {
+  if (MODE == QIL_SCAN_MLSTM) {
+    const bool live = lane < lc;
+    const GateLane g = gate_lane(gates, gate_bias, cap, r0 + (live ? lane : 0), h, heads, live, lane);
+    const double brought = (double)carried[at];
+    double top = g.lead;
+#pragma unroll
+    for (int d = 1; d < QIL_WAVE; d <<= 1) {
+      const double up = __shfl_up(top, d, QIL_WAVE);
+      if (lane >= d) top = fmax(top, up);
+    }
+    top = fmax(top, brought);
+    lead[lane] = g.lead;
+    tops[lane] = top;
+    cw[lane] = expf((float)(brought - top));
+    em[lane] = expf(-(float)(g.sum + top));
+  } else if (MODE == QIL_SCAN_STEP) {
+    const bool live = lane < lc;
+    const StepLane g = step_lane(steps, gate_bias, decay[h], r0 + (live ? lane : 0), h, live, lane);
+    tops[lane] = g.sum;
+    cw[lane] = expf((float)g.sum);
+    em[lane] = g.step;
+  } else if (MODE != QIL_SCAN_CHANNEL) {
+    pw[lane] = decay_power((double)decay[h], lane);
+    if (lane == 0) pw[SCAN_BLOCK] = decay_power((double)decay[h], SCAN_BLOCK);
+  }
 }
 
 // grid (blocks of the longest sequence, sequences x heads, vdim tiles)
@@ -295,33 +383,8 @@ scan_outputs_kernel(const T* __restrict__ proj, int proj_row, int v_off, const f
   if (c * SCAN_BLOCK >= len) return;
   const int r0 = row0 + c * SCAN_BLOCK, lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
   const size_t at = (size_t)block_place(row0, seq, c) * heads + h;
-  if (tid < QIL_WAVE) {
-    if (MODE == QIL_SCAN_MLSTM) {
-      const bool live = tid < lc;
-      const GateLane g = gate_lane(gates, gate_bias, cap, r0 + (live ? tid : 0), h, heads, live, tid);
-      const double brought = (double)carried[at];
-      double top = g.lead;
-#pragma unroll
-      for (int d = 1; d < QIL_WAVE; d <<= 1) {
-        const double up = __shfl_up(top, d, QIL_WAVE);
-        if (tid >= d) top = fmax(top, up);
-      }
-      top = fmax(top, brought);
-      lead[tid] = g.lead;
-      tops[tid] = top;
-      cw[tid] = expf((float)(brought - top));
-      em[tid] = expf(-(float)(g.sum + top));
-    } else if (MODE == QIL_SCAN_STEP) {
-      const bool live = tid < lc;
-      const StepLane g = step_lane(steps, gate_bias, decay[h], r0 + (live ? tid : 0), h, live, tid);
-      tops[tid] = g.sum;
-      cw[tid] = expf((float)g.sum);
-      em[tid] = g.step;
-    } else if (!CHANNEL) {
-      pw[tid] = (float)pow((double)decay[h], (double)tid);
-      if (tid == 0) pw[SCAN_BLOCK] = (float)pow((double)decay[h], (double)SCAN_BLOCK);
-    }
-  }
+  if (tid < QIL_WAVE)
+    outputs_weights<MODE>(gates, gate_bias, cap, decay, carried, steps, h, heads, r0, lc, at, tid, cw, em, pw, lead, tops);
   const int ti = tid / 16, tj = tid % 16;
   const size_t hd = (size_t)heads * dim;
   const int group = MODE == QIL_SCAN_STEP ? h / (heads / steps.groups) : h;
@@ -447,6 +510,309 @@ scan_outputs_kernel(const T* __restrict__ proj, int proj_row, int v_off, const f
   }
 }
 
+// ---- DECAY and MLSTM on the matrix cores: dim 64, 128 or 256, vdim a multiple of 64, values in aligned pairs.
+// v_mfma_f32_32x32x2_f32 takes float32 inputs and adds float32 products into float32 sums, as the vector units do, at twice
+// their rate; what bounds the kernels above is their LDS reads (three 16-byte reads for 16 or 32 multiplications).  The index
+// that a product sums over may be numbered as one likes: step u of group g takes tokens (or state rows) 8 g + u and
+// 8 g + 4 + u, so that a lane's four steps are four neighbours in memory.  Columns are paired the same way (tile j takes
+// the columns 2 lane + j), so that state, values and results move as 8-byte pieces in whole lines, straight between
+// memory and registers.
+typedef float scan_x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ scan_x16 scan_mfma(float a, float b, scan_x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+// row of result register r (of 16) in a 32 x 32 tile, lane half `up`
+__device__ __forceinline__ int scan_tile_row(int r, int up) { return 8 * (r / 4) + 4 * up + r % 4; }
+
+// Two neighbouring values as they lie in memory, and as floats.
+template <typename T> struct ValuePair;
+template <> struct ValuePair<float> {
+  float2 raw;
+  __device__ __forceinline__ void load(const float* p) { raw = *reinterpret_cast<const float2*>(p); }
+  __device__ __forceinline__ float at(int i, bool live) const { return live ? (i ? raw.y : raw.x) : 0.f; }
+};
+template <> struct ValuePair<bf16_t> {
+  uint32_t raw;
+  __device__ __forceinline__ void load(const bf16_t* p) { raw = *reinterpret_cast<const uint32_t*>(p); }
+  __device__ __forceinline__ float at(int i, bool live) const {
+    return live ? __uint_as_float(i ? raw & 0xffff0000u : raw << 16) : 0.f;
+  }
+};
+
+// As scan_sums_kernel.  A wave makes 64 rows by 64 columns of a block's sum over its 64 tokens, 128 products; keys and values
+// come straight from memory (a block's waves share the keys).  grid (blocks of the longest sequence, sequences x heads, dim
+// tiles x groups of column tiles); blockDim.x / 64 column tiles a group.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(256)
+scan_sums_mfma_kernel(const T* __restrict__ proj, int proj_row, int v_off, const float* __restrict__ qk,
+                      const float* __restrict__ gates, const float* __restrict__ gate_bias, float cap,
+                      const float* __restrict__ decay, const float* __restrict__ state, size_t slot_stride,
+                      const int* __restrict__ cu_seqlens, const int* __restrict__ seq_starts, const int* __restrict__ seq_slots,
+                      float* __restrict__ sums, float* __restrict__ norm_sums, double* __restrict__ info,
+                      float* __restrict__ carried, int heads, int dim, int vdim, int dim_tiles) {
+  __shared__ __align__(16) float w[SCAN_BLOCK];
+  const int c = blockIdx.x, seq = blockIdx.y / heads, h = blockIdx.y % heads, tid = threadIdx.x;
+  const int it = blockIdx.z % dim_tiles, jt = blockIdx.z / dim_tiles * (blockDim.x / QIL_WAVE) + tid / QIL_WAVE;
+  const int lane = tid % QIL_WAVE, up = lane / 32, col = lane % 32;
+  const int row0 = cu_seqlens[seq], len = cu_seqlens[seq + 1] - row0;
+  if (c * SCAN_BLOCK >= len) return;
+  const int r0 = row0 + c * SCAN_BLOCK, lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
+  const size_t at = (size_t)block_place(row0, seq, c) * heads + h, hd = (size_t)heads * dim;
+  const float* keys = qk + hd + (size_t)h * dim + it * 64 + 2 * col;
+  const T* values = proj + v_off + h * vdim + jt * 64 + 2 * col;
+  constexpr int AHEAD = 2;
+  float2 k[AHEAD][4];
+  ValuePair<T> v[AHEAD][4];
+  auto ask = [&](int g, int slot) {                              // tokens past the block's end read its last one
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const size_t row = r0 + min(8 * g + 4 * up + u, lc - 1);
+      k[slot][u] = *reinterpret_cast<const float2*>(keys + row * 2 * hd);
+      v[slot][u].load(values + row * proj_row);
+    }
+  };
+#pragma unroll
+  for (int g = 0; g < AHEAD; ++g) ask(g, g);
+  StepInput none{};
+  if (tid < QIL_WAVE)
+    w[tid] = sums_weight<MODE>(gates, gate_bias, cap, decay, state, slot_stride, seq_starts, seq_slots, info, carried, heads,
+                               dim, vdim, none, seq, h, c, r0, lc, at, blockIdx.z == 0, tid);
+  __syncthreads();
+  scan_x16 acc[2][2] = {};
+  float norm[2] = {};
+#pragma unroll
+  for (int g = 0; g < SCAN_BLOCK / 8; ++g) {
+    const float4 w4 = *reinterpret_cast<const float4*>(&w[8 * g + 4 * up]);
+    const float weight[4] = {w4.x, w4.y, w4.z, w4.w};
+    float a[2][4], b[2][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool live = 8 * g + 4 * up + u < lc;
+      a[0][u] = live ? weight[u] * k[g % AHEAD][u].x : 0.f;
+      a[1][u] = live ? weight[u] * k[g % AHEAD][u].y : 0.f;
+      b[0][u] = v[g % AHEAD][u].at(0, live);
+      b[1][u] = v[g % AHEAD][u].at(1, live);
+    }
+    if (g + AHEAD < SCAN_BLOCK / 8) ask(g + AHEAD, g % AHEAD);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (MODE == QIL_SCAN_MLSTM) norm[i] += a[i][u];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = scan_mfma(a[i][u], b[j][u], acc[i][j]);
+      }
+    }
+  }
+  float* to = sums + at * dim * vdim + (size_t)it * 64 * vdim + jt * 64 + 2 * col;
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<float2*>(to + (size_t)(2 * scan_tile_row(r, up) + i) * vdim) = make_float2(acc[i][0][r], acc[i][1][r]);
+  if (MODE == QIL_SCAN_MLSTM && jt == 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float total = norm[i] + __shfl_xor(norm[i], 32, QIL_WAVE);
+      if (up == 0) norm_sums[at * dim + it * 64 + 2 * col + i] = total;
+    }
+  }
+}
+
+// As scan_outputs_kernel: a block makes 64 tokens by 64 columns a wave.  Queries and keys pass through LDS (rows of DIM + 4
+// floats: 16 lanes' 16-byte reads fall on all 64 banks), the state brought in and the values come straight from memory.  The
+// scores are made once a block (the kernel above makes them for every 64 columns again), the quadrant of keys behind the
+// tokens not at all; the weighted scores take the keys' place in LDS.  grid (blocks of the longest sequence, sequences x
+// heads, groups of column tiles).
+template <typename T, int MODE, int DIM>
+__global__ void __launch_bounds__(256, DIM <= 128 ? 2 : 1)
+scan_outputs_mfma_kernel(const T* __restrict__ proj, int proj_row, int v_off, const float* __restrict__ qk,
+                         const float* __restrict__ gates, const float* __restrict__ gate_bias, float cap,
+                         const float* __restrict__ decay, const float* __restrict__ before,
+                         const float* __restrict__ norm_before, const float* __restrict__ carried,
+                         const int* __restrict__ cu_seqlens, float* __restrict__ out, float* __restrict__ below, int heads,
+                         int vdim) {
+  constexpr int ROW = DIM + 4, PROW = SCAN_BLOCK + 4, GROUPS = DIM / 8, AHEAD = MODE == QIL_SCAN_MLSTM ? 2 : 3, VALUES = 2;
+  extern __shared__ __align__(16) float scan_lds[];
+  float* qs = scan_lds;                                          // [64][ROW]
+  float* ks = scan_lds + SCAN_BLOCK * ROW;                       // [64][ROW], later the weighted scores [64][PROW]
+  float* ps = ks;
+  __shared__ __align__(16) float cw[SCAN_BLOCK], em[SCAN_BLOCK], pw[SCAN_BLOCK + 1];
+  __shared__ double lead[SCAN_BLOCK], tops[SCAN_BLOCK];
+  const int c = blockIdx.x, seq = blockIdx.y / heads, h = blockIdx.y % heads, tid = threadIdx.x;
+  const int waves = blockDim.x / QIL_WAVE, wave = tid / QIL_WAVE, lane = tid % QIL_WAVE, up = lane / 32, col = lane % 32;
+  const int row0 = cu_seqlens[seq], len = cu_seqlens[seq + 1] - row0;
+  if (c * SCAN_BLOCK >= len) return;
+  const int r0 = row0 + c * SCAN_BLOCK, lc = min(SCAN_BLOCK, len - c * SCAN_BLOCK);
+  const size_t at = (size_t)block_place(row0, seq, c) * heads + h, hd = (size_t)heads * DIM;
+  const int j0 = (blockIdx.z * waves + wave) * 64 + 2 * col;
+  const float* s_in = before + at * DIM * vdim + (size_t)4 * up * vdim + j0;
+  float2 s[AHEAD][4];
+  auto ask_state = [&](int g, int slot) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s[slot][u] = *reinterpret_cast<const float2*>(s_in + (size_t)(8 * g + u) * vdim);
+  };
+  {                                                              // queries and keys into LDS, rows past the end as zeros
+    const float* src = qk + (size_t)r0 * 2 * hd + (size_t)h * DIM;
+#pragma unroll 8
+    for (int idx = tid; idx < 2 * SCAN_BLOCK * (DIM / 4); idx += blockDim.x) {
+      const int x = idx % (DIM / 4), t = idx / (DIM / 4) % SCAN_BLOCK, key = idx / (DIM / 4) / SCAN_BLOCK;
+      float4 q = *reinterpret_cast<const float4*>(src + (size_t)min(t, lc - 1) * 2 * hd + key * hd + 4 * x);
+      if (t >= lc) q = make_float4(0.f, 0.f, 0.f, 0.f);
+      *reinterpret_cast<float4*>(&qs[(key * SCAN_BLOCK + t) * ROW + 4 * x]) = q;
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < AHEAD; ++g) ask_state(g, g);
+  StepInput none{};
+  if (tid < QIL_WAVE)
+    outputs_weights<MODE>(gates, gate_bias, cap, decay, carried, none, h, heads, r0, lc, at, tid, cw, em, pw, lead, tops);
+  __syncthreads();
+  scan_x16 o[2][2] = {};
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    float a[2][4], b[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const float4 q = *reinterpret_cast<const float4*>(&qs[(32 * t + col) * ROW + 8 * g + 4 * up]);
+      a[t][0] = q.x; a[t][1] = q.y; a[t][2] = q.z; a[t][3] = q.w;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { b[0][u] = s[g % AHEAD][u].x; b[1][u] = s[g % AHEAD][u].y; }
+    if (g + AHEAD < GROUPS) ask_state(g + AHEAD, g % AHEAD);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) o[t][j] = scan_mfma(a[t][u], b[j][u], o[t][j]);
+  }
+  const T* values = proj + v_off + h * vdim + j0;
+  ValuePair<T> v[VALUES][4];
+  auto ask_values = [&](int g, int slot) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[slot][u].load(values + (size_t)(r0 + min(8 * g + 4 * up + u, lc - 1)) * proj_row);
+  };
+#pragma unroll
+  for (int g = 0; g < VALUES; ++g) ask_values(g, g);
+  // the state's part by what a token weighs it with
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int token = 32 * t + scan_tile_row(r, up);
+      const float brought = MODE == QIL_SCAN_MLSTM ? cw[token] : pw[token + 1];
+      o[t][0][r] *= brought;
+      o[t][1][r] *= brought;
+    }
+  // the scores' three quadrants, one a wave where there are four waves: tokens from 32 (n > 0), keys from 32 (n > 1)
+  scan_x16 p[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int n = wave + m * waves;
+    if (n >= 3) continue;
+    p[m] = scan_x16{};
+    const float* a_row = &qs[((n > 0 ? 32 : 0) + col) * ROW + 4 * up];
+    const float* b_row = &ks[((n > 1 ? 32 : 0) + col) * ROW + 4 * up];
+#pragma unroll 8
+    for (int g = 0; g < GROUPS; ++g) {
+      const float4 a = *reinterpret_cast<const float4*>(a_row + 8 * g), b = *reinterpret_cast<const float4*>(b_row + 8 * g);
+      p[m] = scan_mfma(a.x, b.x, p[m]);
+      p[m] = scan_mfma(a.y, b.y, p[m]);
+      p[m] = scan_mfma(a.z, b.z, p[m]);
+      p[m] = scan_mfma(a.w, b.w, p[m]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int n = wave + m * waves, key = (n > 1 ? 32 : 0) + col;
+    if (n >= 3) continue;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int token = (n > 0 ? 32 : 0) + scan_tile_row(r, up);
+      float value = 0.f;
+      if (key <= token && token < lc)
+        value = p[m][r] * (MODE == QIL_SCAN_MLSTM ? expf((float)(lead[key] - tops[token])) : pw[max(token - key, 0)]);
+      ps[token * PROW + key] = value;
+    }
+  }
+  __syncthreads();
+  if (MODE == QIL_SCAN_MLSTM && blockIdx.z == 0 && wave == waves - 1 && lane < lc) {
+    const float* n_in = norm_before + at * DIM;
+    float dot = 0.f, row_sum = 0.f;
+#pragma unroll 2
+    for (int x = 0; x < DIM; x += 4) {
+      const float4 q = *reinterpret_cast<const float4*>(&qs[lane * ROW + x]);
+      dot += q.x * n_in[x];
+      dot += q.y * n_in[x + 1];
+      dot += q.z * n_in[x + 2];
+      dot += q.w * n_in[x + 3];
+    }
+    for (int x = 0; x <= lane; ++x) row_sum += ps[lane * PROW + x];
+    below[(size_t)(r0 + lane) * heads + h] = fmaxf(fabsf(dot * cw[lane] + row_sum), em[lane]) + 1e-6f;
+  }
+#pragma unroll
+  for (int g = 0; g < SCAN_BLOCK / 8; ++g) {
+    float a[2][4], b[2][4];
+#pragma unroll
+    for (int t = g < 4 ? 0 : 1; t < 2; ++t) {                    // the first 32 tokens see none of the last 32 keys
+      const float4 q = *reinterpret_cast<const float4*>(&ps[(32 * t + col) * PROW + 8 * g + 4 * up]);
+      a[t][0] = q.x; a[t][1] = q.y; a[t][2] = q.z; a[t][3] = q.w;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool live = 8 * g + 4 * up + u < lc;
+      b[0][u] = v[g % VALUES][u].at(0, live);
+      b[1][u] = v[g % VALUES][u].at(1, live);
+    }
+    if (g + VALUES < SCAN_BLOCK / 8) ask_values(g + VALUES, g % VALUES);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = g < 4 ? 0 : 1; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) o[t][j] = scan_mfma(a[t][u], b[j][u], o[t][j]);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int token = 32 * t + scan_tile_row(r, up);
+      if (token < lc)
+        *reinterpret_cast<float2*>(out + (size_t)(r0 + token) * heads * vdim + (size_t)h * vdim + j0) =
+            make_float2(o[t][0][r], o[t][1][r]);
+    }
+}
+
+// What the two kernels above take: whole tiles, and rows whose pairs of values are aligned.
+static bool scan_mfma_takes(const void* proj, int dtype, int proj_row, int v_off, const float* workspace, const float* out,
+                            int dim, int vdim) {
+  return (dim == 64 || dim == 128 || dim == 256) && vdim % 64 == 0 && proj_row % 2 == 0 && v_off % 2 == 0 &&
+         (uintptr_t)proj % (dtype == QIL_F32 ? 8 : 4) == 0 && (uintptr_t)workspace % 16 == 0 && (uintptr_t)out % 8 == 0;
+}
+
+template <typename T, int MODE, int DIM>
+static int scan_outputs_mfma(dim3 grid, int threads, const T* proj, int proj_row, int v_off, const float* qk,
+                             const float* gates, const float* gate_bias, float cap, const float* decay, const float* before,
+                             const float* norm_before, const float* carried, const int* cu_seqlens, float* out, float* below,
+                             int heads, int vdim, hipStream_t s) {
+  constexpr size_t lds = 2 * SCAN_BLOCK * (DIM + 4) * sizeof(float);
+  if (lds > 64 * 1024) {
+    static bool granted = false;
+    if (!granted) {
+      hipError_t e = hipFuncSetAttribute((const void*)scan_outputs_mfma_kernel<T, MODE, DIM>,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return (int)e;
+      granted = true;
+    }
+  }
+  hipLaunchKernelGGL((scan_outputs_mfma_kernel<T, MODE, DIM>), grid, dim3(threads), lds, s, proj, proj_row, v_off, qk, gates,
+                     gate_bias, cap, decay, before, norm_before, carried, cu_seqlens, out, below, heads, vdim);
+  return 0;
+}
+
 static size_t chunked_places(int n, int n_seqs) { return (size_t)n / SCAN_BLOCK + n_seqs; }
 
 extern "C" {
@@ -487,21 +853,50 @@ int qil_state_scan_chunked(const void* proj, int dtype, int proj_row, int q_off,
   const int blocks = (max_query + SCAN_BLOCK - 1) / SCAN_BLOCK;
   const int dim_tiles = (dim + 63) / 64, v_tiles = (vdim + 63) / 64;
   const int per_head = dim * vdim + (mode == QIL_SCAN_MLSTM ? dim : 0);
-  const dim3 g_sums(blocks, n_seqs * heads, dim_tiles * v_tiles), g_carry(n_seqs, heads, (per_head + 255) / 256);
+  const bool quads = dim % 4 == 0 && vdim % 4 == 0 && slot_stride % 4 == 0 &&
+                     ((uintptr_t)state | (uintptr_t)workspace) % 16 == 0;
+  const bool matrix_cores = scan_mfma_takes(proj, dtype, proj_row, v_off, workspace, out, dim, vdim);
+  const dim3 g_sums(blocks, n_seqs * heads, dim_tiles * v_tiles);
   const dim3 g_out(blocks, n_seqs * heads, v_tiles);
+  const int units = dim - rot / 2;                               // pairs and single elements of a head that rotate works on
+#define QIL_CARRY(MODE)                                                                                               \
+  if (quads)                                                                                                          \
+    hipLaunchKernelGGL((scan_carry_kernel<MODE, 4>), dim3(n_seqs, heads, (per_head / 4 + 255) / 256), dim3(256), 0, s,  \
+                       sums, norm_sums, info, carried, decay, state, slot_stride, cu_seqlens, seq_starts, seq_slots,   \
+                       heads, dim, vdim, gsum);                                                                       \
+  else                                                                                                                \
+    hipLaunchKernelGGL((scan_carry_kernel<MODE, 1>), dim3(n_seqs, heads, (per_head + 255) / 256), dim3(256), 0, s,     \
+                       sums, norm_sums, info, carried, decay, state, slot_stride, cu_seqlens, seq_starts, seq_slots,   \
+                       heads, dim, vdim, gsum)
 #define QIL_CHUNKED(T, MODE)                                                                                          \
   do {                                                                                                                \
     if (MODE == QIL_SCAN_CHANNEL)                                                                                     \
       hipLaunchKernelGGL(scan_decays_kernel, dim3(blocks, n_seqs, (heads * dim + 255) / 256), dim3(256), 0, s, gates,  \
                          cap, cu_seqlens, gsum, heads * dim);                                                          \
     if (MODE != QIL_SCAN_STEP)                                                                                        \
-    hipLaunchKernelGGL(scan_rotate_kernel<T>, dim3(n), dim3(256), 0, s, (const T*)proj, proj_row, q_off, k_off, freq,  \
-                       rot, q_scale, k_scale, cu_seqlens, seq_starts, n_seqs, qk, heads, dim);                         \
+      hipLaunchKernelGGL(scan_rotate_kernel<T>, dim3(n), dim3(256 / units * units), 0, s, (const T*)proj, proj_row,    \
+                         q_off, k_off, freq, rot, q_scale, k_scale, cu_seqlens, seq_starts, n_seqs, qk, heads, dim);   \
+    if constexpr (MODE == QIL_SCAN_DECAY || MODE == QIL_SCAN_MLSTM)                                                   \
+      if (matrix_cores) {                                                                                             \
+        const int waves = v_tiles % 4 == 0 ? 4 : v_tiles % 2 == 0 ? 2 : 1;                                            \
+        hipLaunchKernelGGL((scan_sums_mfma_kernel<T, MODE>), dim3(blocks, n_seqs * heads, dim_tiles * v_tiles / waves), \
+                           dim3(waves * QIL_WAVE), 0, s, (const T*)proj, proj_row, v_off, qk, gates, gate_bias, cap,   \
+                           decay, state, slot_stride, cu_seqlens, seq_starts, seq_slots, sums, norm_sums, info, carried, \
+                           heads, dim, vdim, dim_tiles);                                                              \
+        QIL_CARRY(MODE);                                                                                              \
+        const auto outputs = dim == 64    ? scan_outputs_mfma<T, MODE, 64>                                            \
+                             : dim == 128 ? scan_outputs_mfma<T, MODE, 128>                                           \
+                                          : scan_outputs_mfma<T, MODE, 256>;                                          \
+        const int status = outputs(dim3(blocks, n_seqs * heads, v_tiles / waves), waves * QIL_WAVE, (const T*)proj,    \
+                                   proj_row, v_off, qk, gates, gate_bias, cap, decay, sums, norm_sums, carried,        \
+                                   cu_seqlens, out, below, heads, vdim, s);                                           \
+        if (status) return status;                                                                                    \
+        break;                                                                                                        \
+      }                                                                                                               \
     hipLaunchKernelGGL((scan_sums_kernel<T, MODE>), g_sums, dim3(256), 0, s, (const T*)proj, proj_row, v_off, qk,      \
                        gates, gate_bias, cap, decay, state, slot_stride, cu_seqlens, seq_starts, seq_slots, sums,      \
                        norm_sums, info, carried, heads, dim, vdim, dim_tiles, gsum, steps);                            \
-    hipLaunchKernelGGL(scan_carry_kernel<MODE>, g_carry, dim3(256), 0, s, sums, norm_sums, info, carried, decay,       \
-                       state, slot_stride, cu_seqlens, seq_starts, seq_slots, heads, dim, vdim, gsum);                 \
+    QIL_CARRY(MODE);                                                                                                  \
     hipLaunchKernelGGL((scan_outputs_kernel<T, MODE>), g_out, dim3(256), 0, s, (const T*)proj, proj_row, v_off, qk,    \
                        gates, gate_bias, cap, decay, sums, norm_sums, carried, cu_seqlens, out, below, heads, dim,     \
                        vdim, gsum, steps);                                                                             \
@@ -518,6 +913,7 @@ int qil_state_scan_chunked(const void* proj, int dtype, int proj_row, int q_off,
     else QIL_CHUNKED(bf16_t, QIL_SCAN_DECAY);
   }
 #undef QIL_CHUNKED
+#undef QIL_CARRY
   QIL_RETURN_LAUNCH_STATUS();
 }
 

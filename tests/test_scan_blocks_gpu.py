@@ -1,0 +1,52 @@
+"""The recurrences in blocks of 64 tokens on the matrix cores, around their tiles' edges, against the token-by-token reference."""
+import pytest
+import torch
+
+import kernel_refs as refs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def ops():
+    from qil_amd import ops
+    ops.library.load()
+    return ops
+
+
+# Heads' sizes: the kernels' three dims, one to four and six column tiles of 64 (four, two or one a block).  Lengths: a block of
+# one token, whole blocks, halves of a block (32), one more and one less; two sequences, the second begun elsewhere.
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('mode', ['decay', 'mlstm'])
+@pytest.mark.parametrize('dim, vdim', [(64, 64), (128, 256), (256, 128), (64, 192), (128, 384)])
+@pytest.mark.parametrize('counts', [(32, 1), (33, 64), (129, 95)])
+@pytest.mark.parametrize('shift', [0, 1])
+def test_blocks_of_tokens_on_the_matrix_cores(ops, dtype, mode, dim, vdim, counts, shift):
+    """``shift`` 1 puts every row's values on odd columns: pairs are not aligned, the general kernels take the step."""
+    heads, n, rot = 2, sum(counts), dim // 2
+    g = torch.Generator().manual_seed(dim + vdim + n)
+    proj = torch.randn(n, 2 * heads * dim + heads * vdim + 2 * shift, generator=g).to(dtype)
+    where = dict(heads=heads, dim=dim, vdim=vdim, q_offset=0, k_offset=heads * dim, v_offset=2 * heads * dim + shift)
+    slot = refs.state_scan_slot(heads=heads, dim=dim, vdim=vdim, mode=mode)
+    state = torch.randn(3, slot, generator=g)
+    index = dict(cu_seqlens=torch.tensor([0, counts[0], n], dtype=torch.int32), seq_starts=torch.tensor([0, 70], dtype=torch.int32),
+                 seq_slots=torch.tensor([2, 0], dtype=torch.int32))
+    extra = dict(frequencies=torch.tensor([50.0 ** (-2 * i / rot) for i in range(rot // 2)]), rot=rot, q_scale=0.9, k_scale=dim ** -0.5)
+    if mode == 'mlstm':
+        tiles, mats = -(-vdim // 16), heads * dim * vdim
+        tops = state[:, mats + heads * dim:].view(3, heads, tiles + 1)
+        tops[:] = tops[:, :, :1].clone()
+        extra.update(gates=torch.randn(n, 2 * heads, generator=g) * 3, gate_bias=torch.randn(2 * heads, generator=g), cap=6.0)
+    else:
+        extra.update(decay=torch.tensor([0.9, 0.999]))
+    on = lambda values: {k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in values.items()}
+    got_state, want_state = state.cuda(), state.clone()
+    want = refs.state_scan(proj, mode=mode, state=want_state, n_seqs=2, **where, **index, **extra)
+    got = ops.state_scan(proj.cuda(), mode=mode, state=got_state, n_seqs=2, max_query=max(counts), **where, **on(index), **on(extra))
+    # every result is a float32 sum of at most 256 (state rows) + 129 (keys) terms, made in another order: 2^-24 sqrt(385) = 1.2e-6
+    # of the largest partial sums on average, ten times that for the worst of 1e5 elements; the reference's own walk, which rounds
+    # the state once a token, is as far off
+    for a, b in ((got[0], want[0]), (got[1], want[1]), (got_state[[0, 2]], want_state[[0, 2]])):
+        if b is not None:
+            torch.testing.assert_close(a.cpu(), b, atol=2.4e-5 * max(1.0, b.abs().max().item()), rtol=2.4e-5)
+    assert torch.equal(got_state[1].cpu(), state[1])
