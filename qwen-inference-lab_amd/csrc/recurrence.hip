@@ -249,6 +249,49 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
   }
 }
 
+// The same with a wave a (row, head) and the head's elements in registers, four neighbours a lane and piece, all asked for
+// before one is taken.  The kernel above has a block for 256 elements, reads them twice and a gate behind a barrier: 3,044 rows
+// of 8 heads of 256 29.9 -> 16.0 us (50 MB), level (4.8) at 8 rows.  grid (rows x heads / waves a block).
+template <typename T, int PIECES>
+__global__ void __launch_bounds__(256)
+head_norm_gate_vec_kernel(const float* __restrict__ o, const float* __restrict__ below, const T* __restrict__ g, int g_row,
+                          int g_off, const float* __restrict__ weight, T* __restrict__ y, int n, int heads, int vdim,
+                          float eps, int act) {
+  const int lane = threadIdx.x % QIL_WAVE, at = blockIdx.x * (blockDim.x / QIL_WAVE) + threadIdx.x / QIL_WAVE;
+  if (at >= n * heads) return;
+  const int row = at / heads, h = at - row * heads;
+  const float* src = o + (size_t)at * vdim;
+  const T* gates = g + (size_t)row * g_row + g_off + h * vdim;
+  float4 v[PIECES], gate[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int j = min((p * QIL_WAVE + lane) * 4, vdim - 4);
+    v[p] = ld4(src + j);
+    gate[p] = ld4(gates + j);
+  }
+  const float divide = below ? below[at] : 1.f;
+  float squares = 0.f;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    v[p].x /= divide; v[p].y /= divide; v[p].z /= divide; v[p].w /= divide;
+    if ((p * QIL_WAVE + lane) * 4 < vdim) squares += v[p].x * v[p].x + v[p].y * v[p].y + v[p].z * v[p].z + v[p].w * v[p].w;
+  }
+  squares = wave_sum(squares);
+  const float unit = 1.f / sqrtf(squares / (float)vdim + eps);
+  auto gated = [&](float value, float z, float w) {
+    const float sig = 1.f / (1.f + expf(-z));
+    return value * unit * w * (act ? z * sig : sig);
+  };
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int j = (p * QIL_WAVE + lane) * 4;
+    if (j >= vdim) continue;
+    const float4 w = weight ? ld4(weight + h * vdim + j) : make_float4(1.f, 1.f, 1.f, 1.f);
+    st4(y + (size_t)at * vdim + j, make_float4(gated(v[p].x, gate[p].x, w.x), gated(v[p].y, gate[p].y, w.y),
+                                               gated(v[p].z, gate[p].z, w.z), gated(v[p].w, gate[p].w, w.w)));
+  }
+}
+
 extern "C" {
 
 // Floats of one state slot.
@@ -313,6 +356,26 @@ int qil_head_norm_gate(const float* o, const float* below, const void* g, int g_
                        int vdim, float eps, int act, int dtype, hipStream_t s) {
   if (n == 0 || heads == 0) return 0;
   if (vdim < 1) return -1;
+  const uintptr_t piece = dtype == QIL_F32 ? 16 : 8;             // bytes of four elements of the model's type
+  if (vdim % 4 == 0 && vdim <= 4 * 4 * QIL_WAVE && g_row % 4 == 0 && g_off % 4 == 0 &&
+      ((uintptr_t)o | (uintptr_t)weight) % 16 == 0 && ((uintptr_t)g | (uintptr_t)y) % piece == 0 &&
+      (size_t)n * heads <= INT32_MAX / 2) {
+    const dim3 grid(((unsigned)n * heads + 3) / 4);
+#define QIL_HNG(T, PIECES)                                                                                            \
+  hipLaunchKernelGGL((head_norm_gate_vec_kernel<T, PIECES>), grid, dim3(256), 0, s, o, below, (const T*)g, g_row, g_off, \
+                     weight, (T*)y, n, heads, vdim, eps, act)
+#define QIL_HNG_PIECES(T)                                                                                             \
+  do {                                                                                                                \
+    if (vdim <= 4 * QIL_WAVE) QIL_HNG(T, 1);                                                                          \
+    else if (vdim <= 8 * QIL_WAVE) QIL_HNG(T, 2);                                                                     \
+    else QIL_HNG(T, 4);                                                                                               \
+  } while (0)
+    if (dtype == QIL_F32) QIL_HNG_PIECES(float);
+    else QIL_HNG_PIECES(bf16_t);
+#undef QIL_HNG_PIECES
+#undef QIL_HNG
+    QIL_RETURN_LAUNCH_STATUS();
+  }
   const int threads = vdim >= 256 ? 256 : (vdim + 63) / 64 * 64;
   if (dtype == QIL_F32)
     hipLaunchKernelGGL(head_norm_gate_kernel<float>, dim3(n, heads), dim3(threads), 0, s, o, below, (const float*)g, g_row, g_off,

@@ -50,3 +50,24 @@ def test_blocks_of_tokens_on_the_matrix_cores(ops, dtype, mode, dim, vdim, count
         if b is not None:
             torch.testing.assert_close(a.cpu(), b, atol=2.4e-5 * max(1.0, b.abs().max().item()), rtol=2.4e-5)
     assert torch.equal(got_state[1].cpu(), state[1])
+
+
+# one, two and four pieces a lane, whole and not, a head's size and an offset that four elements do not divide (general kernel)
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('vdim', [4, 252, 256, 260, 512, 1020, 1024, 1028, 130])
+@pytest.mark.parametrize('offset', [0, 8, 2])
+def test_head_norms_and_gates_of_every_width(ops, dtype, vdim, offset):
+    n, heads = 5, 3                                              # 15 heads: the last block of four waves is not full
+    g = torch.Generator().manual_seed(vdim)
+    o = torch.randn(n, heads * vdim, generator=g) * 5
+    source = torch.randn(n, offset + heads * vdim + 4, generator=g).to(dtype)
+    weight, below = 1 + 0.3 * torch.randn(heads * vdim, generator=g), torch.rand(n, heads, generator=g) + 0.1
+    for gate, w, b in (('sigmoid', weight, below), ('silu', None, None)):
+        got = ops.head_norm_gate(o.cuda(), source.cuda(), gate_offset=offset, heads=heads, vdim=vdim, eps=1e-5, gate=gate, out_dtype=dtype,
+                                 weight=None if w is None else w.cuda(), denominators=None if b is None else b.cuda())
+        v = o.double().view(n, heads, vdim) / (1 if b is None else b.double()[..., None])
+        v = (v / (v.square().mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(n, -1) * (1 if w is None else w.double())
+        z = source[:, offset:offset + heads * vdim].double()
+        want = v * torch.sigmoid(z) * (z if gate == 'silu' else 1)
+        # a sum of vdim squares and a handful of roundings in float32, then one to the type
+        torch.testing.assert_close(got.double().cpu(), want, atol=1e-6, rtol=2e-6 if dtype == torch.float32 else 2.0 ** -8)
