@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "fused_qkv.h"
 #include "key_span.h"
 #include "qk_math.h"
 
@@ -34,32 +35,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define PLAN_MOST_ROWS 128                                 // rows a plan may share the blocks out to
 #define DEC_MAX_WAVES 8                                    // waves of a block; each takes every waves-th 32-key step
-
-// FUSED: the queries do not come from memory but from the partial sums of the q/k/v product, with the
-// head norm and the rotation made here (the arithmetic of qk_rope.hip, shared through qk_math.h); and the
-// wave that meets the row's own position makes the new key and value the same way, writes them into the
-// pages and uses them from its registers.  One kernel less per layer in a decode step.
-struct FusedQKV {
-  const float* qkv;                                        // [splits][rows][(heads + 2 kv_heads) d] partial sums
-  size_t split_stride;
-  int splits;
-  const float* q_weight;                                   // null: no head norm
-  const float* k_weight;
-  float eps;
-  const float* cos_table;                                  // null: no rotation
-  const float* sin_table;                                  // null with a cos_table: that holds rot / 2 frequencies
-  int rot;
-  int rotate_first;                                        // the rotation comes before the head norm
-  int writes;                                              // 0: the cache belongs to another layer, which wrote it
-  int row_elems;                                           // elements of a row of qkv (more than q, k and v where another
-                                                           // branch's columns follow; q alone for a reader without k and v)
-  int v_head;                                              // the head-sized piece of a row at which the values begin
-                                                           // (heads + kv_heads; heads: the values are the keys before norm
-                                                           // and rotation)
-  const float* bias;                                       // null, or the projection's bias by column, added to the sums
-  float temp_coef;                                         // temp_every > 0: the query at position p is multiplied by
-  int temp_every;                                          // 1 + temp_coef * ln(floor((p + 1) / temp_every) + 1) last
-};
 
 // Keys and values are read once a step by one block (the whole group of query heads is served by it).
 __device__ __forceinline__ uint4 once4(const bf16_t* p) {
@@ -74,7 +49,7 @@ __device__ __forceinline__ uint4 shuffle4(uint4 v, int source) {
                     __shfl(v.w, source, QIL_WAVE));
 }
 
-// WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
+// FUSED: fused_qkv.h.  WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
 template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false>
 __global__ void __launch_bounds__(DEC_MAX_WAVES * QIL_WAVE)
 attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_cache,

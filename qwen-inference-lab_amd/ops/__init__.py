@@ -887,10 +887,12 @@ def _places(max_context, window, keep_first):
 
 
 def _rows_part(rows, kv_heads, max_context):
-    """Keys a part of the row kernel: about ROWS_BLOCKS blocks in all, parts of 64 to ATTENTION_PART * 2 keys
-    (measured in float32 at 2,048 keys of 8 kv heads: 1 row 28 us with parts of 64 to 256 against 67 with 512;
-    8 rows 45 us with 128 against 54 with 256 and 62 with 64; 64 rows level from 256 on; 8 rows of 8,192 keys best
-    at 256 and 512)."""
+    """Keys a part of the row kernel and of the float32 matrix-core kernel: about ROWS_BLOCKS blocks in all, parts of 64 to
+    ATTENTION_PART * 2 keys (measured in float32 at 2,048 keys of 8 kv heads: 1 row 28 us with parts of 64 to 256 against 67 with
+    512; 8 rows 45 us with 128 against 54 with 256 and 62 with 64; 64 rows level from 256 on; 8 rows of 8,192 keys best
+    at 256 and 512.  The matrix-core kernel, 16 heads of 128 in 8 groups: 4 rows of 520 keys 9.5 us with 64, 11.1 with 128; 8 of
+    2,048 31.6 / 29.4 / 29.8 / 37.0 with 64 / 128 / 256 / 512; 64 of 2,048 238 / 215 / 195 / 179; a CU draws 36 GB/s at most, so
+    few blocks a CU's worth of keys each are slow: 4 rows of 520 in parts of 512 take 33)."""
     if ATTENTION_PART != 256:                          # a test or tuning run has set it
         return ATTENTION_PART
     wanted = max_context * rows * kv_heads / ROWS_BLOCKS
@@ -969,14 +971,17 @@ def _parts_workspace(rows, heads, head_dim, parts, plan, device):
 
 
 def decode_attention_takes(qkv, *, heads, kv_heads, head_dim, page_size, rotation, dtype):
-    """Whether ``decode_attention`` takes the step: a float32 ``Partials`` q/k/v product, bfloat16 caches, sizes of
-    the fused kernel."""
+    """Whether ``decode_attention`` takes the step: a float32 ``Partials`` q/k/v product, few rows, sizes of the fused
+    kernel of the caches' type."""
     rot = rotation.rot_dim if rotation is not None else 0
     source = qkv.source if isinstance(qkv, Columns) else qkv
     if isinstance(qkv, Columns) and (qkv.offset % 8 or qkv.row % 8):
         return False
-    return isinstance(source, Partials) and qkv.shape[0] <= FUSED_DECODE_MOST_ROWS and dtype == torch.bfloat16 and \
-        bool(library.load().qil_attn_decode_fused_takes(heads, kv_heads, head_dim, page_size, rot))
+    if not isinstance(source, Partials) or qkv.shape[0] > FUSED_DECODE_MOST_ROWS:
+        return False
+    if dtype == torch.float32:
+        return bool(library.load().qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 1, rot))
+    return dtype == torch.bfloat16 and bool(library.load().qil_attn_decode_fused_takes(heads, kv_heads, head_dim, page_size, rot))
 
 
 def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps, rotation, positions, writes, k_cache,
@@ -994,7 +999,7 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     multiplied by its sigmoid (before the rounding, where parts are merged), and comes back merged.  ``plans`` as in
     ``paged_attention``.  Returns what ``paged_attention`` returns."""
     n = qkv.shape[0]
-    dtype = torch.bfloat16
+    dtype = k_cache.dtype
     stored = kv_heads if has_kv else 0
     own = (heads + (1 if values_are_keys else 2) * stored) * head_dim
     if writes and not has_kv:
@@ -1022,15 +1027,23 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     lib = library.load()
     out = torch.empty((n, heads * head_dim), dtype=dtype, device=k_cache.device)
     window_arg = int(window or 0)
-    part, parts, blocks, plan = _decode_shares(n, kv_heads, _places(max_context, window, keep), window_arg, positions, None, plans)
-    workspace = _parts_workspace(n, heads, head_dim, parts, plan, out.device)
-    _check(lib.qil_attn_decode_fused(pointer, splits, _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(cos),
-                                     _ptr(sin), rot, int(bool(writes)), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
-                                     block_tables.shape[1], _ptr(row_seq), _ptr(positions), _ptr(workspace), _ptr(out),
-                                     n, heads, kv_heads, head_dim, page_size, window_arg, float(scale), part, parts,
-                                     DECODE_WAVES, int(bool(rotate_first)), float(softcap or 0.0), int(bool(has_kv)), row - own,
-                                     _ptr(bias), float(coef), int(every), _ptr(sinks), int(bool(values_are_keys)),
-                                     _ptr(slopes), keep, _ptr(plan), blocks, _stream()), 'attn_decode_fused')
+    places = _places(max_context, window, keep)
+    sums = (pointer, splits, _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(cos), _ptr(sin), rot, int(bool(writes)))
+    where = (_ptr(k_cache), _ptr(v_cache), _ptr(block_tables), block_tables.shape[1], _ptr(row_seq), _ptr(positions))
+    forms = (int(bool(rotate_first)), float(softcap or 0.0), int(bool(has_kv)), row - own, _ptr(bias), float(coef), int(every),
+             _ptr(sinks), int(bool(values_are_keys)), _ptr(slopes), keep)
+    if dtype == torch.float32:
+        part = _rows_part(n, kv_heads, places)
+        parts = max(1, -(-places // part))
+        workspace = _parts_workspace(n, heads, head_dim, parts, None, out.device)
+        _check(lib.qil_attn_decode_f32_fused(*sums, *where, _ptr(workspace), _ptr(out), n, heads, kv_heads, head_dim, page_size,
+                                             window_arg, float(scale), part, parts, *forms, _stream()), 'attn_decode_f32_fused')
+    else:
+        part, parts, blocks, plan = _decode_shares(n, kv_heads, places, window_arg, positions, None, plans)
+        workspace = _parts_workspace(n, heads, head_dim, parts, plan, out.device)
+        _check(lib.qil_attn_decode_fused(*sums, *where, _ptr(workspace), _ptr(out), n, heads, kv_heads, head_dim, page_size,
+                                         window_arg, float(scale), part, parts, DECODE_WAVES, *forms, _ptr(plan), blocks,
+                                         _stream()), 'attn_decode_fused')
     if parts > 1:
         if sinks is not None or keep or gate is not None:
             # the merge adds the sinks' term and multiplies by the gate; its parts count places
@@ -1193,6 +1206,21 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
             parts = max(1, -(-places // part))
             nbytes = lib.qil_attn_rows_workspace(rows, heads, head_dim, parts)
             workspace = torch.empty(nbytes // 4, dtype=torch.float32, device=qkv.device) if nbytes else None
+            # heads of 64 and 128 float32 elements run on the matrix cores (caches begin at multiples of 16 bytes)
+            if qkv.dtype == torch.float32 and not (_ptr(qkv) | _ptr(k_cache) | _ptr(v_cache)) & 15 and \
+                    lib.qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 0, 0) and part % 32 == 0:
+                _check(lib.qil_attn_decode_f32(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
+                                               block_tables.shape[1], _ptr(row_seq), _ptr(positions), _ptr(single_rows),
+                                               _ptr(workspace), _ptr(out), rows, heads, kv_heads, head_dim, page_size, window_arg,
+                                               float(scale), part, parts, cap, _ptr(sinks), _ptr(slopes), keep, _stream()),
+                       'attn_decode_f32')
+                if unmerged and slopes is None and parts > 1 and single_rows is None and rows <= UNMERGED_ROWS_MOST:
+                    return Unmerged(workspace, positions, out, heads=heads, head_dim=head_dim, window=window_arg,
+                                    part=part, parts=parts)
+                _check(lib.qil_attn_merge(_ptr(workspace), _ptr(positions), _ptr(single_rows), _ptr(out), rows, heads,
+                                          head_dim, window_arg, part, parts, _code(qkv.dtype), _ptr(sinks), keep,
+                                          *_NO_GATE, _stream()), 'attn_merge')
+                return out
             if unmerged and slopes is None and parts > 1 and single_rows is None and rows <= UNMERGED_ROWS_MOST:
                 _check(lib.qil_attn_rows_unmerged(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache),
                                                   _ptr(block_tables), block_tables.shape[1], _ptr(row_seq),

@@ -227,6 +227,10 @@ def _declare(lib):
     lib.qil_attn_decode_takes.argtypes = [i, i, i, i]
     lib.qil_attn_decode_takes.restype = i
     lib.qil_attn_decode.argtypes = [p, i, p, p, p, i, p, p, p, p, p, i, i, i, i, i, i, f, i, i, i, f, p, p, i, p, i, p]
+    lib.qil_attn_decode_f32_takes.argtypes = [i, i, i, i, i, i]
+    lib.qil_attn_decode_f32_takes.restype = i
+    lib.qil_attn_decode_f32.argtypes = [p, i, p, p, p, i, p, p, p, p, p, i, i, i, i, i, i, f, i, i, f, p, p, i, p]
+    lib.qil_attn_decode_f32_fused.argtypes = [p, i, p, p, f, p, p, i, i, p, p, p, i, p, p, p, p, i, i, i, i, i, i, f, i, i, i, f, i, i, p, f, i, p, i, p, i, p]
     lib.qil_attn_plan.argtypes = [p, p, i, i, i, p, p]
     lib.qil_attn_tile.argtypes = [p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, f, f, i, p, p, i, p]
     lib.qil_gemm_f32.argtypes = [p, p, p, p, i, i, i, i, p]
@@ -411,5 +415,5 @@ def _declare(lib):
     lib.qil_sample_static_prepare.argtypes = []
     lib.qil_sample_static_prepare.restype = i
     for name in ('qil_embed', 'qil_add_rmsnorm', 'qil_silu_mul', 'qil_add_bias', 'qil_qk_norm_rope_store',
-                 'qil_attn_rows', 'qil_attn_merge', 'qil_attn_decode', 'qil_attn_decode_fused', 'qil_attn_tile', 'qil_gemm_f32', 'qil_gemm_bf16', 'qil_gemm_bf16_gated', 'qil_gemm_bf16_unmerged', 'qil_gemm_bf16_normed', 'qil_gemm_bf16_add', 'qil_sample'):
+                 'qil_attn_rows', 'qil_attn_merge', 'qil_attn_decode', 'qil_attn_decode_fused', 'qil_attn_decode_f32', 'qil_attn_decode_f32_fused', 'qil_attn_tile', 'qil_gemm_f32', 'qil_gemm_bf16', 'qil_gemm_bf16_gated', 'qil_gemm_bf16_unmerged', 'qil_gemm_bf16_normed', 'qil_gemm_bf16_add', 'qil_sample'):
         getattr(lib, name).restype = i
