@@ -196,7 +196,8 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
 // buffers are 160 KB exactly: the logits of up to 8 rows at 8B sizes run here unsplit).  The fragment-layout kernel above touches half a cache line per row and load and
 // reaches about 3 TB/s at 8B layer sizes; this one streams at 4.3 to 5.6.  Always writes partial sums
 // C[split, M, N] (one split: the product itself).
-#define FL_WAVES 8                                         // waves of a block: 8, or FL_WIDE_WAVES where fl_plan says so
+#define FL_WAVES 8                                         // waves of a block: 8, or what fl_waves says
+#define FL_NARROW_WAVES 4                                  // small products: twice the blocks
 #define FL_WIDE_WAVES 16                                   // one such block fills a CU: A's slice is staged once for 256 columns
 #define FL_STAGE 64                                        // columns of a stage
 #define FL_PAD 4                                           // floats between rows of a stage of A (the 17-to-64-row kernel)
@@ -493,7 +494,7 @@ static size_t fl_lds_bytes(int M, int K, int splits, int waves = FL_WAVES) {
 static bool fl_takes(int M, int N, int K, int splits, int waves = FL_WAVES, bool all_lds = false) {
   return M >= 1 && M <= 16 && N >= 1 && splits >= 1 && K % (FL_STAGE * splits) == 0 &&
          K / (FL_STAGE * splits) >= FL_DEPTH &&
-         fl_lds_bytes(M, K, splits, waves) <= (waves == FL_WAVES && !all_lds ? FL_LDS_LIMIT : FL_WIDE_LDS_LIMIT);
+         fl_lds_bytes(M, K, splits, waves) <= (waves != FL_WIDE_WAVES && !all_lds ? FL_LDS_LIMIT : FL_WIDE_LDS_LIMIT);
 }
 
 // How well the blocks of `splits` splits and `waves` waves fill their rounds of 256 CUs, less 1.5 % a split for what
@@ -507,11 +508,20 @@ static double fl_score(int M, int N, int K, int splits, int waves) {
   return (double)blocks / (double)slots - 0.015 * splits;
 }
 
-// The waves of a block for a product in `splits` splits: 8, or 16 where only such blocks make one full round of the
+// Products of at most 16 MB take blocks of 4 waves where those fill more CUs: a CU draws 36 GB/s at most, and 64 or 128 blocks of
+// 131 KB each wait for that.  4 rows: 4,096 x 1,024 in four splits 6.7 us with 128 blocks of 8 waves, 5.9 with 256 of 4; 1,024 x
+// 2,048 in eight 6.1 with 64, 4.8 with 128; 1,024 x 3,072 5.8 in 16 splits of 8 blocks, 5.2 in 12 of 16 (16 rows 7.0 / 6.4, 6.3 /
+// 5.3, 6.0 / 5.8).  Larger ones stream for longer than their blocks start and end: 6,144 x 1,024 level, 6,144 x 4,096 20.9 us in
+// 192 blocks of 8 waves, 24.5 in 192 of 4.
+#define FL_NARROW_PRODUCT ((size_t)4 << 20)
+
+// The waves of a block for a product in `splits` splits: 8, 4 for small products, or 16 where only such blocks make one full round of the
 // chip.  Measured with the gate and up products of 8B layer sizes (403 MB, 8 rows): 768 blocks of 8 waves in 4 splits,
 // two a CU and then a third, 81.3 us; 192 blocks of 16 waves in 2 splits, one a CU, 70.3.  Up to 8 rows only: with 16
 // rows of A in LDS the down product in 192 wide blocks of 12 splits took 39.2 us against 37.4 in 512 blocks of 8 waves.
 static int fl_waves(int M, int N, int K, int splits) {
+  if ((size_t)N * K <= FL_NARROW_PRODUCT && fl_score(M, N, K, splits, FL_NARROW_WAVES) > fl_score(M, N, K, splits, FL_WAVES))
+    return FL_NARROW_WAVES;
   return M <= 8 && fl_score(M, N, K, splits, FL_WIDE_WAVES) > fl_score(M, N, K, splits, FL_WAVES) ? FL_WIDE_WAVES : FL_WAVES;
 }
 
@@ -548,6 +558,7 @@ static int launch_f32_lines(const float* A, UnmergedA unmerged, GatedA gated, co
                             int splits, hipStream_t s) {
   const int waves = fl_waves(M, N, K, splits);
   if (!fl_takes(M, N, K, splits, waves, splits == 1)) return -1;
+  if (waves == FL_NARROW_WAVES) return launch_f32_lines_waves<ASRC, FL_NARROW_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s);
   return waves == FL_WAVES ? launch_f32_lines_waves<ASRC, FL_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s)
                            : launch_f32_lines_waves<ASRC, FL_WIDE_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s);
 }
@@ -610,7 +621,7 @@ static bool mfma_wanted(int M, int N, int K, int splits) {
   return matrix < vector;
 }
 
-// Waves of a block of the whole-line kernel for a product of up to 16 rows in `splits` splits (8 or 16; 0: another
+// Waves of a block of the whole-line kernel for a product of up to 16 rows in `splits` splits (4, 8 or 16; 0: another
 // kernel runs it).
 extern "C" int qil_gemm_f32_waves(int M, int N, int K, int splits) {
   if (M < 1 || M > 16 || K % 4 || splits < 1) return 0;

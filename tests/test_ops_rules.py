@@ -140,3 +140,13 @@ def test_whole_products_of_few_rows_that_cannot_split_k(lib):
             assert lib.qil_gemm_bf16_whole_takes(rows, columns, 1280) and lib.qil_gemm_bf16_whole_takes(rows, columns, 2304)
             assert lib.qil_gemm_bf16_whole_takes(rows, columns, 4480) == (rows <= 8)
         assert lib.qil_gemm_bf16_whole_takes(rows, 4112, 1152) and lib.qil_gemm_bf16_whole_takes(rows, 12288, 4480)
+
+
+def test_small_float32_products_take_narrow_blocks(lib):
+    """Blocks of 4 waves where those fill more CUs and the weights are at most 16 MB, else of 8 (or 16 for one full round)."""
+    waves = lambda rows, n, k: lib.qil_gemm_f32_waves(rows, n, k, lib.qil_gemm_f32_splits(rows, n, k))
+    for rows in (1, 4, 16):
+        assert waves(rows, 4096, 1024) == waves(rows, 1024, 2048) == waves(rows, 1024, 3072) == 4
+        assert waves(rows, 4096, 1088) == 8                        # a stage more than 16 MB
+        assert waves(rows, 6144, 1024) == 8
+    assert lib.qil_gemm_f32_splits(4, 1024, 3072) == 12
