@@ -18,6 +18,11 @@ __device__ __forceinline__ float gated_act(float g, float u, int act, float limi
   return (g / (1.f + expf(-g))) * u;
 }
 
+// A gate function and its numbers, as product kernels with the activation in their epilogue take them.
+struct GateFn { int act; float limit, alpha; };
+__device__ __forceinline__ float gated_act(float g, float u, const GateFn& fn) { return gated_act(g, u, fn.act, fn.limit, fn.alpha); }
+inline bool gate_fn_known(int act) { return act == QIL_ACT_SILU || act == QIL_ACT_CLAMPED || act == QIL_ACT_RELU; }
+
 // Activations of experts without a gate branch, by code from QIL_ACT_RELU_SQUARED on:
 //   QIL_ACT_RELU_SQUARED  max(z, 0)^2
 __device__ __forceinline__ float ungated_act(float z, int act) {

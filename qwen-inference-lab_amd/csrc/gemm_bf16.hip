@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gated_act.h"
 #include "merge_parts.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -365,8 +366,8 @@ static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, 
 #define CHUNKS_MOST_ROWS 192
 
 // GATED: W is the [N = 2 inner, K] matrix of a gated feed-forward with gate and up rows interleaved in tiles of 16
-// (gate rows 0-15, up rows 0-15, gate rows 16-31, ...), and C [M, inner] gets silu(A gate^T) * (A up^T)
-// (qil/model.py:71).  A block then owns 64 columns of `inner`, 128 consecutive rows of W: the even waves make gate
+// (gate rows 0-15, up rows 0-15, gate rows 16-31, ...), and C [M, inner] gets act(A gate^T, A up^T)
+// (gated_act.h; qil/model.py:71).  A block then owns 64 columns of `inner`, 128 consecutive rows of W: the even waves make gate
 // products, the odd waves the up products that belong to them; these hand their sums over in LDS and the even waves
 // store the activations.  K is not split: no partial sums in memory and no separate activation pass.  (With the gate
 // rows stacked before the up rows a block would read two regions a power of two apart at the same columns at the
@@ -374,7 +375,7 @@ static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, 
 template <typename OUT, int MT, bool GATED = false>
 __global__ void __launch_bounds__(LINES_WAVES * QIL_WAVE)
 gemm_bf16_chunks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N,
-                        int K, int cols_per_split) {
+                        int K, int cols_per_split, GateFn fn) {
   extern __shared__ __align__(16) bf16_t lds[];            // two stages of A [16 MT][128 + pad], then the waves' buffers
   constexpr int A_ROWS = 16 * MT, SLOT = A_ROWS * CHUNK_ROW;
   constexpr int PIECES = A_ROWS * 16 / (LINES_WAVES * QIL_WAVE);   // 16-byte pieces of a stage of A per thread
@@ -493,7 +494,7 @@ gemm_bf16_chunks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__
         for (int i = 0; i < 4; ++i) {
           const int m = t * 16 + 4 * kb + i, n = inner_n0 + r;
           const float g = acc[t][i];
-          if (m < M && n < inner) store_out(C + (size_t)m * inner + n, (g / (1.f + expf(-g))) * up[i]);
+          if (m < M && n < inner) store_out(C + (size_t)m * inner + n, gated_act(g, up[i], fn));
         }
       }
     }
@@ -529,7 +530,7 @@ static int chunks_splits(int N, int K) {
 }
 
 template <typename OUT, int MT, bool GATED = false>
-static int launch_chunks_tiles(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s) {
+static int launch_chunks_tiles(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, GateFn fn, hipStream_t s) {
   const size_t lds = ((size_t)2 * 16 * MT * CHUNK_ROW + (size_t)LINES_WAVES * 16 * 128) * sizeof(bf16_t);
   auto kernel = gemm_bf16_chunks_kernel<OUT, MT, GATED>;
   static size_t granted = 0;                              // per instantiation
@@ -540,23 +541,23 @@ static int launch_chunks_tiles(const bf16_t* A, const bf16_t* W, OUT* C, int M, 
   }
   // GATED: a block owns 64 columns of the result (N / 2 of them), else 128 of N
   dim3 grid(GATED ? (N / 2 + 63) / 64 : (N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES), 1, splits);
-  hipLaunchKernelGGL(kernel, grid, dim3(LINES_WAVES * QIL_WAVE), lds, s, A, W, C, M, N, K, K / splits);
+  hipLaunchKernelGGL(kernel, grid, dim3(LINES_WAVES * QIL_WAVE), lds, s, A, W, C, M, N, K, K / splits, fn);
   return 0;
 }
 
 template <typename OUT, bool GATED = false>
-static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s) {
-  if (M <= 32) return launch_chunks_tiles<OUT, 2, GATED>(A, W, C, M, N, K, splits, s);
-  if (M <= 64) return launch_chunks_tiles<OUT, 4, GATED>(A, W, C, M, N, K, splits, s);
-  if (M <= 96) return launch_chunks_tiles<OUT, 6, GATED>(A, W, C, M, N, K, splits, s);
-  if (M <= 128) return launch_chunks_tiles<OUT, 8, GATED>(A, W, C, M, N, K, splits, s);
-  if (M <= 160) return launch_chunks_tiles<OUT, 10, GATED>(A, W, C, M, N, K, splits, s);
-  return launch_chunks_tiles<OUT, 12, GATED>(A, W, C, M, N, K, splits, s);
+static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s, GateFn fn = {}) {
+  if (M <= 32) return launch_chunks_tiles<OUT, 2, GATED>(A, W, C, M, N, K, splits, fn, s);
+  if (M <= 64) return launch_chunks_tiles<OUT, 4, GATED>(A, W, C, M, N, K, splits, fn, s);
+  if (M <= 96) return launch_chunks_tiles<OUT, 6, GATED>(A, W, C, M, N, K, splits, fn, s);
+  if (M <= 128) return launch_chunks_tiles<OUT, 8, GATED>(A, W, C, M, N, K, splits, fn, s);
+  if (M <= 160) return launch_chunks_tiles<OUT, 10, GATED>(A, W, C, M, N, K, splits, fn, s);
+  return launch_chunks_tiles<OUT, 12, GATED>(A, W, C, M, N, K, splits, fn, s);
 }
 
 // ---------------------------------------------------------------------------------------------------
 // Gate and up products of a gated feed-forward with the activation in the epilogue:
-//   out[m, n] = silu(A W[n]^T) * (A W[inner + n]^T),  n < inner        (qil/model.py:71)
+//   out[m, n] = act(A W[n]^T, A W[inner + n]^T),  n < inner        (gated_act.h; qil/model.py:71)
 // W is the [2 inner, K] matrix with the gate rows stacked before the up rows, or with both interleaved in tiles of
 // 16 rows (gate rows 0-15, up rows 0-15, gate rows 16-31, ...).  A "pair" is 16 gate rows and the 16 up rows
 // that belong to them.  A block owns `pairs` consecutive pairs and `ksplit` waves per pair, which split
@@ -573,7 +574,7 @@ static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N,
 template <typename OUT>
 __global__ void __launch_bounds__(GATED_MAX_WAVES * QIL_WAVE)
 gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ out, int M,
-                       int inner, int K, int ksplit, int interleaved) {
+                       int inner, int K, int ksplit, int interleaved, GateFn fn) {
   extern __shared__ __align__(16) bf16_t lds[];            // A [8 or 16][K + pad], then a 4 KB buffer per wave
   const int a_rows = M <= 8 ? 8 : 16;                      // rows of A kept (8 or 16: a power of two)
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
@@ -697,7 +698,7 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = 4 * kb + i, n = n0 + r;                 // lane holds D[m = 4 kb + i][n = r]
-      if (m < M) store_out(out + (size_t)m * inner + n, (g[i] / (1.f + expf(-g[i]))) * v[i]);
+      if (m < M) store_out(out + (size_t)m * inner + n, gated_act(g[i], v[i], fn));
     }
   }
 }
@@ -794,16 +795,19 @@ extern "C" int qil_gemm_bf16_gated_takes(int M, int inner, int K, int interleave
          gated_rows_takes(nullptr, nullptr, M, inner, K, interleaved, 0);
 }
 
-// out [M, inner] of out_dtype = silu(A W[:inner]^T) * (A W[inner:]^T).  pairs, ksplit: 0 = chosen here
-// (tuning runs set them).
-extern "C" int qil_gemm_bf16_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype,
-                                   int pairs, int ksplit, int interleaved, hipStream_t s) {
+// out [M, inner] of out_dtype = act(A W[:inner]^T, A W[inner:]^T), act, limit, alpha: a gate function of gated_act.h.
+// pairs, ksplit: 0 = chosen here (tuning runs set them).
+extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype,
+                                       int pairs, int ksplit, int interleaved, int act, float limit, float alpha,
+                                       hipStream_t s) {
+  if (!gate_fn_known(act)) return -1;
+  const GateFn fn{act, limit, alpha};
   if (M == 0 || inner == 0) return 0;
   if (M > 16) {                                              // pairs: the fewest blocks to accept (tests pass 1)
     if (!gated_rows_takes(A, W, M, inner, K, interleaved, pairs)) return -1;
     const int status = out_dtype == QIL_F32
-                           ? launch_chunks<float, true>((const bf16_t*)A, (const bf16_t*)W, (float*)out, M, 2 * inner, K, 1, s)
-                           : launch_chunks<bf16_t, true>((const bf16_t*)A, (const bf16_t*)W, (bf16_t*)out, M, 2 * inner, K, 1, s);
+                           ? launch_chunks<float, true>((const bf16_t*)A, (const bf16_t*)W, (float*)out, M, 2 * inner, K, 1, s, fn)
+                           : launch_chunks<bf16_t, true>((const bf16_t*)A, (const bf16_t*)W, (bf16_t*)out, M, 2 * inner, K, 1, s, fn);
     if (status) return status;
     QIL_RETURN_LAUNCH_STATUS();
   }
@@ -825,11 +829,17 @@ extern "C" int qil_gemm_bf16_gated(const void* A, const void* W, void* out, int 
       if (e != hipSuccess) return (int)e;                                                                            \
       granted = lds;                                                                                                 \
     }                                                                                                                \
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, inner, K, ksplit, interleaved); \
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, inner, K, ksplit, interleaved, fn); \
   }
   if (out_dtype == QIL_F32) QIL_GATED_CASE(float) else QIL_GATED_CASE(bf16_t)
 #undef QIL_GATED_CASE
   QIL_RETURN_LAUNCH_STATUS();
+}
+
+// silu(A W[:inner]^T) * (A W[inner:]^T)
+extern "C" int qil_gemm_bf16_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype,
+                                   int pairs, int ksplit, int interleaved, hipStream_t s) {
+  return qil_gemm_bf16_gated_act(A, W, out, M, inner, K, out_dtype, pairs, ksplit, interleaved, QIL_ACT_SILU, 0.f, 1.f, s);
 }
 
 // Shapes of the kernel that exist: code = MT * 100 + NT * 10 + UNROLL.

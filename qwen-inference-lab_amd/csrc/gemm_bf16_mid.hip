@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "gated_act.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -50,14 +51,14 @@ __host__ __device__ constexpr int mid_a_ring(int mt) {
 
 // MT: row tiles of 32 (M <= 32 MT).  OUT: float (partial sums or the result) or bf16_t (the result, one split).
 // GATED (one split): W holds gate and up rows in turns of 16, a wave's 32 columns are 16 of each, and C [M, N / 2]
-// gets silu(gate) * up (qil/model.py:71), both still in float32.
+// gets act(gate, up) (gated_act.h; qil/model.py:71), both still in float32.
 // Waves 0 to 3 multiply, each with a ring of W of its own; wave 4 loads A for all of them.  A wave waits for its
 // loads by their number in flight (vmcnt counts in order), so loads that must land soon (A, from L2, three stages
 // in LDS) and loads that are sent far ahead (W, from memory) belong to different waves.
 template <int MT, typename OUT, bool GATED>
 __global__ void __launch_bounds__((MID_WAVES + 1) * QIL_WAVE, 1)
 gemm_bf16_mid_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M_all, int N, int K,
-                     int stages, int waves, int turns) {
+                     int stages, int waves, int turns, GateFn fn) {
   constexpr int RW = mid_w_ring(MT), RA = mid_a_ring(MT);
   // more than 32 MT rows: grid.z counts blocks of 32 MT rows, each a product of its own over the same W
   const int row0 = blockIdx.z * (32 * MT), M = min(M_all - row0, 32 * MT);
@@ -178,8 +179,7 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float gate = acc[t][4 * g + e];
-          v[e] = (gate / (1.f + expf(-gate))) * acc[t][4 * (g + 2) + e];
+          v[e] = gated_act(acc[t][4 * g + e], acc[t][4 * (g + 2) + e], fn);
         }
         if constexpr (sizeof(OUT) == 4) *reinterpret_cast<float4*>(row + 8 * g) = make_float4(v[0], v[1], v[2], v[3]);
         else *reinterpret_cast<uint2*>(row + 8 * g) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
@@ -230,7 +230,7 @@ static bool mid_plan(int M, int N, int K, int* waves, int* splits) {
 }
 
 template <int MT, typename OUT, bool GATED>
-static int mid_launch(const void* A, const void* W, void* C, int M, int N, int K, int waves, int splits, hipStream_t s) {
+static int mid_launch(const void* A, const void* W, void* C, int M, int N, int K, int waves, int splits, GateFn fn, hipStream_t s) {
   const size_t lds = (size_t)mid_w_ring(MT) * MID_WAVES * 4096 + (size_t)mid_a_ring(MT) * MT * 4096;
   auto kernel = gemm_bf16_mid_kernel<MT, OUT, GATED>;
   static bool granted = false;                             // per instantiation
@@ -241,17 +241,17 @@ static int mid_launch(const void* A, const void* W, void* C, int M, int N, int K
   }
   dim3 grid((N / 32 + waves - 1) / waves, splits, (M + 32 * MT - 1) / (32 * MT));
   hipLaunchKernelGGL(kernel, grid, dim3((waves + 1) * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N, K,
-                     K / MID_STAGE / splits, waves, splits == 1 ? MID_TURNS : 1);
+                     K / MID_STAGE / splits, waves, splits == 1 ? MID_TURNS : 1, fn);
   QIL_RETURN_LAUNCH_STATUS();
 }
 
 template <bool GATED>
 static int mid_dispatch(const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int waves, int splits,
-                        hipStream_t s) {
+                        hipStream_t s, GateFn fn = {}) {
 #define QIL_MID_CASE(MT)                                                                                      \
   case MT:                                                                                                    \
-    return out_dtype == QIL_F32 ? mid_launch<MT, float, GATED>(A, W, C, M, N, K, waves, splits, s)            \
-                                : mid_launch<MT, bf16_t, GATED>(A, W, C, M, N, K, waves, splits, s)
+    return out_dtype == QIL_F32 ? mid_launch<MT, float, GATED>(A, W, C, M, N, K, waves, splits, fn, s)        \
+                                : mid_launch<MT, bf16_t, GATED>(A, W, C, M, N, K, waves, splits, fn, s)
   // more than 256 rows: blocks of rows of equal size (300 rows: two of 160)
   const int row_blocks = (M + MID_MOST_ROWS - 1) / MID_MOST_ROWS;
   switch (((M + 31) / 32 + row_blocks - 1) / row_blocks) {
@@ -314,14 +314,22 @@ int qil_gemm_bf16_mid_gated_takes(int M, int inner, int K) {
          (2 * inner / 32 + waves - 1) / waves >= 192;
 }
 
-// out [M, inner] of out_dtype = silu(A gate^T) * (A up^T) for W [2 inner, K] with gate and up rows in turns of 16.
-int qil_gemm_bf16_mid_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, hipStream_t s) {
+// out [M, inner] of out_dtype = act(A gate^T, A up^T) for W [2 inner, K] with gate and up rows in turns of 16; act, limit,
+// alpha: a gate function of gated_act.h.
+int qil_gemm_bf16_mid_gated_act(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, int act,
+                                float limit, float alpha, hipStream_t s) {
+  if (!gate_fn_known(act)) return -1;
   if (M == 0 || inner == 0) return 0;
   int waves = 0, splits = 1;
   if (!qil_gemm_bf16_mid_gated_takes(M, inner, K) || !mid_plan(M, 2 * inner, K, &waves, &splits) ||
       ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16 || (out_dtype != QIL_F32 && out_dtype != QIL_BF16))
     return -1;
-  return mid_dispatch<true>(A, W, out, M, 2 * inner, K, out_dtype, waves, 1, s);
+  return mid_dispatch<true>(A, W, out, M, 2 * inner, K, out_dtype, waves, 1, s, GateFn{act, limit, alpha});
+}
+
+// silu(A gate^T) * (A up^T)
+int qil_gemm_bf16_mid_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, hipStream_t s) {
+  return qil_gemm_bf16_mid_gated_act(A, W, out, M, inner, K, out_dtype, QIL_ACT_SILU, 0.f, 1.f, s);
 }
 
 }  // extern "C"

@@ -47,6 +47,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "gated_act.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -61,11 +62,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // RT, CT: tiles of 32 rows and of 32 columns of a wave; DOWN, ACROSS: the block's waves above each other and side by side;
 // AHEAD: stages (even) that a pair's loads go out ahead.  OUT: bf16_t or float (the result; with splits of K float32 partial sums [split][M][N]).  GATED (one split): W holds gate and up rows in turns of 16, a tile of 32 columns is 16
-// of each, and C [M, N / 2] gets silu(gate) * up (qil/model.py:71), both still in float32.
+// of each, and C [M, N / 2] gets act(gate, up) (gated_act.h; qil/model.py:71), both still in float32.
 template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
 __global__ void __launch_bounds__(DOWN * ACROSS * QIL_WAVE, RT * CT <= 4 && AHEAD == 2 ? 2 : 1)
 gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M_all, int N, int K,
-                      int stages, int col_blocks, int row_blocks, int splits, int patch_rows, int patch_cols) {
+                      int stages, int col_blocks, int row_blocks, int splits, int patch_rows, int patch_cols, GateFn fn) {
   constexpr int WAVES = DOWN * ACROSS;
   constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;            // rows and columns of C a block
   constexpr int A_BYTES = ROWS * WIDE_ROW_BYTES, SLOT = A_BYTES + TILE * WIDE_ROW_BYTES;
@@ -234,8 +235,7 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if constexpr (GATED) {                           // columns 0-15 of a tile are gates, 16-31 the ups that belong to them
-            const float gate = acc[i][j][4 * g + e];
-            v[e] = (gate / (1.f + expf(-gate))) * acc[i][j][4 * (g + 2) + e];
+            v[e] = gated_act(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e], fn);
           } else {
             v[e] = acc[i][j][4 * g + e];
           }
@@ -311,7 +311,7 @@ static bool wide_wanted(int M, int N, int K, double us, bool gated) {
 }
 
 template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
-static int wide_launch(const void* A, const void* W, void* C, int M, int N, int K, int splits, hipStream_t s) {
+static int wide_launch(const void* A, const void* W, void* C, int M, int N, int K, int splits, GateFn fn, hipStream_t s) {
   constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;
   const size_t lds = (size_t)(AHEAD + 3) * (ROWS + TILE) * WIDE_ROW_BYTES;
   auto kernel = gemm_bf16_wide_kernel<OUT, RT, CT, DOWN, ACROSS, AHEAD, GATED>;
@@ -323,16 +323,17 @@ static int wide_launch(const void* A, const void* W, void* C, int M, int N, int 
   }
   const WideGrid g = wide_grid(M, N, ROWS, TILE, splits);
   hipLaunchKernelGGL(kernel, dim3(g.blocks), dim3(DOWN * ACROSS * QIL_WAVE), lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)C, M, N,
-                     K, K / WIDE_STAGE / splits, g.col_blocks, g.row_blocks, splits, g.patch_rows, g.patch_cols);
+                     K, K / WIDE_STAGE / splits, g.col_blocks, g.row_blocks, splits, g.patch_rows, g.patch_cols, fn);
   QIL_RETURN_LAUNCH_STATUS();
 }
 
 template <bool GATED>
-static int wide_dispatch(int shape, const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s) {
+static int wide_dispatch(int shape, const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s,
+                         GateFn fn = {}) {
 #define QIL_WIDE_CASE(SHAPE, RT, CT, DOWN, ACROSS, AHEAD)                                                             \
   case SHAPE:                                                                                                         \
-    return out_dtype == QIL_F32 ? wide_launch<float, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, s) \
-                                : wide_launch<bf16_t, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, s)
+    return out_dtype == QIL_F32 ? wide_launch<float, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, fn, s) \
+                                : wide_launch<bf16_t, RT, CT, DOWN, ACROSS, AHEAD, GATED>(A, W, C, M, N, K, splits, fn, s)
   switch (shape) {
     QIL_WIDE_CASE(WIDE_256, 4, 2, 2, 4, 2);
     QIL_WIDE_CASE(WIDE_128, 2, 2, 2, 2, 2);
@@ -416,13 +417,21 @@ int qil_gemm_bf16_wide_gated_wanted(int M, int inner, int K) {
          wide_wanted(M, 2 * inner, K, wide_us(M, 2 * inner, K, 1, wide_shape(M, 2 * inner, K, 1)), true);
 }
 
-// out [M, inner] of out_dtype = silu(A gate^T) * (A up^T) for W [2 inner, K] with gate and up rows in turns of 16.
-int qil_gemm_bf16_wide_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, hipStream_t s) {
+// out [M, inner] of out_dtype = act(A gate^T, A up^T) for W [2 inner, K] with gate and up rows in turns of 16; act, limit,
+// alpha: a gate function of gated_act.h.
+int qil_gemm_bf16_wide_gated_act(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, int act,
+                                 float limit, float alpha, hipStream_t s) {
+  if (!gate_fn_known(act)) return -1;
   if (M == 0 || inner == 0) return 0;
   if (!qil_gemm_bf16_wide_gated_takes(M, inner, K) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16 ||
       (out_dtype != QIL_F32 && out_dtype != QIL_BF16))
     return -1;
-  return wide_dispatch<true>(wide_shape(M, 2 * inner, K, 1), A, W, out, M, 2 * inner, K, out_dtype, 1, s);
+  return wide_dispatch<true>(wide_shape(M, 2 * inner, K, 1), A, W, out, M, 2 * inner, K, out_dtype, 1, s, GateFn{act, limit, alpha});
+}
+
+// silu(A gate^T) * (A up^T)
+int qil_gemm_bf16_wide_gated(const void* A, const void* W, void* out, int M, int inner, int K, int out_dtype, hipStream_t s) {
+  return qil_gemm_bf16_wide_gated_act(A, W, out, M, inner, K, out_dtype, QIL_ACT_SILU, 0.f, 1.f, s);
 }
 
 }  // extern "C"

@@ -724,9 +724,10 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
     """act(x @ gate^T, x @ up^T) -> [N, I] (``activation``: a name of ``GATE_FUNCTIONS``; silu(gate) * up unless said), with ``weight`` the [2 I, K] matrix of both: the gate rows stacked
     before the up rows, or (``interleaved``) both in turns of 16 rows, which the kernels read faster.
 
-    One kernel when a fused kernel takes the sizes (bfloat16; up to 16 rows, or up to 256 rows of an interleaved
+    One kernel when a fused kernel takes the sizes, whatever the gate function (bfloat16; up to 16 rows, or up to 256 rows of an interleaved
     matrix large enough to fill the chip, or more rows of one whose product is short (``qil_gemm_bf16_wide_gated_wanted``),
-    or from 512 rows on under ``OWN_LARGE_PRODUCTS``); otherwise the product followed by ``silu_mul``.  Both add in float32.
+    or from 512 rows on under ``OWN_LARGE_PRODUCTS``); otherwise the product followed by ``silu_mul`` or ``gated_act``.  Both add in float32.  (8 rows of 12,288 x 2,048 with a
+    clamped swish: 10.2 us and 5.1 for the activation, 12.7 as one kernel; a step of six such layers 496 -> 481 us.)
     ``lazy``: a few float32 rows may come back as ``Gated`` (the product's partial sums) for ``linear`` to finish."""
     if isinstance(x, Normed):
         x = x.materialize()
@@ -743,32 +744,33 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
         raise ValueError(f'gated_linear: x {tuple(x.shape)}, weight {tuple(weight.shape)}')
     out_dtype = out_dtype or x.dtype
     lib = library.load()
-    if activation != 'silu':                       # the product, then the activation kernel
-        return gated_act(linear(x, weight, None, partials=True), out_dtype, activation=activation, limit=limit, alpha=alpha,
-                         interleaved=interleaved)
+    act = (GATE_FUNCTIONS[activation], float(limit), float(alpha))
+    inside = activation == 'silu' or not (x.data_ptr() | weight.data_ptr()) & 15     # (the others at any address: as products)
     # 17 to 256 rows of an interleaved matrix: the 32 x 32 tile kernel where it takes the sizes (measured against the
     # staged 16 x 16 kernel with the same epilogue at 17 to 64 rows: 37 to 38 us against 38 to 43 at Qwen3-8B sizes,
     # 73 to 85 against 87 to 102 at 14B sizes)
-    if x.dtype == torch.bfloat16 and interleaved and MID_GATED_FEWEST_ROWS <= n <= MID_GEMM_MOST_ROWS and \
+    if x.dtype == torch.bfloat16 and interleaved and inside and MID_GATED_FEWEST_ROWS <= n <= MID_GEMM_MOST_ROWS and \
             lib.qil_gemm_bf16_mid_gated_takes(n, both // 2, k):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_mid_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
+        _check(lib.qil_gemm_bf16_mid_gated_act(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), *act, _stream()),
                'gemm_bf16_mid_gated')
         return out
-    if x.dtype == torch.bfloat16 and n and lib.qil_gemm_bf16_gated_takes(n, both // 2, k, int(interleaved)):
+    if x.dtype == torch.bfloat16 and n and inside and lib.qil_gemm_bf16_gated_takes(n, both // 2, k, int(interleaved)):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_gated(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), 0, 0,
-                                       int(interleaved), _stream()), 'gemm_bf16_gated')
+        _check(lib.qil_gemm_bf16_gated_act(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), 0, 0,
+                                           int(interleaved), *act, _stream()), 'gemm_bf16_gated')
         return out
     at_x, at_weight = x.data_ptr(), weight.data_ptr()
     if x.dtype == torch.bfloat16 and interleaved and \
             ((OWN_LARGE_PRODUCTS and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k)) or
              (not (at_x | at_weight) & 15 and lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k))):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
-        _check(lib.qil_gemm_bf16_wide_gated(at_x, at_weight, _ptr(out), n, both // 2, k, _code(out_dtype), _stream()),
+        _check(lib.qil_gemm_bf16_wide_gated_act(at_x, at_weight, _ptr(out), n, both // 2, k, _code(out_dtype), *act, _stream()),
                'gemm_bf16_wide_gated')
         return out
     sums = linear(x, weight, None, partials=True)
+    if activation != 'silu':
+        return gated_act(sums, out_dtype, activation=activation, limit=limit, alpha=alpha, interleaved=interleaved)
     if lazy and x.dtype == torch.float32 and out_dtype == torch.float32 and n <= GATED_OPERAND_MOST_ROWS:
         return Gated(sums if isinstance(sums, Partials) else Partials(sums[None]), interleaved, out_dtype)
     return silu_mul(sums, out_dtype, interleaved=interleaved)

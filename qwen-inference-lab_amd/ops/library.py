@@ -274,6 +274,7 @@ def _declare(lib):
     lib.qil_gemm_bf16_unmerged_takes.argtypes = [i, i, i, i, i]
     lib.qil_gemm_bf16_unmerged_takes.restype = i
     lib.qil_gemm_bf16_gated.argtypes = [p, p, p, i, i, i, i, i, i, i, p]
+    lib.qil_gemm_bf16_gated_act.argtypes = [p, p, p, i, i, i, i, i, i, i, i, f, f, p]
     lib.qil_gemm_bf16_gated_takes.argtypes = [i, i, i, i]
     lib.qil_gemm_bf16_gated_takes.restype = i
     lib.qil_gemm_bf16_normed_takes.argtypes = [i, i, i, i]
@@ -293,6 +294,7 @@ def _declare(lib):
     lib.qil_gemm_bf16_mid_gated_takes.argtypes = [i, i, i]
     lib.qil_gemm_bf16_mid_gated_takes.restype = i
     lib.qil_gemm_bf16_mid_gated.argtypes = [p, p, p, i, i, i, i, p]
+    lib.qil_gemm_bf16_mid_gated_act.argtypes = [p, p, p, i, i, i, i, i, f, f, p]
     lib.qil_gemm_bf16_wide_takes.argtypes = [i, i, i, i]
     lib.qil_gemm_bf16_wide_takes.restype = i
     lib.qil_gemm_bf16_wide_shape.argtypes = [i, i, i, i]
@@ -305,6 +307,7 @@ def _declare(lib):
     lib.qil_gemm_bf16_wide_gated_takes.argtypes = [i, i, i]
     lib.qil_gemm_bf16_wide_gated_takes.restype = i
     lib.qil_gemm_bf16_wide_gated.argtypes = [p, p, p, i, i, i, i, p]
+    lib.qil_gemm_bf16_wide_gated_act.argtypes = [p, p, p, i, i, i, i, i, f, f, p]
     lib.qil_add_norm.argtypes = [p, p, i, i, i, f, p, p, p, p, i, i, f, i, i, i, p]
     lib.qil_gated_act.argtypes = [p, i, i, i, p, i, i, i, i, i, f, f, p]
     lib.qil_latent_prepare.argtypes = [p, i, i, i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, f, i, p, p, i, p]
