@@ -1693,6 +1693,13 @@ def state_scan(proj, *, mode, heads, dim, vdim, q_offset, k_offset, v_offset, st
                                      _ptr(seq_starts), _ptr(seq_slots), _ptr(out), _ptr(workspace), n, n_seqs,
                                      int(max_query), heads, shared, dim, vdim, _stream()), 'step_scan')
             return out, None
+    if max_query == 1 and n == n_seqs and \
+            lib.qil_state_token_takes(_ptr(proj), _ptr(state), code, width, v_offset, dim, vdim, rot, SCAN_MODES[mode]):
+        _check(lib.qil_state_token(_ptr(proj), code, width, q_offset, k_offset, v_offset, _ptr(gates), float(cap), _ptr(decay),
+                                   _ptr(frequencies) if rot else None, rot, float(q_scale), float(k_scale), _ptr(state),
+                                   _ptr(seq_starts), _ptr(seq_slots), _ptr(out), n, heads, dim, vdim, SCAN_MODES[mode],
+                                   _stream()), 'state_token')
+        return out, None
     below = torch.empty((n, heads), dtype=torch.float32, device=proj.device) if mode == 'mlstm' else None
     if max_query is not None and max_query >= SCAN_BLOCKS_FROM:
         floats = lib.qil_state_scan_chunked_workspace(n, n_seqs, heads, dim, vdim, SCAN_MODES[mode])

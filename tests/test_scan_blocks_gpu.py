@@ -71,3 +71,37 @@ def test_head_norms_and_gates_of_every_width(ops, dtype, vdim, offset):
         want = v * torch.sigmoid(z) * (z if gate == 'silu' else 1)
         # a sum of vdim squares and a handful of roundings in float32, then one to the type
         torch.testing.assert_close(got.double().cpu(), want, atol=1e-6, rtol=2e-6 if dtype == torch.float32 else 2.0 ** -8)
+
+
+# one row group's last row and beyond (16 groups), whole and odd sizes of a head, one and several blocks of 64 columns; sequences that
+# begin, continue and share nothing; a state that holds NaN where a sequence begins
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('mode', ['decay', 'channel'])
+@pytest.mark.parametrize('dim, vdim, rot', [(1, 64, 0), (17, 64, 16), (64, 128, 64), (128, 256, 128), (130, 64, 2), (256, 192, 128)])
+def test_one_token_a_sequence(ops, dtype, mode, dim, vdim, rot):
+    heads, n = 3, 5
+    g = torch.Generator().manual_seed(dim + vdim)
+    pad = -(heads * dim * 2) % 4                                  # the values' columns begin at a multiple of four elements
+    proj = torch.randn(n, 2 * heads * dim + pad + heads * vdim + (-(2 * heads * dim + pad + heads * vdim)) % 4, generator=g).to(dtype)
+    where = dict(heads=heads, dim=dim, vdim=vdim, q_offset=0, k_offset=heads * dim, v_offset=2 * heads * dim + pad)
+    state = torch.randn(7, heads * dim * vdim, generator=g)
+    state[3] = float('nan')                                      # the slot of a sequence that begins
+    index = dict(cu_seqlens=torch.arange(n + 1, dtype=torch.int32), seq_starts=torch.tensor([5, 0, 1000, 31, 7], dtype=torch.int32),
+                 seq_slots=torch.tensor([6, 3, 0, 1, 4], dtype=torch.int32))
+    extra = dict(frequencies=torch.tensor([50.0 ** (-2 * i / max(rot, 2)) for i in range(rot // 2)]) if rot else None, rot=rot,
+                 q_scale=0.9, k_scale=dim ** -0.5)
+    extra.update(dict(decay=torch.tensor([0.9, 0.999, 0.5])) if mode == 'decay' else dict(gates=torch.randn(n, heads * dim, generator=g), cap=4.0))
+    on = lambda values: {k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in values.items()}
+    got_state, want_state = state.cuda(), state.clone()
+    takes = ops.library.load().qil_state_token_takes
+    moved = proj.cuda()
+    assert takes(moved.data_ptr(), got_state.data_ptr(), int(dtype == torch.bfloat16), proj.shape[1], where['v_offset'], dim, vdim, rot,
+                 ops.SCAN_MODES[mode])
+    want, _ = refs.state_scan(proj, mode=mode, state=want_state, n_seqs=n, **where, **index, **extra)
+    got, below = ops.state_scan(moved, mode=mode, state=got_state, n_seqs=n, max_query=1, **where, **on(index), **on(extra))
+    assert below is None
+    # a state element is one product and one sum, a result a float32 sum of ``dim`` products; positions of 1,000 turn by angles that
+    # float32 holds to 6e-5
+    for a, b in ((got.cpu(), want), (got_state[index['seq_slots'].long()].cpu(), want_state[index['seq_slots'].long()])):
+        torch.testing.assert_close(a, b, atol=1e-4 * max(1.0, b.abs().max().item()), rtol=2e-5)
+    assert torch.equal(got_state[[2, 5]].cpu(), state[[2, 5]])
