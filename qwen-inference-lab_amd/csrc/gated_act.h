@@ -18,10 +18,16 @@ __device__ __forceinline__ float gated_act(float g, float u, int act, float limi
   return (g / (1.f + expf(-g))) * u;
 }
 
-// A gate function and its numbers, as product kernels with the activation in their epilogue take them.
+// A gate function and its numbers, as product kernels with the activation in their epilogue take them.  SILU: a kernel of its own
+// for silu, whose few instructions are all there is (one kernel for all of them took 6.9 us for one row of 6,144 x 1,024 where that
+// one takes 6.1: the other functions' code has to be fetched past).
 struct GateFn { int act; float limit, alpha; };
-__device__ __forceinline__ float gated_act(float g, float u, const GateFn& fn) { return gated_act(g, u, fn.act, fn.limit, fn.alpha); }
+template <bool SILU>
+__device__ __forceinline__ float gate_by(float g, float u, const GateFn& fn) {
+  return SILU ? (g / (1.f + expf(-g))) * u : gated_act(g, u, fn.act, fn.limit, fn.alpha);
+}
 inline bool gate_fn_known(int act) { return act == QIL_ACT_SILU || act == QIL_ACT_CLAMPED || act == QIL_ACT_RELU; }
+enum { QIL_UNGATED = 0, QIL_GATED_SILU = 1, QIL_GATED_OTHER = 2 };                  // what a product kernel does with its sums
 
 // Activations of experts without a gate branch, by code from QIL_ACT_RELU_SQUARED on:
 //   QIL_ACT_RELU_SQUARED  max(z, 0)^2

@@ -191,16 +191,16 @@ struct NormedA {
 };
 
 // ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA)
-template <typename OUT, int ASRC>
-__global__ void __launch_bounds__(LINES_WAVES * QIL_WAVE)
-gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, UnmergedA unmerged, NormedA normed, const bf16_t* __restrict__ W,
-                       OUT* __restrict__ C, int M, int N, int K, int cols_per_split) {
+template <typename OUT, int ASRC, int WAVES = LINES_WAVES>
+__global__ void __launch_bounds__(WAVES * QIL_WAVE)
+gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N, int K,
+                       int cols_per_split, UnmergedA unmerged, NormedA normed) {
   constexpr bool MERGE = ASRC == 1;
   extern __shared__ __align__(16) bf16_t lds[];            // A slice [8 or 16][cols + pad], then the waves' buffers
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
   const int a_rows = M <= 8 ? 8 : 16;                      // rows of A kept (8 or 16: a power of two)
-  const int n0 = (blockIdx.x * LINES_WAVES + wave) * 16, split = blockIdx.z;
+  const int n0 = (blockIdx.x * WAVES + wave) * 16, split = blockIdx.z;
   const int k_begin = split * cols_per_split, stages = cols_per_split / 128;
   const int row_width = cols_per_split + GEMM_LDS_PAD;
   bf16_t* a_lds = lds;
@@ -218,31 +218,68 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, UnmergedA unmerged, NormedA
   // A slice first: a wait for it after W's requests would cover the first stages of W as well (unless A goes
   // straight into LDS, below)
   if (ASRC == 2) {
-    // 1 / rms of the rows: wave m (and m + 8) adds the row's pieces lane by lane, then across the wave
-    float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + LINES_WAVES * (16 * 128));
-    for (int m = wave; m < M; m += LINES_WAVES) {
-      float sum = 0.f;
-      for (int p = lane; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + m];
-      sum = wave_sum(sum);
-      if (lane == 0) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += LINES_WAVES * QIL_WAVE) {
-      const int m = idx / (cols_per_split / 8), c = (idx - m * (cols_per_split / 8)) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m < M) {
-        float x[8], g[8];
-        ld8(normed.stream + (size_t)m * K + k_begin + c, x);
-        ld8(normed.weight + k_begin + c, g);
-        const float scale = rstd[m];
+    // 1 / rms of the rows: a wave adds the pieces of two rows lane by lane, then across the wave.  Their sums of squares are asked
+    // for first and, right behind them, what the first two pieces of A a thread are made of: one wait for all of it, and the
+    // sums are made while the rest arrives.  (Both are held in place: the compiler otherwise moves loads whose use stands
+    // under a condition down to it.)
+    float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
+    const int pieces = cols_per_split / 8, all = M * pieces;
+    constexpr int EARLY = 2, THREADS = WAVES * QIL_WAVE, SQUARES = 4;
+    float x[EARLY][8], g[EARLY][8], squares[2][SQUARES];
+    auto ask = [&](int idx, float (&to_x)[8], float (&to_g)[8]) {
+      const int m = idx / pieces, c = (idx - m * pieces) * 8;
+      ld8(normed.stream + (size_t)m * K + k_begin + c, to_x);
+      ld8(normed.weight + k_begin + c, to_g);
+    };
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = round_to<bf16_t>(x[e] * scale) * g[e];
-        v = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7]));
+    for (int i = 0; i < SQUARES; ++i) {
+      const float* from = normed.squares + (size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M;
+      squares[0][i] = from[min(wave, M - 1)];
+      squares[1][i] = from[min(wave + WAVES, M - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u) ask(min((int)threadIdx.x + u * THREADS, all - 1), x[u], g[u]);
+#pragma unroll
+    for (int r2 = 0; r2 < 2; ++r2) {                        // (2 WAVES rows are all there are)
+      const int m = wave + r2 * WAVES;
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < SQUARES; ++i) {
+        asm volatile("" : "+v"(squares[r2][i]));
+        if (lane + i * QIL_WAVE < normed.pieces) sum += squares[r2][i];
       }
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = v;
+      for (int p = lane + SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
+      sum = wave_sum(sum);
+      if (lane == 0 && m < M) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
+    }
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(x[u][e]), "+v"(g[u][e]));
+    __syncthreads();
+    auto put = [&](int idx, const float (&from_x)[8], const float (&from_g)[8]) {
+      const int m = idx / pieces, c = (idx - m * pieces) * 8;
+      const float scale = rstd[m];
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = round_to<bf16_t>(from_x[e] * scale) * from_g[e];
+      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) =
+          make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+    };
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+      if ((int)threadIdx.x + u * THREADS < all) put(threadIdx.x + u * THREADS, x[u], g[u]);
+    for (int idx = threadIdx.x + EARLY * THREADS; idx < all; idx += THREADS) {
+      ask(idx, x[0], g[0]);
+      put(idx, x[0], g[0]);
+    }
+    // rows past M: zeros
+    for (int idx = all + threadIdx.x; idx < a_rows * pieces; idx += THREADS) {
+      const int m = idx / pieces, c = (idx - m * pieces) * 8;
+      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = make_uint4(0, 0, 0, 0);
     }
   } else if (MERGE) {
-    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += LINES_WAVES * QIL_WAVE) {
+    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += WAVES * QIL_WAVE) {
       const int m = idx / (cols_per_split / 8), c = (idx - m * (cols_per_split / 8)) * 8;
       uint4 v = make_uint4(0, 0, 0, 0);
       if (m < M) v = merged8(unmerged, m, k_begin + c);
@@ -253,7 +290,7 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, UnmergedA unmerged, NormedA
     // here: W's first stages are asked for right behind it (loads complete in order, so waiting for A later
     // does not wait for them).  Rows past M repeat the last one; their products are never stored.
     const int row_loads = (cols_per_split + 511) / 512;
-    for (int j = wave; j < a_rows * row_loads; j += LINES_WAVES) {
+    for (int j = wave; j < a_rows * row_loads; j += WAVES) {
       const int m = __builtin_amdgcn_readfirstlane(j / row_loads), c0 = __builtin_amdgcn_readfirstlane(j - m * row_loads) * 512;
       if (c0 + lane * 8 < cols_per_split)
         __builtin_amdgcn_global_load_lds(
@@ -325,9 +362,9 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, UnmergedA unmerged, NormedA
   }
 }
 
-static size_t lines_lds(int M, int K, int splits) {
+static size_t lines_lds(int M, int K, int splits, int waves = LINES_WAVES) {
   const int rows = M <= 8 ? 8 : 16;
-  return ((size_t)rows * (K / splits + GEMM_LDS_PAD) + (size_t)LINES_WAVES * 16 * 128) * sizeof(bf16_t) + 16 * sizeof(float);
+  return ((size_t)rows * (K / splits + GEMM_LDS_PAD) + (size_t)waves * 16 * 128) * sizeof(bf16_t) + 16 * sizeof(float);
 }
 
 // Whether the whole-line kernel takes the product with this many splits.
@@ -338,20 +375,34 @@ static bool lines_takes(const void* A, const void* W, const float* bias, int M, 
   return lines_lds(M, K, splits) <= LINES_LDS_LIMIT;
 }
 
-template <typename OUT, int ASRC = 0>
-static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
-                        UnmergedA unmerged = UnmergedA(), NormedA normed = NormedA()) {
-  const size_t lds = lines_lds(M, K, splits);
-  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC>;
+template <typename OUT, int ASRC, int WAVES>
+static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
+                              UnmergedA unmerged, NormedA normed) {
+  const size_t lds = lines_lds(M, K, splits, WAVES);
+  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC, WAVES>;
   static size_t granted = 0;                              // per instantiation
   if (lds > 64 * 1024 && lds > granted) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
     granted = lds;
   }
-  dim3 grid((N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES), 1, splits);
-  hipLaunchKernelGGL(kernel, grid, dim3(LINES_WAVES * QIL_WAVE), lds, s, A, unmerged, normed, W, C, M, N, K, K / splits);
+  dim3 grid((N + 16 * WAVES - 1) / (16 * WAVES), 1, splits);
+  hipLaunchKernelGGL(kernel, grid, dim3(WAVES * QIL_WAVE), lds, s, A, W, C, M, N, K, K / splits, unmerged, normed);
   return 0;
+}
+
+// Blocks of 4 waves where those of 8 leave half of the CUs without one: a CU draws 36 GB/s at most.  One row, inside a step:
+// 1,024 x 2,048 behind the merge in 4 splits 6.0 us with 32 blocks of 8, 4.6 with 64 of 4; 4,096 x 1,024 behind the norm in 2 5.9 with
+// 64, 5.4 with 128 (its operands asked for in one batch); 8 rows of 2,048 x 2,048 in 4 5.3 with 64, 4.5 with 128.  Up to 8 rows:
+// with 16 half the threads stage twice the rows.
+#define LINES_FEW_WAVES 4
+template <typename OUT, int ASRC = 0>
+static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
+                        UnmergedA unmerged = UnmergedA(), NormedA normed = NormedA()) {
+  const long blocks = (long)((N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES)) * splits;
+  if (M <= 8 && blocks <= QIL_CUS / 2)
+    return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
+  return launch_lines_waves<OUT, ASRC, LINES_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -372,7 +423,7 @@ static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, 
 // store the activations.  K is not split: no partial sums in memory and no separate activation pass.  (With the gate
 // rows stacked before the up rows a block would read two regions a power of two apart at the same columns at the
 // same time, which loads a few memory channels only: 59 us against 45 for 64 rows at 8B sizes.)
-template <typename OUT, int MT, bool GATED = false>
+template <typename OUT, int MT, int GATED = QIL_UNGATED>
 __global__ void __launch_bounds__(LINES_WAVES * QIL_WAVE)
 gemm_bf16_chunks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N,
                         int K, int cols_per_split, GateFn fn) {
@@ -494,7 +545,7 @@ gemm_bf16_chunks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__
         for (int i = 0; i < 4; ++i) {
           const int m = t * 16 + 4 * kb + i, n = inner_n0 + r;
           const float g = acc[t][i];
-          if (m < M && n < inner) store_out(C + (size_t)m * inner + n, gated_act(g, up[i], fn));
+          if (m < M && n < inner) store_out(C + (size_t)m * inner + n, gate_by<GATED == QIL_GATED_SILU>(g, up[i], fn));
         }
       }
     }
@@ -529,7 +580,7 @@ static int chunks_splits(int N, int K) {
   return splits;
 }
 
-template <typename OUT, int MT, bool GATED = false>
+template <typename OUT, int MT, int GATED = false>
 static int launch_chunks_tiles(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, GateFn fn, hipStream_t s) {
   const size_t lds = ((size_t)2 * 16 * MT * CHUNK_ROW + (size_t)LINES_WAVES * 16 * 128) * sizeof(bf16_t);
   auto kernel = gemm_bf16_chunks_kernel<OUT, MT, GATED>;
@@ -545,7 +596,7 @@ static int launch_chunks_tiles(const bf16_t* A, const bf16_t* W, OUT* C, int M, 
   return 0;
 }
 
-template <typename OUT, bool GATED = false>
+template <typename OUT, int GATED = QIL_UNGATED>
 static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s, GateFn fn = {}) {
   if (M <= 32) return launch_chunks_tiles<OUT, 2, GATED>(A, W, C, M, N, K, splits, fn, s);
   if (M <= 64) return launch_chunks_tiles<OUT, 4, GATED>(A, W, C, M, N, K, splits, fn, s);
@@ -571,7 +622,7 @@ static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N,
 #define GATED_ROWS_FEWEST_BLOCKS 128                       // of the 17-to-192-row kernel: see gated_rows_takes
 #define GATED_ROWS_MOST 64                                 // beyond, the product and a separate activation are faster
 
-template <typename OUT>
+template <typename OUT, bool SILU>
 __global__ void __launch_bounds__(GATED_MAX_WAVES * QIL_WAVE)
 gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ out, int M,
                        int inner, int K, int ksplit, int interleaved, GateFn fn) {
@@ -698,7 +749,7 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = 4 * kb + i, n = n0 + r;                 // lane holds D[m = 4 kb + i][n = r]
-      if (m < M) store_out(out + (size_t)m * inner + n, gated_act(g[i], v[i], fn));
+      if (m < M) store_out(out + (size_t)m * inner + n, gate_by<SILU>(g[i], v[i], fn));
     }
   }
 }
@@ -805,9 +856,11 @@ extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, 
   if (M == 0 || inner == 0) return 0;
   if (M > 16) {                                              // pairs: the fewest blocks to accept (tests pass 1)
     if (!gated_rows_takes(A, W, M, inner, K, interleaved, pairs)) return -1;
-    const int status = out_dtype == QIL_F32
-                           ? launch_chunks<float, true>((const bf16_t*)A, (const bf16_t*)W, (float*)out, M, 2 * inner, K, 1, s, fn)
-                           : launch_chunks<bf16_t, true>((const bf16_t*)A, (const bf16_t*)W, (bf16_t*)out, M, 2 * inner, K, 1, s, fn);
+#define QIL_CHUNKS_GATED(OUT, GATED) \
+  launch_chunks<OUT, GATED>((const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, 2 * inner, K, 1, s, fn)
+    const int status = out_dtype == QIL_F32 ? (act == QIL_ACT_SILU ? QIL_CHUNKS_GATED(float, QIL_GATED_SILU) : QIL_CHUNKS_GATED(float, QIL_GATED_OTHER))
+                                            : (act == QIL_ACT_SILU ? QIL_CHUNKS_GATED(bf16_t, QIL_GATED_SILU) : QIL_CHUNKS_GATED(bf16_t, QIL_GATED_OTHER));
+#undef QIL_CHUNKS_GATED
     if (status) return status;
     QIL_RETURN_LAUNCH_STATUS();
   }
@@ -820,9 +873,9 @@ extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, 
   if (lds > 160 * 1024) return -1;
   const int all_pairs = inner / 16;
   dim3 grid((all_pairs + pairs - 1) / pairs), block(pairs * ksplit * QIL_WAVE);
-#define QIL_GATED_CASE(OUT)                                                                                          \
+#define QIL_GATED_CASE(OUT, SILU)                                                                                       \
   {                                                                                                                  \
-    auto kernel = gemm_bf16_gated_kernel<OUT>;                                                                       \
+    auto kernel = gemm_bf16_gated_kernel<OUT, SILU>;                                                                 \
     static size_t granted = 0;                                                                                       \
     if (lds > 64 * 1024 && lds > granted) {                                                                          \
       hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
@@ -831,7 +884,12 @@ extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, 
     }                                                                                                                \
     hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, inner, K, ksplit, interleaved, fn); \
   }
-  if (out_dtype == QIL_F32) QIL_GATED_CASE(float) else QIL_GATED_CASE(bf16_t)
+  const bool silu = act == QIL_ACT_SILU;
+  if (out_dtype == QIL_F32) {
+    if (silu) QIL_GATED_CASE(float, true) else QIL_GATED_CASE(float, false)
+  } else {
+    if (silu) QIL_GATED_CASE(bf16_t, true) else QIL_GATED_CASE(bf16_t, false)
+  }
 #undef QIL_GATED_CASE
   QIL_RETURN_LAUNCH_STATUS();
 }

@@ -55,7 +55,7 @@ __host__ __device__ constexpr int mid_a_ring(int mt) {
 // Waves 0 to 3 multiply, each with a ring of W of its own; wave 4 loads A for all of them.  A wave waits for its
 // loads by their number in flight (vmcnt counts in order), so loads that must land soon (A, from L2, three stages
 // in LDS) and loads that are sent far ahead (W, from memory) belong to different waves.
-template <int MT, typename OUT, bool GATED>
+template <int MT, typename OUT, int GATED>
 __global__ void __launch_bounds__((MID_WAVES + 1) * QIL_WAVE, 1)
 gemm_bf16_mid_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M_all, int N, int K,
                      int stages, int waves, int turns, GateFn fn) {
@@ -167,7 +167,7 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
 
   // acc[t][e]: row m = 32 t + l32, column n0 + 8 (e / 4) + 4 half + e % 4
   if (n0 >= N) return;
-  if constexpr (GATED) {                                   // columns 0-15 of the wave are gates, 16-31 the ups that belong to them
+  if constexpr (GATED != QIL_UNGATED) {                                   // columns 0-15 of the wave are gates, 16-31 the ups that belong to them
     const int inner = N / 2;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
@@ -179,7 +179,7 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          v[e] = gated_act(acc[t][4 * g + e], acc[t][4 * (g + 2) + e], fn);
+          v[e] = gate_by<GATED == QIL_GATED_SILU>(acc[t][4 * g + e], acc[t][4 * (g + 2) + e], fn);
         }
         if constexpr (sizeof(OUT) == 4) *reinterpret_cast<float4*>(row + 8 * g) = make_float4(v[0], v[1], v[2], v[3]);
         else *reinterpret_cast<uint2*>(row + 8 * g) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
@@ -229,7 +229,7 @@ static bool mid_plan(int M, int N, int K, int* waves, int* splits) {
   return found;
 }
 
-template <int MT, typename OUT, bool GATED>
+template <int MT, typename OUT, int GATED>
 static int mid_launch(const void* A, const void* W, void* C, int M, int N, int K, int waves, int splits, GateFn fn, hipStream_t s) {
   const size_t lds = (size_t)mid_w_ring(MT) * MID_WAVES * 4096 + (size_t)mid_a_ring(MT) * MT * 4096;
   auto kernel = gemm_bf16_mid_kernel<MT, OUT, GATED>;
@@ -245,7 +245,7 @@ static int mid_launch(const void* A, const void* W, void* C, int M, int N, int K
   QIL_RETURN_LAUNCH_STATUS();
 }
 
-template <bool GATED>
+template <int GATED>
 static int mid_dispatch(const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int waves, int splits,
                         hipStream_t s, GateFn fn = {}) {
 #define QIL_MID_CASE(MT)                                                                                      \
@@ -303,7 +303,7 @@ int qil_gemm_bf16_mid(const void* A, const void* W, void* C, int M, int N, int K
   if (splits < 0 || splits > 16 || !mid_plan(M, N, K, &waves, &splits) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16)
     return -1;
   if ((splits > 1 && out_dtype != QIL_F32) || (out_dtype != QIL_F32 && out_dtype != QIL_BF16)) return -1;
-  return mid_dispatch<false>(A, W, C, M, N, K, out_dtype, waves, splits, s);
+  return mid_dispatch<QIL_UNGATED>(A, W, C, M, N, K, out_dtype, waves, splits, s);
 }
 
 // 1 if qil_gemm_bf16_mid_gated takes these sizes: those of the product with 2 * inner columns, which in one split must
@@ -324,7 +324,9 @@ int qil_gemm_bf16_mid_gated_act(const void* A, const void* W, void* out, int M, 
   if (!qil_gemm_bf16_mid_gated_takes(M, inner, K) || !mid_plan(M, 2 * inner, K, &waves, &splits) ||
       ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16 || (out_dtype != QIL_F32 && out_dtype != QIL_BF16))
     return -1;
-  return mid_dispatch<true>(A, W, out, M, 2 * inner, K, out_dtype, waves, 1, s, GateFn{act, limit, alpha});
+  const GateFn fn{act, limit, alpha};
+  return act == QIL_ACT_SILU ? mid_dispatch<QIL_GATED_SILU>(A, W, out, M, 2 * inner, K, out_dtype, waves, 1, s, fn)
+                             : mid_dispatch<QIL_GATED_OTHER>(A, W, out, M, 2 * inner, K, out_dtype, waves, 1, s, fn);
 }
 
 // silu(A gate^T) * (A up^T)

@@ -63,7 +63,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // RT, CT: tiles of 32 rows and of 32 columns of a wave; DOWN, ACROSS: the block's waves above each other and side by side;
 // AHEAD: stages (even) that a pair's loads go out ahead.  OUT: bf16_t or float (the result; with splits of K float32 partial sums [split][M][N]).  GATED (one split): W holds gate and up rows in turns of 16, a tile of 32 columns is 16
 // of each, and C [M, N / 2] gets act(gate, up) (gated_act.h; qil/model.py:71), both still in float32.
-template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
+template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, int GATED>
 __global__ void __launch_bounds__(DOWN * ACROSS * QIL_WAVE, RT * CT <= 4 && AHEAD == 2 ? 2 : 1)
 gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M_all, int N, int K,
                       int stages, int col_blocks, int row_blocks, int splits, int patch_rows, int patch_cols, GateFn fn) {
@@ -234,8 +234,8 @@ gemm_bf16_wide_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if constexpr (GATED) {                           // columns 0-15 of a tile are gates, 16-31 the ups that belong to them
-            v[e] = gated_act(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e], fn);
+          if constexpr (GATED != QIL_UNGATED) {                           // columns 0-15 of a tile are gates, 16-31 the ups that belong to them
+            v[e] = gate_by<GATED == QIL_GATED_SILU>(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e], fn);
           } else {
             v[e] = acc[i][j][4 * g + e];
           }
@@ -310,7 +310,7 @@ static bool wide_wanted(int M, int N, int K, double us, bool gated) {
   return us <= WIDE_HOST_US && (M > WIDE_GRAPH_ROWS || us <= blas_us(M, N, K, gated) + WIDE_LEVEL_US);
 }
 
-template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, bool GATED>
+template <typename OUT, int RT, int CT, int DOWN, int ACROSS, int AHEAD, int GATED>
 static int wide_launch(const void* A, const void* W, void* C, int M, int N, int K, int splits, GateFn fn, hipStream_t s) {
   constexpr int ROWS = 32 * RT * DOWN, TILE = 32 * CT * ACROSS;
   const size_t lds = (size_t)(AHEAD + 3) * (ROWS + TILE) * WIDE_ROW_BYTES;
@@ -327,7 +327,7 @@ static int wide_launch(const void* A, const void* W, void* C, int M, int N, int 
   QIL_RETURN_LAUNCH_STATUS();
 }
 
-template <bool GATED>
+template <int GATED>
 static int wide_dispatch(int shape, const void* A, const void* W, void* C, int M, int N, int K, int out_dtype, int splits, hipStream_t s,
                          GateFn fn = {}) {
 #define QIL_WIDE_CASE(SHAPE, RT, CT, DOWN, ACROSS, AHEAD)                                                             \
@@ -402,7 +402,7 @@ int qil_gemm_bf16_wide(const void* A, const void* W, void* C, int M, int N, int 
   if (M == 0 || N == 0) return 0;
   if (!wide_takes(M, N, K, splits) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) return -1;
   if ((splits > 1 && out_dtype != QIL_F32) || (out_dtype != QIL_F32 && out_dtype != QIL_BF16)) return -1;
-  return wide_dispatch<false>(wide_shape(M, N, K, splits), A, W, C, M, N, K, out_dtype, splits, s);
+  return wide_dispatch<QIL_UNGATED>(wide_shape(M, N, K, splits), A, W, C, M, N, K, out_dtype, splits, s);
 }
 
 // 1 if qil_gemm_bf16_wide_gated takes these sizes: those of the product with 2 * inner columns in one split.
@@ -426,7 +426,10 @@ int qil_gemm_bf16_wide_gated_act(const void* A, const void* W, void* out, int M,
   if (!qil_gemm_bf16_wide_gated_takes(M, inner, K) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16 ||
       (out_dtype != QIL_F32 && out_dtype != QIL_BF16))
     return -1;
-  return wide_dispatch<true>(wide_shape(M, 2 * inner, K, 1), A, W, out, M, 2 * inner, K, out_dtype, 1, s, GateFn{act, limit, alpha});
+  const GateFn fn{act, limit, alpha};
+  const int shape = wide_shape(M, 2 * inner, K, 1);
+  return act == QIL_ACT_SILU ? wide_dispatch<QIL_GATED_SILU>(shape, A, W, out, M, 2 * inner, K, out_dtype, 1, s, fn)
+                             : wide_dispatch<QIL_GATED_OTHER>(shape, A, W, out, M, 2 * inner, K, out_dtype, 1, s, fn);
 }
 
 // silu(A gate^T) * (A up^T)

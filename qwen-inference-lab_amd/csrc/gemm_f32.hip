@@ -216,8 +216,8 @@ struct GatedA {
 // ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = the activation of a gated feed-forward (GatedA)
 template <int ASRC, int WAVES>
 __global__ void __launch_bounds__(WAVES * QIL_WAVE)
-gemm_f32_lines_kernel(const float* __restrict__ A, UnmergedA unmerged, GatedA gated, const float* __restrict__ W,
-                      float* __restrict__ C, int M, int N, int K, int cols_per_split) {
+gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K,
+                      int cols_per_split, UnmergedA unmerged, GatedA gated) {
   extern __shared__ __align__(16) float fl_lds[];           // A slice [8 or 16][cols + pad], then the waves' buffers
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
@@ -549,7 +549,7 @@ static int launch_f32_lines_waves(const float* A, UnmergedA unmerged, GatedA gat
     granted = lds;
   }
   dim3 grid((N + 16 * WAVES - 1) / (16 * WAVES), 1, splits);
-  hipLaunchKernelGGL(kernel, grid, dim3(WAVES * QIL_WAVE), lds, s, A, unmerged, gated, W, C, M, N, K, K / splits);
+  hipLaunchKernelGGL(kernel, grid, dim3(WAVES * QIL_WAVE), lds, s, A, W, C, M, N, K, K / splits, unmerged, gated);
   QIL_RETURN_LAUNCH_STATUS();
 }
 
