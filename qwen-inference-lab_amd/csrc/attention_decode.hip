@@ -49,17 +49,19 @@ __device__ __forceinline__ uint4 shuffle4(uint4 v, int source) {
                     __shfl(v.w, source, QIL_WAVE));
 }
 
-// FUSED: fused_qkv.h.  WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
-template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false>
+// What the first loads need stands in the first 56 bytes of the arguments, which arrive in registers; the rest and the row's
+// position and sequence are asked for in batches (a dozen reads of arguments, each waited for by itself, and 10 KB of sines to fetch
+// past stood before the first load of data: 8 rows of 2,000 keys 18.8 -> 17.9 us).
+// FUSED: fused_qkv.h; FREQUENCIES: its rotation is made from frequencies, not read from tables.  WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
+template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false, bool FREQUENCIES = false>
 __global__ void __launch_bounds__(DEC_MAX_WAVES * QIL_WAVE)
-attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_cache,
-                   const bf16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int table_stride,
-                   const int* __restrict__ row_seq, const int* __restrict__ positions,
-                   const int* __restrict__ row_index, float* __restrict__ part_acc, float* __restrict__ part_m,
-                   float* __restrict__ part_l, bf16_t* __restrict__ out, int heads, int kv_heads, int d,
-                   int page_size, int window, float scale, int P, int parts, float softcap,
-                   const float* __restrict__ sinks, const float* __restrict__ slopes, int keep,
-                   const int* __restrict__ plan, int* __restrict__ part_keys) {
+attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positions, const int* __restrict__ row_seq,
+                   const int* __restrict__ block_tables, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+                   int table_stride, int P, int heads, int kv_heads, int page_size, int window, int keep, int d, int parts,
+                   float scale, float softcap, const int* __restrict__ row_index, const float* __restrict__ sinks,
+                   const float* __restrict__ slopes, const bf16_t* __restrict__ q, int q_stride, float* __restrict__ part_acc,
+                   float* __restrict__ part_m, float* __restrict__ part_l, bf16_t* __restrict__ out, int* __restrict__ part_keys,
+                   FusedQKV fused) {
   constexpr int QFRAGS = DMAX / 32, DTILES = DMAX / 16;
   constexpr int TG = DMAX / 8, HPP = QIL_WAVE / TG;          // lanes of a head (8 elements each), heads a wave
   if (WHOLE) d = DMAX;                                      // what the host has checked, known to the compiler: no
@@ -67,7 +69,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
   extern __shared__ float lds[];
   int slot_row = blockIdx.x, part = blockIdx.z;
   const int kvh = blockIdx.y;
-  if (plan) {                                               // the rows' parts one behind another (attn_plan_kernel)
+  if (__builtin_expect(plan != nullptr, 0)) {               // the rows' parts one behind another (attn_plan_kernel)
     const int job = plan[1 + blockIdx.x];
     P = plan[0];
     if (blockIdx.x == 0 && kvh == 0 && threadIdx.x == 0) *part_keys = P;       // for whoever merges the parts
@@ -75,9 +77,11 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
     slot_row = job >> 16;
     part = job & 0xffff;
   }
-  const int row = row_index ? row_index[slot_row] : slot_row;
+  if constexpr (FUSED) ask_fields(fused);
+  const int row = !FUSED && row_index ? row_index[slot_row] : slot_row;
   const int g = heads / kv_heads;
-  const int pos = positions[row], ctx = pos + 1;
+  const int pos = positions[row], sequence = row_seq[row], ctx = pos + 1;
+  asm volatile("" ::"s"(pos), "s"(sequence), "s"(slopes));     // one wait for the three
   const KeySpan span(pos, window, keep);
   const int begin = max(part * P, span.first_place()), end = min((part + 1) * P, span.places());      // places
   if (begin >= end) return;
@@ -86,7 +90,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE, waves = blockDim.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
   const int dt = d / 16;
-  const int* table = block_tables + (size_t)row_seq[row] * table_stride;
+  const int* table = block_tables + (size_t)sequence * table_stride;
 
   const int first_step = begin / 32;                       // steps of 32 places, numbered from the first place
   const int last_step = (end - 1) / 32;
@@ -254,7 +258,7 @@ attn_decode_kernel(FusedQKV fused, const bf16_t* __restrict__ q, int q_stride, c
     }
     const float* weight = query ? fused.q_weight : fused.k_weight;
     if (weight) load_eight(weight + chunk * 8, factors.w);
-    if (fused.cos_table && fused.rot > 0) load_turns(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
+    if (fused.cos_table && fused.rot > 0) load_turns<FREQUENCIES>(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
   };
   auto answer = [&](bool query, int head, float (&x)[8], float (&plain)[8]) __attribute__((always_inline)) {
 #pragma unroll
@@ -522,11 +526,11 @@ extern "C" int qil_attn_decode(const void* q, int q_stride, const void* k_cache,
   // 16 heads of 64 in 8 groups 30.8 / 29.2, but 16 rows of 1,000 keys 12.9 / 13.4; heads of 128 48.6 / 53.
   const bool pairs = (plan ? (long)blocks : (long)rows * parts) * kv_heads <= QIL_CUS && d < 128 &&
                      (plan || (d == 64 ? P >= 128 * waves : P > 32 * waves));
-#define QIL_DEC_LAUNCH(DMAX, FUSED, WHOLE, PAIRS, FIELDS)                                                          \
-  hipLaunchKernelGGL((attn_decode_kernel<DMAX, FUSED, WHOLE, PAIRS>), grid, dim3(waves * QIL_WAVE), lds, s, FIELDS,        \
-                     (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,       \
-                     table_stride, row_seq, positions, row_index, acc, m, l, (bf16_t*)out, heads, kv_heads, d,        \
-                     page_size, window, scale, P, parts, softcap, sinks, slopes, keep, plan, part_keys)
+#define QIL_DEC_LAUNCH(DMAX, FUSED, WHOLE, PAIRS, FIELDS, ...)                                                          \
+  hipLaunchKernelGGL((attn_decode_kernel<DMAX, FUSED, WHOLE, PAIRS, ##__VA_ARGS__>), grid, dim3(waves * QIL_WAVE), lds, s, plan,   \
+                     positions, row_seq, block_tables, (const bf16_t*)k_cache, (const bf16_t*)v_cache, table_stride, P, heads,     \
+                     kv_heads, page_size, window, keep, d, parts, scale, softcap, row_index, sinks, slopes, (const bf16_t*)q,     \
+                     q_stride, acc, m, l, (bf16_t*)out, part_keys, FIELDS)
   if (d == 64 && pairs) QIL_DEC_LAUNCH(64, false, true, true, none);
   else if (d == 64) QIL_DEC_LAUNCH(64, false, true, false, none);
   else if (d < 64 && pairs) QIL_DEC_LAUNCH(64, false, false, true, none);
@@ -596,8 +600,13 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
-  if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused);
-  else QIL_DEC_LAUNCH(128, true, true, false, fused);
+  if (cos_table && !sin_table) {
+    if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused, true);
+    else QIL_DEC_LAUNCH(128, true, true, false, fused, true);
+  } else {
+    if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused);
+    else QIL_DEC_LAUNCH(128, true, true, false, fused);
+  }
 #undef QIL_DEC_LAUNCH
   QIL_RETURN_LAUNCH_STATUS();
 }

@@ -33,20 +33,23 @@ __device__ __forceinline__ f32x4 once_f4(const float* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
 }
 
-template <int D, bool FUSED>
+// FUSED: fused_qkv.h; FREQUENCIES: its rotation is made from frequencies, not read from tables.
+template <int D, bool FUSED, bool FREQUENCIES = false>
 __global__ void __launch_bounds__(DEC32_WAVES * QIL_WAVE)
-attn_decode_f32_kernel(FusedQKV fused, const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
-                       const float* __restrict__ v_cache, const int* __restrict__ block_tables, int table_stride,
-                       const int* __restrict__ row_seq, const int* __restrict__ positions, const int* __restrict__ row_index,
-                       float* __restrict__ part_acc, float* __restrict__ part_m, float* __restrict__ part_l,
-                       float* __restrict__ out, int heads, int kv_heads, int page_size, int window, float scale, int P,
-                       int parts, float softcap, const float* __restrict__ sinks, const float* __restrict__ slopes, int keep) {
+attn_decode_f32_kernel(const int* __restrict__ positions, const int* __restrict__ row_seq, const int* __restrict__ block_tables,
+                       const float* __restrict__ k_cache, const float* __restrict__ v_cache, int table_stride, int P, int heads,
+                       int kv_heads, int page_size, int window, int keep, int parts, float scale, float softcap,
+                       const int* __restrict__ row_index, const float* __restrict__ sinks, const float* __restrict__ slopes,
+                       const float* __restrict__ q, int q_stride, float* __restrict__ part_acc, float* __restrict__ part_m,
+                       float* __restrict__ part_l, float* __restrict__ out, FusedQKV fused) {
   constexpr int PIECES = D / 16, TG = D / 8, HPP = QIL_WAVE / TG, CELL = D + 2, waves = DEC32_WAVES;
   extern __shared__ __align__(16) float lds[];
   const int slot_row = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
-  const int row = row_index ? row_index[slot_row] : slot_row;
+  if constexpr (FUSED) ask_fields(fused);
+  const int row = !FUSED && row_index ? row_index[slot_row] : slot_row;
   const int g = heads / kv_heads;
-  const int pos = positions[row], ctx = pos + 1;
+  const int pos = positions[row], sequence = row_seq[row], ctx = pos + 1;
+  asm volatile("" ::"s"(pos), "s"(sequence), "s"(slopes));     // one wait for the three
   const KeySpan span(pos, window, keep);
   const int begin = max(part * P, span.first_place()), end = min((part + 1) * P, span.places());      // places
   if (begin >= end) return;
@@ -54,7 +57,7 @@ attn_decode_f32_kernel(FusedQKV fused, const float* __restrict__ q, int q_stride
 
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
-  const int* table = block_tables + (size_t)row_seq[row] * table_stride;
+  const int* table = block_tables + (size_t)sequence * table_stride;
   const int first_step = begin / DEC32_STEP, last_step = (end - 1) / DEC32_STEP;
   const float slope = (slopes && r < g) ? slopes[kvh * g + r] : 0.f;
 
@@ -168,7 +171,7 @@ attn_decode_f32_kernel(FusedQKV fused, const float* __restrict__ q, int q_stride
     ask_sums(query, head, 0);
     const float* weight = query ? fused.q_weight : fused.k_weight;
     if (weight) load_eight(weight + chunk * 8, factors.w);
-    if (fused.cos_table && fused.rot > 0) load_turns(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
+    if (fused.cos_table && fused.rot > 0) load_turns<FREQUENCIES>(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
   };
   auto answer = [&](bool query, int head, float (&x)[8], float (&plain)[8]) __attribute__((always_inline)) {
 #pragma unroll
@@ -326,11 +329,11 @@ int qil_attn_decode_f32(const void* q, int q_stride, const void* k_cache, const 
   const size_t lds = dec32_lds(g, d, false);
   const dim3 grid(rows, kv_heads, parts);
   const FusedQKV none = {};
-#define QIL_DEC32(D, FUSED, FIELDS)                                                                                   \
-  hipLaunchKernelGGL((attn_decode_f32_kernel<D, FUSED>), grid, dim3(DEC32_WAVES * QIL_WAVE), lds, s, FIELDS, (const float*)q, \
-                     q_stride, (const float*)k_cache, (const float*)v_cache, block_tables, table_stride, row_seq,      \
-                     positions, row_index, acc, m, l, (float*)out, heads, kv_heads, page_size, window, scale, P, parts, \
-                     softcap, sinks, slopes, keep)
+#define QIL_DEC32(D, FUSED, FIELDS, ...)                                                                              \
+  hipLaunchKernelGGL((attn_decode_f32_kernel<D, FUSED, ##__VA_ARGS__>), grid, dim3(DEC32_WAVES * QIL_WAVE), lds, s, positions, row_seq, \
+                     block_tables, (const float*)k_cache, (const float*)v_cache, table_stride, P, heads, kv_heads,      \
+                     page_size, window, keep, parts, scale, softcap, row_index, sinks, slopes, (const float*)q, q_stride, \
+                     acc, m, l, (float*)out, FIELDS)
   if (d == 64) QIL_DEC32(64, false, none);
   else QIL_DEC32(128, false, none);
   QIL_RETURN_LAUNCH_STATUS();
@@ -373,8 +376,13 @@ int qil_attn_decode_f32_fused(const float* qkv, int splits, const float* q_weigh
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
-  if (d == 64) QIL_DEC32(64, true, fused);
-  else QIL_DEC32(128, true, fused);
+  if (cos_table && !sin_table) {
+    if (d == 64) QIL_DEC32(64, true, fused, true);
+    else QIL_DEC32(128, true, fused, true);
+  } else {
+    if (d == 64) QIL_DEC32(64, true, fused);
+    else QIL_DEC32(128, true, fused);
+  }
 #undef QIL_DEC32
   QIL_RETURN_LAUNCH_STATUS();
 }

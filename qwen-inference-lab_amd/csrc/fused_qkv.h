@@ -27,3 +27,11 @@ struct FusedQKV {
   float temp_coef;                                         // temp_every > 0: the query at position p is multiplied by
   int temp_every;                                          // 1 + temp_coef * ln(floor((p + 1) / temp_every) + 1) last
 };
+
+// Reads the fields at a kernel's start, all with one wait: where each is read at its use, a wave waits for a dozen of them in
+// turn before its first load of data.
+__device__ __forceinline__ void ask_fields(const FusedQKV& f) {
+  asm volatile("" ::"s"(f.qkv), "s"(f.split_stride), "s"(f.splits), "s"(f.q_weight), "s"(f.k_weight), "s"(f.eps), "s"(f.cos_table),
+               "s"(f.sin_table), "s"(f.rot), "s"(f.rotate_first), "s"(f.writes), "s"(f.row_elems), "s"(f.v_head), "s"(f.bias),
+               "s"(f.temp_coef), "s"(f.temp_every));
+}

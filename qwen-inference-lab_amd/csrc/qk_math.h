@@ -84,12 +84,15 @@ __device__ __forceinline__ void load_eight(const float* p, float (&to)[8]) {
   const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 4);
   to[0] = lo.x; to[1] = lo.y; to[2] = lo.z; to[3] = lo.w; to[4] = hi.x; to[5] = hi.y; to[6] = hi.z; to[7] = hi.w;
 }
+// FREQUENCIES: 1 made from frequencies, 0 read from tables, -1 as the arguments say (a kernel that knows does not carry the code
+// for both: eight sines and cosines are 10 KB, and kernels of a few us wait for the instruction cache).
+template <int FREQUENCIES = -1>
 __device__ __forceinline__ void load_turns(HeadFactors& f, int chunk, const float* __restrict__ cos_table,
                                            const float* __restrict__ sin_table, int position, int rot) {
   const int half_chunks = rot >> 4;                   // chunks in half of the rotated width (a power of two)
   if (chunk < 2 * half_chunks) {
     const int pair = chunk < half_chunks ? chunk : chunk - half_chunks;
-    if (sin_table) {
+    if (FREQUENCIES == 0 || (FREQUENCIES < 0 && sin_table)) {
       const size_t at = (size_t)position * (rot >> 1) + pair * 8;
       load_eight(cos_table + at, f.c);
       load_eight(sin_table + at, f.sn);
