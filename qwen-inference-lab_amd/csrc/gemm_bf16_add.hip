@@ -23,44 +23,45 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define ADD_DEPTH 3                                        // stages in flight per wave
 #define ADD_LDS_LIMIT (160 * 1024)
 
-// AROWS: rows of A kept (8 or 16).  INTO: the result goes into the stream; else out [M, N] of bfloat16 gets it (squares null).
-template <int AROWS, bool INTO>
-__global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE, AROWS == 8 ? 4 : 3)
+// AROWS: rows of A kept (8 or 16).  COLS: columns of a group, 16 or 8 (the matrix cores then make every column twice and memory
+// is read once: twice the groups, where those of 16 leave half of the CUs without a block).  INTO: the result goes into the stream; else out [M, N] of bfloat16 gets it (squares null).
+template <int AROWS, bool INTO, int COLS = 16>
+__global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE, COLS == 8 ? 2 : AROWS == 8 ? 4 : 3)
 gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ stream,
                      bf16_t* __restrict__ out, float* __restrict__ squares, int M, int N, int K, int ksplit) {
   extern __shared__ __align__(16) bf16_t lds[];            // per wave: 4 KB for W, AROWS x 256 bytes for A
-  constexpr int ALOADS = AROWS / 4, PER_WAVE = (16 + AROWS) * 128;
+  constexpr int ALOADS = AROWS / 4, WLOADS = COLS / 4, PER_WAVE = (COLS + AROWS) * 128;
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
   const int group = wave / ksplit, part = wave - group * ksplit;
   const int groups = blockDim.x / QIL_WAVE / ksplit;
   const int mine = blockIdx.x * groups + group;
-  const bool stores = mine * 16 < N;
-  const int n0 = min(mine, N / 16 - 1) * 16;               // a group past the end repeats the last one and stores nothing
+  const bool stores = mine * COLS < N && (lane & 15) < COLS;
+  const int n0 = min(mine, N / COLS - 1) * COLS;               // a group past the end repeats the last one and stores nothing
   const int cols = K / ksplit, k_begin = part * cols, stages = cols / 128;
   // Every wave walks its K range from a start of its own and wraps around: waves that all read the same columns
   // of their rows at the same time load a few memory channels only.
-  const int turn = (n0 / 16) % stages;
+  const int turn = (n0 / COLS) % stages;
   auto column = [&](int stage) { const int st = stage + turn; return (st >= stages ? st - stages : st) * 128; };
   bf16_t* buffer = lds + wave * PER_WAVE;
-  bf16_t* a_buffer = buffer + 16 * 128;
+  bf16_t* a_buffer = buffer + COLS * 128;
 
   const int load_row = lane >> 4, piece = lane & 15;
-  const bf16_t* source[4];
+  const bf16_t* source[WLOADS];
   const bf16_t* a_source[ALOADS];                          // rows past the last read it again: rows of D never stored
   int place[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int row = 4 * u + load_row;
-    source[u] = W + (size_t)(n0 + row) * K + k_begin + piece * 8;
+    if (u < WLOADS) source[u] = W + (size_t)(n0 + row) * K + k_begin + piece * 8;
     place[u] = row * 128 + ((piece ^ row) & 15) * 8;
     if (u < ALOADS) a_source[u] = A + (size_t)min(row, M - 1) * K + k_begin + piece * 8;
   }
-  u32x4 w0[4], w1[4], w2[4], a0[ALOADS], a1[ALOADS], a2[ALOADS];   // named, so that none is indexed at run time
-  auto request = [&](u32x4 (&stage_w)[4], u32x4 (&stage_a)[ALOADS], int stage) {
+  u32x4 w0[WLOADS], w1[WLOADS], w2[WLOADS], a0[ALOADS], a1[ALOADS], a2[ALOADS];   // named, so that none is indexed at run time
+  auto request = [&](u32x4 (&stage_w)[WLOADS], u32x4 (&stage_a)[ALOADS], int stage) {
     const int at = column(stage);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) stage_w[u] = load_once(source[u] + at);
+    for (int u = 0; u < WLOADS; ++u) stage_w[u] = load_once(source[u] + at);
 #pragma unroll
     for (int u = 0; u < ALOADS; ++u) stage_a[u] = *reinterpret_cast<const u32x4*>(a_source[u] + at);
   };
@@ -69,17 +70,17 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
   request(w2, a2, 2);
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int a_row = r & (AROWS - 1);
-  auto step = [&](u32x4 (&stage_w)[4], u32x4 (&stage_a)[ALOADS], int next, bool more) {
+  const int a_row = r & (AROWS - 1), w_row = r & (COLS - 1);
+  auto step = [&](u32x4 (&stage_w)[WLOADS], u32x4 (&stage_a)[ALOADS], int next, bool more) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) *reinterpret_cast<u32x4*>(buffer + place[u]) = stage_w[u];
+    for (int u = 0; u < WLOADS; ++u) *reinterpret_cast<u32x4*>(buffer + place[u]) = stage_w[u];
 #pragma unroll
     for (int u = 0; u < ALOADS; ++u) *reinterpret_cast<u32x4*>(a_buffer + place[u]) = stage_a[u];
     if (more) request(stage_w, stage_a, next);
     __builtin_amdgcn_wave_barrier();                        // LDS operations of one wave complete in order: no wait
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) {
-      const u32x4 b = *reinterpret_cast<const u32x4*>(buffer + r * 128 + (((4 * s4 + kb) ^ r) & 15) * 8);
+      const u32x4 b = *reinterpret_cast<const u32x4*>(buffer + w_row * 128 + (((4 * s4 + kb) ^ w_row) & 15) * 8);
       const u32x4 a = *reinterpret_cast<const u32x4*>(a_buffer + a_row * 128 + (((4 * s4 + kb) ^ a_row) & 15) * 8);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0,
                                                     0, 0);
@@ -122,20 +123,27 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
         value = *cell + total[i];
         *cell = value;
       }
-      if (squares) {                                        // the 16 lanes of a row add their squares: one order for all
+      if (squares) {                                        // the lanes of a row add their squares: one order for all
         float square = value * value;
         square += __shfl_xor(square, 1, QIL_WAVE);
         square += __shfl_xor(square, 2, QIL_WAVE);
         square += __shfl_xor(square, 4, QIL_WAVE);
-        square += __shfl_xor(square, 8, QIL_WAVE);
+        if (COLS == 16) square += __shfl_xor(square, 8, QIL_WAVE);
         if (r == 0 && m < M && stores) squares[(size_t)mine * M + m] = square;
       }
     }
   }
 }
 
-static size_t add_lds_bytes(int M, int waves) {
-  return (size_t)waves * (16 + (M <= 8 ? 8 : 16)) * 128 * sizeof(bf16_t);     // also holds the waves' sums (1 KB a wave)
+static size_t add_lds_bytes(int M, int waves, int cols = 16) {
+  return (size_t)waves * (cols + (M <= 8 ? 8 : 16)) * 128 * sizeof(bf16_t);   // also holds the waves' sums (1 KB a wave)
+}
+
+// Groups of 8 columns instead of 16: up to 8 rows of products whose groups of 16 fill at most half of the CUs with a block each
+// (a CU draws 36 GB/s at most): 1,024 x 3,072, one row, 6.4 -> 5.8 us inside a step (64 blocks of 98 KB, 128 of 49), 2,048 x 6,144,
+// 8 rows, 10.7 -> 9.2.
+static bool add_narrow(int M, int N, int K) {
+  return M <= 8 && N >= 512 && N <= 16 * QIL_CUS / 2 && K % 1024 == 0 && K / 1024 >= ADD_DEPTH;
 }
 
 // Waves a group and groups a block for these sizes; false if the kernel does not take them.
@@ -182,6 +190,11 @@ static int add_launch(const void* A, const void* W, float* stream, void* out, fl
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)stream) % 16) return -1;
   int planned_groups, planned_ksplit;
   if (!add_plan(M, N, K, &planned_groups, &planned_ksplit)) return -1;
+  if (INTO && !groups && !ksplit && add_narrow(M, N, K)) {
+    hipLaunchKernelGGL((gemm_bf16_add_kernel<8, INTO, 8>), dim3(N / 8), dim3(ADD_WAVES * QIL_WAVE), add_lds_bytes(M, ADD_WAVES, 8), s,
+                       (const bf16_t*)A, (const bf16_t*)W, stream, (bf16_t*)out, squares, M, N, K, ADD_WAVES);
+    QIL_RETURN_LAUNCH_STATUS();
+  }
   if (!groups) groups = planned_groups;
   if (!ksplit) ksplit = planned_ksplit;
   if (groups < 1 || ksplit < 1 || groups * ksplit > ADD_WAVES || K % (128 * ksplit) || K / (128 * ksplit) < ADD_DEPTH)
@@ -199,8 +212,11 @@ static int add_launch(const void* A, const void* W, float* stream, void* out, fl
 
 extern "C" {
 
-// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [N / 16][M] that gets the rows' sums of squares
-// of the new stream in pieces of 16 columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set them).
+// Pieces of a row whose sums of squares qil_gemm_bf16_add leaves (groups and ksplit 0): N / 16, or N / 8.
+int qil_gemm_bf16_add_pieces(int M, int N, int K) { return add_narrow(M, N, K) ? N / 8 : N / 16; }
+
+// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [pieces][M] that gets the rows' sums of squares
+// of the new stream in pieces of 16 (or 8) columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set both; then 16).
 int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* squares, int M, int N, int K, int groups,
                       int ksplit, hipStream_t s) {
   return add_launch<true>(A, W, stream, nullptr, squares, M, N, K, groups, ksplit, s);

@@ -200,7 +200,7 @@ class Gated:
 
 class Added:
     """What ``linear`` returns when it has added its result into ``add_to`` itself.  ``squares`` [pieces, N] float32:
-    the rows' sums of squares of the stream as it is now, in pieces of 16 columns."""
+    the rows' sums of squares of the stream as it is now, in pieces of 16 or 8 columns."""
 
     def __init__(self, squares):
         self.squares = squares
@@ -609,7 +609,7 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
             _require(x, 'x')
             _require(weight, 'weight', x.dtype, (o, k))
             _require(add_to, 'add_to', torch.float32, (n, o))
-            squares = torch.empty((o // 16, n), dtype=torch.float32, device=x.device)
+            squares = torch.empty((lib.qil_gemm_bf16_add_pieces(n, o, k), n), dtype=torch.float32, device=x.device)
             _check(lib.qil_gemm_bf16_add(_ptr(x), _ptr(weight), _ptr(add_to), _ptr(squares), n, o, k, 0, 0, _stream()),
                    'gemm_bf16_add')
             return Added(squares)
