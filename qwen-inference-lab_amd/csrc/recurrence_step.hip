@@ -25,7 +25,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define STEP_L 128                                         // tokens a block
-#define STEP_ROW (STEP_L + 8)                              // elements of a transposed row in LDS
+// A block's tokens pass through LDS in halves: with dim = 128 all of them take 53 KB, three blocks a CU, and 2,048 tokens of 64
+// heads are four; a half takes 29 and every block runs at once.  And no load waits behind a condition: past the end the last
+// row or column is loaded, and becomes zero on its way on.  dim 128, vdim 64, us: sums 26.5, halves 23.8, loads ahead 22.4 (50 MB);
+// outputs 48.6, 42.2, 37.6 (84 MB: loads, the state taken apart by each of the four waves, scores, stores, about 10 us each and
+// one after another, since all blocks begin together).
+#define STEP_HALF (STEP_L / 2)
+#define STEP_ROW (STEP_HALF + 8)                           // elements of a transposed row in LDS
 
 struct StepGates {
   Operand raw;                                             // [n, row]: the raw step size of head h at column h
@@ -34,19 +40,35 @@ struct StepGates {
   const float* rates;                                      // [heads], natural logarithm's units
 };
 
+__device__ __forceinline__ float softplus_step(float v) { return v > 20.f ? v : log1pf(expf(v)); }
 __device__ __forceinline__ float step_size(const StepGates& g, int row, int h) {
-  const float v = operand_at(g.raw, (size_t)row * g.row + h) + g.bias[h];
-  return v > 20.f ? v : log1pf(expf(v));
+  return softplus_step(operand_at(g.raw, (size_t)row * g.row + h) + g.bias[h]);
 }
 
-// The first wave: F_t (log2 units) and d_t of the block's tokens into LDS; tokens past the end have d = 0 and F unchanged.
-__device__ __forceinline__ void step_prefix(const StepGates& g, int r0, int lc, int h, int lane, double* F, float* d) {
+// The first wave: F_t (log2 units) and d_t of the block's tokens into LDS; tokens past the end have d = 0 and F unchanged.  In
+// two halves, the loads of a plain array and what becomes of them (the sums of splits are read by the second).
+struct AskedSteps { uint32_t bits[STEP_L / QIL_WAVE]; };
+__device__ __forceinline__ AskedSteps step_ask(const StepGates& g, int r0, int lc, int h, int lane) {
+  AskedSteps asked{};
+#pragma unroll
+  for (int u = 0; u < STEP_L / QIL_WAVE; ++u) {
+    const size_t at = (size_t)(r0 + min(lane + u * QIL_WAVE, lc - 1)) * g.row + h;
+    if (g.raw.code == QIL_BF16) asked.bits[u] = (uint32_t)reinterpret_cast<const bf16_t*>(g.raw.data)[at] << 16;
+    else if (g.raw.splits == 1) asked.bits[u] = reinterpret_cast<const uint32_t*>(g.raw.data)[at];
+  }
+  return asked;
+}
+__device__ __forceinline__ void step_prefix(const StepGates& g, const AskedSteps& asked, int r0, int lc, int h, int lane, double* F,
+                                            float* d) {
   const double rate = (double)g.rates[h] * 1.4426950408889634;
+  const float bias = g.bias[h];
   float mine[STEP_L / QIL_WAVE];
 #pragma unroll
   for (int u = 0; u < STEP_L / QIL_WAVE; ++u) {
     const int t = lane + u * QIL_WAVE;
-    mine[u] = t < lc ? step_size(g, r0 + t, h) : 0.f;
+    const float raw = g.raw.code == QIL_BF16 || g.raw.splits == 1 ? __uint_as_float(asked.bits[u])
+                                                                  : operand_at(g.raw, (size_t)(r0 + min(t, lc - 1)) * g.row + h);
+    mine[u] = t < lc ? softplus_step(raw + bias) : 0.f;
   }
   double before = 0.0;
 #pragma unroll
@@ -85,20 +107,32 @@ __device__ __forceinline__ Split3 split3(const float (&v)[8]) {
 }
 __device__ __forceinline__ bf16x8 lds_fragment(const bf16_t* p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p)); }
 
-// Columns [first, first + 8 chunks) of the block's rows, transposed into LDS: to[column][token].  Two tokens at a time: a
-// dword holds the same column of both.  Columns from `columns` on and tokens from lc on are zeros.
-__device__ __forceinline__ void stage_transposed(const bf16_t* __restrict__ src, int src_row, int r0, int lc, int columns,
-                                                 int chunks, bf16_t* __restrict__ to) {
-  for (int item = threadIdx.x; item < chunks * (STEP_L / 2); item += blockDim.x) {
-    const int chunk = (item & 7) + ((item >> 3) / (STEP_L / 2)) * 8, s = ((item >> 3) % (STEP_L / 2)) * 2;
-    if (chunk >= chunks) continue;
-    uint4 a = make_uint4(0, 0, 0, 0), b = make_uint4(0, 0, 0, 0);
-    if (chunk * 8 < columns) {
-      const bf16_t* p = src + (size_t)(r0 + s) * src_row + chunk * 8;
-      if (s < lc) a = *reinterpret_cast<const uint4*>(p);
-      if (s + 1 < lc) b = *reinterpret_cast<const uint4*>(p + src_row);
-    }
-    const uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+// 64 N columns of STEP_HALF rows from r0 on their way to LDS, transposed: to[column][token].  Two tokens at a time: a dword holds
+// the same column of both.  Columns from `columns` on and tokens from lc on (lc >= 1) are zeros; what is loaded for them is the
+// last one's, so that no load has a condition to wait behind.
+template <int N> struct TokenPairs { uint4 a[N], b[N]; };
+template <int N>
+__device__ __forceinline__ TokenPairs<N> ask_pairs(const bf16_t* __restrict__ src, int src_row, int r0, int lc, int columns) {
+  TokenPairs<N> x;
+  const int s = threadIdx.x / 8 * 2;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const bf16_t* p = src + min((int)(threadIdx.x % 8 + 8 * n) * 8, columns - 8);
+    x.a[n] = *reinterpret_cast<const uint4*>(p + (size_t)(r0 + min(s, lc - 1)) * src_row);
+    x.b[n] = *reinterpret_cast<const uint4*>(p + (size_t)(r0 + min(s + 1, lc - 1)) * src_row);
+  }
+  return x;
+}
+template <int N>
+__device__ __forceinline__ void store_transposed(const TokenPairs<N>& pairs, int lc, int columns, bf16_t* __restrict__ to) {
+  const int s = threadIdx.x / 8 * 2;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int chunk = threadIdx.x % 8 + 8 * n;
+    const bool column = chunk * 8 < columns, first = column && s < lc, second = column && s + 1 < lc;
+    const uint4 a = pairs.a[n], b = pairs.b[n];
+    const uint32_t x[4] = {first ? a.x : 0u, first ? a.y : 0u, first ? a.z : 0u, first ? a.w : 0u};
+    const uint32_t y[4] = {second ? b.x : 0u, second ? b.y : 0u, second ? b.z : 0u, second ? b.w : 0u};
     uint32_t* out = reinterpret_cast<uint32_t*>(to + (size_t)chunk * 8 * STEP_ROW + s);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -114,7 +148,7 @@ __device__ __forceinline__ size_t step_place(int row0, int seq, int c) { return 
 
 // grid (blocks of the longest sequence, sequences x heads, value tiles of 64); NT: 16-row tiles of i a wave (dim <= 64 NT)
 template <int NT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NT <= 2 ? 4 : 2)
 step_sums_kernel(const bf16_t* __restrict__ proj, int proj_row, int k_off, int v_off, StepGates gates,
                  const int* __restrict__ cu_seqlens, float* __restrict__ states, float* __restrict__ keeps, int heads,
                  int groups, int dim, int vdim) {
@@ -130,8 +164,13 @@ step_sums_kernel(const bf16_t* __restrict__ proj, int proj_row, int k_off, int v
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE, r = lane & 15, kb = lane >> 4;
   const int group = h / (heads / groups);
   const size_t at = step_place(row0, seq, c) * heads + h;
+  const bf16_t *keys = proj + k_off + group * dim, *values = proj + v_off + h * vdim + j0;
+  AskedSteps asked{};
+  if (wave == 0) asked = step_ask(gates, r0, lc, h, lane);
+  TokenPairs<NT> kp = ask_pairs<NT>(keys, proj_row, r0, lc, dim);
+  TokenPairs<1> xp = ask_pairs<1>(values, proj_row, r0, lc, vdim - j0);
   if (wave == 0) {
-    step_prefix(gates, r0, lc, h, lane, F, w);
+    step_prefix(gates, asked, r0, lc, h, lane, F, w);
     const double end = F[lc - 1];                          // (a wave's LDS operations are in order)
 #pragma unroll
     for (int u = 0; u < STEP_L / QIL_WAVE; ++u) {
@@ -140,31 +179,39 @@ step_sums_kernel(const bf16_t* __restrict__ proj, int proj_row, int k_off, int v
     }
     if (lane == 0 && blockIdx.z == 0) keeps[at] = exp2f((float)end);
   }
-  stage_transposed(proj + k_off + group * dim, proj_row, r0, lc, dim, NT * 8, kT);
-  stage_transposed(proj + v_off + h * vdim + j0, proj_row, r0, lc, vdim - j0, 8, xT);
-  __syncthreads();
   f32x4 acc[NT][4];
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) acc[n][jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < lc; s0 += 32) {
-    float ws[8];
-    ld8(w + s0 + 8 * kb, ws);
-    bf16x8 k[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) k[n] = lds_fragment(kT + ((wave * NT + n) * 16 + r) * STEP_ROW + s0 + 8 * kb);
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-      float x[8];
-      ld8(xT + (jt * 16 + r) * STEP_ROW + s0 + 8 * kb, x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] *= ws[e];
-      const Split3 xs = split3(x);
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) acc[n][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[n], xs.part[p], acc[n][jt], 0, 0, 0);
+  for (int half = 0; half < lc; half += STEP_HALF) {
+    if (half > 0) __syncthreads();
+    store_transposed(kp, lc - half, dim, kT);
+    store_transposed(xp, lc - half, vdim - j0, xT);
+    __syncthreads();
+    const int next = half + STEP_HALF;
+    if (next < lc) {
+      kp = ask_pairs<NT>(keys, proj_row, r0 + next, lc - next, dim);
+      xp = ask_pairs<1>(values, proj_row, r0 + next, lc - next, vdim - j0);
+    }
+    for (int s0 = 0; s0 < min(STEP_HALF, lc - half); s0 += 32) {
+      float ws[8];
+      ld8(w + half + s0 + 8 * kb, ws);
+      bf16x8 k[NT];
+  #pragma unroll
+      for (int n = 0; n < NT; ++n) k[n] = lds_fragment(kT + ((wave * NT + n) * 16 + r) * STEP_ROW + s0 + 8 * kb);
+  #pragma unroll
+      for (int jt = 0; jt < 4; ++jt) {
+        float x[8];
+        ld8(xT + (jt * 16 + r) * STEP_ROW + s0 + 8 * kb, x);
+  #pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= ws[e];
+        const Split3 xs = split3(x);
+  #pragma unroll
+        for (int n = 0; n < NT; ++n)
+  #pragma unroll
+          for (int p = 0; p < 3; ++p) acc[n][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[n], xs.part[p], acc[n][jt], 0, 0, 0);
+      }
     }
   }
   // lane: U[i = tile + 4 kb ..][j = jt * 16 + r]: four neighbours of a row [j][i]
@@ -225,14 +272,14 @@ step_carry_kernel(float* __restrict__ states, const float* __restrict__ keeps, f
 // grid (blocks of the longest sequence, sequences x heads, value tiles of 64); dim <= 32 NF.  A wave owns the 16-token
 // tiles `wave` and 7 - wave: the early one has few keys, the late one many.
 template <int NF>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NF <= 4 ? 4 : 2)
 step_outputs_kernel(const bf16_t* __restrict__ proj, int proj_row, int q_off, int k_off, int v_off, StepGates gates,
                     const int* __restrict__ cu_seqlens, const float* __restrict__ states, float* __restrict__ out, int heads,
                     int groups, int dim, int vdim) {
-  constexpr int K_ROW = NF * 32 + 8;
+  constexpr int K_ROW = NF * 32 + 8, AHEAD = 2;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16_t* Ks = reinterpret_cast<bf16_t*>(lds_raw);         // [STEP_L][K_ROW]
-  bf16_t* xT = Ks + STEP_L * K_ROW;                        // [64][STEP_ROW]
+  bf16_t* Ks = reinterpret_cast<bf16_t*>(lds_raw);         // [STEP_HALF][K_ROW]
+  bf16_t* xT = Ks + STEP_HALF * K_ROW;                        // [64][STEP_ROW]
   double* F = reinterpret_cast<double*>(xT + 64 * STEP_ROW);
   float* d = reinterpret_cast<float*>(F + STEP_L);
   const int c = blockIdx.x, seq = blockIdx.y / heads, h = blockIdx.y % heads, j0 = blockIdx.z * 64;
@@ -244,68 +291,101 @@ step_outputs_kernel(const bf16_t* __restrict__ proj, int proj_row, int q_off, in
   const bf16_t* keys = proj + k_off + group * dim;
   const bf16_t* queries = proj + q_off + group * dim;
   const int tiles[2] = {wave, 7 - wave};
+  const bf16_t* values = proj + v_off + h * vdim + j0;
+  // every load of the first half before the first is taken; rows and columns past the end are the last one's, and the queries'
+  // zeros there keep them out of the products
+  AskedSteps asked{};
+  if (wave == 0) asked = step_ask(gates, r0, lc, h, lane);
   bf16x8 q[2][NF];
+  uint4 raw[2][NF];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int ks = 0; ks < NF; ++ks)
+      raw[b][ks] = *reinterpret_cast<const uint4*>(queries + (size_t)(r0 + min(tiles[b] * 16 + r, lc - 1)) * proj_row +
+                                                   min(ks * 32 + 8 * kb, dim - 8));
+  uint4 kr[NF];
+  TokenPairs<1> xp;
+  const auto ask = [&](int half) {
+#pragma unroll
+    for (int n = 0; n < NF; ++n) {
+      const int item = threadIdx.x + 256 * n, s = item / (NF * 4), i = item % (NF * 4) * 8;
+      kr[n] = *reinterpret_cast<const uint4*>(keys + (size_t)(r0 + min(half + s, lc - 1)) * proj_row + min(i, dim - 8));
+    }
+    xp = ask_pairs<1>(values, proj_row, r0 + half, lc - half, vdim - j0);
+  };
+  const auto put = [&](int half) {
+#pragma unroll
+    for (int n = 0; n < NF; ++n) {
+      const int item = threadIdx.x + 256 * n, s = item / (NF * 4), i = item % (NF * 4) * 8;
+      const bool live = half + s < lc && i < dim;
+      *reinterpret_cast<uint4*>(Ks + s * K_ROW + i) =
+          make_uint4(live ? kr[n].x : 0u, live ? kr[n].y : 0u, live ? kr[n].z : 0u, live ? kr[n].w : 0u);
+    }
+    store_transposed(xp, lc - half, vdim - j0, xT);
+  };
+  ask(0);
+  const float* s_in = states + (step_place(row0, seq, c) * heads + h) * dim * vdim;
+  float v[AHEAD][8];                                       // eight along i of row j: the pieces AHEAD of the one in hand
+  const auto ask_state = [&](int piece) {
+    const unsigned at = min(j0 + piece % 4 * 16 + r, vdim - 1) * dim + min(piece / 4 * 32 + 8 * kb, dim - 8);
+    ld8(s_in + at, v[piece % AHEAD]);
+  };
+#pragma unroll
+  for (int piece = 0; piece < AHEAD; ++piece) ask_state(piece);
 #pragma unroll
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int ks = 0; ks < NF; ++ks) {
-      const int t = tiles[b] * 16 + r, i = ks * 32 + 8 * kb;
-      uint4 raw = make_uint4(0, 0, 0, 0);
-      if (t < lc && i < dim) raw = *reinterpret_cast<const uint4*>(queries + (size_t)(r0 + t) * proj_row + i);
-      q[b][ks] = __builtin_bit_cast(bf16x8, raw);
+      const bool live = tiles[b] * 16 + r < lc && ks * 32 + 8 * kb < dim;
+      const uint4 x = raw[b][ks];
+      q[b][ks] = __builtin_bit_cast(bf16x8, make_uint4(live ? x.x : 0u, live ? x.y : 0u, live ? x.z : 0u, live ? x.w : 0u));
     }
-  for (int item = threadIdx.x; item < STEP_L * NF * 4; item += 256) {
-    const int s = item / (NF * 4), i = item % (NF * 4) * 8;
-    uint4 raw = make_uint4(0, 0, 0, 0);
-    if (s < lc && i < dim) raw = *reinterpret_cast<const uint4*>(keys + (size_t)(r0 + s) * proj_row + i);
-    *reinterpret_cast<uint4*>(Ks + s * K_ROW + i) = raw;
-  }
-  stage_transposed(proj + v_off + h * vdim + j0, proj_row, r0, lc, vdim - j0, 8, xT);
-  if (wave == 0) step_prefix(gates, r0, lc, h, lane, F, d);
+  put(0);
+  if (wave == 0) step_prefix(gates, asked, r0, lc, h, lane, F, d);
   f32x4 o[2][4];
 #pragma unroll
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) o[b][jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
   // what came in: rows j of S_in^T (float32, taken apart) with the queries
-  const float* s_in = states + (step_place(row0, seq, c) * heads + h) * dim * vdim;
 #pragma unroll
-  for (int ks = 0; ks < NF; ++ks) {
-    const int i = ks * 32 + 8 * kb;
+  for (int piece = 0; piece < NF * 4; ++piece) {
+    const int ks = piece / 4, jt = piece % 4;
+    const bool live = ks * 32 + 8 * kb < dim;
+    float (&mine)[8] = v[piece % AHEAD];
 #pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-      const int j = j0 + jt * 16 + r;
-      float v[8];
+    for (int e = 0; e < 8; ++e) mine[e] = live ? mine[e] : 0.f;
+    const Split3 s = split3(mine);
+    if (piece + AHEAD < NF * 4) ask_state(piece + AHEAD);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 0.f;
-      if (i < dim && j < vdim) ld8(s_in + (size_t)j * dim + i, v);
-      const Split3 s = split3(v);
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) o[b][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.part[p], q[b][ks], o[b][jt], 0, 0, 0);
-    }
+      for (int p = 0; p < 3; ++p) o[b][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.part[p], q[b][ks], o[b][jt], 0, 0, 0);
   }
   __syncthreads();
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int t = tiles[b] * 16 + r;
-    const double mine = F[t];
-    const float brought = exp2f((float)mine);
+    const float brought = exp2f((float)F[tiles[b] * 16 + r]);
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[b][jt][e] *= brought;
-    if (tiles[b] * 16 >= lc) continue;
-    for (int s0 = 0; s0 <= tiles[b] * 16 + 15; s0 += 32) {
+  }
+  // the keys from `from` on, of the half in LDS, that the tile's queries see
+  const auto add_keys = [&](int b, int from) {
+    const int t = tiles[b] * 16 + r, end = min(tiles[b] * 16 + 16, from + STEP_HALF);
+    if (tiles[b] * 16 >= lc) return;
+    const double mine = F[t];
+    for (int s0 = from; s0 < end; s0 += 32) {
       f32x4 score[2];
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        score[half] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        const bf16_t* row = Ks + (s0 + 8 * (r >> 2) + 4 * half + (r & 3)) * K_ROW + 8 * kb;
+      for (int part = 0; part < 2; ++part) {
+        score[part] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        const bf16_t* row = Ks + (s0 - from + 8 * (r >> 2) + 4 * part + (r & 3)) * K_ROW + 8 * kb;
 #pragma unroll
         for (int ks = 0; ks < NF; ++ks)
-          score[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_fragment(row + ks * 32), q[b][ks], score[half], 0, 0, 0);
+          score[part] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_fragment(row + ks * 32), q[b][ks], score[part], 0, 0, 0);
       }
       float p[8];
 #pragma unroll
@@ -316,20 +396,33 @@ step_outputs_kernel(const bf16_t* __restrict__ proj, int proj_row, int q_off, in
       const Split3 ps = split3(p);
 #pragma unroll
       for (int jt = 0; jt < 4; ++jt) {
-        const bf16x8 x = lds_fragment(xT + (jt * 16 + r) * STEP_ROW + s0 + 8 * kb);
+        const bf16x8 x = lds_fragment(xT + (jt * 16 + r) * STEP_ROW + s0 - from + 8 * kb);
 #pragma unroll
         for (int k = 0; k < 3; ++k) o[b][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ps.part[k], o[b][jt], 0, 0, 0);
       }
     }
-    if (t < lc) {
-      float* row = out + (size_t)(r0 + t) * heads * vdim + (size_t)h * vdim;
+  };
+  const auto store = [&](int b) {
+    const int t = tiles[b] * 16 + r;
+    if (t >= lc) return;
+    float* row = out + (size_t)(r0 + t) * heads * vdim + (size_t)h * vdim;
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        const int j = j0 + jt * 16 + 4 * kb;
-        if (j < vdim) *reinterpret_cast<f32x4*>(row + j) = o[b][jt];
-      }
+    for (int jt = 0; jt < 4; ++jt) {
+      const int j = j0 + jt * 16 + 4 * kb;
+      if (j < vdim) *reinterpret_cast<f32x4*>(row + j) = o[b][jt];
     }
+  };
+  add_keys(0, 0);
+  store(0);                                                // (tile `wave` ends in the first half)
+  add_keys(1, 0);
+  if (lc > STEP_HALF) {
+    ask(STEP_HALF);                                        // (earlier: 33 registers spilled)
+    __syncthreads();
+    put(STEP_HALF);
+    __syncthreads();
+    add_keys(1, STEP_HALF);
   }
+  store(1);
 }
 
 // One token a sequence.  grid (sequences, heads), 256 threads: thread (c, g) takes the columns 4 c .. 4 c + 3 and the rows
@@ -431,11 +524,6 @@ int qil_step_scan(const void* proj, int proj_row, int q_off, int k_off, int v_of
 #define QIL_STEP_SUMS(NT)                                                                                             \
   do {                                                                                                                \
     const size_t lds = (size_t)(NT + 1) * 64 * STEP_ROW * sizeof(bf16_t) + tail;                                      \
-    if (lds > 64 * 1024) {                                                                                            \
-      hipError_t e = hipFuncSetAttribute((const void*)step_sums_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                         (int)lds);                                                                   \
-      if (e != hipSuccess) return (int)e;                                                                             \
-    }                                                                                                                 \
     hipLaunchKernelGGL(step_sums_kernel<NT>, grid, dim3(256), lds, s, (const bf16_t*)proj, proj_row, k_off, v_off,     \
                        gates, cu_seqlens, states, keeps, heads, groups, dim, vdim);                                   \
   } while (0)
@@ -448,12 +536,7 @@ int qil_step_scan(const void* proj, int proj_row, int q_off, int k_off, int v_of
                      (size_t)heads * dim * vdim, cu_seqlens, seq_starts, seq_slots, heads, dim, vdim, i_tiles);
 #define QIL_STEP_OUT(NF)                                                                                              \
   do {                                                                                                                \
-    const size_t lds = ((size_t)STEP_L * (NF * 32 + 8) + 64 * STEP_ROW) * sizeof(bf16_t) + tail;                      \
-    if (lds > 64 * 1024) {                                                                                            \
-      hipError_t e = hipFuncSetAttribute((const void*)step_outputs_kernel<NF>,                                        \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                       \
-      if (e != hipSuccess) return (int)e;                                                                             \
-    }                                                                                                                 \
+    const size_t lds = ((size_t)STEP_HALF * (NF * 32 + 8) + 64 * STEP_ROW) * sizeof(bf16_t) + tail;                      \
     hipLaunchKernelGGL(step_outputs_kernel<NF>, grid, dim3(256), lds, s, (const bf16_t*)proj, proj_row, q_off, k_off,  \
                        v_off, gates, cu_seqlens, states, out, heads, groups, dim, vdim);                              \
   } while (0)
