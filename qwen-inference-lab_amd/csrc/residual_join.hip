@@ -115,6 +115,50 @@ __global__ void residual_join_kernel(float* __restrict__ stream, JoinInputs in, 
   }
 }
 
+// Plain operands of bfloat16 (the products of many rows), all of them there but b: eight columns a thread, every operand asked
+// for before one is taken, the row in registers.  Where each operand's kind is found out at run time its load waits inside its
+// branch: 2,048 rows of 2,048 columns, two mixers and a feed-forward, 23.0 -> 19.4 us (84 MB; the quotients and exponentials of
+// the gates are about 6 of them).  blockDim.x = width / 8.
+template <bool TWO>
+__global__ void __launch_bounds__(1024)
+residual_join_plain_kernel(float* __restrict__ stream, const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
+                           const bf16_t* __restrict__ f, const bf16_t* __restrict__ gates, int a_row, int b_row, int f_row,
+                           int g_row, float a_scale, float b_scale, const float* __restrict__ bias,
+                           const float* __restrict__ weight, bf16_t* __restrict__ out, int width, float eps) {
+  __shared__ float scratch[16];
+  const size_t m = blockIdx.x;
+  const int i = threadIdx.x * 8;
+  float* x = stream + m * width + i;
+  float v[8], t[8], u[8], y[8], g1[8], g2[8], b1[8], b2[8], w[8];
+  ld8(x, v);
+  ld8(a + m * a_row + i, t);
+  if (TWO) ld8(b + m * b_row + i, u);
+  ld8(f + m * f_row + i, y);
+  ld8(gates + m * g_row + i, g1);
+  ld8(gates + m * g_row + width + i, g2);
+  ld8(bias + i, b1);
+  ld8(bias + width + i, b2);
+  ld8(weight + i, w);
+  float squares = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float mixed = t[e] * a_scale;
+    if (TWO) mixed += b_scale * u[e];
+    mixed = mixed / (1.f + expf(-(g1[e] + b1[e])));
+    mixed += y[e] / (1.f + expf(-(g2[e] + b2[e])));
+    v[e] += mixed;
+    squares += v[e] * v[e];
+  }
+  st4(x, make_float4(v[0], v[1], v[2], v[3]));
+  st4(x + 4, make_float4(v[4], v[5], v[6], v[7]));
+  squares = block_sum(squares, scratch);
+  const float unit = 1.f / sqrtf(squares / (float)width + eps);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = v[e] * unit * w[e];
+  *reinterpret_cast<uint4*>(out + m * width + i) =
+      make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+}
+
 extern "C" {
 
 // a, b, f, gates: (pointer or null, code, splits, elements of a row); the split stride is total_rows times the row.
@@ -144,6 +188,19 @@ int qil_residual_join(float* stream, const void* a, int a_code, int a_splits, in
   vec = vec && (((uintptr_t)stream | (uintptr_t)bias | (uintptr_t)plus | (uintptr_t)step | (uintptr_t)weight | (uintptr_t)out) % 16) == 0;
   const size_t lds = (size_t)width * sizeof(float);
   if (lds > 128 * 1024) return -1;
+  // whole waves of eight columns a thread, up to 1,024 threads; other widths, kinds and partial sums: the general kernel
+  bool plain = vec && out_dtype == QIL_BF16 && a && f && gates && !plus && !step && !rows && update && width % 512 == 0 && width <= 8192;
+  for (int k = 0; k < 4; ++k) plain = plain && (!data[k] || (codes[k] == QIL_BF16 && row[k] % 8 == 0));
+  if (plain) {
+#define QIL_JOIN_PLAIN(TWO)                                                                                           \
+  hipLaunchKernelGGL(residual_join_plain_kernel<TWO>, dim3(n_out), dim3(width / 8), 0, s, stream, (const bf16_t*)a,    \
+                     (const bf16_t*)b, (const bf16_t*)f, (const bf16_t*)gates, a_row, b_row, f_row, g_row, a_scale,    \
+                     b_scale, bias, weight, (bf16_t*)out, width, eps)
+    if (b) QIL_JOIN_PLAIN(true);
+    else QIL_JOIN_PLAIN(false);
+#undef QIL_JOIN_PLAIN
+    QIL_RETURN_LAUNCH_STATUS();
+  }
   const int lanes = vec ? width / 4 : width;
   const int threads = lanes >= 1024 ? 1024 : (lanes + 63) / 64 * 64;
 #define QIL_JOIN(T, V)                                                                                               \
