@@ -1,11 +1,11 @@
 // A few-row bfloat16 product that adds its result into the float32 residual stream:
 //   stream[M, N] += A[M, K] W[N, K]^T,   M <= 16, float32 accumulation.
-// A block owns `groups` groups of 16 output columns and `ksplit` waves per group, which split K among themselves and
+// A block owns `groups` groups of 16 (or 8, below) output columns and `ksplit` waves per group, which split K among themselves and
 // add their float32 sums in LDS in wave order (the scheme of the gated kernel in gemm_bf16.hip): no partial sums in
 // memory, every element of the stream is read, added to and written by one lane, after its sum is complete.  The
 // kernel that follows finds the stream complete: it needs no sum over partial results, and the norm it would start
 // with can be made by the product after it (gemm_bf16.hip, NormedA), for which this kernel leaves the rows' sums of
-// squares in pieces: squares[piece][m] = sum over the 16 columns of group `piece` of stream[m, .]^2.
+// squares in pieces: squares[piece][m] = sum over the columns of group `piece` of stream[m, .]^2.
 // W and A both travel in whole cache lines (4 rows x 256 bytes a load), three stages of 128 columns ahead in
 // registers, through buffers of the wave's own in LDS that turn them into matrix-core fragments (see the whole-line
 // kernel in gemm_bf16.hip); A comes from L2.  K may be any length (the down product of a gated feed-forward).
@@ -24,7 +24,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define ADD_LDS_LIMIT (160 * 1024)
 
 // AROWS: rows of A kept (8 or 16).  COLS: columns of a group, 16 or 8 (the matrix cores then make every column twice and memory
-// is read once: twice the groups, where those of 16 leave half of the CUs without a block).  INTO: the result goes into the stream; else out [M, N] of bfloat16 gets it (squares null).
+// is read once: twice the groups, where those of 16 leave half of the CUs without a block).  INTO: the result goes into the
+// stream; else out [M, N] of bfloat16 gets it (squares null).
 template <int AROWS, bool INTO, int COLS = 16>
 __global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE, COLS == 8 ? 2 : AROWS == 8 ? 4 : 3)
 gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ stream,

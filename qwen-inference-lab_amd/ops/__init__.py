@@ -46,7 +46,7 @@ DECODE_MAX_PART = 8192
 # launch (64 rows of 2048 keys: 111 us against 94 + 5; whole steps at 8B sizes: 24 and 32 rows gain 0.8 %
 # with the fused kernel, 48 rows lose 2 %).
 FUSED_DECODE_MOST_ROWS = 32
-# Rows up to which the row kernel leaves its parts unmerged when the caller allows (the product after it merges them).
+# Rows up to which the decode and row kernels leave their parts unmerged when the caller allows (the product after it merges them).
 UNMERGED_ROWS_MOST = 16
 
 
@@ -1094,8 +1094,9 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
 
     Sequences with two or more rows (``cu_seqlens``, ``seq_starts``) go to the matrix-core tile
     kernel; rows alone in their sequence (``single_rows``: their indices, or None when every row is
-    alone, i.e. ``max_query == 1``) go to the split-context row kernel.  With ``unmerged`` the result may
-    come back as ``Unmerged`` (every row alone, context in several parts) for ``linear`` to merge.
+    alone, i.e. ``max_query == 1``) go to a split-context kernel: on the matrix cores where
+    type, head and page sizes allow it, else the row kernel.  With ``unmerged`` the result may come back as ``Unmerged``
+    (every row alone, context in several parts) for ``linear`` to merge.
     ``tile_seqs``: the caller has put the sequences of two or more rows first and there are this many; the tile
     kernel then gets blocks for these only (None: for every sequence; those of one row leave at once).
     ``softcap`` c: scores are scaled, then capped softly, c * tanh(score / c), before the softmax.  The kernels
@@ -1103,7 +1104,7 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
     ``sinks`` float32 [heads]: exp(sinks[h]) joins the divisor of head h's softmax once (no key, no value, not
     scaled).  It enters where a row's result is normalised: in the kernel when the keys are in one piece, in the merge
     of the parts otherwise.  The general tile kernel, the bfloat16 prompt kernel for heads of 128, the matrix-core
-    decode kernel and the row kernel take it; steps with sinks run on those and come back merged.
+    decode kernels and the row kernel take it; steps with sinks run on those and come back merged.
     ``slopes`` float32 [heads]: slopes[h] * (position - key) is taken off head h's score after the scale (and the cap).
     ``keep_first``: with a window, the first so many keys stay visible: row n sees j <= positions[n] with
     j > positions[n] - window or j < keep_first.  Both run on the kernels that take sinks; with kept keys the parts of a
