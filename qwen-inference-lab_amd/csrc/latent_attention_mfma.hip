@@ -32,7 +32,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define LM_AHEAD 8                                          // LDS fragments asked for ahead of the product that takes them
 #define LM_SLACK 5.5f                                      // how far a score may pass the exponentials' reference
 
-// EXACT: the sizes are the template's (rank + rot == 32 QF up to padding, rank == 16 VT): no size guards the products.
+// EXACT: the sizes are the template's (rank + rot == 32 QF, rank == 16 VT): no size guards the products, and no dim of a
+// query or key is masked.  Where rank + rot is short of 32 QF the dims behind a row are zeros in both (not EXACT).
 // SPLIT (steps of single rows): the block's columns are at most 16, one wave's; every wave takes the scores of all of
 // them and a quarter of the latent's dims in the second product, so that four waves work where one would, each holds
 // a quarter of the sums, and two blocks fit a compute unit.
@@ -463,7 +464,8 @@ int qil_latent_mfma(const float* q, const void* latent, const void* rope, const 
       page_size, scale, rt, hb, P, parts, window
 #define QIL_LM(QF, VT, EXACT) \
   status = single ? lm_launch<QF, VT, EXACT, true>(QIL_LM_ARGS) : lm_launch<QF, VT, EXACT, false>(QIL_LM_ARGS)
-  if (qf == 18 && vt == 32) QIL_LM(18, 32, true);
+  if (rank + rot == 18 * 32 && vt == 32) QIL_LM(18, 32, true);
+  else if (qf == 18) QIL_LM(18, 32, false);
   else if (qf <= 8 && vt <= 8) QIL_LM(8, 8, false);
   else if (qf <= 12 && vt <= 16) QIL_LM(12, 16, false);
   else QIL_LM(20, 32, false);

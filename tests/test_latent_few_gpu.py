@@ -124,3 +124,34 @@ def test_single_rows_over_latents(ops, monkeypatch, heads, rank, rot, key_parts,
                                positions=positions.cuda(), sink=sink, gate=gate, cu_seqlens=cu.cuda(),
                                seq_starts=positions.cuda(), n_seqs=n, max_query=1, max_context=max(lengths), **plain)
     torch.testing.assert_close(got.cpu(), want, atol=1e-2, rtol=1e-2)
+
+
+# sizes that fill the template of 512 + 64 dims and sizes that end short of it, whose last dims are padding: what lies behind a
+# query (the next head's, or nothing behind the last) and behind a key (its first dims stand in) must not reach a score
+@pytest.mark.parametrize('heads,rank,rot', [(3, 512, 40), (16, 512, 48), (5, 512, 56), (5, 512, 64), (2, 496, 72)])
+@pytest.mark.parametrize('rows', [(1, 1, 1, 1), (41, 1, 67, 3)])
+@pytest.mark.parametrize('key_parts', [None, (64, 1), (32, 4)])
+def test_dims_behind_a_row_stay_out_of_the_scores(ops, monkeypatch, heads, rank, rot, rows, key_parts):
+    """Queries whose heads differ a hundredfold, so that a neighbour's dims would outweigh every score.  bfloat16 queries,
+    probabilities and latents: eight bits each."""
+    monkeypatch.setattr(ops, 'LATENT_KEY_PARTS', key_parts)
+    starts, page = [50, 0, 31, 64], 16
+    n, n_seqs, most = sum(rows), len(rows), max(a + b for a, b in zip(starts, rows))
+    pages = -(-most // page)
+    latent, rope = rand(n_seqs * pages, page, rank, dtype=torch.bfloat16), rand(n_seqs * pages, page, rot, dtype=torch.bfloat16, seed=1)
+    tables = torch.randperm(n_seqs * pages, generator=torch.Generator().manual_seed(5)).to(torch.int32).view(n_seqs, pages)
+    size = torch.tensor([1.0, 100.0]).repeat(heads)[:heads].repeat_interleave(rank + rot).cuda()
+    q = rand(n, heads * (rank + rot), seed=2) * size
+    positions = torch.tensor([a + i for a, b in zip(starts, rows) for i in range(b)], dtype=torch.int32)
+    row_seq = torch.tensor([s for s, b in enumerate(rows) for _ in range(b)], dtype=torch.int32)
+    cu = torch.tensor([sum(rows[:s]) for s in range(n_seqs + 1)], dtype=torch.int32)
+    plain = dict(page_size=page, scale=(rank + rot) ** -0.5, heads=heads, rank=rank, rot=rot)
+    want = refs.latent_attention(q.cpu().to(torch.bfloat16).float(), latent=latent.cpu(), rope=rope.cpu(), block_tables=tables,
+                                 row_seq=row_seq, positions=positions, sink=None, **plain)
+    got = ops.latent_attention(q, latent=latent, rope=rope, block_tables=tables.cuda(), row_seq=row_seq.cuda(),
+                               positions=positions.cuda(), sink=None, cu_seqlens=cu.cuda(),
+                               seq_starts=torch.tensor(starts, dtype=torch.int32).cuda(), n_seqs=n_seqs, max_query=max(rows),
+                               max_context=most, **plain)
+    small = slice(None, None, 2)                             # (the large heads' softmax hangs on a score's last bits)
+    got, want = (v.view(n, heads, rank)[:, small] for v in (got.cpu(), want))
+    torch.testing.assert_close(got, want, atol=1e-2, rtol=1e-2)
