@@ -972,18 +972,26 @@ def _parts_workspace(rows, heads, head_dim, parts, plan, device):
     return torch.empty(floats + (4 if plan is not None else 0), dtype=torch.float32, device=device) if floats else None
 
 
-def decode_attention_takes(qkv, *, heads, kv_heads, head_dim, page_size, rotation, dtype):
+def decode_attention_takes(qkv, *, heads, kv_heads, head_dim, page_size, rotation, dtype, operands=()):
     """Whether ``decode_attention`` takes the step: a float32 ``Partials`` q/k/v product, few rows, sizes of the fused
-    kernel of the caches' type."""
+    kernel of the caches' type.  ``operands``: the step's caches, norm weights and bias (None: not there).  The float32 kernel
+    reads everything in pieces of 16 bytes and its keys in whole steps: a float32 step with an operand that begins between two
+    pieces, or with parts of other sizes, stays with ``qk_norm_rope_store`` and ``paged_attention``."""
     rot = rotation.rot_dim if rotation is not None else 0
     source = qkv.source if isinstance(qkv, Columns) else qkv
     if isinstance(qkv, Columns) and (qkv.offset % 8 or qkv.row % 8):
         return False
     if not isinstance(source, Partials) or qkv.shape[0] > FUSED_DECODE_MOST_ROWS:
         return False
-    if dtype == torch.float32:
-        return bool(library.load().qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 1, rot))
-    return dtype == torch.bfloat16 and bool(library.load().qil_attn_decode_fused_takes(heads, kv_heads, head_dim, page_size, rot))
+    if dtype != torch.float32:
+        return dtype == torch.bfloat16 and bool(library.load().qil_attn_decode_fused_takes(heads, kv_heads, head_dim, page_size, rot))
+    frequencies = getattr(rotation, 'frequencies', None)
+    tables = (frequencies,) if rotation is None or frequencies is not None else (rotation.cos, rotation.sin)
+    at = source.tensor.data_ptr()
+    for operand in (*operands, *tables):
+        at |= 0 if operand is None else operand.data_ptr()
+    return not at & 15 and ATTENTION_PART % 32 == 0 and \
+        bool(library.load().qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 1, rot))
 
 
 def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps, rotation, positions, writes, k_cache,

@@ -225,7 +225,8 @@ class Attention(Mixer):
             return self._forward_extended(qkv, rotation, norms, sizes, ctx, cache)
         # (the kernel that makes its queries itself norms over the whole head it sees: not for padded heads)
         if ctx.max_query == 1 and self.padded_dim == self.head_dim and \
-                ops.decode_attention_takes(qkv, page_size=cache.page_size, rotation=rotation, dtype=self.dtype, **sizes):
+                ops.decode_attention_takes(qkv, page_size=cache.page_size, rotation=rotation, dtype=self.dtype,
+                                           operands=(cache.k, cache.v, norms['q_weight'], norms['k_weight']), **sizes):
             # every row alone in its sequence: norm, rotation and cache write happen inside the attention kernel
             attended = ops.decode_attention(
                 qkv, rotation=rotation, positions=ctx.positions, writes=cache.writes, k_cache=cache.k, v_cache=cache.v,
@@ -259,7 +260,9 @@ class Attention(Mixer):
                      keep_first=self.keep_first)
         rows = self.qk_norm == 'row'
         if not rows and ctx.max_query == 1 and self.padded_dim == self.head_dim and \
-                ops.decode_attention_takes(qkv, page_size=cache.page_size, rotation=rotation, dtype=self.dtype, **sizes):
+                ops.decode_attention_takes(qkv, page_size=cache.page_size, rotation=rotation, dtype=self.dtype,
+                                           operands=(cache.k, cache.v, norms['q_weight'], norms['k_weight'], self.b_qkv_own),
+                                           **sizes):
             # every row alone in its sequence: bias, norm, rotation, temperature and cache write inside the attention kernel
             attended = ops.decode_attention(
                 qkv, rotation=rotation, positions=ctx.positions, writes=cache.writes, k_cache=cache.k, v_cache=cache.v,

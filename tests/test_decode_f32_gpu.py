@@ -101,3 +101,55 @@ def test_caches_at_other_addresses(ops):
     got = ops.paged_attention(q, k_cache=shifted, v_cache=v_cache, **step, **rest)
     want = refs.paged_attention(q.double(), k_cache=k_cache.double(), v_cache=v_cache.double(), accumulate=torch.float64, **step, **rest)
     torch.testing.assert_close(got.double(), want.double(), **NEAR)
+
+
+@pytest.mark.parametrize('moved', ['k', 'v', 'q_weight', 'k_weight', 'bias', 'cos', 'part'])
+def test_steps_with_operands_at_other_addresses(ops, monkeypatch, moved):
+    """A float32 step of an attention part, one operand beginning between multiples of 16 bytes (or parts of the keys that are
+    no whole steps): not the kernel that makes its queries itself, and the same results and cache."""
+    from qil_amd.cache.manager import KVView
+    from qil_amd.engine.batch import StepContext
+    from qil_amd.parts import Attention, Rotary
+    heads, kv_heads, d, width, lengths = 4, 2, 64, 512, [33, 200, 1]
+    rotary = Rotary(d, 10000.0, 256, device='cuda')
+    extended = dict(bias=True, gate=True) if moved == 'bias' else dict(bias=False)
+    part = Attention(width=width, heads=heads, kv_heads=kv_heads, head_dim=d, qk_norm_eps=1e-6, scale=d ** -0.5, position=rotary,
+                     dtype=torch.float32, **extended)
+    for index, (name, spec) in enumerate(part.param_specs().items()):
+        part.set_param(name, rand(*spec.shape, scale=spec.shape[-1] ** -0.5, seed=30 + index))
+    part.finalize()
+    k_cache, v_cache, step, rest = task(lengths, 16, heads, kv_heads, d)
+    rows, positions, table = len(lengths), step['positions'], step['block_tables']
+    slots = (table[step['row_seq'].long(), (positions // 16).long()] * 16 + positions % 16).to(torch.int32)
+    single = dict(cu_seqlens=torch.arange(rows + 1, dtype=torch.int32).cuda(), seq_starts=positions, seq_slots=None, single_rows=None)
+    ctx = StepContext(n_tokens=rows, n_seqs=rows, n_logit_rows=0, token_ids=None, positions=positions, row_seq=step['row_seq'],
+                      logit_rows=None, max_query=1, max_context=max(lengths), **single)
+    h = rand(rows, width, seed=41)
+    asked = []
+    plain = ops.decode_attention
+    monkeypatch.setattr(ops, 'decode_attention', lambda *a, **kw: (asked.append(1), plain(*a, **kw))[1])
+
+    def shifted(tensor):
+        return torch.empty(tensor.numel() + 1, dtype=tensor.dtype, device='cuda')[1:].view(tensor.shape).copy_(tensor)
+
+    def attend(k, v):
+        view = KVView(k=k, v=v, page_size=16, writes=True, group=0, block_tables=table, slots=slots)
+        out = part.forward(h, ctx, view)
+        return (out.sum() if isinstance(out, ops.Partials) else out), k, v
+    want = attend(k_cache.clone(), v_cache.clone())
+    assert asked
+    asked.clear()
+    k, v = (shifted(c) if moved == name else c.clone() for c, name in ((k_cache, 'k'), (v_cache, 'v')))
+    if moved in ('q_weight', 'k_weight'):
+        part.p[moved[0] + '_norm.weight'] = shifted(part.p[moved[0] + '_norm.weight'])
+    elif moved == 'bias':
+        part.b_qkv_own = shifted(part.b_qkv_own)
+    elif moved == 'cos':
+        rotation = rotary.rotation()
+        monkeypatch.setattr(rotary, 'rotation', lambda: type(rotation)(shifted(rotation.cos), rotation.sin, rotation.rot_dim))
+    elif moved == 'part':
+        monkeypatch.setattr(ops, 'ATTENTION_PART', 48)
+    got = attend(k, v)
+    assert not asked
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, equal_nan=True, **NEAR)
