@@ -1010,6 +1010,7 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     ``paged_attention``.  Returns what ``paged_attention`` returns."""
     n = qkv.shape[0]
     dtype = k_cache.dtype
+    _code(dtype)                                       # kernels of two types: other caches are refused
     stored = kv_heads if has_kv else 0
     own = (heads + (1 if values_are_keys else 2) * stored) * head_dim
     if writes and not has_kv:

@@ -150,3 +150,16 @@ def test_small_float32_products_take_narrow_blocks(lib):
         assert waves(rows, 4096, 1088) == 8                        # a stage more than 16 MB
         assert waves(rows, 6144, 1024) == 8
     assert lib.qil_gemm_f32_splits(4, 1024, 3072) == 12
+
+
+def test_decode_attention_refuses_caches_of_other_types():
+    """Its kernels read bfloat16 and float32 pages; caches of another type of two bytes must not be taken for bfloat16 ones."""
+    import torch
+    d, rows = 64, 2
+    for dtype in (torch.float16, torch.float64, torch.int16):
+        k, v = torch.zeros(3, 1, 16, d, dtype=dtype), torch.zeros(3, 1, d, 16, dtype=dtype)
+        with pytest.raises(ops.UnsupportedShape):
+            ops.decode_attention(ops.Partials(torch.zeros(1, rows, 3 * d)), heads=1, kv_heads=1, head_dim=d, q_weight=None,
+                                 k_weight=None, eps=1e-6, rotation=None, positions=torch.zeros(rows, dtype=torch.int32), writes=False,
+                                 k_cache=k, v_cache=v, page_size=16, block_tables=torch.zeros(rows, 1, dtype=torch.int32),
+                                 row_seq=torch.zeros(rows, dtype=torch.int32), max_context=1, scale=1.0, window=None)
