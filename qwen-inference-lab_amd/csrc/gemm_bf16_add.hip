@@ -30,7 +30,7 @@ template <int AROWS, bool INTO, int COLS = 16>
 __global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE, COLS == 8 ? 2 : AROWS == 8 ? 4 : 3)
 gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ stream,
                      bf16_t* __restrict__ out, float* __restrict__ squares, int M, int N, int K, int ksplit) {
-  extern __shared__ __align__(16) bf16_t lds[];            // per wave: 4 KB for W, AROWS x 256 bytes for A
+  extern __shared__ __align__(16) bf16_t lds[];            // per wave: COLS x 256 bytes for W, AROWS x 256 for A
   constexpr int ALOADS = AROWS / 4, WLOADS = COLS / 4, PER_WAVE = (COLS + AROWS) * 128;
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
@@ -186,12 +186,12 @@ int qil_gemm_bf16_add_takes(int M, int N, int K) {
 
 template <bool INTO>
 static int add_launch(const void* A, const void* W, float* stream, void* out, float* squares, int M, int N, int K, int groups,
-                      int ksplit, hipStream_t s) {
+                      int ksplit, hipStream_t s, bool narrow = false) {
   if (M == 0 || N == 0) return 0;
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)stream) % 16) return -1;
   int planned_groups, planned_ksplit;
   if (!add_plan(M, N, K, &planned_groups, &planned_ksplit)) return -1;
-  if (INTO && !groups && !ksplit && add_narrow(M, N, K)) {
+  if (INTO && narrow) {
     hipLaunchKernelGGL((gemm_bf16_add_kernel<8, INTO, 8>), dim3(N / 8), dim3(ADD_WAVES * QIL_WAVE), add_lds_bytes(M, ADD_WAVES, 8), s,
                        (const bf16_t*)A, (const bf16_t*)W, stream, (bf16_t*)out, squares, M, N, K, ADD_WAVES);
     QIL_RETURN_LAUNCH_STATUS();
@@ -213,14 +213,21 @@ static int add_launch(const void* A, const void* W, float* stream, void* out, fl
 
 extern "C" {
 
-// Pieces of a row whose sums of squares qil_gemm_bf16_add leaves (groups and ksplit 0): N / 16, or N / 8.
-int qil_gemm_bf16_add_pieces(int M, int N, int K) { return add_narrow(M, N, K) ? N / 8 : N / 16; }
-
-// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [pieces][M] that gets the rows' sums of squares
-// of the new stream in pieces of 16 (or 8) columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set both; then 16).
+// stream float32 [M, N] += A[M, K] W[N, K]^T.  squares: null, or float32 [N / 16][M] that gets the rows' sums of squares of
+// the new stream in pieces of 16 columns.  groups, ksplit: 0 = chosen here (tuning runs and tests set them).
 int qil_gemm_bf16_add(const void* A, const void* W, float* stream, float* squares, int M, int N, int K, int groups,
                       int ksplit, hipStream_t s) {
   return add_launch<true>(A, W, stream, nullptr, squares, M, N, K, groups, ksplit, s);
+}
+
+// The same in groups of 16 or 8 columns, whichever these sizes run better in.  squares: float32 [pieces][M]; pieces, the size
+// of the caller's array, has to be what qil_gemm_bf16_add_pieces says (N / 16, or N / 8).
+int qil_gemm_bf16_add_pieces(int M, int N, int K) { return add_narrow(M, N, K) ? N / 8 : N / 16; }
+int qil_gemm_bf16_add_in_pieces(const void* A, const void* W, float* stream, float* squares, int pieces, int M, int N, int K,
+                                hipStream_t s) {
+  if (M == 0 || N == 0) return 0;
+  if (pieces != qil_gemm_bf16_add_pieces(M, N, K)) return -1;
+  return add_launch<true>(A, W, stream, nullptr, squares, M, N, K, 0, 0, s, add_narrow(M, N, K));
 }
 
 // 1 if a product of up to 16 rows whose result has to be whole and of bfloat16 should run here (qil_gemm_bf16_whole): where

@@ -609,8 +609,9 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
             _require(x, 'x')
             _require(weight, 'weight', x.dtype, (o, k))
             _require(add_to, 'add_to', torch.float32, (n, o))
-            squares = torch.empty((lib.qil_gemm_bf16_add_pieces(n, o, k), n), dtype=torch.float32, device=x.device)
-            _check(lib.qil_gemm_bf16_add(_ptr(x), _ptr(weight), _ptr(add_to), _ptr(squares), n, o, k, 0, 0, _stream()),
+            pieces = lib.qil_gemm_bf16_add_pieces(n, o, k)
+            squares = torch.empty((pieces, n), dtype=torch.float32, device=x.device)
+            _check(lib.qil_gemm_bf16_add_in_pieces(_ptr(x), _ptr(weight), _ptr(add_to), _ptr(squares), pieces, n, o, k, _stream()),
                    'gemm_bf16_add')
             return Added(squares)
     if isinstance(x, Unmerged):

@@ -284,6 +284,8 @@ def _declare(lib):
     lib.qil_gemm_bf16_add_takes.restype = i
     lib.qil_gemm_bf16_add_pieces.argtypes = [i, i, i]
     lib.qil_gemm_bf16_add_pieces.restype = i
+    lib.qil_gemm_bf16_add_in_pieces.argtypes = [p, p, p, p, i, i, i, i, p]
+    lib.qil_gemm_bf16_add_in_pieces.restype = i
     lib.qil_gemm_bf16_whole_takes.argtypes = [i, i, i]
     lib.qil_gemm_bf16_whole_takes.restype = i
     lib.qil_gemm_bf16_whole.argtypes = [p, p, p, i, i, i, p]

@@ -39,3 +39,18 @@ def test_adds_in_groups_of_eight_columns(ops, m, n, k, narrow):
     want = ops.linear(ops.add_rmsnorm(stream, None, weight, 1e-6, torch.bfloat16), q, None, partials=True)
     value = lambda y: y.tensor.sum(0) if isinstance(y, ops.Partials) else y.float()
     torch.testing.assert_close(value(got), value(want), atol=2.0 ** -6, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize('m,n,k', [(1, 1024, 3072), (8, 2048, 6144), (9, 1024, 3072)])
+def test_adds_by_the_older_entry_leave_pieces_of_sixteen(ops, m, n, k):
+    """qil_gemm_bf16_add writes N / 16 pieces a row whatever the sizes, and nothing behind them."""
+    lib = ops.library.load()
+    x, w = rand(m, k, dtype=torch.bfloat16), rand(n, k, dtype=torch.bfloat16, seed=3, scale=k ** -0.5)
+    stream, squares = rand(m, n, scale=2.0, seed=7), torch.full((n // 8, m), 7.0, device='cuda')
+    want = stream.double() + x.double() @ w.double().t()
+    assert lib.qil_gemm_bf16_add(x.data_ptr(), w.data_ptr(), stream.data_ptr(), squares.data_ptr(), m, n, k, 0, 0, ops._stream()) == 0
+    # as above: a float32 sum of k products of unit variance, added to values of size two
+    torch.testing.assert_close(stream.double(), want, atol=2e-5, rtol=1e-5)
+    pieces = stream.double().square().reshape(m, n // 16, 16).sum(-1).t()
+    torch.testing.assert_close(squares[:n // 16].double(), pieces, atol=1e-5, rtol=1e-5)
+    assert (squares[n // 16:] == 7).all()

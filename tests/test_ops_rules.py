@@ -163,3 +163,13 @@ def test_decode_attention_refuses_caches_of_other_types():
                                  k_weight=None, eps=1e-6, rotation=None, positions=torch.zeros(rows, dtype=torch.int32), writes=False,
                                  k_cache=k, v_cache=v, page_size=16, block_tables=torch.zeros(rows, 1, dtype=torch.int32),
                                  row_seq=torch.zeros(rows, dtype=torch.int32), max_context=1, scale=1.0, window=None)
+
+
+def test_adds_are_told_how_many_pieces_their_array_holds(lib):
+    """Groups of 8 columns leave twice the pieces of groups of 16: an array sized for the other number is refused before
+    anything is launched (the addresses are never read)."""
+    for m, n, k in ((1, 1024, 3072), (8, 2048, 6144), (9, 1024, 3072), (8, 1024, 2048)):
+        pieces = lib.qil_gemm_bf16_add_pieces(m, n, k)
+        assert pieces in (n // 16, n // 8)
+        for other in (0, n // 16 + n // 8 - pieces, pieces + 1):
+            assert lib.qil_gemm_bf16_add_in_pieces(16, 16, 16, 16, other, m, n, k, None) == -1
