@@ -1532,6 +1532,8 @@ def latent_query(q, k_up, *, heads, dim, rot, rank, frequencies, positions):
     """Queries in the latent's space.  ``q`` [N, heads * (dim + rot)] (a head's unrotated part first), ``k_up``
     [heads, dim, rank] (the key expansion, a head's rows, as stored) -> float32 [N, heads, rank + rot]:
     k_up_h^T q_h, then the head's rotated part turned by the row's position."""
+    if rot < 2 or rot % 2:
+        raise RuntimeError(f'latent_query: {rot} rotated elements: size not taken by the kernel')
     n = q.shape[0]
     _require(q, 'q', None, (n, heads * (dim + rot)))
     _require(k_up, 'k_up', q.dtype, (heads, dim, rank))

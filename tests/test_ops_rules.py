@@ -173,3 +173,12 @@ def test_adds_are_told_how_many_pieces_their_array_holds(lib):
         assert pieces in (n // 16, n // 8)
         for other in (0, n // 16 + n // 8 - pieces, pieces + 1):
             assert lib.qil_gemm_bf16_add_in_pieces(16, 16, 16, 16, other, m, n, k, None) == -1
+
+
+def test_queries_in_the_latents_space_need_a_rotated_part():
+    """Pairs of elements are turned: none, or an odd number of them, is refused as ever."""
+    import torch
+    for rot in (0, 1, 7):
+        with pytest.raises(RuntimeError, match='size not taken'):
+            ops.latent_query(torch.zeros(2, 3 * (8 + rot)), torch.zeros(3, 8, 16), heads=3, dim=8, rot=rot, rank=16,
+                             frequencies=torch.zeros(rot // 2), positions=torch.zeros(2, dtype=torch.int32))
