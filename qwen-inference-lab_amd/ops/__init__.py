@@ -745,7 +745,8 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
         raise ValueError(f'gated_linear: x {tuple(x.shape)}, weight {tuple(weight.shape)}')
     out_dtype = out_dtype or x.dtype
     lib = library.load()
-    act = (GATE_FUNCTIONS[activation], float(limit), float(alpha))
+    # (silu has no numbers: whatever stands in their place is not looked at)
+    act = (0, 0.0, 1.0) if activation == 'silu' else (GATE_FUNCTIONS[activation], float(limit), float(alpha))
     inside = activation == 'silu' or not (x.data_ptr() | weight.data_ptr()) & 15     # (the others at any address: as products)
     # 17 to 256 rows of an interleaved matrix: the 32 x 32 tile kernel where it takes the sizes (measured against the
     # staged 16 x 16 kernel with the same epilogue at 17 to 64 rows: 37 to 38 us against 38 to 43 at Qwen3-8B sizes,

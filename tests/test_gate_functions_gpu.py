@@ -68,3 +68,10 @@ def test_gate_functions_that_do_not_exist(ops):
     raw = torch.cuda.current_stream().cuda_stream
     for act in (-1, 3, 16):
         assert lib.qil_gemm_bf16_gated_act(x.data_ptr(), w.data_ptr(), out.data_ptr(), 8, 48, 256, 1, 0, 0, 1, act, 0.0, 1.0, raw) == -1
+
+
+def test_silu_looks_at_no_numbers(ops):
+    x, w = rand(3, 256, seed=1), rand(512, 256, seed=3, scale=0.06)
+    for interleaved in (False, True):
+        got = ops.gated_linear(x, w, interleaved=interleaved, limit=None, alpha=None)
+        assert torch.equal(got, ops.gated_linear(x, w, interleaved=interleaved))
