@@ -141,16 +141,17 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ stream, const TD* __restr
   }
 }
 
-// The same for width % 4 == 0 and width <= 4 * J * THREADS: every access is a 16-byte (8-byte for
-// bfloat16) vector, all loads (stream, delta or its partial sums, weight) are issued before the first
+// The same for width % 4 == 0 and width <= 4 * J * THREADS: every access is a 16-byte (8-byte for bfloat16) vector, all loads (stream, delta or its partial sums, weight) are issued before the first
 // is used, and the row stays in registers between the statistics and the output.
-// AT_ONCE: the splits that are asked for at once (1, 4, 8 or, for one piece a thread, 16; the rest one by one; past the last it is
-// read again and not added).  A template's business: with the choice made in the kernel the norm of one row and four splits
-// took 4.4 us instead of 3.4, the branches' targets waiting for the instruction cache.  No load stands under a condition (a lane
-// past the row's end reads its last elements), and `pin` keeps it so: the compiler otherwise moves a load whose value is added
-// under a condition down to it, behind the wait for all others.  What the loads need stands in the first 56 bytes of the
-// arguments, which arrive in registers.  One row of 1,024 with four splits behind it 3.0 -> 2.6 us, 4 float32 rows with eight
-// and twelve 4.7 -> 3.9 (eight at a time, each under a condition, before); rows of 4,096 are level.
+// AT_ONCE: the splits that are asked for at once (1, 4, 8 or 16; past the last it is read again and not added).  A template's
+// business: with the choice made in the kernel the norm of one row and four splits took 4.4 us instead of 3.4, the branches'
+// targets waiting for the instruction cache.  No load stands under a condition (a lane past the row's end reads its last
+// elements), and `pin` keeps it so: the compiler otherwise moves a load whose value is added under a condition down to it,
+// behind the wait for all others.  What the loads need stands in the first 56 bytes of the arguments, which arrive in
+// registers.  One row of 1,024 with four splits behind it 2.5 -> 2.3 us, with sixteen 3.0 -> 2.75.
+// AT_ONCE 0: the splits in eights, each under a condition, and no more loads than there are: what is read again or past the end
+// costs more than the conditions where rows are wide.  us with eights / all at once, one row: 5,120 and 2 splits 3.2 / 3.8, 6
+// 3.8 / 4.8, 16 5.2 / 6.7; 4,096 and 4 3.4 / 3.0, 6 3.5 / 3.7, 16 4.5 / 5.4; 2,048 and 8 2.8 / 2.7, 12 3.1 / 3.3; 1,152 and 5 2.57 / 2.67.
 __device__ __forceinline__ void pin(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 template <typename TD, typename T, int THREADS, int J, int AT_ONCE>
 __global__ void __launch_bounds__(THREADS)
@@ -161,40 +162,51 @@ add_rmsnorm_vec_kernel(float* __restrict__ stream, const TD* __restrict__ delta,
   const int m = blockIdx.x;
   const size_t r = rows ? (size_t)rows[m] : (size_t)m;
   float* x = stream + r * width;
-  float4 cache[J], w[J], part[J][AT_ONCE];
+  constexpr bool EIGHTS = AT_ONCE == 0;
+  float4 cache[J], w[J], part[J][EIGHTS ? 1 : AT_ONCE];
+  if constexpr (EIGHTS) {
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int i = min((int)(threadIdx.x + j * THREADS) * 4, width - 4);
-    cache[j] = load4(x + i);
-    w[j] = load4(weight + i);
-  }
-  if (delta) {
-    const TD* base = delta + r * width;
-#pragma unroll
-    for (int u = 0; u < AT_ONCE; ++u) {
-#pragma unroll
-      for (int j = 0; j < J; ++j) part[j][u] = load4(base + min((int)(threadIdx.x + j * THREADS) * 4, width - 4));
-      if (u + 1 < splits) base += split_stride;
+    for (int j = 0; j < J; ++j) {
+      const int i = (threadIdx.x + j * THREADS) * 4;
+      const bool live = i < width;
+      cache[j] = live ? load4(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+      w[j] = live ? load4(weight + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+      part[j][0] = (live && delta) ? load_sum4(delta, r * width + i, splits, split_stride) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
-    for (int u = 0; u < AT_ONCE; ++u)
+    for (int j = 0; j < J; ++j) {
+      cache[j].x += part[j][0].x; cache[j].y += part[j][0].y; cache[j].z += part[j][0].z; cache[j].w += part[j][0].w;
+    }
+  } else {
 #pragma unroll
-      for (int j = 0; j < J; ++j) pin(part[j][u]);
+    for (int j = 0; j < J; ++j) {
+      const int i = min((int)(threadIdx.x + j * THREADS) * 4, width - 4);
+      cache[j] = load4(x + i);
+      w[j] = load4(weight + i);
+    }
+    if (delta) {
+      const TD* base = delta + r * width;
+#pragma unroll
+      for (int u = 0; u < AT_ONCE; ++u) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) part[j][u] = load4(base + min((int)(threadIdx.x + j * THREADS) * 4, width - 4));
+        if (u + 1 < splits) base += split_stride;
+      }
+#pragma unroll
+      for (int u = 0; u < AT_ONCE; ++u)
+#pragma unroll
+        for (int j = 0; j < J; ++j) pin(part[j][u]);
+    }
   }
   float sum = 0.f;
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int i = (threadIdx.x + j * THREADS) * 4;
-    if (delta) {
+    if (!EIGHTS && delta) {
       float4 d = part[j][0];
 #pragma unroll
       for (int u = 1; u < AT_ONCE; ++u)
         if (u < splits) { d.x += part[j][u].x; d.y += part[j][u].y; d.z += part[j][u].z; d.w += part[j][u].w; }
-      if constexpr (AT_ONCE >= 8)
-        for (int u = AT_ONCE; u < splits; ++u) {
-          const float4 more = load4(delta + r * width + u * split_stride + min(i, width - 4));
-          d.x += more.x; d.y += more.y; d.z += more.z; d.w += more.w;
-        }
       cache[j].x += d.x; cache[j].y += d.y; cache[j].z += d.z; cache[j].w += d.w;
     }
     if (i < width) {
@@ -327,13 +339,17 @@ int qil_add_rmsnorm(float* stream, const void* delta, int delta_dtype, int split
 #define QIL_NORM_SPLITS(TD, T, THREADS, J, AT_ONCE)                                                                  \
   hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, T, THREADS, J, AT_ONCE>), dim3(n_out), dim3(THREADS), 0, s, stream,   \
                      (const TD*)delta, rows, weight, width, splits, stride, eps, update, (T*)out)
+// (how many splits at once: the kernel's comment has both sides' figures)
 #define QIL_NORM_VEC(TD, T, THREADS, J)                                                                              \
   do {                                                                                                               \
+    constexpr int MOST = J > 1 ? (THREADS > 512 ? 1 : 4) : (THREADS > 256 ? 8 : 16);                                 \
     if (sizeof(TD) == 2 || splits == 1) QIL_NORM_SPLITS(TD, T, THREADS, J, 1);                                       \
     else if constexpr (sizeof(TD) == 4) {                                                                            \
-      if (splits <= 4) QIL_NORM_SPLITS(TD, T, THREADS, J, 4);                                                        \
-      else if (splits <= 8) QIL_NORM_SPLITS(TD, T, THREADS, J, 8);                                                   \
-      else QIL_NORM_SPLITS(TD, T, THREADS, J, J == 1 ? 16 : 8);                                                      \
+      if (splits > MOST || (THREADS > 256 && (splits == 5 || splits == 6)))                                          \
+        QIL_NORM_SPLITS(TD, T, THREADS, J, 0);                                                                       \
+      else if (MOST >= 4 && splits <= 4) QIL_NORM_SPLITS(TD, T, THREADS, J, (MOST < 4 ? 0 : 4));                     \
+      else if (MOST >= 8 && splits <= 8) QIL_NORM_SPLITS(TD, T, THREADS, J, (MOST < 8 ? 0 : 8));                     \
+      else if (MOST >= 16) QIL_NORM_SPLITS(TD, T, THREADS, J, (MOST < 16 ? 0 : 16));                                 \
     }                                                                                                                \
   } while (0)
 #define QIL_NORM_CASE(TD, T)                                                                                         \
