@@ -459,7 +459,11 @@ int qil_head_norm_gate(const float* o, const float* below, const void* g, int g_
   if (n == 0 || heads == 0) return 0;
   if (vdim < 1) return -1;
   const uintptr_t piece = dtype == QIL_F32 ? 16 : 8;             // bytes of four elements of the model's type
-  if (vdim % 4 == 0 && vdim <= 4 * 4 * QIL_WAVE && g_row % 4 == 0 && g_off % 4 == 0 &&
+  // A wave a head: its lanes are all at work from 256 elements on, with heads of 64 a quarter of them (us, block a head / wave a
+  // head: 3,000 rows of 32 heads of 64 27.9 / 45.4, of 16 of 80 25.6 / 24.2, of 96 25.8 / 23.8).  More than 512 elements are many
+  // loads a lane: where there are heads enough to hide them (1,200 heads of 768 4.7 / 5.0, 2,000 6.1 / 5.3, 33 of 1,024 4.0 / 4.1).
+  const bool waves = vdim >= 80 && (vdim <= 512 || (size_t)n * heads >= 1536);
+  if (waves && vdim % 4 == 0 && vdim <= 4 * 4 * QIL_WAVE && g_row % 4 == 0 && g_off % 4 == 0 &&
       ((uintptr_t)o | (uintptr_t)weight) % 16 == 0 && ((uintptr_t)g | (uintptr_t)y) % piece == 0 &&
       (size_t)n * heads <= INT32_MAX / 2) {
     const dim3 grid(((unsigned)n * heads + 3) / 4);

@@ -105,3 +105,15 @@ def test_one_token_a_sequence(ops, dtype, mode, dim, vdim, rot):
     for a, b in ((got.cpu(), want), (got_state[index['seq_slots'].long()].cpu(), want_state[index['seq_slots'].long()])):
         torch.testing.assert_close(a, b, atol=1e-4 * max(1.0, b.abs().max().item()), rtol=2e-5)
     assert torch.equal(got_state[[2, 5]].cpu(), state[[2, 5]])
+
+
+# on both sides of where a wave takes a head: heads of 76 and 80 elements, and 1,534 and 1,536 heads of 768
+@pytest.mark.parametrize('n,heads,vdim', [(5, 3, 76), (5, 3, 80), (767, 2, 768), (768, 2, 768), (3, 2, 1024), (600, 4, 64)])
+def test_head_norms_where_their_form_changes(ops, n, heads, vdim):
+    g = torch.Generator().manual_seed(vdim)
+    o, source = torch.randn(n, heads * vdim, generator=g).cuda(), torch.randn(n, 8 + heads * vdim, generator=g).bfloat16().cuda()
+    weight = (1 + 0.2 * torch.randn(heads * vdim, generator=g)).cuda()
+    got = ops.head_norm_gate(o, source, gate_offset=8, heads=heads, vdim=vdim, weight=weight, eps=1e-5, gate='silu', out_dtype=torch.bfloat16)
+    x, z = o.double().view(n, heads, vdim), source[:, 8:].double()
+    want = (x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt()).view(n, -1) * weight.double() * z * torch.sigmoid(z)
+    torch.testing.assert_close(got.double(), want, atol=1e-6, rtol=2.0 ** -8 + 1e-5)      # float32, then one rounding to bfloat16
