@@ -721,13 +721,32 @@ def interleave_gate_up(gate, up):
     return torch.stack((gate.view(inner // 16, 16, k), up.view(inner // 16, 16, k)), dim=1).reshape(2 * inner, k).contiguous()
 
 
+def _few_function_wanted(n, inner, k):
+    """Whether a gate function other than silu belongs into a product of up to 16 rows.  A long K is split over blocks where the
+    product is one of partial sums, here over a block's waves.  us as product and activation / as one: 8 rows of 6,144 x 2,048 13.8 /
+    12.7, 10,240 x 5,120 40.4 / 38.1, but 2,048 x 4,096 11.6 / 12.1 and 6,144 x 8,192 40.0 / 60.4; 16 rows of 8,192 x 3,072 21.3 / 20.7,
+    10,240 x 4,096 35.5 / 31.2, but 5,120 x 4,096 19.2 / 25.7 and 8,192 x 4,096 26.5 / 27.3."""
+    if n <= 8:
+        return k <= 3072 or (k <= 5120 and inner >= 3072)
+    return k <= 3072 or (k <= 4096 and inner >= 10240)
+
+
+def _wide_function_wanted(n, inner, k):
+    """Whether a gate function other than silu belongs into a product of more than 256 rows whose kernel with silu is wanted (a
+    count that allows 3 us on the GPU for a launch less on the host).  us as product and activation / as one: 300 rows of 1,024 x
+    1,024 14.1 / 15.6, 2,048 x 1,024 20.6 / 15.8, 3,072 x 1,024 20.1 / 16.6; 400 of 1,536 x 1,024 13.6 / 15.7, 2,048 x 1,024 15.7 / 15.7;
+    450 of 2,048 x 2,048 20.9 / 24.9, 600 26.3 / 26.1, 700 25.6 / 25.1; 300 of 4,096 x 1,024 18.2 / 17.1, 257 of 6,144 x 1,024 22.2 /
+    25.4, 513 of 8,192 x 512 31.9 / 35.9."""
+    return 2048 <= inner <= 4096 and (k <= 1024 or n > 512)
+
+
 def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activation='silu', limit=0.0, alpha=1.0):
     """act(x @ gate^T, x @ up^T) -> [N, I] (``activation``: a name of ``GATE_FUNCTIONS``; silu(gate) * up unless said), with ``weight`` the [2 I, K] matrix of both: the gate rows stacked
     before the up rows, or (``interleaved``) both in turns of 16 rows, which the kernels read faster.
 
-    One kernel when a fused kernel takes the sizes, whatever the gate function (bfloat16; up to 16 rows, or up to 256 rows of an interleaved
+    One kernel when a fused kernel takes the sizes and is ahead (bfloat16; up to 16 rows, or up to 256 rows of an interleaved
     matrix large enough to fill the chip, or more rows of one whose product is short (``qil_gemm_bf16_wide_gated_wanted``),
-    or from 512 rows on under ``OWN_LARGE_PRODUCTS``); otherwise the product followed by ``silu_mul`` or ``gated_act``.  Both add in float32.  (8 rows of 12,288 x 2,048 with a
+    or from 512 rows on under ``OWN_LARGE_PRODUCTS``; gate functions other than silu at fewer of these sizes); otherwise the product followed by ``silu_mul`` or ``gated_act``.  Both add in float32.  (8 rows of 12,288 x 2,048 with a
     clamped swish: 10.2 us and 5.1 for the activation, 12.7 as one kernel; a step of six such layers 496 -> 481 us.)
     ``lazy``: a few float32 rows may come back as ``Gated`` (the product's partial sums) for ``linear`` to finish."""
     if isinstance(x, Normed):
@@ -747,23 +766,35 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
     lib = library.load()
     # (silu has no numbers: whatever stands in their place is not looked at)
     act = (0, 0.0, 1.0) if activation == 'silu' else (GATE_FUNCTIONS[activation], float(limit), float(alpha))
-    inside = activation == 'silu' or not (x.data_ptr() | weight.data_ptr()) & 15     # (the others at any address: as products)
+    silu = activation == 'silu'
+    aligned = silu or not (x.data_ptr() | weight.data_ptr()) & 15            # (the others at any address: as products)
     # 17 to 256 rows of an interleaved matrix: the 32 x 32 tile kernel where it takes the sizes (measured against the
     # staged 16 x 16 kernel with the same epilogue at 17 to 64 rows: 37 to 38 us against 38 to 43 at Qwen3-8B sizes,
     # 73 to 85 against 87 to 102 at 14B sizes)
-    if x.dtype == torch.bfloat16 and interleaved and inside and MID_GATED_FEWEST_ROWS <= n <= MID_GEMM_MOST_ROWS and \
-            lib.qil_gemm_bf16_mid_gated_takes(n, both // 2, k):
+    # Other functions run inside a product where that is ahead of the product and the activation kernel: ``_few_function_wanted``;
+    # from 17 to 256 rows where the product itself is whole, or K is short (us as two / as one: 9,728 x 2,560 17 rows 27.1 / 21.0,
+    # 256 rows 47.4 / 46.4; split in K, 6,144 x 4,096 22.8 / 29.6 and 45.1 / 59.2, 8,192 x 2,048 32 rows 18.9 / 16.2, 256 rows 34.7 /
+    # 36.6, 7,168 x 1,536 64 rows 18.0 / 15.3, 256 rows 32.9 / 30.0); beyond, ``_wide_function_wanted``.
+    if silu or n > MID_GEMM_MOST_ROWS:
+        whole = True
+    elif n < MID_GATED_FEWEST_ROWS:
+        whole = _few_function_wanted(n, both // 2, k)
+    else:
+        whole = lib.qil_gemm_bf16_mid_splits(n, both, k) == 1
+    if x.dtype == torch.bfloat16 and interleaved and aligned and MID_GATED_FEWEST_ROWS <= n <= MID_GEMM_MOST_ROWS and \
+            (whole or k <= (2048 if n <= 32 else 1536)) and lib.qil_gemm_bf16_mid_gated_takes(n, both // 2, k):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
         _check(lib.qil_gemm_bf16_mid_gated_act(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), *act, _stream()),
                'gemm_bf16_mid_gated')
         return out
-    if x.dtype == torch.bfloat16 and n and inside and lib.qil_gemm_bf16_gated_takes(n, both // 2, k, int(interleaved)):
+    if x.dtype == torch.bfloat16 and n and aligned and whole and \
+            lib.qil_gemm_bf16_gated_takes(n, both // 2, k, int(interleaved)):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)
         _check(lib.qil_gemm_bf16_gated_act(_ptr(x), _ptr(weight), _ptr(out), n, both // 2, k, _code(out_dtype), 0, 0,
                                            int(interleaved), *act, _stream()), 'gemm_bf16_gated')
         return out
     at_x, at_weight = x.data_ptr(), weight.data_ptr()
-    if x.dtype == torch.bfloat16 and interleaved and \
+    if x.dtype == torch.bfloat16 and interleaved and (silu or _wide_function_wanted(n, both // 2, k)) and \
             ((OWN_LARGE_PRODUCTS and n >= WIDE_GEMM_FEWEST_ROWS and lib.qil_gemm_bf16_wide_gated_takes(n, both // 2, k)) or
              (not (at_x | at_weight) & 15 and lib.qil_gemm_bf16_wide_gated_wanted(n, both // 2, k))):
         out = torch.empty((n, both // 2), dtype=out_dtype, device=x.device)

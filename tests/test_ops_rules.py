@@ -182,3 +182,19 @@ def test_queries_in_the_latents_space_need_a_rotated_part():
         with pytest.raises(RuntimeError, match='size not taken'):
             ops.latent_query(torch.zeros(2, 3 * (8 + rot)), torch.zeros(3, 8, 16), heads=3, dim=8, rot=rot, rank=16,
                              frequencies=torch.zeros(rot // 2), positions=torch.zeros(2, dtype=torch.int32))
+
+
+def test_gate_functions_inside_products_of_many_rows():
+    """Where a function other than silu joins a product of more than 256 rows: 2,048 to 4,096 columns, and a short K or more rows
+    than a graph replays."""
+    assert ops._wide_function_wanted(300, 2048, 1024) and ops._wide_function_wanted(512, 3072, 1024)
+    assert not ops._wide_function_wanted(400, 1536, 1024) and not ops._wide_function_wanted(300, 512, 512)
+    assert not ops._wide_function_wanted(450, 2048, 2048) and ops._wide_function_wanted(600, 2048, 2048)
+    assert not ops._wide_function_wanted(600, 1024, 2048) and not ops._wide_function_wanted(257, 6144, 1024)
+
+
+def test_gate_functions_inside_products_of_few_rows():
+    """A short K, or more columns with it: what a long K loses when a block's waves share it instead of blocks."""
+    assert ops._few_function_wanted(1, 48, 256) and ops._few_function_wanted(8, 10240, 5120) and ops._few_function_wanted(16, 10240, 4096)
+    assert not ops._few_function_wanted(8, 2048, 4096) and not ops._few_function_wanted(8, 6144, 8192)
+    assert not ops._few_function_wanted(9, 5120, 4096) and not ops._few_function_wanted(16, 8192, 4096)
