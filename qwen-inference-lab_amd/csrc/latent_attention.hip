@@ -238,11 +238,15 @@ __global__ void head_product_kernel(const TX* __restrict__ x, int x_row, int x_h
 // not written), and the partial sums of a wave meet by exchanging halves (a step leaves half as many sums a lane: 60
 // shuffles for 64 sums over 16 lanes, 256 if every lane kept them all), then through LDS between the four waves.
 // 8 rows of 16 heads: 512 x 128 a head 13.8 us -> 6.6, 128 x 512 and the turned parts (a kernel of their own
-// before) 8.8 + 3.9 -> 6.0; up to 255 rows it beats the plain kernel above, whose reads of W wait one by one (64 rows 32.9 and
-// 11.9 us, here 7.8 and 7.7; 255 rows 34.3 and 22.8, here 12.8 and 20.2), and from 256 rows on bfloat16 is the GPU BLAS's.
+// before) 8.8 + 3.9 -> 6.0.  Up to 255 rows it is ahead of the plain kernel above, whose reads of W wait one by one, or level (64
+// rows 32.9 and 11.9 us, here 7.8 and 7.7; 255 rows 34.8 and 20.1, here 13.9 and 20.8), and from 256 rows on bfloat16 is the GPU
+// BLAS's.  With a k of less than 128 a thread has one or two of the weights it asks for ahead, and where there are many blocks the
+// plain kernel's few waits are hidden: us there / here 64 rows of 4 heads of 64 x 64 6.3 / 4.1, 96 of 16 of 64 x 256 level (768 blocks
+// here), 200 of them 7.1 / 9.1, 64 of 16 of 32 x 256 4.5 / 5.3, 33 of 4 of 16 x 64 3.4 / 4.1, 224 of 16 of 96 x 256 9.4 / 10.4 (1,792).
 // With `tail` the last blocks of grid.z turn the heads' rotated parts (see rotate_tail_kernel) instead.
 #define HP_AHEAD 8
 #define HP_FEW_ROWS 255
+#define HP_LONG_K 128
 template <typename TX, typename TW, typename TO, int OT>
 __global__ void __launch_bounds__(256)
 head_product_few_kernel(const TX* __restrict__ x, int x_row, int x_head, const TW* __restrict__ w, TO* __restrict__ out,
@@ -562,7 +566,9 @@ int qil_head_product(const void* x, int x_dtype, int x_row, int x_head, const vo
   const int threads = o_dim >= 256 ? 256 : (o_dim + 63) / 64 * 64;
   dim3 grid((n + rows - 1) / rows, heads, (o_dim + threads - 1) / threads);
   const size_t w_bytes = w_dtype == QIL_F32 ? 4 : 2, x_bytes = x_dtype == QIL_F32 ? 4 : 2;
-  const bool few = n <= HP_FEW_ROWS && o_dim % 8 == 0 && (size_t)w % (8 * w_bytes) == 0 &&
+  const long few_blocks = (long)((n + 7) / 8) * heads * ((o_dim + 63) / 64);
+  const bool ahead = n <= 32 || (n <= HP_FEW_ROWS && (k_dim >= HP_LONG_K || few_blocks <= 24L * k_dim - 768));
+  const bool few = ahead && o_dim % 8 == 0 && (size_t)w % (8 * w_bytes) == 0 &&
                    lds + 4 * 8 * 64 * sizeof(float) <= 64 * 1024;
   const int wide = k_dim % 4 == 0 && x_row % 4 == 0 && x_head % 4 == 0 && (size_t)x % (4 * x_bytes) == 0;
   const RotatedTail tail{tail_freq, positions, tail_offset, tail_rot};

@@ -155,3 +155,12 @@ def test_dims_behind_a_row_stay_out_of_the_scores(ops, monkeypatch, heads, rank,
     small = slice(None, None, 2)                             # (the large heads' softmax hangs on a score's last bits)
     got, want = (v.view(n, heads, rank)[:, small] for v in (got.cpu(), want))
     torch.testing.assert_close(got, want, atol=1e-2, rtol=1e-2)
+
+
+# on both sides of where the few-row product per head ends with a short k: by blocks (24 k - 768 of 64 outputs for eight rows) and rows
+@pytest.mark.parametrize('n,heads,k,o', [(33, 2, 16, 64), (40, 4, 64, 64), (96, 16, 64, 256), (104, 16, 64, 256), (32, 16, 32, 256), (33, 3, 33, 24),
+                                         (225, 16, 96, 256), (255, 2, 127, 64), (255, 2, 128, 64)])
+def test_products_per_head_where_their_form_changes(ops, n, heads, k, o):
+    x, w = rand(n, heads * k), rand(heads, k, o, dtype=torch.bfloat16, seed=1)
+    want = torch.einsum('nhk,hko->nho', x.double().view(n, heads, k), w.double()).reshape(n, -1)
+    near_sum(ops.head_product(x, w, heads=heads, out_dtype=torch.bfloat16), want, k, torch.bfloat16)
