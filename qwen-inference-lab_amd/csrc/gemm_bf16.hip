@@ -394,13 +394,15 @@ static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, i
 // Blocks of 4 waves where those of 8 leave half of the CUs without one: a CU draws 36 GB/s at most.  One row, inside a step:
 // 1,024 x 2,048 behind the merge in 4 splits 6.0 us with 32 blocks of 8, 4.6 with 64 of 4; 4,096 x 1,024 behind the norm in 2 5.9 with
 // 64, 5.4 with 128 (its operands asked for in one batch); 8 rows of 2,048 x 2,048 in 4 5.3 with 64, 4.5 with 128.  Up to 8 rows:
-// with 16 half the threads stage twice the rows.
+// with 16 half the threads stage twice the rows.  Behind the merge up to 4 rows: every block merges all of its rows' parts, and twice
+// the blocks of half the threads take longer for that than they gain (8 rows and 63 parts 16.7 us with 8 waves, 22.5 with 4; 6 rows
+// and 2 parts 5.5 / 5.9; 4 rows 4 is ahead at any number of parts).
 #define LINES_FEW_WAVES 4
 template <typename OUT, int ASRC = 0>
 static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
                         UnmergedA unmerged = UnmergedA(), NormedA normed = NormedA()) {
   const long blocks = (long)((N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES)) * splits;
-  if (M <= 8 && blocks <= QIL_CUS / 2)
+  if (M <= (ASRC == 1 ? 4 : 8) && blocks <= QIL_CUS / 2)
     return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
   return launch_lines_waves<OUT, ASRC, LINES_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
 }
