@@ -217,11 +217,36 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
   }
   // A slice first: a wait for it after W's requests would cover the first stages of W as well (unless A goes
   // straight into LDS, below)
-  if (ASRC == 2) {
-    // 1 / rms of the rows: a wave adds the pieces of two rows lane by lane, then across the wave.  Their sums of squares are asked
+  if (ASRC == 2 && WAVES == LINES_WAVES) {
+    // 1 / rms of the rows: wave m (and m + 8) adds the row's pieces lane by lane, then across the wave
+    float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
+    for (int m = wave; m < M; m += WAVES) {
+      float sum = 0.f;
+      for (int p = lane; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + m];
+      sum = wave_sum(sum);
+      if (lane == 0) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += WAVES * QIL_WAVE) {
+      const int m = idx / (cols_per_split / 8), c = (idx - m * (cols_per_split / 8)) * 8;
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (m < M) {
+        float x[8], g[8];
+        ld8(normed.stream + (size_t)m * K + k_begin + c, x);
+        ld8(normed.weight + k_begin + c, g);
+        const float scale = rstd[m];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = round_to<bf16_t>(x[e] * scale) * g[e];
+        v = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7]));
+      }
+      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = v;
+    }
+  } else if (ASRC == 2) {
+    // The same in blocks of few waves, of which a CU has one or two: a wave adds the pieces of two rows.  Their sums of squares are asked
     // for first and, right behind them, what the first two pieces of A a thread are made of: one wait for all of it, and the
     // sums are made while the rest arrives.  (Both are held in place: the compiler otherwise moves loads whose use stands
-    // under a condition down to it.)
+    // under a condition down to it.)  In blocks of 8 waves the loads for rows that are not there cost more than the wait: 8 rows of
+    // 6,144 x 2,048 8.1 us as above, 9.0 this way, 16 of 4,096 x 1,024 6.7 / 7.0.
     float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
     const int pieces = cols_per_split / 8, all = M * pieces;
     constexpr int EARLY = 2, THREADS = WAVES * QIL_WAVE, SQUARES = 4;
