@@ -32,12 +32,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define LM_AHEAD 8                                          // LDS fragments asked for ahead of the product that takes them
 #define LM_SLACK 5.5f                                      // how far a score may pass the exponentials' reference
 
-// EXACT: the sizes are the template's (rank + rot == 32 QF, rank == 16 VT): no size guards the products, and no dim of a
-// query or key is masked.  Where rank + rot is short of 32 QF the dims behind a row are zeros in both (not EXACT).
+// EXACT: the sizes are the template's (rank + rot == 32 QF up to padding, rank == 16 VT): no size guards the products.
+// PADDED: rank + rot may be short of 32 QF, the dims behind a row are made zeros in queries and keys (always so where not EXACT).
 // SPLIT (steps of single rows): the block's columns are at most 16, one wave's; every wave takes the scores of all of
 // them and a quarter of the latent's dims in the second product, so that four waves work where one would, each holds
 // a quarter of the sums, and two blocks fit a compute unit.
-template <int QF, int VT, bool EXACT, bool SPLIT>
+template <int QF, int VT, bool EXACT, bool SPLIT, bool PADDED>
 __global__ void __launch_bounds__(LM_THREADS, SPLIT ? 2 : 1)
 latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ latent, const bf16_t* __restrict__ rope,
                    const int* __restrict__ tables, int table_stride, const int* __restrict__ cu_seqlens,
@@ -104,7 +104,9 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
   int place[2];                                             // the cache slots of keys 2 jp, 2 jp + 1 of a step
   // Keys behind the block's last one stand in as that last key (their scores are masked), so that neither the look-ups
   // nor the rows' loads are under a condition; dims behind the row (other sizes than the template's) are read from its
-  // start and made zero.
+  // start and made zero.  SMALL: in steps of several rows of small sizes, whose blocks are many, a wave leaves out turns of units and
+  // fragments of queries that lie behind its row (320 rows of 16 heads of 128 + 32 23.8 us, now 22.2).
+  constexpr bool SMALL = QF <= 12 && !SPLIT;
   auto lookup = [&](int j0) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -116,13 +118,14 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int chunk = c0 + CSTEP * u, dim = chunk * 8, from = dim < d ? dim : 0;
+      if (SMALL && wave * (QIL_WAVE / (LM_KEYS / 2)) + CSTEP * u >= chunks) break;
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const bf16_t* row = from < rank ? latent + (size_t)place[e] * rank + from : rope + (size_t)place[e] * rot + (from - rank);
         ahead[u][e] = *reinterpret_cast<const uint4*>(row);
       }
     }
-    if constexpr (!EXACT) {
+    if constexpr (PADDED) {
 #pragma unroll
       for (int u = 0; u < NU; ++u)
         if ((c0 + CSTEP * u) * 8 >= d) ahead[u][0] = ahead[u][1] = make_uint4(0, 0, 0, 0);
@@ -161,19 +164,21 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
       qb[f] = *reinterpret_cast<const bf16x8*>(ks + r * krow + (EXACT || f < qf ? 32 * f : 0) + 8 * kb);
   } else {
     const float* qrow = q + gcol * d;
-    constexpr int G = QF % 6 == 0 ? 6 : 4;                  // fragments in flight: all of them would spill
+    constexpr int G = QF <= 8 ? QF : QF % 6 == 0 ? 6 : 4;     // fragments in flight: more of them would spill
 #pragma unroll
     for (int f0 = 0; f0 < QF; f0 += G) {
       float4 x[G][2];
 #pragma unroll
       for (int f = 0; f < G; ++f) {
-        const float* src = qrow + (EXACT || 32 * (f0 + f) + 8 * kb < d ? 32 * (f0 + f) + 8 * kb : 0);
+        if (SMALL && f0 + f >= qf) break;                   // fragments that no product takes
+        const float* src = qrow + (!PADDED || 32 * (f0 + f) + 8 * kb < d ? 32 * (f0 + f) + 8 * kb : 0);
         x[f][0] = *reinterpret_cast<const float4*>(src);
         x[f][1] = *reinterpret_cast<const float4*>(src + 4);
       }
 #pragma unroll
       for (int f = 0; f < G; ++f) {
-        const uint32_t mask = valid && (EXACT || 32 * (f0 + f) + 8 * kb < d) ? ~0u : 0u;
+        if (SMALL && f0 + f >= qf) break;
+        const uint32_t mask = valid && (!PADDED || 32 * (f0 + f) + 8 * kb < d) ? ~0u : 0u;
         const float4 a = x[f][0], b = x[f][1];
         qb[f0 + f] = __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(a.x, a.y) & mask, pack_bf16(a.z, a.w) & mask,
                                                            pack_bf16(b.x, b.y) & mask, pack_bf16(b.z, b.w) & mask));
@@ -319,12 +324,14 @@ latent_mfma_kernel(const float* __restrict__ q, const bf16_t* __restrict__ laten
 
 // out[column] = sum_p w_p acc_p / (sum_p w_p l_p + exp(sink - M)), w_p = exp(m_p - M), M the largest of the parts'
 // references and the sink, over the parts that the row's position reaches.  One block per (row, head): a thread holds four
-// neighbouring elements of every Gth part (G = threads / (rank / 4)) and asks for the first LMM_AHEAD of them before the
+// neighbouring elements of every Gth part (G = threads / (rank / 4)) and asks for the first AHEAD of them before the
 // parts' weights are made, none under a condition (a place behind the last part reads that part with weight zero); the G
 // groups' sums meet in LDS.  Dynamic LDS: [parts] weights, then 4 floats a thread.
 // What bounds it is its waits: with one element and four parts in flight a thread, 8 rows of 16 heads of 33 parts of 512
-// elements (8.7 MB) took 9.6 us; now 5.5.
+// elements (8.7 MB) took 9.6 us; now 5.5.  AHEAD: LMM_AHEAD, or one or two where no group has more parts (prompts in a few
+// parts have thousands of blocks: eight loads for one that counts kept the memory at work).
 #define LMM_AHEAD 8
+template <int AHEAD>
 __global__ void __launch_bounds__(512)
 latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_m, const float* __restrict__ part_l,
                     const int* __restrict__ positions, const float* __restrict__ sink, const float* __restrict__ gate,
@@ -340,10 +347,10 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   const int from = window > 0 ? max(0, position - window + 1) / P : 0;     // the part of the row's oldest visible key
   const int quads = rank / 4, groups = nt / quads, group = tid / quads, quad = tid - group * quads;
   const float* acc_p = part_acc + column * parts * rank + 4 * quad;
-  float4 ahead[LMM_AHEAD];
+  float4 ahead[AHEAD];
   auto fetch = [&](int p0) {
 #pragma unroll
-    for (int u = 0; u < LMM_AHEAD; ++u) ahead[u] = ld4(acc_p + (size_t)min(p0 + groups * u, reached - 1) * rank);
+    for (int u = 0; u < AHEAD; ++u) ahead[u] = ld4(acc_p + (size_t)min(p0 + groups * u, reached - 1) * rank);
   };
   fetch(from + group);
   const float floor_ = sink ? sink[h] : -INFINITY;
@@ -363,10 +370,10 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   below = block_sum(below, scratch);                        // its barriers also publish the weights
   const float inv = (gate ? gate[column] : 1.f) / below;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int p0 = from + group; p0 < reached; p0 += groups * LMM_AHEAD) {
+  for (int p0 = from + group; p0 < reached; p0 += groups * AHEAD) {
     if (p0 != from + group) fetch(p0);
 #pragma unroll
-    for (int u = 0; u < LMM_AHEAD; ++u) {
+    for (int u = 0; u < AHEAD; ++u) {
       const int p = p0 + groups * u;
       const float w = p < reached ? weight[p] : 0.f;
       acc.x += w * ahead[u].x; acc.y += w * ahead[u].y; acc.z += w * ahead[u].z; acc.w += w * ahead[u].w;
@@ -388,13 +395,13 @@ static int lm_lds_bytes(int rank, int rot) {
   return (LM_KEYS * (dp + 8) + rank * LM_VROW) * (int)sizeof(bf16_t);
 }
 
-template <int QF, int VT, bool EXACT, bool SPLIT>
+template <int QF, int VT, bool EXACT, bool SPLIT, bool PADDED>
 static int lm_launch(dim3 grid, size_t lds, hipStream_t s, const float* q, const bf16_t* latent, const bf16_t* rope,
                      const int* tables, int table_stride, const int* cu_seqlens, const int* seq_starts, int n_seqs,
                      int single, const float* sink, const float* gate, float* out, float* part_acc, float* part_m,
                      float* part_l, int heads, int rank, int rot, int page_size, float scale, int rt, int hb, int P, int parts,
                      int window) {
-  auto kernel = latent_mfma_kernel<QF, VT, EXACT, SPLIT>;
+  auto kernel = latent_mfma_kernel<QF, VT, EXACT, SPLIT, PADDED>;
   static bool raised = false;                                // per instantiation
   if (lds > 64 * 1024 && !raised) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -462,13 +469,13 @@ int qil_latent_mfma(const float* q, const void* latent, const void* rope, const 
   grid, lds, s, q, (const bf16_t*)latent, (const bf16_t*)rope, tables, table_stride, cu_seqlens, seq_starts, n_seqs, \
       single, parts == 1 ? sink : nullptr, parts == 1 ? gate : nullptr, out, part_acc, part_m, part_l, heads, rank, rot,     \
       page_size, scale, rt, hb, P, parts, window
-#define QIL_LM(QF, VT, EXACT) \
-  status = single ? lm_launch<QF, VT, EXACT, true>(QIL_LM_ARGS) : lm_launch<QF, VT, EXACT, false>(QIL_LM_ARGS)
-  if (rank + rot == 18 * 32 && vt == 32) QIL_LM(18, 32, true);
-  else if (qf == 18) QIL_LM(18, 32, false);
-  else if (qf <= 8 && vt <= 8) QIL_LM(8, 8, false);
-  else if (qf <= 12 && vt <= 16) QIL_LM(12, 16, false);
-  else QIL_LM(20, 32, false);
+#define QIL_LM(QF, VT, EXACT, PADDED) \
+  status = single ? lm_launch<QF, VT, EXACT, true, PADDED>(QIL_LM_ARGS) : lm_launch<QF, VT, EXACT, false, PADDED>(QIL_LM_ARGS)
+  if (qf == 18 && vt == 32 && rank + rot == 18 * 32) QIL_LM(18, 32, true, false);
+  else if (qf == 18 && vt == 32) QIL_LM(18, 32, true, true);
+  else if (qf <= 8 && vt <= 8) QIL_LM(8, 8, false, true);
+  else if (qf <= 12 && vt <= 16) QIL_LM(12, 16, false, true);
+  else QIL_LM(20, 32, false, true);
 #undef QIL_LM
 #undef QIL_LM_ARGS
   if (status) return status;
@@ -476,7 +483,9 @@ int qil_latent_mfma(const float* q, const void* latent, const void* rope, const 
     // parts in turns of as many threads as hold them all in LMM_AHEAD loads each, as far as 512 threads go
     const int want = rank / 4 * ((parts + LMM_AHEAD - 1) / LMM_AHEAD);
     const int threads = want >= 512 ? 512 : want <= 128 ? 128 : (want + 63) / 64 * 64;
-    hipLaunchKernelGGL(latent_merge_kernel, dim3(n_rows, heads), dim3(threads), (parts + 4 * threads) * sizeof(float), s,
+    const int groups = threads / (rank / 4);
+    const auto merge = parts <= groups ? latent_merge_kernel<1> : parts <= 2 * groups ? latent_merge_kernel<2> : latent_merge_kernel<LMM_AHEAD>;
+    hipLaunchKernelGGL(merge, dim3(n_rows, heads), dim3(threads), (parts + 4 * threads) * sizeof(float), s,
                        part_acc, part_m, part_l, positions, sink, gate, out, heads, rank, P, parts, window);
   }
   QIL_RETURN_LAUNCH_STATUS();
