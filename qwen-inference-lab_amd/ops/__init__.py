@@ -921,20 +921,48 @@ def _places(max_context, window, keep_first):
     return min(max_context, -(-keep_first // 32) * 32 + window + 31)
 
 
-def _rows_part(rows, kv_heads, max_context):
-    """Keys a part of the row kernel and of the float32 matrix-core kernel: about ROWS_BLOCKS blocks in all, parts of 64 to
-    ATTENTION_PART * 2 keys (measured in float32 at 2,048 keys of 8 kv heads: 1 row 28 us with parts of 64 to 256 against 67 with
-    512; 8 rows 45 us with 128 against 54 with 256 and 62 with 64; 64 rows level from 256 on; 8 rows of 8,192 keys best
-    at 256 and 512.  The matrix-core kernel, 16 heads of 128 in 8 groups: 4 rows of 520 keys 9.5 us with 64, 11.1 with 128; 8 of
-    2,048 31.6 / 29.4 / 29.8 / 37.0 with 64 / 128 / 256 / 512; 64 of 2,048 238 / 215 / 195 / 179; a CU draws 36 GB/s at most, so
-    few blocks a CU's worth of keys each are slow: 4 rows of 520 in parts of 512 take 33)."""
+def _rows_part(rows, kv_heads, max_context, blocks=ROWS_BLOCKS):
+    """Keys a part of the row kernel: about ``blocks`` blocks in all, parts of 64 to ATTENTION_PART * 2 keys
+    (measured in float32 at 2,048 keys of 8 kv heads: 1 row 28 us with parts of 64 to 256 against 67 with 512;
+    8 rows 45 us with 128 against 54 with 256 and 62 with 64; 64 rows level from 256 on; 8 rows of 8,192 keys best
+    at 256 and 512)."""
     if ATTENTION_PART != 256:                          # a test or tuning run has set it
         return ATTENTION_PART
-    wanted = max_context * rows * kv_heads / ROWS_BLOCKS
+    wanted = max_context * rows * kv_heads / blocks
     part = 64
     while part < 2 * ATTENTION_PART and part * 1.41 < wanted:      # the nearest of 64, 128, 256, 512
         part *= 2
     return part
+
+
+# Blocks the float32 matrix-core kernel aims for by the size of a head: two a CU with heads of 128 and four with heads of 64 are what
+# its registers leave room for, and with twice as many a second round is as long as the first (keys and values from memory, 16
+# heads of 128 in 8 groups, us for 1,024 blocks / 512: 8 rows of 2,048 keys 38.2 / 32.2, 16 of 1,000 36.8 / 31.9, 4 of 4,000 39.4 /
+# 33.0; 12 rows of 2,048 are better in 768 than in 384).
+MATRIX_BLOCKS = {128: 576, 64: 1024}
+
+
+def _matrix_part(rows, kv_heads, head_dim, places):
+    """Keys a part of the float32 matrix-core kernel.  A CU draws 36 GB/s at most, so that few blocks are slow: 4 rows of 520 keys of
+    8 groups in parts of 64 9.5 us, in parts of 512 33."""
+    return _rows_part(rows, kv_heads, places, MATRIX_BLOCKS[head_dim])
+
+
+def _matrix_attention_wanted(rows, heads, kv_heads, head_dim, places):
+    """Whether single float32 rows whose queries are made already belong on the matrix cores where both kernels take the sizes.
+    Groups of two heads and more: always (never more than 3 % behind in 304 sizes).  A group of one head uses one column of sixteen.
+    With heads of 128 the row kernel, which has more blocks a CU, is then ahead where the blocks make between one round and a dozen
+    (us there / on the matrix cores: 16 rows of 300 keys of 16 heads 21.9 / 24.6, 33 of 520 60.1 / 77.3, 33 of 2,048 of 2 35.2 / 44.5, and
+    33 of 20 of 16 in a step 27.2 / 29.8;
+    but 33 of 300 of 2 16.4 / 13.5, 48 of 1,000 of 16 174.6 / 142.2); with heads of 64 where they are just more than one (33 of 2,048
+    of 4 33.8 / 36.4, 1,056 blocks; 24 of 2,048 28.9 / 26.6)."""
+    if heads > kv_heads:
+        return True
+    if head_dim == 64:
+        blocks = rows * kv_heads * -(-places // _matrix_part(rows, kv_heads, head_dim, places))
+        return not MATRIX_BLOCKS[64] < blocks <= MATRIX_BLOCKS[64] * 9 // 8
+    work = rows * kv_heads * places
+    return (work <= 40000 and rows * kv_heads <= 512) or work >= 750000
 
 
 def _decode_parts(rows, kv_heads, max_context):
@@ -1077,7 +1105,7 @@ def decode_attention(qkv, *, heads, kv_heads, head_dim, q_weight, k_weight, eps,
     forms = (int(bool(rotate_first)), float(softcap or 0.0), int(bool(has_kv)), row - own, _ptr(bias), float(coef), int(every),
              _ptr(sinks), int(bool(values_are_keys)), _ptr(slopes), keep)
     if dtype == torch.float32:
-        part = _rows_part(n, kv_heads, places)
+        part = _matrix_part(n, kv_heads, head_dim, places)
         parts = max(1, -(-places // part))
         workspace = _parts_workspace(n, heads, head_dim, parts, None, out.device)
         _check(lib.qil_attn_decode_f32_fused(*sums, *where, _ptr(workspace), _ptr(out), n, heads, kv_heads, head_dim, page_size,
@@ -1247,13 +1275,15 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
                                       head_dim, window_arg, part, parts, _code(qkv.dtype), _ptr(sinks), keep,
                                       *_NO_GATE, _stream()), 'attn_merge')
         else:
-            part = _rows_part(rows, kv_heads, places)
+            # heads of 64 and 128 float32 elements run on the matrix cores (caches begin at multiples of 16 bytes)
+            matrix = qkv.dtype == torch.float32 and not (_ptr(qkv) | _ptr(k_cache) | _ptr(v_cache)) & 15 and \
+                lib.qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 0, 0) and ATTENTION_PART % 32 == 0 and \
+                _matrix_attention_wanted(rows, heads, kv_heads, head_dim, places)
+            part = _matrix_part(rows, kv_heads, head_dim, places) if matrix else _rows_part(rows, kv_heads, places)
             parts = max(1, -(-places // part))
             nbytes = lib.qil_attn_rows_workspace(rows, heads, head_dim, parts)
             workspace = torch.empty(nbytes // 4, dtype=torch.float32, device=qkv.device) if nbytes else None
-            # heads of 64 and 128 float32 elements run on the matrix cores (caches begin at multiples of 16 bytes)
-            if qkv.dtype == torch.float32 and not (_ptr(qkv) | _ptr(k_cache) | _ptr(v_cache)) & 15 and \
-                    lib.qil_attn_decode_f32_takes(heads, kv_heads, head_dim, page_size, 0, 0) and part % 32 == 0:
+            if matrix:
                 _check(lib.qil_attn_decode_f32(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
                                                block_tables.shape[1], _ptr(row_seq), _ptr(positions), _ptr(single_rows),
                                                _ptr(workspace), _ptr(out), rows, heads, kv_heads, head_dim, page_size, window_arg,

@@ -153,3 +153,15 @@ def test_steps_with_operands_at_other_addresses(ops, monkeypatch, moved):
     assert not asked
     for a, b in zip(got, want):
         torch.testing.assert_close(a, b, equal_nan=True, **NEAR)
+
+
+# groups of one head on both sides of the lines between the kernels, and parts of every size (64 to 512 keys)
+@pytest.mark.parametrize('heads,kv_heads,d,lengths', [(16, 16, 128, [60] * 41), (16, 16, 128, [60, 33] * 21), (4, 4, 64, [2048, 700, 9] * 11),
+                                                      (8, 8, 128, [1500] * 62 + [7]), (8, 8, 128, [1500] * 63), (16, 8, 128, [2048, 100, 1999] * 3),
+                                                      (4, 1, 64, [9000, 64, 8000])])
+def test_rows_alone_where_their_kernel_changes(ops, heads, kv_heads, d, lengths):
+    k_cache, v_cache, step, rest = task(lengths, 16, heads, kv_heads, d)
+    q = rand(len(lengths), heads * d, seed=5)
+    got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step, **rest)
+    want = refs.paged_attention(q.double(), k_cache=k_cache.double(), v_cache=v_cache.double(), accumulate=torch.float64, **step, **rest)
+    torch.testing.assert_close(got.double(), want.double(), **NEAR)

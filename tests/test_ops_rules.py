@@ -198,3 +198,16 @@ def test_gate_functions_inside_products_of_few_rows():
     assert ops._few_function_wanted(1, 48, 256) and ops._few_function_wanted(8, 10240, 5120) and ops._few_function_wanted(16, 10240, 4096)
     assert not ops._few_function_wanted(8, 2048, 4096) and not ops._few_function_wanted(8, 6144, 8192)
     assert not ops._few_function_wanted(9, 5120, 4096) and not ops._few_function_wanted(16, 8192, 4096)
+
+
+def test_float32_decode_parts_and_kernels():
+    """Two blocks a CU with heads of 128, four with heads of 64; groups of one head on the matrix cores where the work is less than
+    a round of blocks or many rounds (heads of 128), or not just more than one (heads of 64); other groups always."""
+    assert ops._matrix_part(8, 8, 128, 2048) == 256 and ops._matrix_part(8, 8, 64, 2048) == 128
+    assert ops._matrix_part(1, 8, 128, 512) == 64 and ops._matrix_part(64, 8, 128, 8192) == 512
+    for rows, kv_heads, places in ((1, 8, 100), (16, 16, 300), (33, 2, 4000), (64, 8, 16000)):
+        assert ops._matrix_attention_wanted(rows, 2 * kv_heads, kv_heads, 128, places)
+        assert ops._matrix_attention_wanted(rows, 2 * kv_heads, kv_heads, 64, places)
+    assert ops._matrix_attention_wanted(33, 2, 2, 128, 300) and ops._matrix_attention_wanted(48, 16, 16, 128, 1000)
+    assert not ops._matrix_attention_wanted(33, 16, 16, 128, 20) and not ops._matrix_attention_wanted(16, 16, 16, 128, 300) and not ops._matrix_attention_wanted(33, 16, 16, 128, 520)
+    assert not ops._matrix_attention_wanted(33, 4, 4, 64, 2048) and ops._matrix_attention_wanted(24, 4, 4, 64, 2048)
