@@ -10,11 +10,12 @@
 // 16-byte load, and a lane's four scores (rows 4 kb + i of a tile) are the probabilities that its four values meet.  A wave's
 // step is 16 keys: 8 + 8 loads a lane in flight with heads of 128.
 //
-// What bounds it: memory (64 products of 32 cycles a step and wave, 16 KB: 2 KB a CU and nanosecond if memory kept up); for
-// few short rows the chain position, page, key, score, value and the launch.  The row kernel walks the keys once for the
-// scores and once for the values with three barriers between, and adds every score over 16 lanes on the vector units.  Alone, 16
-// heads in 8 groups, row kernel / here: 4 rows of 520 keys 10.7 / 9.5 us, 8 of 2,048 31.0 / 29.4, 64 of 300 40.8 / 33.8, 33 of
-// 1,000 76.7 / 59.2, 32 heads and 64 rows of 2,048 215.8 / 179.2 (6.0 TB/s); 32 heads of 64 in 2 groups, 8 rows of 1,000, 32.3 / 8.3.
+// What bounds it: memory where rows are long (64 products of 32 cycles a step of 16 KB: a CU's four matrix cores ask for 32 bytes
+// a cycle, 77 B/ns, twice what memory brings a CU); for few short rows the chain position, page, key, score, value and the launch.
+// The row kernel walks the keys once for the scores and once for the values with three barriers between, and adds every score
+// over 16 lanes on the vector units.  Alone, keys and values from memory, 16 heads in 8 groups, us row kernel / here: 4 rows of 520
+// keys 16.8 / 13.0, 8 of 2,048 35.8 / 32.2, 64 of 300 44.4 / 33.7, 33 of 1,000 81.2 / 65.8, 32 heads and 64 rows of 2,048 221.6 /
+// 195.4 (5.5 TB/s); 32 heads of 64 in 2 groups, 8 rows of 1,000, 36.2 / 10.9.  (The parts: ops._matrix_part.)
 // With the queries, the new key and the new value made inside, a float32 step of 4 rows of 512 keys at 0.6B sizes takes 1,492 us
 // instead of 1,662 (12.6 + 5.1 us a layer -> 12.1).
 #include <algorithm>

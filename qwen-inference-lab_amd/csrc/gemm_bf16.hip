@@ -179,8 +179,8 @@ __device__ __forceinline__ uint4 merged8(const UnmergedA& u, int m, int k) {
 }
 
 // A given as the float32 residual stream whose RMSNorm is to be taken (qil/model.py:15-23), with the rows' sums of
-// squares already there in pieces: squares [pieces][M], one piece per 16 columns of the stream, left by the kernel that
-// completed the stream (gemm_bf16_cols.hip).  The block adds the pieces in a fixed order, normalises its slice of the
+// squares already there in pieces: squares [pieces][M], a piece for every 16 (or 8) columns of the stream, left by the kernel
+// that completed the stream (gemm_bf16_add.hip).  The block adds the pieces in a fixed order, normalises its slice of the
 // row (round, then the weight, as add_rmsnorm in elementwise.hip does) and needs no norm kernel before it.
 struct NormedA {
   const float* stream;                                     // [M, K]

@@ -259,7 +259,7 @@ scan_sums_kernel(const T* __restrict__ proj, int proj_row, int v_off, const floa
 }
 
 // grid (sequences, heads, elements of a head's state / 256 V): a thread takes V neighbouring elements of S (or of n) block
-// after block.  Four where they are aligned and lie in one row of S (V == 4: dim and vdim multiples of 4): 28 blocks of
+// after block.  Four where they are aligned and lie in one row of S (V == 4: dim and vdim multiples of 4): 48 blocks of
 // 8 heads of 128 x 256 26.8 -> 18.0 us (102 MB).
 #define CARRY_AHEAD 8
 template <int MODE, int V>

@@ -939,13 +939,17 @@ def _rows_part(rows, kv_heads, max_context, blocks=ROWS_BLOCKS):
 # its registers leave room for, and with twice as many a second round is as long as the first (keys and values from memory, 16
 # heads of 128 in 8 groups, us for 1,024 blocks / 512: 8 rows of 2,048 keys 38.2 / 32.2, 16 of 1,000 36.8 / 31.9, 4 of 4,000 39.4 /
 # 33.0; 12 rows of 2,048 are better in 768 than in 384).
-MATRIX_BLOCKS = {128: 576, 64: 1024}
+MATRIX_BLOCKS = {128: 552, 64: 1024}
 
 
 def _matrix_part(rows, kv_heads, head_dim, places):
     """Keys a part of the float32 matrix-core kernel.  A CU draws 36 GB/s at most, so that few blocks are slow: 4 rows of 520 keys of
-    8 groups in parts of 64 9.5 us, in parts of 512 33."""
-    return _rows_part(rows, kv_heads, places, MATRIX_BLOCKS[head_dim])
+    8 groups in parts of 64 13.0 us, in parts of 512 37.  Heads of 128: where a few blocks more than a round's 512 would run alone,
+    parts of half the size (33 rows of 1,000 keys of 8 groups: 528 blocks 76.4, 1,056 blocks 65.8)."""
+    part = _rows_part(rows, kv_heads, places, MATRIX_BLOCKS[head_dim])
+    if head_dim == 128 and part > 64 and ATTENTION_PART == 256 and 512 < rows * kv_heads * -(-places // part) <= 563:
+        part //= 2
+    return part
 
 
 def _matrix_attention_wanted(rows, heads, kv_heads, head_dim, places):

@@ -205,6 +205,7 @@ def test_float32_decode_parts_and_kernels():
     a round of blocks or many rounds (heads of 128), or not just more than one (heads of 64); other groups always."""
     assert ops._matrix_part(8, 8, 128, 2048) == 256 and ops._matrix_part(8, 8, 64, 2048) == 128
     assert ops._matrix_part(1, 8, 128, 512) == 64 and ops._matrix_part(64, 8, 128, 8192) == 512
+    assert ops._matrix_part(33, 8, 128, 1000) == 256          # 1,056 blocks, not 528
     for rows, kv_heads, places in ((1, 8, 100), (16, 16, 300), (33, 2, 4000), (64, 8, 16000)):
         assert ops._matrix_attention_wanted(rows, 2 * kv_heads, kv_heads, 128, places)
         assert ops._matrix_attention_wanted(rows, 2 * kv_heads, kv_heads, 64, places)
