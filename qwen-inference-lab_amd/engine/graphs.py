@@ -40,7 +40,9 @@ BUCKET = 512          # contexts are rounded up to a multiple of this many token
 MAX_GRAPHS = 24
 DECODE_REPLACE_AT = 3   # comings of a decode batch's (rows, context bucket) before it may push a graph out of a full store
 MIXED_BUCKET = 2048   # ... and of this many for a step with prompt portions (a portion moves on by its size a step)
-MIXED_MOST_ROWS = 512  # steps of more rows are bound by their kernels, not by their launches
+# Steps of more rows are bound by their kernels at 8B sizes (2,048 rows 9.1 ms, first passes included 9.8); at 0.6B sizes launches and
+# kernels are alike (643 rows: 2.7 ms on the host, 2.5 on the GPU), but such shapes are prompts' lengths, which seldom come again.
+MIXED_MOST_ROWS = 512
 MAX_MIXED_GRAPHS = 32  # each keeps the step's activations: tens of MB at 8B sizes and 512 rows
 MIXED_CAPTURE_AT = 2   # sightings of a shape before it is captured ...
 MIXED_REPLACE_AT = 4   # ... and before it may push the least recently replayed graph out of a full store
