@@ -171,13 +171,6 @@ static int launch_stream(const bf16_t* A, const bf16_t* W, const float* bias, OU
 #define LINES_DEPTH 3                                      // stages of W in flight per wave
 #define LINES_LDS_LIMIT (100 * 1024)                       // one block of 8 waves on a CU when A is long, two otherwise
 
-// Eight merged values of row m starting at column k (all of one head: d % 8 == 0), as bfloat16.
-__device__ __forceinline__ uint4 merged8(const UnmergedA& u, int m, int k) {
-  float v[8];
-  merged_values<8>(u, m, k, v);
-  return make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
-}
-
 // A given as the float32 residual stream whose RMSNorm is to be taken (qil/model.py:15-23), with the rows' sums of
 // squares already there in pieces: squares [pieces][M], a piece for every 16 (or 8) columns of the stream, left by the kernel
 // that completed the stream (gemm_bf16_add.hip).  The block adds the pieces in a fixed order, normalises its slice of the
@@ -190,8 +183,9 @@ struct NormedA {
   float eps;
 };
 
-// ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA)
-template <typename OUT, int ASRC, int WAVES = LINES_WAVES>
+// ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA).  AHEAD (ASRC 1): W's first requests
+// go out ahead of the parts' arrival (launch_lines).
+template <typename OUT, int ASRC, int WAVES = LINES_WAVES, bool AHEAD = true>
 __global__ void __launch_bounds__(WAVES * QIL_WAVE)
 gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N, int K,
                        int cols_per_split, UnmergedA unmerged, NormedA normed) {
@@ -215,72 +209,72 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
     source[u] = W + (size_t)min(n0 + row, N - 1) * K + k_begin + piece * 8;
     place[u] = row * 128 + ((piece ^ row) & 15) * 8;
   }
-  // A slice first: a wait for it after W's requests would cover the first stages of W as well (unless A goes
-  // straight into LDS, below)
-  if (ASRC == 2 && WAVES == LINES_WAVES) {
-    // 1 / rms of the rows: wave m (and m + 8) adds the row's pieces lane by lane, then across the wave
-    float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
-    for (int m = wave; m < M; m += WAVES) {
-      float sum = 0.f;
-      for (int p = lane; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + m];
-      sum = wave_sum(sum);
-      if (lane == 0) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += WAVES * QIL_WAVE) {
-      const int m = idx / (cols_per_split / 8), c = (idx - m * (cols_per_split / 8)) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m < M) {
-        float x[8], g[8];
-        ld8(normed.stream + (size_t)m * K + k_begin + c, x);
-        ld8(normed.weight + k_begin + c, g);
-        const float scale = rstd[m];
+  // Every wave walks its K range from a start of its own and wraps around: waves that all read the
+  // same columns of their rows at the same time load a few memory channels only.
+  const int turn = (n0 / 16) % stages;
+  auto column = [&](int stage) { const int st = stage + turn; return (st >= stages ? st - stages : st) * 128; };
+  // three stages in flight, each in registers of its own (named, so that none is indexed at run time)
+  u32x4 w0[4], w1[4], w2[4];
+  auto request = [&](u32x4 (&stage_w)[4], int stage) {
+    const int at = column(stage);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = round_to<bf16_t>(x[e] * scale) * g[e];
-        v = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7]));
-      }
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = v;
-    }
-  } else if (ASRC == 2) {
-    // The same in blocks of few waves, of which a CU has one or two: a wave adds the pieces of two rows.  Their sums of squares are asked
-    // for first and, right behind them, what the first two pieces of A a thread are made of: one wait for all of it, and the
-    // sums are made while the rest arrives.  (Both are held in place: the compiler otherwise moves loads whose use stands
-    // under a condition down to it.)  In blocks of 8 waves the loads for rows that are not there cost more than the wait: 8 rows of
-    // 6,144 x 2,048 8.1 us as above, 9.0 this way, 16 of 4,096 x 1,024 6.7 / 7.0.
+    for (int u = 0; u < 4; ++u) stage_w[u] = load_once(source[u] + at);
+  };
+  auto request_first = [&]() {
+    request(w0, 0);                                         // the host sees to stages >= 3
+    request(w1, 1);
+    request(w2, 2);
+  };
+  // What A is made of is asked for first and W's first stages right behind it, before anything is waited for (loads come back in
+  // order, so waiting for A does not wait for W).  With W asked for behind A's arrival the two waits stood one behind the other: one
+  // row of 4,096 x 1,024 behind the norm in 2 splits 5.1 -> 4.2 us, 8 rows 5.6 -> 5.1, 8 of 6,144 x 4,096 12.6 -> 12.2, 16 of 6,144 x 2,048
+  // 9.0 -> 8.5 (a step of 28 layers and one row 966 -> 932 with the merge's part of it, launch_lines).
+  constexpr int THREADS = WAVES * QIL_WAVE;
+  const int pieces = cols_per_split / 8, all = M * pieces;  // (rows past M stay as they are in LDS: their products are never stored)
+  if (ASRC == 2) {
+    // A wave adds the pieces of two rows' sums of squares; they are asked for together with what a thread's first two pieces of A are
+    // made of.  (All are held in place: the compiler otherwise moves loads whose use stands under a condition down to it.)
     float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
-    const int pieces = cols_per_split / 8, all = M * pieces;
-    constexpr int EARLY = 2, THREADS = WAVES * QIL_WAVE, SQUARES = 4;
+    constexpr int EARLY = 2, SQUARES = 4;
     float x[EARLY][8], g[EARLY][8], squares[2][SQUARES];
     auto ask = [&](int idx, float (&to_x)[8], float (&to_g)[8]) {
       const int m = idx / pieces, c = (idx - m * pieces) * 8;
       ld8(normed.stream + (size_t)m * K + k_begin + c, to_x);
       ld8(normed.weight + k_begin + c, to_g);
     };
+    const bool both_rows = M > WAVES, both_pieces = all > THREADS;
 #pragma unroll
-    for (int i = 0; i < SQUARES; ++i) {
-      const float* from = normed.squares + (size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M;
-      squares[0][i] = from[min(wave, M - 1)];
-      squares[1][i] = from[min(wave + WAVES, M - 1)];
-    }
+    for (int r2 = 0; r2 < 2; ++r2)
+      if (!r2 || both_rows)
 #pragma unroll
-    for (int u = 0; u < EARLY; ++u) ask(min((int)threadIdx.x + u * THREADS, all - 1), x[u], g[u]);
+        for (int i = 0; i < SQUARES; ++i)
+          squares[r2][i] = normed.squares[(size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M + min(wave + r2 * WAVES, M - 1)];
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+      if (!u || both_pieces) ask(min((int)threadIdx.x + u * THREADS, all - 1), x[u], g[u]);
+    __builtin_amdgcn_sched_barrier(0);
+    request_first();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r2 = 0; r2 < 2; ++r2) {                        // (2 WAVES rows are all there are)
       const int m = wave + r2 * WAVES;
       float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < SQUARES; ++i) {
+        if (r2 && !both_rows) break;
         asm volatile("" : "+v"(squares[r2][i]));
         if (lane + i * QIL_WAVE < normed.pieces) sum += squares[r2][i];
       }
       for (int p = lane + SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
       sum = wave_sum(sum);
       if (lane == 0 && m < M) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
+      if (!both_rows) break;
     }
 #pragma unroll
     for (int u = 0; u < EARLY; ++u)
+      if (!u || both_pieces)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(x[u][e]), "+v"(g[u][e]));
+        for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(x[u][e]), "+v"(g[u][e]));
     __syncthreads();
     auto put = [&](int idx, const float (&from_x)[8], const float (&from_g)[8]) {
       const int m = idx / pieces, c = (idx - m * pieces) * 8;
@@ -298,17 +292,45 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
       ask(idx, x[0], g[0]);
       put(idx, x[0], g[0]);
     }
-    // rows past M: zeros
-    for (int idx = all + threadIdx.x; idx < a_rows * pieces; idx += THREADS) {
-      const int m = idx / pieces, c = (idx - m * pieces) * 8;
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = make_uint4(0, 0, 0, 0);
-    }
   } else if (MERGE) {
-    for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 8); idx += WAVES * QIL_WAVE) {
-      const int m = idx / (cols_per_split / 8), c = (idx - m * (cols_per_split / 8)) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m < M) v = merged8(unmerged, m, k_begin + c);
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = v;
+    MergeParts<8, 4> parts;
+    const int P = merge_part_keys(unmerged);
+    int idx = threadIdx.x, m, c;
+    auto ask = [&](int of) {
+      m = of / pieces;
+      c = (of - m * pieces) * 8;
+      merge_ask(unmerged, P, m, k_begin + c, parts);
+    };
+    auto put = [&]() {
+      float v[8];
+      merge_finish(unmerged, P, m, k_begin + c, parts, v);
+      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) =
+          make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+    };
+    if constexpr (!AHEAD) {
+      for (; idx < all; idx += THREADS) {
+        ask(idx);
+        put();
+      }
+      request_first();
+    } else if constexpr (WAVES < LINES_WAVES) {
+      ask(min(idx, all - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      request_first();
+      parts.arrived();                                      // (in the loop this would be a wait for W as well)
+      if (idx < all) put();
+      for (idx += THREADS; idx < all; idx += THREADS) {
+        ask(idx);
+        put();
+      }
+    } else {
+      ask(min(idx, all - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      request(w0, 0);                                       // (all three stages of eight waves are in the way of the slower waves' parts)
+      parts.arrived();
+      if (idx < all) put();                                 // (a piece a thread: launch_lines)
+      request(w1, 1);
+      request(w2, 2);
     }
   } else {
     // A as it is goes from memory straight into LDS, 512 columns of a row an instruction, and is not waited for
@@ -322,21 +344,8 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
             (const __attribute__((address_space(1))) void*)(A + (size_t)min(m, M - 1) * K + k_begin + c0 + lane * 8),
             (__attribute__((address_space(3))) void*)(a_lds + m * row_width + c0), 16, 0, 0);
     }
+    request_first();
   }
-  // Every wave walks its K range from a start of its own and wraps around: waves that all read the
-  // same columns of their rows at the same time load a few memory channels only.
-  const int turn = (n0 / 16) % stages;
-  auto column = [&](int stage) { const int st = stage + turn; return (st >= stages ? st - stages : st) * 128; };
-  // three stages in flight, each in registers of its own (named, so that none is indexed at run time)
-  u32x4 w0[4], w1[4], w2[4];
-  auto request = [&](u32x4 (&stage_w)[4], int stage) {
-    const int at = column(stage);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) stage_w[u] = load_once(source[u] + at);
-  };
-  request(w0, 0);                                           // the host sees to stages >= 3
-  request(w1, 1);
-  request(w2, 2);
   if (ASRC == 0) {
     // A has landed, W's 12 loads need not: s_waitcnt vmcnt(12) lgkmcnt(0).  As a builtin and with the LDS counter
     // in it, because the compiler treats a load into LDS as an access of both kinds and, until it sees one wait
@@ -400,11 +409,11 @@ static bool lines_takes(const void* A, const void* W, const float* bias, int M, 
   return lines_lds(M, K, splits) <= LINES_LDS_LIMIT;
 }
 
-template <typename OUT, int ASRC, int WAVES>
+template <typename OUT, int ASRC, int WAVES, bool AHEAD = true>
 static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
                               UnmergedA unmerged, NormedA normed) {
   const size_t lds = lines_lds(M, K, splits, WAVES);
-  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC, WAVES>;
+  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC, WAVES, AHEAD>;
   static size_t granted = 0;                              // per instantiation
   if (lds > 64 * 1024 && lds > granted) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -422,13 +431,23 @@ static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, i
 // with 16 half the threads stage twice the rows.  Behind the merge up to 4 rows: every block merges all of its rows' parts, and twice
 // the blocks of half the threads take longer for that than they gain (8 rows and 63 parts 16.7 us with 8 waves, 22.5 with 4; 6 rows
 // and 2 parts 5.5 / 5.9; 4 rows 4 is ahead at any number of parts).
+// Behind the merge W's first stages are asked for ahead of the parts' arrival (AHEAD) where all parts come in one turn: up to four of
+// them for blocks of 4 waves, a piece of A a thread for those of 8; a second turn's loads would come back behind W.  us without / with:
+// 1 row of 1,024 x 2,048, 2 parts 4.5 / 4.4 alone and 5.7 / 5.3 inside a step, 9 parts 5.9 / 5.9; 8 rows of 4,096 x 4,096, 4 parts
+// 8.7 / 8.1; 16 rows of 1,024 x 2,048, 2 parts (two pieces a thread) 6.8 / 7.2.
 #define LINES_FEW_WAVES 4
 template <typename OUT, int ASRC = 0>
 static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
                         UnmergedA unmerged = UnmergedA(), NormedA normed = NormedA()) {
   const long blocks = (long)((N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES)) * splits;
-  if (M <= (ASRC == 1 ? 4 : 8) && blocks <= QIL_CUS / 2)
-    return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
+  const bool few = M <= (ASRC == 1 ? 4 : 8) && blocks <= QIL_CUS / 2;
+  if constexpr (ASRC == 1) {
+    const bool ahead = few ? unmerged.parts <= 4 : (long)M * (K / splits / 8) <= LINES_WAVES * QIL_WAVE;
+    if (!ahead)
+      return few ? launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES, false>(A, W, C, M, N, K, splits, s, unmerged, normed)
+                 : launch_lines_waves<OUT, ASRC, LINES_WAVES, false>(A, W, C, M, N, K, splits, s, unmerged, normed);
+  }
+  if (few) return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
   return launch_lines_waves<OUT, ASRC, LINES_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
 }
 

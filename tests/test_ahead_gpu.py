@@ -1,0 +1,68 @@
+"""Few-row kernels that ask for their weights ahead of their operand's arrival: the edges of the rules and of the loads."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def ops():
+    from qil_amd import ops
+    ops.library.load()
+    return ops
+
+
+def rand(*shape, dtype=torch.float32, scale=1.0, seed=0):
+    g = torch.Generator().manual_seed(seed + sum(shape))
+    return (torch.randn(*shape, generator=g) * scale).to(dtype).cuda()
+
+
+# blocks of four and of eight waves; one turn of parts (4), a second one (5) and a third batch of maxima (21); a piece of A a thread
+# and more; a window that leaves the first parts without keys
+@pytest.mark.parametrize('m', [1, 4, 5, 8, 16])
+@pytest.mark.parametrize('parts', [1, 4, 5, 21])
+@pytest.mark.parametrize('n,heads,d,window', [(1024, 16, 128, 0), (64, 6, 64, 0), (4096, 32, 128, 40)])
+def test_products_behind_the_merge(ops, m, parts, n, heads, d, window):
+    """The parts past a row's keys hold NaN, which nothing may read into a sum.  The operand is rounded to bfloat16 (2^-9 of each of k
+    terms) and multiplied in float32."""
+    lib, part = ops.library.load(), 32
+    k, splits = heads * d, ops.library.load().qil_gemm_bf16_splits(m, n, heads * d)
+    assert lib.qil_gemm_bf16_unmerged_takes(m, n, heads, d, splits)
+    positions = torch.tensor([(r * 37 + 5) % (parts * part) for r in range(m - 1)] + [parts * part - 1], dtype=torch.int32).cuda()
+    acc, top, total = rand(m, heads, parts, d), rand(m, heads, parts, seed=1), rand(m, heads, parts, seed=2).abs() + 1
+    index = torch.arange(parts, device='cuda')
+    last = positions // part
+    first = (positions + 1 - window).clamp(min=0) // part if window else torch.zeros_like(last)
+    live = (index >= first[:, None]) & (index <= last[:, None])
+    weights = torch.where(live[:, None], top.double(), -torch.inf).softmax(-1)           # exp(m_p - max) over its sum
+    divisor = (weights * total.double().where(live[:, None], 0)).sum(-1)
+    want = (weights[..., None] * acc.double()).sum(2) / divisor[..., None]
+    workspace = torch.cat([acc.where(live[:, None, :, None], torch.nan).flatten(), top.where(live[:, None], torch.nan).flatten(),
+                           total.where(live[:, None], torch.nan).flatten()])
+    w = rand(n, k, dtype=torch.bfloat16, scale=k ** -0.5, seed=3)
+    out = torch.empty(splits, m, n, device='cuda')
+    assert lib.qil_gemm_bf16_unmerged(workspace.data_ptr(), positions.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, heads, d,
+                                      window, part, parts, splits, torch.cuda.current_stream().cuda_stream) == 0
+    rounded = want.reshape(m, k).to(torch.float32).to(torch.bfloat16).double()
+    # (a value that lies at a rounding's edge may go either way: one in a few hundred, 2^-8 of its size and 1 / sqrt(k) of the row's)
+    torch.testing.assert_close(out.double().sum(0), rounded @ w.double().t(), atol=2.0 ** -8 * 4 * k ** -0.5 * want.abs().max().item(), rtol=1e-5)
+
+
+# a thread's first and second piece of A and more; one and two rows a wave; pieces of 8 and of 16 columns, more than 256 of them
+@pytest.mark.parametrize('m', [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize('n,k,columns', [(4096, 1024, 8), (64, 384, 16), (6144, 4096, 16), (512, 4608, 16)])
+def test_products_behind_the_norm(ops, m, n, k, columns):
+    """As above, with the operand as the norm rounds it: the row over its root mean square, then the weight."""
+    lib = ops.library.load()
+    splits = lib.qil_gemm_bf16_splits(m, n, k)
+    if not lib.qil_gemm_bf16_normed_takes(m, n, k, splits):
+        pytest.skip('not a size of this kernel')
+    stream, weight = rand(m, k, scale=3.0), 1 + 0.1 * rand(k, seed=1)
+    squares = stream.square().reshape(m, k // columns, columns).sum(-1).t().contiguous()
+    normed = (stream.double() / torch.sqrt(stream.double().square().mean(-1, keepdim=True) + 1e-6)).float().bfloat16().float() * weight
+    w = rand(n, k, dtype=torch.bfloat16, scale=k ** -0.5, seed=2)
+    out = torch.empty(splits, m, n, device='cuda')
+    assert lib.qil_gemm_bf16_normed(stream.data_ptr(), weight.data_ptr(), squares.data_ptr(), k // columns, 1e-6, w.data_ptr(),
+                                    out.data_ptr(), m, n, k, splits, torch.cuda.current_stream().cuda_stream) == 0
+    torch.testing.assert_close(out.double().sum(0), normed.bfloat16().double() @ w.double().t(),
+                               atol=2.0 ** -8 * 4 * k ** -0.5 * normed.abs().max().item(), rtol=1e-5)
