@@ -674,7 +674,7 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
                        int inner, int K, int ksplit, int interleaved, GateFn fn) {
   extern __shared__ __align__(16) bf16_t lds[];            // A [8 or 16][K + pad], then a 4 KB buffer per wave
   const int a_rows = M <= 8 ? 8 : 16;                      // rows of A kept (8 or 16: a power of two)
-  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
+  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
   const int r = lane & 15, kb = lane >> 4;
   const int pair = wave / ksplit, part = wave - pair * ksplit;
   const int pairs = blockDim.x / QIL_WAVE / ksplit;
@@ -709,38 +709,27 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
 #pragma unroll
     for (int u = 0; u < 4; ++u) w[u] = load_once(gate_source[u] + offset + at);
   };
-  // A long A (more than two 16-byte pieces a thread): W's first two stages are requested first, then A is staged
-  // four pieces a thread at a time with all four loads before the first store; a loop of load, wait, store pays
-  // a round trip to L2 for every piece, six of them at K = 4096.  Measured in one process, 8 rows: 36.9 -> 35.6 us
-  // at 8B sizes, 26.8 -> 22.2 at 4B sizes.  Rows past M repeat row M - 1 and pieces past the end repeat the last
-  // one (a load under a condition would make every later wait a wait for all loads): their products are rows
-  // of D that are never stored.  A short A keeps the old order, which is 0.5 us faster at 0.6B sizes.
-  const int per_row = K / 8, total = a_rows * per_row;
-  if (total <= 2 * (int)blockDim.x) {                       // a short A: one or two pieces a thread, A first
-    for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-      const int m = idx / per_row, c = (idx - m * per_row) * 8;
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) = *reinterpret_cast<const uint4*>(A + (size_t)min(m, M - 1) * K + c);
-    }
-    request(g0, 0, 0); request(u0, up_offset, 0);
-    request(g1, 0, 1); request(u1, up_offset, 1);
-  } else {
-    request(g0, 0, 0); request(u0, up_offset, 0);           // the host sees to stages >= 2
-    request(g1, 0, 1); request(u1, up_offset, 1);
-    for (int base = threadIdx.x; base < total; base += 4 * blockDim.x) {
-      uint4 v[4];
-      int to[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int idx = min(base + j * (int)blockDim.x, total - 1);
-        const int m = idx / per_row, c = (idx - m * per_row) * 8;
-        v[j] = *reinterpret_cast<const uint4*>(A + (size_t)min(m, M - 1) * K + c);
-        to[j] = m * row_width + c;
+  // A goes straight into LDS, 512 columns of a row an instruction, with W's first two stages asked for right behind it: loads complete
+  // in order, so A is waited for without W, and W without A.  (In registers, with A behind W, A was there when all of W's first
+  // requests were, and with A ahead W was asked for only when A was there: 3,072 x 1,024,
+  // one row 5.3 -> 4.6 us, 16 rows 6.4 -> 5.3; 9,728 x 2,560, 8 rows 19.9 -> 19.2, 16 rows 20.5 -> 19.4.)  Rows past M stay as they are in LDS: their products are rows of D that are never stored.
+  const int waves = blockDim.x / QIL_WAVE;
+  for (int c0 = 0; c0 < K; c0 += 512)
+    if (c0 + lane * 8 < K) {
+      const bf16_t* from = A + (size_t)wave * K + c0 + lane * 8;
+      bf16_t* to = a_lds + wave * row_width + c0;
+#pragma unroll 4
+      for (int m = wave; m < M; m += waves) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                         (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+        from += (size_t)waves * K;
+        to += waves * row_width;
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(a_lds + to[j]) = v[j];
     }
-  }
-  __syncthreads();
+  request(g0, 0, 0); request(u0, up_offset, 0);             // the host sees to stages >= 2
+  request(g1, 0, 1); request(u1, up_offset, 1);
+  __builtin_amdgcn_s_waitcnt(0x4070);                       // vmcnt(16) lgkmcnt(0): see the whole-line kernel
+  __builtin_amdgcn_s_barrier();
 
   f32x4 gate = {0.f, 0.f, 0.f, 0.f}, up = {0.f, 0.f, 0.f, 0.f};
   // lanes past the kept rows read the rows again: their products are rows of D that are never stored
@@ -780,17 +769,17 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
     pass(u0); multiply(stage + 2, up);
   }
 
-  // the waves' sums meet in LDS (in the buffers, which every wave has finished with): [wave][gate, up][lane][4]
-  __syncthreads();
+  // the waves' sums meet in LDS (each wave's in its own buffer, which it has finished with): [gate, up][lane][4]
   float* sums = reinterpret_cast<float*>(lds + a_rows * row_width);
-  *reinterpret_cast<f32x4*>(sums + ((wave * 2 + 0) * QIL_WAVE + lane) * 4) = gate;
-  *reinterpret_cast<f32x4*>(sums + ((wave * 2 + 1) * QIL_WAVE + lane) * 4) = up;
+  constexpr int BUFFER = 16 * 128 / 2;                       // floats of a wave's buffer
+  *reinterpret_cast<f32x4*>(sums + wave * BUFFER + lane * 4) = gate;
+  *reinterpret_cast<f32x4*>(sums + wave * BUFFER + (QIL_WAVE + lane) * 4) = up;
   __syncthreads();
   if (part == 0 && stores) {
     f32x4 g = {0.f, 0.f, 0.f, 0.f}, v = {0.f, 0.f, 0.f, 0.f};
     for (int w = wave; w < wave + ksplit; ++w) {            // fixed order
-      g += *reinterpret_cast<const f32x4*>(sums + ((w * 2 + 0) * QIL_WAVE + lane) * 4);
-      v += *reinterpret_cast<const f32x4*>(sums + ((w * 2 + 1) * QIL_WAVE + lane) * 4);
+      g += *reinterpret_cast<const f32x4*>(sums + w * BUFFER + lane * 4);
+      v += *reinterpret_cast<const f32x4*>(sums + w * BUFFER + (QIL_WAVE + lane) * 4);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -815,15 +804,14 @@ static bool gated_plan(const void* A, const void* W, int M, int inner, int K, in
   for (int c = 8; c >= 1 && !ks; c /= 2)
     if (K % (128 * c) == 0 && K / (128 * c) >= (c == 1 || (long)(inner / 16) * c <= 8 * QIL_CUS ? 2 : 16)) ks = c;
   if (!ks) return false;
-  // Pairs that are fewer than the CUs: a CU each, and waves that have four stages where K is long enough (3,072 x 1,024: 192
-  // blocks of two waves instead of 96 of eight, part of 1,098 -> 1,053 us for a step of 28 layers and one row; 8 rows of 4,096 x
-  // 768 7.8 -> 6.2 us, 3,072 x 768 7.6 -> 6.0).  With many stages both shapes fill the CUs alike, also where the products are
-  // large enough for the count below: 4,096 x 6,144 20.8 us (21.1 by that count), 4,096 x 7,168 23.6 (24.1).
+  // Pairs that are fewer than the CUs: a CU each, and up to four waves with two stages or more, all on their way at once where they
+  // are two (8 rows, two waves / four: 3,072 x 1,024 5.3 / 5.3 us, 4,096 x 4,096 13.9 / 13.3, with eight 16.4; one / two: 768 x 512
+  // 4.3 / 3.7, 2,048 x 768 5.6 / 4.9).
   if (inner / 16 <= QIL_CUS && gated_lds(M, K, 8) <= 156 * 1024) {
     *pairs = 1;
     *ksplit = 1;
-    for (int c = 2; c <= 8; c *= 2)
-      if (K % (128 * c) == 0 && K / (128 * c) >= 4) *ksplit = c;
+    for (int c = 2; c <= 4; c *= 2)
+      if (K % (128 * c) == 0 && K / (128 * c) >= 2) *ksplit = c;
     return true;
   }
   // Pairs a block: what a CU has to do in all (its blocks one after the other, as many at a time as LDS and
