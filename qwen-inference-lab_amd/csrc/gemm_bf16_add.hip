@@ -23,6 +23,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define ADD_DEPTH 3                                        // stages in flight per wave
 #define ADD_LDS_LIMIT (160 * 1024)
 
+// The value of another lane of the same 16, by data-parallel move (a shuffle is a trip through LDS).
+template <int CONTROL>
+__device__ __forceinline__ float lanes_across(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CONTROL, 0xF, 0xF, true));
+}
+
 // AROWS: rows of A kept (8 or 16).  COLS: columns of a group, 16 or 8 (the matrix cores then make every column twice and memory
 // is read once: twice the groups, where those of 16 leave half of the CUs without a block).  INTO: the result goes into the
 // stream; else out [M, N] of bfloat16 gets it (squares null).
@@ -32,7 +38,7 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                      bf16_t* __restrict__ out, float* __restrict__ squares, int M, int N, int K, int ksplit) {
   extern __shared__ __align__(16) bf16_t lds[];            // per wave: COLS x 256 bytes for W, AROWS x 256 for A
   constexpr int ALOADS = AROWS / 4, WLOADS = COLS / 4, PER_WAVE = (COLS + AROWS) * 128;
-  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
+  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
   const int r = lane & 15, kb = lane >> 4;
   const int group = wave / ksplit, part = wave - group * ksplit;
   const int groups = blockDim.x / QIL_WAVE / ksplit;
@@ -47,28 +53,38 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
   bf16_t* buffer = lds + wave * PER_WAVE;
   bf16_t* a_buffer = buffer + COLS * 128;
 
+  // a load's address is a scalar base (the wave's rows and columns) and an offset of the lane's
   const int load_row = lane >> 4, piece = lane & 15;
-  const bf16_t* source[WLOADS];
-  const bf16_t* a_source[ALOADS];                          // rows past the last read it again: rows of D never stored
+  const char* w_base = reinterpret_cast<const char*>(W + (size_t)n0 * K + k_begin);
+  const char* a_base = reinterpret_cast<const char*>(A + k_begin);
+  const uint32_t w_offset = (uint32_t)load_row * (uint32_t)K * 2 + piece * 16;
+  uint32_t a_offset[ALOADS];                               // (rows of A past the last read it again: rows of D never stored)
   int place[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int row = 4 * u + load_row;
-    if (u < WLOADS) source[u] = W + (size_t)(n0 + row) * K + k_begin + piece * 8;
     place[u] = row * 128 + ((piece ^ row) & 15) * 8;
-    if (u < ALOADS) a_source[u] = A + (size_t)min(row, M - 1) * K + k_begin + piece * 8;
+    if (u < ALOADS) a_offset[u] = (uint32_t)min(row, M - 1) * (uint32_t)K * 2 + piece * 16;
   }
   u32x4 w0[WLOADS], w1[WLOADS], w2[WLOADS], a0[ALOADS], a1[ALOADS], a2[ALOADS];   // named, so that none is indexed at run time
   auto request = [&](u32x4 (&stage_w)[WLOADS], u32x4 (&stage_a)[ALOADS], int stage) {
-    const int at = column(stage);
+    const size_t at = (size_t)column(stage) * 2;
 #pragma unroll
-    for (int u = 0; u < WLOADS; ++u) stage_w[u] = load_once(source[u] + at);
+    for (int u = 0; u < WLOADS; ++u) stage_w[u] = load_once(w_base + at + (size_t)(4 * u) * K * 2 + w_offset);
 #pragma unroll
-    for (int u = 0; u < ALOADS; ++u) stage_a[u] = *reinterpret_cast<const u32x4*>(a_source[u] + at);
+    for (int u = 0; u < ALOADS; ++u) stage_a[u] = *reinterpret_cast<const u32x4*>(a_base + at + a_offset[u]);
   };
   request(w0, a0, 0);
   request(w1, a1, 1);
   request(w2, a2, 2);
+
+  // The cells of the stream that this lane will add to come in behind the first stages: read when the sums are there, they were one
+  // more trip to memory at the kernel's end (with the barrier that the sums' own buffers save and the squares' shuffles: one row of 1,024 x
+  // 3,072 5.3 -> 4.7 us, 8 rows 6.7 -> 5.3, 8 of 4,096 x 12,288 19.4 -> 18.0, 16 of 4,096 x 4,096 10.4 -> 9.1).
+  float cell[4] = {0.f, 0.f, 0.f, 0.f};
+  if (INTO)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cell[i] = stream[(size_t)min(4 * kb + i, M - 1) * N + n0 + (r & (COLS - 1))];
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const int a_row = r & (AROWS - 1), w_row = r & (COLS - 1);
@@ -101,16 +117,15 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
   if (left > 3) step(w0, a0, 0, false);
   if (left > 4) step(w1, a1, 0, false);
 
-  // The waves' sums meet in LDS ([wave][lane][4] floats, in the buffers, which every wave has finished with); part 0 of
+  // The waves' sums meet in LDS ([lane][4] floats, each wave's in its own buffer, which it has finished with); part 0 of
   // each group adds them in wave order; the lane that holds D[m = 4 kb + i][n = r] adds it into the stream.
   float* sums = reinterpret_cast<float*>(lds);
-  __syncthreads();
-  *reinterpret_cast<f32x4*>(sums + (wave * QIL_WAVE + lane) * 4) = acc;
+  *reinterpret_cast<f32x4*>(sums + wave * (PER_WAVE / 2) + lane * 4) = acc;
   __syncthreads();
   if (part == 0) {
     f32x4 total = {0.f, 0.f, 0.f, 0.f};
     for (int v = wave; v < wave + ksplit; ++v)              // fixed order
-      total += *reinterpret_cast<const f32x4*>(sums + (v * QIL_WAVE + lane) * 4);
+      total += *reinterpret_cast<const f32x4*>(sums + v * (PER_WAVE / 2) + lane * 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = 4 * kb + i;
@@ -120,16 +135,15 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
         continue;
       }
       if (m < M && stores) {
-        float* cell = stream + (size_t)m * N + n0 + r;
-        value = *cell + total[i];
-        *cell = value;
+        value = cell[i] + total[i];
+        stream[(size_t)m * N + n0 + r] = value;
       }
       if (squares) {                                        // the lanes of a row add their squares: one order for all
         float square = value * value;
-        square += __shfl_xor(square, 1, QIL_WAVE);
-        square += __shfl_xor(square, 2, QIL_WAVE);
-        square += __shfl_xor(square, 4, QIL_WAVE);
-        if (COLS == 16) square += __shfl_xor(square, 8, QIL_WAVE);
+        square += lanes_across<0xB1>(square);               // quads (1, 0, 3, 2): the neighbour
+        square += lanes_across<0x4E>(square);               // quads (2, 3, 0, 1)
+        square += lanes_across<0x141>(square);              // halves of 16 mirrored: the other quad, whose lanes agree by now
+        if (COLS == 16) square += lanes_across<0x140>(square);          // 16 mirrored: the other half
         if (r == 0 && m < M && stores) squares[(size_t)mine * M + m] = square;
       }
     }
@@ -149,7 +163,7 @@ static bool add_narrow(int M, int N, int K) {
 
 // Waves a group and groups a block for these sizes; false if the kernel does not take them.
 static bool add_plan(int M, int N, int K, int* groups, int* ksplit) {
-  if (M < 1 || M > 16 || N < 16 || N % 16 || K < 128 * ADD_DEPTH || K % 128) return false;
+  if (M < 1 || M > 16 || N < 16 || N % 16 || K < 128 * ADD_DEPTH || K % 128 || K > 1 << 27) return false;     // (a lane's offset: 32 bits)
   const int all_groups = N / 16;
   int best_groups = 0, best_ksplit = 0;
   double best_cost = 0;

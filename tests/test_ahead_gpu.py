@@ -66,3 +66,33 @@ def test_products_behind_the_norm(ops, m, n, k, columns):
                                     out.data_ptr(), m, n, k, splits, torch.cuda.current_stream().cuda_stream) == 0
     torch.testing.assert_close(out.double().sum(0), normed.bfloat16().double() @ w.double().t(),
                                atol=2.0 ** -8 * 4 * k ** -0.5 * normed.abs().max().item(), rtol=1e-5)
+
+
+# rows of A that the waves share unevenly, a last piece of A that half of the lanes load, waves with two stages and with more
+@pytest.mark.parametrize('m', [1, 3, 8, 9, 16])
+@pytest.mark.parametrize('inner,k', [(3072, 1024), (48, 256), (768, 640), (4096, 4096), (6144, 2176), (12288, 4096)])
+def test_gated_products_of_few_rows(ops, m, inner, k):
+    """silu(gate) * up of float32 sums of k products, rounded once.  (What stands in LDS past the rows is whatever ran before.)"""
+    assert m > 8 or ops.library.load().qil_gemm_bf16_gated_takes(m, inner, k, 1)       # (more rows of a long k do not fit LDS)
+    x, w = rand(m, k, dtype=torch.bfloat16), rand(2 * inner, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5)
+    y = x.double() @ w.double().t()
+    want = torch.nn.functional.silu(y[:, :inner]) * y[:, inner:]
+    got = ops.gated_linear(x, ops.interleave_gate_up(w[:inner].contiguous(), w[inner:].contiguous()), interleaved=True)
+    torch.testing.assert_close(got.double(), want, atol=3e-5 * want.abs().max().item(), rtol=2.0 ** -8)
+
+
+# groups of 8 and of 16 columns, one group a block and several, one wave and eight a group, a block that holds groups past the end
+@pytest.mark.parametrize('m', [1, 5, 8, 9, 16])
+@pytest.mark.parametrize('n,k', [(1024, 3072), (512, 1024), (16, 384), (4112, 1152), (4096, 4096), (80, 3200)])
+def test_products_that_add_into_the_stream(ops, m, n, k):
+    """Float32 sums of k products; the pieces of the squares are those of the stream as it is afterwards."""
+    lib = ops.library.load()
+    x, w = rand(m, k, dtype=torch.bfloat16), rand(n, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5)
+    stream = rand(m, n, seed=2)
+    want = stream.double() + x.double() @ w.double().t()
+    pieces = lib.qil_gemm_bf16_add_pieces(m, n, k)
+    squares = torch.empty(pieces, m, device='cuda')
+    assert lib.qil_gemm_bf16_add_in_pieces(x.data_ptr(), w.data_ptr(), stream.data_ptr(), squares.data_ptr(), pieces, m, n, k,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+    torch.testing.assert_close(stream.double(), want, atol=3e-6 * want.abs().max().item(), rtol=0)
+    torch.testing.assert_close(squares.double(), stream.double().square().reshape(m, pieces, n // pieces).sum(-1).t(), atol=0, rtol=1e-6)
