@@ -23,12 +23,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define ADD_DEPTH 3                                        // stages in flight per wave
 #define ADD_LDS_LIMIT (160 * 1024)
 
-// The value of another lane of the same 16, by data-parallel move (a shuffle is a trip through LDS).
-template <int CONTROL>
-__device__ __forceinline__ float lanes_across(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CONTROL, 0xF, 0xF, true));
-}
-
 // AROWS: rows of A kept (8 or 16).  COLS: columns of a group, 16 or 8 (the matrix cores then make every column twice and memory
 // is read once: twice the groups, where those of 16 leave half of the CUs without a block).  INTO: the result goes into the
 // stream; else out [M, N] of bfloat16 gets it (squares null).
@@ -140,10 +134,10 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
       }
       if (squares) {                                        // the lanes of a row add their squares: one order for all
         float square = value * value;
-        square += lanes_across<0xB1>(square);               // quads (1, 0, 3, 2): the neighbour
-        square += lanes_across<0x4E>(square);               // quads (2, 3, 0, 1)
-        square += lanes_across<0x141>(square);              // halves of 16 mirrored: the other quad, whose lanes agree by now
-        if (COLS == 16) square += lanes_across<0x140>(square);          // 16 mirrored: the other half
+        square += lane_move<0xB1>(square);               // quads (1, 0, 3, 2): the neighbour
+        square += lane_move<0x4E>(square);               // quads (2, 3, 0, 1)
+        square += lane_move<0x141>(square);              // halves of 16 mirrored: the other quad, whose lanes agree by now
+        if (COLS == 16) square += lane_move<0x140>(square);          // 16 mirrored: the other half
         if (r == 0 && m < M && stores) squares[(size_t)mine * M + m] = square;
       }
     }

@@ -108,7 +108,14 @@ __device__ __forceinline__ void head_norm8(float (&x)[8], int TG, const HeadFact
   float sum = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) sum += x[e] * x[e];
-  for (int o = TG >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, QIL_WAVE);
+  if (TG == 16) {                                       // rows of the data-parallel moves: the same additions without trips through LDS
+    sum += lane_move<0x128>(sum);                       // rotated by 8: the lane ^ 8
+    sum += lane_move<0x124>(sum);                       // by 4 (eight lanes agree with the other eight by now)
+    sum += lane_move<0x4E>(sum);
+    sum += lane_move<0xB1>(sum);
+  } else {
+    for (int o = TG >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, QIL_WAVE);
+  }
   const float rstd = rsqrtf(sum / (float)d + eps);
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = round_to<T>(x[e] * rstd) * f.w[e];
