@@ -44,10 +44,6 @@ __device__ __forceinline__ uint4 once4(const bf16_t* p) {
 __device__ __forceinline__ uint4 pack8(const float* v) {
   return make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
 }
-__device__ __forceinline__ uint4 shuffle4(uint4 v, int source) {
-  return make_uint4(__shfl(v.x, source, QIL_WAVE), __shfl(v.y, source, QIL_WAVE), __shfl(v.z, source, QIL_WAVE),
-                    __shfl(v.w, source, QIL_WAVE));
-}
 
 // What the first loads need stands in the first 56 bytes of the arguments, which arrive in registers; the rest and the row's
 // position and sequence are asked for in batches (a dozen reads of arguments, each waited for by itself, and 10 KB of sines to fetch
@@ -87,7 +83,7 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   if (begin >= end) return;
   const int pos_place = pos - span.hole;                   // the row's own key lies behind the hole
 
-  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE, waves = blockDim.x / QIL_WAVE;
+  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE), waves = blockDim.x / QIL_WAVE;
   const int r = lane & 15, kb = lane >> 4;
   const int dt = d / 16;
   const int* table = block_tables + (size_t)sequence * table_stride;
@@ -98,7 +94,9 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
 
   // Q fragments: B operand, column r = head kvh * g + r (filled below, after the first loads are on their way)
   bf16x8 qb[QFRAGS];
-  uint4 new_k = make_uint4(0, 0, 0, 0), new_v = make_uint4(0, 0, 0, 0);   // FUSED: chunk lane % (DMAX / 8) of the new key / value
+  // FUSED, behind the cells in which the waves' results meet: the queries [g][TG] chunks, the new key, the new value
+  uint4* shared_q = reinterpret_cast<uint4*>(lds + (blockDim.x / QIL_WAVE * g * (d + 2) + 3) / 4 * 4);
+  uint4* shared_new = shared_q + g * TG;
   // FUSED: the block whose keys end with the row's own position makes the new key and value, its last wave does that;
   // `owner` is the wave that meets the position among its steps
   const bool new_here = FUSED && fused.writes && pos_place >= begin && pos_place < end;
@@ -108,6 +106,11 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   f32x4 o[DTILES];
 #pragma unroll
   for (int t = 0; t < DTILES; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  // The page of a key and its place there (a division by a number that is not known takes forty instructions a lane).
+  const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
+  auto page_of = [&](int key) __attribute__((always_inline)) { return __builtin_expect(page_shift >= 0, 1) ? key >> page_shift : key / page_size; };
+  auto place_in = [&](int key) __attribute__((always_inline)) { return __builtin_expect(page_shift >= 0, 1) ? key & (page_size - 1) : key % page_size; };
 
   // What one 32-key step needs from memory: the K rows of both 16-key sub-tiles and the V^T fragments
   // of every dim tile, found through three entries of the block table.
@@ -121,15 +124,15 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
     for (int jt = 0; jt < 2; ++jt)
       // row r of sub-tile jt is key 8 (r / 4) + 4 jt + r % 4 of the step, so that a lane's eight
       // scores (rows 4 kb + i of both sub-tiles) are the eight consecutive keys 8 kb .. 8 kb + 7
-      page[jt] = table[min(k0 + 8 * (r >> 2) + 4 * jt + (r & 3), ctx - 1) / page_size];   // clamped: an invisible key's score is replaced
-    page[2] = table[(min(k0 + 8 * kb, ctx - 1) & ~7) / page_size];
+      page[jt] = table[page_of(min(k0 + 8 * (r >> 2) + 4 * jt + (r & 3), ctx - 1))];   // clamped: an invisible key's score is replaced
+    page[2] = table[page_of(min(k0 + 8 * kb, ctx - 1) & ~7)];
   };
   auto request = [&](int step, const int (&page)[3], StepData& data) __attribute__((always_inline)) {
     const int k0 = span.key(step * 32);
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt) {
       const int key = min(k0 + 8 * (r >> 2) + 4 * jt + (r & 3), ctx - 1);
-      const bf16_t* krow = k_cache + (((size_t)page[jt] * kv_heads + kvh) * page_size + (key % page_size)) * (size_t)d;
+      const bf16_t* krow = k_cache + (((size_t)page[jt] * kv_heads + kvh) * page_size + place_in(key)) * (size_t)d;
 #pragma unroll
       for (int ks = 0; ks < QFRAGS; ++ks) {
         const int dim = ks * 32 + kb * 8;
@@ -137,7 +140,7 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
       }
     }
     const int key = min(k0 + 8 * kb, ctx - 1) & ~7;
-    const bf16_t* vbase = v_cache + ((size_t)page[2] * kv_heads + kvh) * (size_t)d * page_size + (key % page_size);
+    const bf16_t* vbase = v_cache + ((size_t)page[2] * kv_heads + kvh) * (size_t)d * page_size + place_in(key);
 #pragma unroll
     for (int t = 0; t < DTILES; ++t)
       data.v[t] = t < dt ? once4(vbase + (size_t)(t * 16 + r) * page_size) : make_uint4(0, 0, 0, 0);
@@ -145,31 +148,31 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   auto attend = [&](int step, StepData& data) __attribute__((always_inline)) {
     const int k0 = span.key(step * 32);
     if constexpr (FUSED) {
-      if (owner && step == (pos_place >> 5)) {                   // the new key and value come from this wave's registers
+      if (owner && step == (pos_place >> 5)) {               // the new key and value are not in the pages yet: from LDS
         const int local = pos & 31;                          // key 8 (rr / 4) + 4 jt + rr % 4 of the step
         const int jt_new = (local >> 2) & 1, rr = ((local >> 3) << 2) | (local & 3);
+        uint4 piece[QFRAGS];
+        uint32_t value[DTILES];
 #pragma unroll
-        for (int ks = 0; ks < QFRAGS; ++ks) {
-          const uint4 piece = shuffle4(new_k, 4 * ks + kb);
+        for (int ks = 0; ks < QFRAGS; ++ks) piece[ks] = shared_new[4 * ks + kb];
+#pragma unroll
+        for (int t = 0; t < DTILES; ++t) value[t] = reinterpret_cast<const bf16_t*>(shared_new + TG)[16 * t + r];
+#pragma unroll
+        for (int ks = 0; ks < QFRAGS; ++ks)
 #pragma unroll
           for (int jt = 0; jt < 2; ++jt)
-            if (r == rr && jt == jt_new) data.k[jt][ks] = piece;
-        }
+            if (r == rr && jt == jt_new) data.k[jt][ks] = piece[ks];
         const int j = local & 7;                             // element of the lanes with kb == local / 8
+        uint32_t put[4];                                     // the bits of a lane's four words that the new value takes
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put[i] = kb == (local >> 3) && i == (j >> 1) ? 0xffffu << ((j & 1) * 16) : 0u;
 #pragma unroll
         for (int t = 0; t < DTILES; ++t) {
-          const uint4 piece = shuffle4(new_v, 2 * t + (r >> 3));             // chunk of dim 16 t + r
-          const int e = r & 7;
-          const uint32_t word = (e >> 1) == 0 ? piece.x : (e >> 1) == 1 ? piece.y : (e >> 1) == 2 ? piece.z : piece.w;
-          const uint32_t value = (word >> ((e & 1) * 16)) & 0xffffu;
-          if (kb == (local >> 3)) {
-            const uint32_t shift = (j & 1) * 16, keep = ~(0xffffu << shift), put = value << shift;
-            uint32_t w[4] = {data.v[t].x, data.v[t].y, data.v[t].z, data.v[t].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (i == (j >> 1)) w[i] = (w[i] & keep) | put;
-            data.v[t] = make_uint4(w[0], w[1], w[2], w[3]);
-          }
+          const uint32_t both = value[t] * 0x10001u;
+          data.v[t].x = (data.v[t].x & ~put[0]) | (both & put[0]);
+          data.v[t].y = (data.v[t].y & ~put[1]) | (both & put[1]);
+          data.v[t].z = (data.v[t].z & ~put[2]) | (both & put[2]);
+          data.v[t].w = (data.v[t].w & ~put[3]) | (both & put[3]);
         }
       }
     }
@@ -237,7 +240,10 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   };
   // FUSED: a wave makes HPP of the group's queries, or (the last wave, in its first lane groups) the new key and value.
   // Everything that takes is asked for ahead of the wave's keys and values, behind which it would wait otherwise: a
-  // wave's loads come back in order.  (With the pages looked up a step ahead: one row of 100 keys at 0.6B sizes 1,102 ->
+  // wave's loads come back in order.  What a wave waits for and how many instructions the slowest one has is what binds rows with few
+  // keys: with the new key's page looked up first, no load on the way under a condition, the new key and value from LDS (48
+  // shuffles before) and the waves' results read at once, a step of 28 layers and one row took 902 -> 888 us, of 12 layers and 8 rows
+  // of 2,048 keys 1,352 -> 1,341.  (With the pages looked up a step ahead: one row of 100 keys at 0.6B sizes 1,102 ->
   // 1,068 us a step of 28 layers, eight of 2,000 1,501 -> 1,467; two steps' keys and values in flight a wave do not fit
   // the registers, and blocks of four waves, three a CU, took 30 us where these take 19.)
   const int chunk = lane % TG, sub = lane / TG;
@@ -256,29 +262,50 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
       sum_lo[u] = *reinterpret_cast<const float4*>(p);
       sum_hi[u] = *reinterpret_cast<const float4*>(p + 4);
     }
+    // (what a step has no use for is read from where something stands: a load under a condition would make every wait behind it one
+    // for all loads, the keys' and values' too)
     const float* weight = query ? fused.q_weight : fused.k_weight;
-    if (weight) load_eight(weight + chunk * 8, factors.w);
-    if (fused.cos_table && fused.rot > 0) load_turns<FREQUENCIES>(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
+    load_eight((weight ? weight : fused.qkv) + chunk * 8, factors.w);
+    if constexpr (!FREQUENCIES) {
+      const bool turns = fused.cos_table && chunk < 2 * (fused.rot >> 4);
+      const int half_chunks = fused.rot >> 4, pair = chunk < half_chunks ? chunk : chunk - half_chunks;
+      const size_t at = (size_t)pos * (fused.rot >> 1) + pair * 8;
+      load_eight(turns ? fused.cos_table + at : fused.qkv, factors.c);
+      load_eight(turns ? fused.sin_table + at : fused.qkv, factors.sn);
+    } else {
+      load_turns<1>(factors, chunk, fused.cos_table, fused.sin_table, pos, fused.rot);
+    }
+  };
+  // A wave's own sums and factors have arrived (the keys and values asked for behind them need not have).
+  auto arrived = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) asm volatile("" : "+v"(sum_lo[u].x), "+v"(sum_lo[u].y), "+v"(sum_lo[u].z), "+v"(sum_lo[u].w),
+                                                 "+v"(sum_hi[u].x), "+v"(sum_hi[u].y), "+v"(sum_hi[u].z), "+v"(sum_hi[u].w));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(factors.w[e]), "+v"(factors.c[e]), "+v"(factors.sn[e]));
   };
   auto answer = [&](bool query, int head, float (&x)[8], float (&plain)[8]) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = 0.f;
-    for (int s0 = 0; s0 < fused.splits; s0 += AHEAD) {
-      if (s0) {
-        const float* from = fused.qkv + (size_t)row * fused.row_elems + column(query, head);
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-          const float* p = from + (size_t)min(s0 + u, fused.splits - 1) * fused.split_stride;
-          sum_lo[u] = *reinterpret_cast<const float4*>(p);
-          sum_hi[u] = *reinterpret_cast<const float4*>(p + 4);
-        }
-      }
+    auto add = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < AHEAD; ++u)
         if (s0 + u < fused.splits) {
           x[0] += sum_lo[u].x; x[1] += sum_lo[u].y; x[2] += sum_lo[u].z; x[3] += sum_lo[u].w;
           x[4] += sum_hi[u].x; x[5] += sum_hi[u].y; x[6] += sum_hi[u].z; x[7] += sum_hi[u].w;
         }
+    };
+    add(0);
+    for (int s0 = AHEAD; s0 < fused.splits; s0 += AHEAD) {
+      const float* from = fused.qkv + (size_t)row * fused.row_elems + column(query, head);
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const float* p = from + (size_t)min(s0 + u, fused.splits - 1) * fused.split_stride;
+        sum_lo[u] = *reinterpret_cast<const float4*>(p);
+        sum_hi[u] = *reinterpret_cast<const float4*>(p + 4);
+      }
+      arrived();
+      add(s0);
     }
     add_bias8(x, fused.bias, column(query, head));
 #pragma unroll
@@ -286,58 +313,59 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
     norm_rope8<bf16_t>(x, chunk, TG, factors, fused.q_weight != nullptr, DMAX, fused.eps, fused.cos_table && fused.rot > 0,
                        fused.rot, fused.rotate_first != 0);
   };
+  // The table's entries come first of all: of the wave's first step and of the new key (asked for at its use, behind the keys and values,
+  // its wait was one for all of them, before the barrier that everyone's queries stand behind).
+  int new_page = 0;
   auto make_queries = [&]() __attribute__((always_inline)) {
     if constexpr (FUSED) {
-      uint4* shared_q = reinterpret_cast<uint4*>(lds);       // [g][TG] chunks; the end of the kernel uses the LDS again
-      uint4* shared_new = shared_q + g * TG;                 // the new key, then the new value
-      if (makes_q || makes_new) {
-        bool query = makes_q;
-        for (int base = wave * HPP;;) {                      // once, unless the group is large for the block's waves
-          float x[8], plain[8];
-          answer(query, base + sub, x, plain);
-          if (query) {
-            if (fused.temp_every > 0) {
-              const float temperature = query_temperature(pos, fused.temp_coef, fused.temp_every);
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[e] *= temperature;
-            }
-            if (base + sub < g) shared_q[(base + sub) * TG + chunk] = pack8(x);
-          } else {
-            const bool value = sub & 1;
-            const uint4 made = value ? pack8(plain) : pack8(x);
-            if (sub < 2) {                                   // into the pages (qil/cache.py:79-82), and for this row's own step
-              shared_new[sub * TG + chunk] = made;
-              const size_t page = table[pos / page_size];
-              const int offset = pos % page_size;
-              if (!value) {
-                bf16_t* k_row = const_cast<bf16_t*>(k_cache) + ((page * kv_heads + kvh) * page_size + offset) * (size_t)DMAX;
-                *reinterpret_cast<uint4*>(k_row + chunk * 8) = made;
-              } else {
-                bf16_t* column = const_cast<bf16_t*>(v_cache) + ((page * kv_heads + kvh) * (size_t)DMAX + chunk * 8) * page_size + offset;
-                const uint32_t words[4] = {made.x, made.y, made.z, made.w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) column[(size_t)e * page_size] = (bf16_t)(words[e >> 1] >> ((e & 1) * 16));
-              }
+      auto make = [&](bool query, int base) __attribute__((always_inline)) {
+        float x[8], plain[8];
+        answer(query, base + sub, x, plain);
+        if (query) {
+          if (fused.temp_every > 0) {
+            const float temperature = query_temperature(pos, fused.temp_coef, fused.temp_every);
+  #pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] *= temperature;
+          }
+          if (base + sub < g) shared_q[(base + sub) * TG + chunk] = pack8(x);
+        } else {
+          const bool value = sub & 1;
+          const uint4 made = value ? pack8(plain) : pack8(x);
+          if (sub < 2) {                                   // into the pages (qil/cache.py:79-82), and for this row's own step
+            shared_new[sub * TG + chunk] = made;
+            const size_t page = new_page;
+            const int offset = place_in(pos);
+            if (!value) {
+              bf16_t* k_row = const_cast<bf16_t*>(k_cache) + ((page * kv_heads + kvh) * page_size + offset) * (size_t)DMAX;
+              *reinterpret_cast<uint4*>(k_row + chunk * 8) = made;
+            } else {
+              bf16_t* column = const_cast<bf16_t*>(v_cache) + ((page * kv_heads + kvh) * (size_t)DMAX + chunk * 8) * page_size + offset;
+              const uint32_t words[4] = {made.x, made.y, made.z, made.w};
+  #pragma unroll
+              for (int e = 0; e < 8; ++e) column[(size_t)e * page_size] = (bf16_t)(words[e >> 1] >> ((e & 1) * 16));
             }
           }
-          if (!query) break;
+        }
+      };
+      if (makes_q || makes_new) {
+        bool query = makes_q;
+        int base = wave * HPP;
+        make(query, base);
+        while (query) {                                      // (once, unless the group is large for the block's waves)
           base += waves * HPP;
           if (base >= g) {
             if (!makes_new) break;
             query = false;
           }
           ask(query, base + sub);
+          arrived();                                         // (no load of this rare way may be open where the ways meet)
+          make(query, base);
         }
       }
       __syncthreads();
 #pragma unroll
       for (int ks = 0; ks < QFRAGS; ++ks)                    // fragment ks of head r = chunk 4 ks + kb of that head
         qb[ks] = __builtin_bit_cast(bf16x8, r < g ? shared_q[r * TG + 4 * ks + kb] : make_uint4(0, 0, 0, 0));
-      if (owner) {
-        new_k = shared_new[chunk];
-        new_v = shared_new[TG + chunk];
-      }
-      __syncthreads();                                       // the LDS is free again
     } else {
 #pragma unroll
       for (int ks = 0; ks < QFRAGS; ++ks) {
@@ -348,9 +376,6 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
       }
     }
   };
-  if constexpr (FUSED) {
-    if (makes_q || makes_new) ask(makes_q, wave * HPP + sub);
-  }
   // The loads of a wave's first step go out before its queries are made, so that the two waits overlap, and the table's
   // entries are looked up a step ahead of the loads that need them.
   constexpr bool EARLY = FUSED;
@@ -376,12 +401,27 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   } else {
     int page[3];
     StepData here;
-    if (step <= last_step) {
+    if constexpr (EARLY) {
+      // (every wave looks up and asks: one without a step of its own for the block's last; conditions would cost the waits' counts)
+      look_up(min(step, last_step), page);
+      if (new_here) new_page = table[page_of(pos)];
+      asm volatile("" : "+v"(new_page));
+      __builtin_amdgcn_sched_barrier(0);
+      if (makes_q || makes_new) {
+        ask(makes_q, wave * HPP + sub);
+        __builtin_amdgcn_sched_barrier(0);
+        request(min(step, last_step), page, here);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived();
+      } else {
+        request(min(step, last_step), page, here);
+      }
+    } else if (step <= last_step) {
       look_up(step, page);
       request(step, page, here);
-      if (EARLY) look_up(step + waves, page);                // (clamped: any entry will do where there is no such step)
     }
     make_queries();
+    if (EARLY) look_up(step + waves, page);                  // (clamped: any entry will do where there is no such step)
     if (step <= last_step)
       for (;;) {
         attend(step, here);
@@ -409,14 +449,25 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
   __syncthreads();
   for (int idx = threadIdx.x; idx < g * d; idx += blockDim.x) {
     const int h = idx / d, e = idx - h * d;
-    float mm = -INFINITY;
-    for (int w = 0; w < waves; ++w) mm = fmaxf(mm, lds[((size_t)w * g + h) * cell + d]);
+    // every wave's cells asked for at once (waves the block does not have: the last one's, not used)
+    float mw[DEC_MAX_WAVES], lw[DEC_MAX_WAVES], ow[DEC_MAX_WAVES], mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < DEC_MAX_WAVES; ++w) {
+      const float* theirs = lds + ((size_t)min(w, waves - 1) * g + h) * cell;
+      mw[w] = theirs[d];
+      lw[w] = theirs[d + 1];
+      ow[w] = theirs[e];
+    }
+#pragma unroll
+    for (int w = 0; w < DEC_MAX_WAVES; ++w) mm = fmaxf(mm, mw[w]);
     float total = 0.f, ll = 0.f;
-    for (int w = 0; w < waves; ++w) {                       // fixed order
-      const float mw = lds[((size_t)w * g + h) * cell + d];
-      const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw - mm) * 1.44269504088896f);
-      total += lds[((size_t)w * g + h) * cell + e] * f;
-      ll += lds[((size_t)w * g + h) * cell + d + 1] * f;
+#pragma unroll
+    for (int w = 0; w < DEC_MAX_WAVES; ++w) {               // fixed order
+      const float f = w >= waves || mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw[w] - mm) * 1.44269504088896f);
+      if (w < waves) {
+        total += ow[w] * f;
+        ll += lw[w] * f;
+      }
     }
     const int head = kvh * g + h;
     if (parts == 1) {
@@ -583,7 +634,7 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   float* acc = (float*)workspace;
   float* m = acc ? acc + (size_t)rows * heads * parts * d : nullptr;
   float* l = m ? m + (size_t)rows * heads * parts : nullptr;
-  const size_t lds = std::max((size_t)waves * g * (d + 2) * sizeof(float), (size_t)(g + 2) * d * sizeof(bf16_t));
+  const size_t lds = ((size_t)waves * g * (d + 2) + 3) / 4 * 4 * sizeof(float) + (size_t)(g + 2) * d * sizeof(bf16_t);
   const dim3 grid = plan ? dim3(blocks, kv_heads) : dim3(rows, kv_heads, parts);
   int* part_keys = plan ? reinterpret_cast<int*>(l + (size_t)rows * heads * parts) : nullptr;
   FusedQKV fused;
@@ -600,13 +651,25 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
+#define QIL_DEC_FUSED(DMAX, FREQUENCIES)                                                                                          \
+  do {                                                                                                                             \
+    static bool granted = false;                           /* per instantiation: more LDS than a kernel has without asking */      \
+    if (lds > 64 * 1024 && !granted) {                                                                                             \
+      const hipError_t e = hipFuncSetAttribute((const void*)attn_decode_kernel<DMAX, true, true, false, FREQUENCIES>,              \
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);                             \
+      if (e != hipSuccess) return (int)e;                                                                                          \
+      granted = true;                                                                                                              \
+    }                                                                                                                              \
+    QIL_DEC_LAUNCH(DMAX, true, true, false, fused, FREQUENCIES);                                                                   \
+  } while (0)
   if (cos_table && !sin_table) {
-    if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused, true);
-    else QIL_DEC_LAUNCH(128, true, true, false, fused, true);
+    if (d == 64) QIL_DEC_FUSED(64, true);
+    else QIL_DEC_FUSED(128, true);
   } else {
-    if (d == 64) QIL_DEC_LAUNCH(64, true, true, false, fused);
-    else QIL_DEC_LAUNCH(128, true, true, false, fused);
+    if (d == 64) QIL_DEC_FUSED(64, false);
+    else QIL_DEC_FUSED(128, false);
   }
+#undef QIL_DEC_FUSED
 #undef QIL_DEC_LAUNCH
   QIL_RETURN_LAUNCH_STATUS();
 }

@@ -2,6 +2,9 @@
 import pytest
 import torch
 
+import kernel_refs as refs
+from test_kernels_gpu import Rot, build_cache
+
 pytestmark = pytest.mark.gpu
 
 
@@ -96,3 +99,33 @@ def test_products_that_add_into_the_stream(ops, m, n, k):
                                            torch.cuda.current_stream().cuda_stream) == 0
     torch.testing.assert_close(stream.double(), want, atol=3e-6 * want.abs().max().item(), rtol=0)
     torch.testing.assert_close(squares.double(), stream.double().square().reshape(m, pieces, n // pieces).sum(-1).t(), atol=0, rtol=1e-6)
+
+
+# groups of fifteen heads (more LDS than a kernel has without asking) and of one; pages whose size is no power of two; four sums at a
+# time and a fifth; neither norm nor rotation; new keys at every place of a step's lanes, in a block's first and last step
+@pytest.mark.parametrize('d,heads,kv_heads,page_size', [(128, 15, 1, 16), (128, 16, 8, 24), (64, 4, 4, 8), (64, 16, 1, 40)])
+@pytest.mark.parametrize('splits,plain,window', [(2, False, None), (5, False, 40), (1, True, None)])
+def test_decode_attention_that_makes_its_queries(ops, d, heads, kv_heads, page_size, splits, plain, window):
+    """Keys and values in the pages bit for bit those of the q/k kernel; the result against the float32 reference, one rounding to
+    bfloat16 and its neighbour."""
+    lengths = [1, 2, 31, 32, 33, 40, 100, 255, 256, 257, 300, 517]
+    dtype, rows = torch.bfloat16, len(lengths)
+    k_cache, v_cache, table, _ = build_cache(lengths, page_size, kv_heads, d, dtype)
+    positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32).cuda()
+    row_seq = torch.arange(rows, dtype=torch.int32).cuda()
+    sizes = dict(heads=heads, kv_heads=kv_heads, head_dim=d)
+    step = dict(page_size=page_size, block_tables=table, row_seq=row_seq, positions=positions, max_context=max(lengths),
+                scale=d ** -0.5, window=window, **sizes)
+    rest = dict(cu_seqlens=None, seq_starts=None, single_rows=None, n_seqs=rows, max_query=1)
+    slots = (table[row_seq.long(), (positions // page_size).long()] * page_size + positions % page_size).to(torch.int32)
+    qkv = ops.Partials(rand(splits, rows, (heads + 2 * kv_heads) * d, scale=splits ** -0.5, seed=21))
+    norms = dict(q_weight=None, k_weight=None, eps=0.0, rotation=None) if plain else \
+        dict(q_weight=1 + 0.1 * rand(d, seed=22), k_weight=1 + 0.1 * rand(d, seed=23), eps=1e-6, rotation=Rot(d, 10000.0, max(lengths), d))
+    k_fused, v_fused = k_cache.clone(), v_cache.clone()
+    fused = ops.decode_attention(qkv, writes=True, k_cache=k_fused, v_cache=v_fused, **norms, **step)
+    q = ops.qk_norm_rope_store(qkv, positions=positions, slots=slots, k_cache=k_cache, v_cache=v_cache, page_size=page_size,
+                               dtype=dtype, **norms, **sizes)
+    assert torch.equal(k_fused.view(torch.int16), k_cache.view(torch.int16))
+    assert torch.equal(v_fused.view(torch.int16), v_cache.view(torch.int16))
+    want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step, **rest).float()
+    torch.testing.assert_close(fused.float(), want, atol=2.0 ** -8, rtol=2.0 ** -7)
