@@ -214,12 +214,13 @@ struct GatedA {
 };
 
 // ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = the activation of a gated feed-forward (GatedA)
-template <int ASRC, int WAVES>
+// AHEAD (ASRC 1 and 2): W's first requests go out ahead of the operand's arrival (launch_f32_lines).
+template <int ASRC, int WAVES, bool AHEAD = false>
 __global__ void __launch_bounds__(WAVES * QIL_WAVE)
 gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K,
                       int cols_per_split, UnmergedA unmerged, GatedA gated) {
   extern __shared__ __align__(16) float fl_lds[];           // A slice [8 or 16][cols + pad], then the waves' buffers
-  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = threadIdx.x / QIL_WAVE;
+  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
   const int r = lane & 15, kb = lane >> 4;
   const int a_rows = M <= 8 ? 8 : 16;                      // rows of A kept (a power of two)
   const int n0 = (blockIdx.x * WAVES + wave) * 16, split = blockIdx.z;
@@ -237,43 +238,6 @@ gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, 
     source[u] = W + (size_t)min(n0 + row, N - 1) * K + k_begin + piece * 4;
     place[u] = row * FL_STAGE + ((piece ^ row) & 15) * 4;
   }
-  // A slice first: its wait would otherwise cover the first stages of W as well
-  for (int idx = threadIdx.x; idx < a_rows * (cols_per_split / 4); idx += WAVES * QIL_WAVE) {
-    const int m = idx / (cols_per_split / 4), c = (idx - m * (cols_per_split / 4)) * 4;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (m < M) {
-      if (ASRC == 1) {
-        float merged[4];
-        merged_values<4, 16>(unmerged, m, k_begin + c, merged);
-        v = make_float4(merged[0], merged[1], merged[2], merged[3]);
-      } else if (ASRC == 2) {
-        const int k = k_begin + c;                          // four columns of one tile of 16
-        const size_t at = (size_t)m * 2 * K + (gated.interleaved ? (size_t)(k >> 4) * 32 + (k & 15) : (size_t)k);
-        const size_t stride = (size_t)M * 2 * K;
-        float4 g = make_float4(0.f, 0.f, 0.f, 0.f), u = g;
-        for (int s0 = 0; s0 < gated.splits; s0 += 4) {       // four splits' loads at a time; the sums in split order
-          float4 gs[4], us[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const size_t from = (size_t)min(s0 + j, gated.splits - 1) * stride + at;
-            gs[j] = *reinterpret_cast<const float4*>(gated.sums + from);
-            us[j] = *reinterpret_cast<const float4*>(gated.sums + from + (gated.interleaved ? 16 : K));
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (s0 + j < gated.splits) {
-              g.x += gs[j].x; g.y += gs[j].y; g.z += gs[j].z; g.w += gs[j].w;
-              u.x += us[j].x; u.y += us[j].y; u.z += us[j].z; u.w += us[j].w;
-            }
-        }
-        v = make_float4((g.x / (1.f + expf(-g.x))) * u.x, (g.y / (1.f + expf(-g.y))) * u.y,
-                        (g.z / (1.f + expf(-g.z))) * u.z, (g.w / (1.f + expf(-g.w))) * u.w);
-      } else {
-        v = *reinterpret_cast<const float4*>(A + (size_t)m * K + k_begin + c);
-      }
-    }
-    *reinterpret_cast<float4*>(a_lds + m * row_width + (c ^ ((m & 7) << 2))) = v;
-  }
   // every wave walks its K range from a start of its own and wraps around (waves that read the same columns
   // of their rows at the same time load a few memory channels only)
   const int turn = (n0 / 16) % stages;
@@ -284,10 +248,98 @@ gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, 
 #pragma unroll
     for (int u = 0; u < 4; ++u) stage_w[u] = __builtin_bit_cast(f32x4v, load_once(source[u] + at));
   };
-  request(w0, 0);                                           // the host sees to stages >= 3
-  request(w1, 1);
-  request(w2, 2);
-  __syncthreads();
+  auto request_first = [&]() {
+    request(w0, 0);                                         // the host sees to stages >= 3
+    request(w1, 1);
+    request(w2, 2);
+  };
+  // A slice first, W's first stages right behind it where that is possible: loads come back in order, so A's arrival is waited for
+  // without W's.  (Rows past M stay as they are in LDS: their products are never stored.)
+  constexpr int THREADS = WAVES * QIL_WAVE;
+  const int pieces = cols_per_split / 4, all = M * pieces;
+  if constexpr (ASRC == 0) {
+    // straight into LDS, 256 columns of a row an instruction (lane l's 16 bytes land at piece l: it fetches the piece that belongs there)
+    for (int c0 = 0; c0 < cols_per_split; c0 += 256)
+      if (c0 + lane * 4 < cols_per_split) {
+#pragma unroll 4
+        for (int m = wave; m < M; m += WAVES)
+          __builtin_amdgcn_global_load_lds(
+              (const __attribute__((address_space(1))) void*)(A + (size_t)m * K + k_begin + c0 + ((lane ^ (m & 7)) << 2)),
+              (__attribute__((address_space(3))) void*)(a_lds + m * row_width + c0), 16, 0, 0);
+      }
+    request_first();
+    __builtin_amdgcn_s_waitcnt(0x07C);                      // vmcnt(12) lgkmcnt(0): see the whole-line kernel in gemm_bf16.hip
+    __builtin_amdgcn_s_barrier();
+  } else {
+    MergeParts<4, WAVES == FL_WIDE_WAVES ? 8 : 16> parts;     // (ASRC 1; sixteen parts do not fit the registers of 16 waves)
+    const int P = ASRC == 1 ? merge_part_keys(unmerged) : 0;
+    float4 gs[4], us[4];                                    // (ASRC 2: four splits of gate and up)
+    const size_t stride = (size_t)M * 2 * K;
+    int m, c;
+    auto ask_sums = [&](int s0) __attribute__((always_inline)) {
+      const int k = k_begin + c;                            // four columns of one tile of 16
+      const size_t at = (size_t)m * 2 * K + (gated.interleaved ? (size_t)(k >> 4) * 32 + (k & 15) : (size_t)k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const size_t from = (size_t)min(s0 + j, gated.splits - 1) * stride + at;
+        gs[j] = *reinterpret_cast<const float4*>(gated.sums + from);
+        us[j] = *reinterpret_cast<const float4*>(gated.sums + from + (gated.interleaved ? 16 : K));
+      }
+    };
+    auto ask = [&](int idx) __attribute__((always_inline)) {
+      m = idx / pieces;
+      c = (idx - m * pieces) * 4;
+      if constexpr (ASRC == 1) merge_ask(unmerged, P, m, k_begin + c, parts);
+      else ask_sums(0);
+    };
+    auto put = [&]() __attribute__((always_inline)) {
+      float4 v;
+      if constexpr (ASRC == 1) {
+        float merged[4];
+        merge_finish(unmerged, P, m, k_begin + c, parts, merged);
+        v = make_float4(merged[0], merged[1], merged[2], merged[3]);
+      } else {
+        float4 g = make_float4(0.f, 0.f, 0.f, 0.f), u = g;
+        auto add = [&](int s0) __attribute__((always_inline)) {           // in split order
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (s0 + j < gated.splits) {
+              g.x += gs[j].x; g.y += gs[j].y; g.z += gs[j].z; g.w += gs[j].w;
+              u.x += us[j].x; u.y += us[j].y; u.z += us[j].z; u.w += us[j].w;
+            }
+        };
+        add(0);
+        if constexpr (!AHEAD)
+          for (int s0 = 4; s0 < gated.splits; s0 += 4) {
+            ask_sums(s0);
+            add(s0);
+          }
+        v = make_float4((g.x / (1.f + expf(-g.x))) * u.x, (g.y / (1.f + expf(-g.y))) * u.y,
+                        (g.z / (1.f + expf(-g.z))) * u.z, (g.w / (1.f + expf(-g.w))) * u.w);
+      }
+      *reinterpret_cast<float4*>(a_lds + m * row_width + (c ^ ((m & 7) << 2))) = v;
+    };
+    if constexpr (AHEAD) {                                  // (a piece a thread, in one turn of loads: launch_f32_lines)
+      ask(min((int)threadIdx.x, all - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      request_first();
+      if constexpr (ASRC == 1) {
+        parts.arrived();
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          asm volatile("" : "+v"(gs[j].x), "+v"(gs[j].y), "+v"(gs[j].z), "+v"(gs[j].w), "+v"(us[j].x), "+v"(us[j].y), "+v"(us[j].z), "+v"(us[j].w));
+      }
+      if ((int)threadIdx.x < all) put();
+    } else {
+      for (int idx = threadIdx.x; idx < all; idx += THREADS) {
+        ask(idx);
+        put();
+      }
+      request_first();
+    }
+    __syncthreads();
+  }
 
   f32x4v acc = {0.f, 0.f, 0.f, 0.f};
   // lanes past the kept rows read the rows again: their products are rows of D that are never stored
@@ -537,11 +589,11 @@ static int fl_splits(int M, int N, int K) {
   return fit;
 }
 
-template <int ASRC, int WAVES>
+template <int ASRC, int WAVES, bool AHEAD = false>
 static int launch_f32_lines_waves(const float* A, UnmergedA unmerged, GatedA gated, const float* W, float* C, int M, int N,
                                   int K, int splits, hipStream_t s) {
   const size_t lds = fl_lds_bytes(M, K, splits, WAVES);
-  auto kernel = gemm_f32_lines_kernel<ASRC, WAVES>;
+  auto kernel = gemm_f32_lines_kernel<ASRC, WAVES, AHEAD>;
   static size_t granted = 0;                              // per instantiation
   if (lds > 64 * 1024 && lds > granted) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -558,6 +610,13 @@ static int launch_f32_lines(const float* A, UnmergedA unmerged, GatedA gated, co
                             int splits, hipStream_t s) {
   const int waves = fl_waves(M, N, K, splits);
   if (!fl_takes(M, N, K, splits, waves, splits == 1)) return -1;
+  // W ahead of an operand that is made here: in blocks of 4 waves whose threads make one piece each from one turn of loads
+  // (4 rows, us behind / ahead: 2,048 x 2,048 behind the merge of 16 parts 7.9 / 6.8, 1,024 x 3,072 behind the activation of four sums 5.9 /
+  // 5.0; with A as it is straight into LDS, 16 rows of 4,096 x 1,024 6.3 / 5.7; a step of 28 layers, 4 rows 1,366 -> 1,323).
+  if constexpr (ASRC != 0)
+    if (waves == FL_NARROW_WAVES && (long)M * (K / splits / 4) <= FL_NARROW_WAVES * QIL_WAVE &&
+        (ASRC == 1 ? unmerged.parts <= 16 : gated.splits <= 4))
+      return launch_f32_lines_waves<ASRC, FL_NARROW_WAVES, true>(A, unmerged, gated, W, C, M, N, K, splits, s);
   if (waves == FL_NARROW_WAVES) return launch_f32_lines_waves<ASRC, FL_NARROW_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s);
   return waves == FL_WAVES ? launch_f32_lines_waves<ASRC, FL_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s)
                            : launch_f32_lines_waves<ASRC, FL_WIDE_WAVES>(A, unmerged, gated, W, C, M, N, K, splits, s);

@@ -129,3 +129,49 @@ def test_decode_attention_that_makes_its_queries(ops, d, heads, kv_heads, page_s
     assert torch.equal(v_fused.view(torch.int16), v_cache.view(torch.int16))
     want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step, **rest).float()
     torch.testing.assert_close(fused.float(), want, atol=2.0 ** -8, rtol=2.0 ** -7)
+
+
+# blocks of four waves with a piece of A a thread and with more, of eight and of sixteen; one turn of parts (16) or sums (4) and a second
+@pytest.mark.parametrize('m', [1, 3, 4, 5, 9, 16])
+@pytest.mark.parametrize('n,heads,d,parts', [(1024, 16, 128, 16), (1024, 16, 128, 17), (96, 6, 64, 3), (6144, 32, 128, 4)])
+def test_float32_products_behind_the_merge(ops, m, n, heads, d, parts):
+    """The parts past a row's keys hold NaN.  Float32 sums of k products."""
+    lib, part, k = ops.library.load(), 64, heads * d
+    splits = lib.qil_gemm_f32_splits(m, n, k)
+    if not lib.qil_gemm_f32_unmerged_takes(m, n, heads, d, splits):
+        pytest.skip('not a size of this kernel')
+    positions = torch.tensor([(r * 71 + 5) % (parts * part) for r in range(m - 1)] + [parts * part - 1], dtype=torch.int32).cuda()
+    acc, top, total = rand(m, heads, parts, d), rand(m, heads, parts, seed=1), rand(m, heads, parts, seed=2).abs() + 1
+    live = torch.arange(parts, device='cuda') <= (positions // part)[:, None]
+    weights = torch.where(live[:, None], top.double(), -torch.inf).softmax(-1)
+    want = (weights[..., None] * acc.double()).sum(2) / (weights * total.double()).sum(-1)[..., None]
+    workspace = torch.cat([acc.where(live[:, None, :, None], torch.nan).flatten(), top.where(live[:, None], torch.nan).flatten(),
+                           total.where(live[:, None], torch.nan).flatten()])
+    w = rand(n, k, scale=k ** -0.5, seed=3)
+    out = torch.empty(splits, m, n, device='cuda')
+    assert lib.qil_gemm_f32_unmerged(workspace.data_ptr(), positions.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, heads, d, 0,
+                                     part, parts, splits, torch.cuda.current_stream().cuda_stream) == 0
+    want = want.reshape(m, k) @ w.double().t()
+    torch.testing.assert_close(out.double().sum(0), want, atol=3e-6 * want.abs().max().item(), rtol=0)
+
+
+@pytest.mark.parametrize('m', [1, 3, 4, 5, 9, 16])
+@pytest.mark.parametrize('n,k,sums', [(1024, 3072, 4), (1024, 3072, 5), (64, 192, 1), (4096, 12288, 2)])
+@pytest.mark.parametrize('interleaved', [False, True])
+def test_float32_products_of_few_rows(ops, m, n, k, sums, interleaved):
+    """Behind the activation, and of an operand as it is.  Float32 sums of k products."""
+    lib, stream = ops.library.load(), torch.cuda.current_stream().cuda_stream
+    splits = lib.qil_gemm_f32_splits(m, n, k)
+    w, parts = rand(n, k, scale=k ** -0.5, seed=3), rand(sums, m, 2 * k, scale=sums ** -0.5)
+    out = torch.empty(splits, m, n, device='cuda')
+    total = parts.double().sum(0)
+    gate, up = (total.reshape(m, k // 16, 2, 16).unbind(2) if interleaved else total.reshape(m, 2, k).unbind(1))
+    operand = (torch.nn.functional.silu(gate) * up).reshape(m, k)
+    if lib.qil_gemm_f32_gated_takes(m, n, k, int(interleaved), splits):
+        assert lib.qil_gemm_f32_gated(parts.data_ptr(), sums, int(interleaved), w.data_ptr(), out.data_ptr(), m, n, k, splits, stream) == 0
+        want = operand @ w.double().t()
+        torch.testing.assert_close(out.double().sum(0), want, atol=3e-6 * want.abs().max().item(), rtol=0)
+    x = operand.float()
+    assert lib.qil_gemm_f32(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, splits, stream) == 0
+    want = x.double() @ w.double().t()
+    torch.testing.assert_close(out.double().sum(0), want, atol=3e-6 * want.abs().max().item(), rtol=0)
