@@ -183,6 +183,75 @@ struct NormedA {
   float eps;
 };
 
+// A block's slice of such an operand, columns k_begin .. k_begin + cols, on its way into LDS: ask() sends the first loads, put() waits for
+// them (not for what was asked for in between) and leaves the rows in LDS, to be met behind a barrier.  M at most twice the waves.
+// A wave adds the pieces of two rows' sums of squares; they are asked for together with what a thread's first two pieces of A are
+// made of.  (All are held in place: the compiler otherwise moves loads whose use stands under a condition down to it.)
+struct NormedStage {
+  static constexpr int EARLY = 2, SQUARES = 4;
+  const NormedA& normed;
+  float* rstd;                                             // 16 floats of LDS
+  const int M, K, k_begin, pieces, all, threads, lane, wave, waves;
+  float x[EARLY][8], g[EARLY][8], squares[2][SQUARES];
+  __device__ __forceinline__ NormedStage(const NormedA& n, void* scratch, int m, int k, int first, int cols, int w, int ws)
+      : normed(n), rstd(reinterpret_cast<float*>(scratch)), M(m), K(k), k_begin(first), pieces(cols / 8), all(m * (cols / 8)),
+        threads(ws * QIL_WAVE), lane(threadIdx.x & (QIL_WAVE - 1)), wave(w), waves(ws) {}
+  __device__ __forceinline__ void ask_piece(int idx, float (&to_x)[8], float (&to_g)[8]) {
+    const int m = idx / pieces, c = (idx - m * pieces) * 8;
+    ld8(normed.stream + (size_t)m * K + k_begin + c, to_x);
+    ld8(normed.weight + k_begin + c, to_g);
+  }
+  __device__ __forceinline__ void ask() {
+#pragma unroll
+    for (int r2 = 0; r2 < 2; ++r2)
+      if (!r2 || M > waves)
+#pragma unroll
+        for (int i = 0; i < SQUARES; ++i)
+          squares[r2][i] = normed.squares[(size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M + min(wave + r2 * waves, M - 1)];
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+      if (!u || all > threads) ask_piece(min((int)threadIdx.x + u * threads, all - 1), x[u], g[u]);
+  }
+  __device__ __forceinline__ void put_piece(int idx, const float (&from_x)[8], const float (&from_g)[8], bf16_t* a_lds, int row_width) {
+    const int m = idx / pieces, c = (idx - m * pieces) * 8;
+    const float scale = rstd[m];
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = round_to<bf16_t>(from_x[e] * scale) * from_g[e];
+    *reinterpret_cast<uint4*>(a_lds + m * row_width + c) =
+        make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+  }
+  __device__ __forceinline__ void put(bf16_t* a_lds, int row_width) {
+#pragma unroll
+    for (int r2 = 0; r2 < 2; ++r2) {                        // (twice the waves: all rows there are)
+      if (r2 && M <= waves) break;
+      const int m = wave + r2 * waves;
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < SQUARES; ++i) {
+        asm volatile("" : "+v"(squares[r2][i]));
+        if (lane + i * QIL_WAVE < normed.pieces) sum += squares[r2][i];
+      }
+      for (int p = lane + SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
+      sum = wave_sum(sum);
+      if (lane == 0 && m < M) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
+    }
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+      if (!u || all > threads)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(x[u][e]), "+v"(g[u][e]));
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < EARLY; ++u)
+      if ((int)threadIdx.x + u * threads < all) put_piece(threadIdx.x + u * threads, x[u], g[u], a_lds, row_width);
+    for (int idx = threadIdx.x + EARLY * threads; idx < all; idx += threads) {
+      ask_piece(idx, x[0], g[0]);
+      put_piece(idx, x[0], g[0], a_lds, row_width);
+    }
+  }
+};
+
 // ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA).  AHEAD (ASRC 1): W's first requests
 // go out ahead of the parts' arrival (launch_lines).
 template <typename OUT, int ASRC, int WAVES = LINES_WAVES, bool AHEAD = true>
@@ -232,66 +301,12 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
   constexpr int THREADS = WAVES * QIL_WAVE;
   const int pieces = cols_per_split / 8, all = M * pieces;  // (rows past M stay as they are in LDS: their products are never stored)
   if (ASRC == 2) {
-    // A wave adds the pieces of two rows' sums of squares; they are asked for together with what a thread's first two pieces of A are
-    // made of.  (All are held in place: the compiler otherwise moves loads whose use stands under a condition down to it.)
-    float* rstd = reinterpret_cast<float*>(lds + a_rows * row_width + WAVES * (16 * 128));
-    constexpr int EARLY = 2, SQUARES = 4;
-    float x[EARLY][8], g[EARLY][8], squares[2][SQUARES];
-    auto ask = [&](int idx, float (&to_x)[8], float (&to_g)[8]) {
-      const int m = idx / pieces, c = (idx - m * pieces) * 8;
-      ld8(normed.stream + (size_t)m * K + k_begin + c, to_x);
-      ld8(normed.weight + k_begin + c, to_g);
-    };
-    const bool both_rows = M > WAVES, both_pieces = all > THREADS;
-#pragma unroll
-    for (int r2 = 0; r2 < 2; ++r2)
-      if (!r2 || both_rows)
-#pragma unroll
-        for (int i = 0; i < SQUARES; ++i)
-          squares[r2][i] = normed.squares[(size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M + min(wave + r2 * WAVES, M - 1)];
-#pragma unroll
-    for (int u = 0; u < EARLY; ++u)
-      if (!u || both_pieces) ask(min((int)threadIdx.x + u * THREADS, all - 1), x[u], g[u]);
+    NormedStage stage(normed, lds + a_rows * row_width + WAVES * (16 * 128), M, K, k_begin, cols_per_split, wave, WAVES);
+    stage.ask();
     __builtin_amdgcn_sched_barrier(0);
     request_first();
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r2 = 0; r2 < 2; ++r2) {                        // (2 WAVES rows are all there are)
-      const int m = wave + r2 * WAVES;
-      float sum = 0.f;
-#pragma unroll
-      for (int i = 0; i < SQUARES; ++i) {
-        if (r2 && !both_rows) break;
-        asm volatile("" : "+v"(squares[r2][i]));
-        if (lane + i * QIL_WAVE < normed.pieces) sum += squares[r2][i];
-      }
-      for (int p = lane + SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
-      sum = wave_sum(sum);
-      if (lane == 0 && m < M) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
-      if (!both_rows) break;
-    }
-#pragma unroll
-    for (int u = 0; u < EARLY; ++u)
-      if (!u || both_pieces)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(x[u][e]), "+v"(g[u][e]));
-    __syncthreads();
-    auto put = [&](int idx, const float (&from_x)[8], const float (&from_g)[8]) {
-      const int m = idx / pieces, c = (idx - m * pieces) * 8;
-      const float scale = rstd[m];
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = round_to<bf16_t>(from_x[e] * scale) * from_g[e];
-      *reinterpret_cast<uint4*>(a_lds + m * row_width + c) =
-          make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
-    };
-#pragma unroll
-    for (int u = 0; u < EARLY; ++u)
-      if ((int)threadIdx.x + u * THREADS < all) put(threadIdx.x + u * THREADS, x[u], g[u]);
-    for (int idx = threadIdx.x + EARLY * THREADS; idx < all; idx += THREADS) {
-      ask(idx, x[0], g[0]);
-      put(idx, x[0], g[0]);
-    }
+    stage.put(a_lds, row_width);
   } else if (MERGE) {
     MergeParts<8, 4> parts;
     const int P = merge_part_keys(unmerged);
@@ -668,10 +683,11 @@ static int launch_chunks(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N,
 #define GATED_ROWS_FEWEST_BLOCKS 128                       // of the 17-to-192-row kernel: see gated_rows_takes
 #define GATED_ROWS_MOST 64                                 // beyond, the product and a separate activation are faster
 
-template <typename OUT, bool SILU>
+// NORMED: A is the norm of the residual stream (NormedA), made by every block while W is on its way (M at most twice the waves).
+template <typename OUT, bool SILU, bool NORMED = false>
 __global__ void __launch_bounds__(GATED_MAX_WAVES * QIL_WAVE)
 gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ out, int M,
-                       int inner, int K, int ksplit, int interleaved, GateFn fn) {
+                       int inner, int K, int ksplit, int interleaved, GateFn fn, NormedA normed) {
   extern __shared__ __align__(16) bf16_t lds[];            // A [8 or 16][K + pad], then a 4 KB buffer per wave
   const int a_rows = M <= 8 ? 8 : 16;                      // rows of A kept (8 or 16: a power of two)
   const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
@@ -714,22 +730,35 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
   // requests were, and with A ahead W was asked for only when A was there: 3,072 x 1,024,
   // one row 5.3 -> 4.6 us, 16 rows 6.4 -> 5.3; 9,728 x 2,560, 8 rows 19.9 -> 19.2, 16 rows 20.5 -> 19.4.)  Rows past M stay as they are in LDS: their products are rows of D that are never stored.
   const int waves = blockDim.x / QIL_WAVE;
-  for (int c0 = 0; c0 < K; c0 += 512)
-    if (c0 + lane * 8 < K) {
-      const bf16_t* from = A + (size_t)wave * K + c0 + lane * 8;
-      bf16_t* to = a_lds + wave * row_width + c0;
+  auto request_first = [&]() {
+    request(g0, 0, 0); request(u0, up_offset, 0);           // the host sees to stages >= 2
+    request(g1, 0, 1); request(u1, up_offset, 1);
+  };
+  if constexpr (NORMED) {
+    NormedStage stage(normed, lds + a_rows * row_width + waves * (16 * 128), M, K, 0, K, wave, waves);
+    stage.ask();
+    __builtin_amdgcn_sched_barrier(0);
+    request_first();
+    __builtin_amdgcn_sched_barrier(0);
+    stage.put(a_lds, row_width);
+    __syncthreads();
+  } else {
+    for (int c0 = 0; c0 < K; c0 += 512)
+      if (c0 + lane * 8 < K) {
+        const bf16_t* from = A + (size_t)wave * K + c0 + lane * 8;
+        bf16_t* to = a_lds + wave * row_width + c0;
 #pragma unroll 4
-      for (int m = wave; m < M; m += waves) {
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
-                                         (__attribute__((address_space(3))) void*)to, 16, 0, 0);
-        from += (size_t)waves * K;
-        to += waves * row_width;
+        for (int m = wave; m < M; m += waves) {
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                           (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+          from += (size_t)waves * K;
+          to += waves * row_width;
+        }
       }
-    }
-  request(g0, 0, 0); request(u0, up_offset, 0);             // the host sees to stages >= 2
-  request(g1, 0, 1); request(u1, up_offset, 1);
-  __builtin_amdgcn_s_waitcnt(0x4070);                       // vmcnt(16) lgkmcnt(0): see the whole-line kernel
-  __builtin_amdgcn_s_barrier();
+    request_first();
+    __builtin_amdgcn_s_waitcnt(0x4070);                     // vmcnt(16) lgkmcnt(0): see the whole-line kernel
+    __builtin_amdgcn_s_barrier();
+  }
 
   f32x4 gate = {0.f, 0.f, 0.f, 0.f}, up = {0.f, 0.f, 0.f, 0.f};
   // lanes past the kept rows read the rows again: their products are rows of D that are never stored
@@ -916,7 +945,8 @@ extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, 
       if (e != hipSuccess) return (int)e;                                                                            \
       granted = lds;                                                                                                 \
     }                                                                                                                \
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, inner, K, ksplit, interleaved, fn); \
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)A, (const bf16_t*)W, (OUT*)out, M, inner, K, ksplit, interleaved, fn, \
+                       NormedA());                                                                                   \
   }
   const bool silu = act == QIL_ACT_SILU;
   if (out_dtype == QIL_F32) {
@@ -925,6 +955,37 @@ extern "C" int qil_gemm_bf16_gated_act(const void* A, const void* W, void* out, 
     if (silu) QIL_GATED_CASE(bf16_t, true) else QIL_GATED_CASE(bf16_t, false)
   }
 #undef QIL_GATED_CASE
+  QIL_RETURN_LAUNCH_STATUS();
+}
+
+// 1 if qil_gemm_bf16_gated_normed takes these sizes.
+extern "C" int qil_gemm_bf16_gated_normed_takes(int M, int inner, int K) {
+  int pairs, ksplit;
+  return gated_plan(nullptr, nullptr, M, inner, K, &pairs, &ksplit) && M <= 2 * pairs * ksplit &&
+         gated_lds(M, K, pairs * ksplit) + 16 * sizeof(float) <= 160 * 1024;
+}
+
+// out bfloat16 [M, inner] = silu(A gate^T) * (A up^T) for W with gate and up rows in turns of 16, A the norm of the float32 stream [M, K]
+// (round, then the weight), made from its sums of squares in pieces as qil_gemm_bf16_normed does.
+extern "C" int qil_gemm_bf16_gated_normed(const float* stream, const float* weight, const float* squares, int pieces, float eps,
+                                          const void* W, void* out, int M, int inner, int K, hipStream_t s) {
+  if (M == 0 || inner == 0) return 0;
+  int pairs, ksplit;
+  if (!qil_gemm_bf16_gated_normed_takes(M, inner, K) || !gated_plan(nullptr, W, M, inner, K, &pairs, &ksplit) || pieces < 1 ||
+      (((uintptr_t)stream | (uintptr_t)weight) % 16))
+    return -1;
+  const NormedA normed{stream, weight, squares, pieces, eps};
+  const size_t lds = gated_lds(M, K, pairs * ksplit) + 16 * sizeof(float);
+  auto kernel = gemm_bf16_gated_kernel<bf16_t, true, true>;
+  static size_t granted = 0;
+  if (lds > 64 * 1024 && lds > granted) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return (int)e;
+    granted = lds;
+  }
+  const int all_pairs = inner / 16;
+  hipLaunchKernelGGL(kernel, dim3((all_pairs + pairs - 1) / pairs), dim3(pairs * ksplit * QIL_WAVE), lds, s, (const bf16_t*)nullptr,
+                     (const bf16_t*)W, (bf16_t*)out, M, inner, K, ksplit, 1, GateFn{QIL_ACT_SILU, 0.f, 1.f}, normed);
   QIL_RETURN_LAUNCH_STATUS();
 }
 

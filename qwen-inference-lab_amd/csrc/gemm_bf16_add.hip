@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "merge_parts.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -144,6 +145,95 @@ gemm_bf16_add_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
   }
 }
 
+// The same behind split-context attention, few rows: A [M, K = heads * d] is merged from the attention's parts (merge_parts.h) while W is
+// on its way.  A block owns 8 columns and 8 waves share K, whose STAGES stages of 128 columns a wave are all asked for at once; every
+// block merges all of its rows (from L2).  With the stream complete behind it and its squares left, the next product makes the second
+// norm of a layer itself: one kernel less.  What bounds it is the chain parts, merge, products, sums, stream.
+template <int STAGES>
+__global__ void __launch_bounds__(ADD_WAVES * QIL_WAVE)
+gemm_bf16_merge_add_kernel(const bf16_t* __restrict__ W, float* __restrict__ stream, float* __restrict__ squares, int M, int N, int K,
+                           UnmergedA unmerged) {
+  extern __shared__ __align__(16) bf16_t lds[];            // A [8][K + 8], then 8 x 256 bytes of W a wave
+  constexpr int COLS = 8, A_ROWS = 8, THREADS = ADD_WAVES * QIL_WAVE, PER_WAVE = COLS * 128;
+  const int lane = threadIdx.x & (QIL_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / QIL_WAVE);
+  const int r = lane & 15, kb = lane >> 4, load_row = lane >> 4, piece = lane & 15;
+  const int n0 = blockIdx.x * COLS, k_begin = wave * STAGES * 128, row_width = K + 8;
+  bf16_t* buffer = lds + A_ROWS * row_width + wave * PER_WAVE;
+  const int pieces = K / 8, all = M * pieces, P = merge_part_keys(unmerged);
+  MergeParts<8, 4> parts;
+  int idx = threadIdx.x, m0, c0;
+  auto ask = [&](int of) __attribute__((always_inline)) {
+    m0 = of / pieces;
+    c0 = (of - m0 * pieces) * 8;
+    merge_ask(unmerged, P, m0, c0, parts);
+  };
+  auto put = [&]() __attribute__((always_inline)) {
+    float v[8];
+    merge_finish(unmerged, P, m0, c0, parts, v);
+    *reinterpret_cast<uint4*>(lds + m0 * row_width + c0) =
+        make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+  };
+  ask(min(idx, all - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4 w[STAGES][2];
+#pragma unroll
+  for (int st = 0; st < STAGES; ++st)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      w[st][u] = load_once(W + (size_t)(n0 + 4 * u + load_row) * K + k_begin + st * 128 + piece * 8);
+  float cell[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cell[i] = stream[(size_t)min(4 * kb + i, M - 1) * N + n0 + (r & (COLS - 1))];
+  __builtin_amdgcn_sched_barrier(0);
+  parts.arrived();
+  if (idx < all) put();
+  for (idx += THREADS; idx < all; idx += THREADS) {
+    ask(idx);
+    put();
+  }
+  __syncthreads();
+
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int w_row = r & (COLS - 1);
+  const bf16_t* a_row = lds + (r & (A_ROWS - 1)) * row_width + k_begin + kb * 8;     // (rows past M: products that are never stored)
+#pragma unroll
+  for (int st = 0; st < STAGES; ++st) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 4 * u + load_row;
+      *reinterpret_cast<u32x4*>(buffer + row * 128 + ((piece ^ row) & 15) * 8) = w[st][u];
+    }
+    __builtin_amdgcn_wave_barrier();                        // LDS operations of one wave complete in order: no wait
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      const u32x4 b = *reinterpret_cast<const u32x4*>(buffer + w_row * 128 + (((4 * s4 + kb) ^ w_row) & 15) * 8);
+      const u32x4 a = *reinterpret_cast<const u32x4*>(a_row + st * 128 + s4 * 32);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  float* sums = reinterpret_cast<float*>(lds + A_ROWS * row_width);      // the waves' sums, each in its own buffer
+  *reinterpret_cast<f32x4*>(sums + wave * (PER_WAVE / 2) + lane * 4) = acc;
+  __syncthreads();
+  if (wave == 0) {
+    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < ADD_WAVES; ++v) total += *reinterpret_cast<const f32x4*>(sums + v * (PER_WAVE / 2) + lane * 4);   // fixed order
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = 4 * kb + i;
+      const bool stores = m < M && r < COLS;
+      const float value = stores ? cell[i] + total[i] : 0.f;
+      if (stores) stream[(size_t)m * N + n0 + r] = value;
+      float square = value * value;
+      square += lane_move<0xB1>(square);
+      square += lane_move<0x4E>(square);
+      square += lane_move<0x141>(square);
+      if (stores && r == 0) squares[(size_t)blockIdx.x * M + m] = square;
+    }
+  }
+}
+
 static size_t add_lds_bytes(int M, int waves, int cols = 16) {
   return (size_t)waves * (cols + (M <= 8 ? 8 : 16)) * 128 * sizeof(bf16_t);   // also holds the waves' sums (1 KB a wave)
 }
@@ -255,6 +345,53 @@ int qil_gemm_bf16_whole_takes(int M, int N, int K) {
 // out bfloat16 [M, N] = A[M, K] W[N, K]^T, K split over a block's waves.
 int qil_gemm_bf16_whole(const void* A, const void* W, void* out, int M, int N, int K, hipStream_t s) {
   return add_launch<false>(A, W, nullptr, out, nullptr, M, N, K, 0, 0, s);
+}
+
+// 1 if qil_gemm_bf16_unmerged_add takes these sizes: up to MERGE_ADD_ROWS rows, at most a block of 8 columns a CU, one to four stages a
+// wave; parts in one turn of loads.
+#define MERGE_ADD_ROWS 4
+int qil_gemm_bf16_unmerged_add_takes(int M, int N, int heads, int d, int parts) {
+  if (M < 1 || M > MERGE_ADD_ROWS || N < 8 || N % 8 || N > 8 * QIL_CUS || heads < 1 || d < 8 || d % 8 || heads > 65536 || d > 65536) return 0;
+  const long K = (long)heads * d;
+  return K % 1024 == 0 && K <= 4096 && parts >= 1 && parts <= 4;
+}
+
+// stream float32 [M, N] += merge(workspace) W^T, the workspace as qil_gemm_bf16_unmerged takes it; squares float32 [N / 8][M]: the rows'
+// sums of squares of the new stream in pieces of 8 columns.
+int qil_gemm_bf16_unmerged_add(const void* workspace, const int* positions, const void* W, float* stream, float* squares, int M, int N,
+                               int heads, int d, int window, int P, int parts, hipStream_t s) {
+  if (M == 0 || N == 0) return 0;
+  if (!qil_gemm_bf16_unmerged_add_takes(M, N, heads, d, parts) || P < 0 || !squares ||
+      (((uintptr_t)W | (uintptr_t)workspace | (uintptr_t)stream) % 16))
+    return -1;
+  const int K = heads * d;
+  UnmergedA u;
+  u.acc = (const float*)workspace;
+  u.m = u.acc + (size_t)M * heads * parts * d;
+  u.l = u.m + (size_t)M * heads * parts;
+  u.positions = positions;
+  u.heads = heads; u.d = d; u.parts = parts; u.P = P; u.window = window;
+  u.part_keys = planned_keys(u.l, (size_t)M * heads * parts, P);
+  const size_t lds = ((size_t)8 * (K + 8) + ADD_WAVES * 8 * 128) * sizeof(bf16_t);
+#define QIL_MERGE_ADD(STAGES)                                                                                                    \
+  {                                                                                                                              \
+    auto kernel = gemm_bf16_merge_add_kernel<STAGES>;                                                                            \
+    static bool granted = false;                             /* per instantiation */                                             \
+    if (lds > 64 * 1024 && !granted) {                                                                                           \
+      const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);       \
+      if (e != hipSuccess) return (int)e;                                                                                        \
+      granted = true;                                                                                                            \
+    }                                                                                                                            \
+    hipLaunchKernelGGL(kernel, dim3(N / 8), dim3(ADD_WAVES * QIL_WAVE), lds, s, (const bf16_t*)W, stream, squares, M, N, K, u);  \
+  }
+  switch (K / 1024) {
+    case 1: QIL_MERGE_ADD(1) break;
+    case 2: QIL_MERGE_ADD(2) break;
+    case 3: QIL_MERGE_ADD(3) break;
+    default: QIL_MERGE_ADD(4)
+  }
+#undef QIL_MERGE_ADD
+  QIL_RETURN_LAUNCH_STATUS();
 }
 
 }  // extern "C"

@@ -619,9 +619,16 @@ def linear(x, weight, bias=None, out_dtype=None, partials=False, add_to=None):
         n, k = x.shape
         o = weight.shape[0]
         _require(weight, 'weight', x.dtype, (o, k))
+        plain = partials and bias is None and out_dtype in (None, x.dtype) and x.dtype == torch.bfloat16
+        if add_to is not None and plain and lib.qil_gemm_bf16_unmerged_add_takes(n, o, x.heads, x.head_dim, x.parts):
+            _require(add_to, 'add_to', torch.float32, (n, o))
+            squares = torch.empty((o // 8, n), dtype=torch.float32, device=x.device)
+            _check(lib.qil_gemm_bf16_unmerged_add(_ptr(x.workspace), _ptr(x.positions), _ptr(weight), _ptr(add_to), _ptr(squares), n, o,
+                                                  x.heads, x.head_dim, x.window, x.part, x.parts, _stream()),
+                   'gemm_bf16_unmerged_add')
+            return Added(squares)
         splits = lib.qil_gemm_bf16_splits(n, o, k)
-        if partials and bias is None and out_dtype in (None, x.dtype) and x.dtype == torch.bfloat16 and \
-                lib.qil_gemm_bf16_unmerged_takes(n, o, x.heads, x.head_dim, splits):
+        if plain and lib.qil_gemm_bf16_unmerged_takes(n, o, x.heads, x.head_dim, splits):
             out = torch.empty((splits, n, o), dtype=torch.float32, device=x.device)
             _check(lib.qil_gemm_bf16_unmerged(_ptr(x.workspace), _ptr(x.positions), _ptr(weight), _ptr(out), n, o,
                                               x.heads, x.head_dim, x.window, x.part, x.parts, splits, _stream()),
@@ -750,6 +757,18 @@ def gated_linear(x, weight, out_dtype=None, interleaved=False, lazy=False, activ
     clamped swish: 10.2 us and 5.1 for the activation, 12.7 as one kernel; a step of six such layers 496 -> 481 us.)
     ``lazy``: a few float32 rows may come back as ``Gated`` (the product's partial sums) for ``linear`` to finish."""
     if isinstance(x, Normed):
+        n, k = x.shape
+        both, lib = weight.shape[0], library.load()
+        if activation == 'silu' and interleaved and x.dtype == torch.bfloat16 and weight.dtype == x.dtype and both % 32 == 0 and \
+                out_dtype in (None, x.dtype) and n and not weight.data_ptr() & 15 and lib.qil_gemm_bf16_gated_normed_takes(n, both // 2, k):
+            _require(x.stream, 'stream', torch.float32, (n, k))
+            _require(x.weight, 'norm weight', torch.float32, (k,))
+            _require(x.squares, 'squares', torch.float32, (x.squares.shape[0], n))
+            _require(weight, 'weight', x.dtype, (both, k))
+            out = torch.empty((n, both // 2), dtype=x.dtype, device=x.device)
+            _check(lib.qil_gemm_bf16_gated_normed(_ptr(x.stream), _ptr(x.weight), _ptr(x.squares), x.squares.shape[0], x.eps,
+                                                  _ptr(weight), _ptr(out), n, both // 2, k, _stream()), 'gemm_bf16_gated_normed')
+            return out
         x = x.materialize()
     if isinstance(x, SharedInput):
         if id(weight) in x.places:                  # the stack's product, then the activation kernel

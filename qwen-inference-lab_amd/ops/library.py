@@ -280,6 +280,14 @@ def _declare(lib):
     lib.qil_gemm_bf16_normed_takes.argtypes = [i, i, i, i]
     lib.qil_gemm_bf16_normed_takes.restype = i
     lib.qil_gemm_bf16_normed.argtypes = [p, p, p, i, f, p, p, i, i, i, i, p]
+    lib.qil_gemm_bf16_gated_normed_takes.argtypes = [i, i, i]
+    lib.qil_gemm_bf16_gated_normed_takes.restype = i
+    lib.qil_gemm_bf16_gated_normed.argtypes = [p, p, p, i, f, p, p, i, i, i, p]
+    lib.qil_gemm_bf16_gated_normed.restype = i
+    lib.qil_gemm_bf16_unmerged_add_takes.argtypes = [i, i, i, i, i]
+    lib.qil_gemm_bf16_unmerged_add_takes.restype = i
+    lib.qil_gemm_bf16_unmerged_add.argtypes = [p, p, p, p, p, i, i, i, i, i, i, i, p]
+    lib.qil_gemm_bf16_unmerged_add.restype = i
     lib.qil_gemm_bf16_add_takes.argtypes = [i, i, i]
     lib.qil_gemm_bf16_add_takes.restype = i
     lib.qil_gemm_bf16_add_pieces.argtypes = [i, i, i]

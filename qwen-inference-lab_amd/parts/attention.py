@@ -52,6 +52,7 @@ class Attention(Mixer):
     """
     graph_safe = True
     takes_lazy_norm = True       # h goes into ops.linear only, which takes a norm not computed yet
+    adds_to_stream = True
 
     def __init__(self, *, width, heads, kv_heads, head_dim, bias, qk_norm_eps, scale,
                  position=None, window=None, dtype=torch.bfloat16, value_dim=None, softcap=None, qk_norm_weights=True,
@@ -207,7 +208,7 @@ class Attention(Mixer):
         super().place_matrix(name, tensor)
         self.w_qkv = self.p['qkv_proj.weight']
 
-    def forward(self, h, ctx, cache):
+    def forward(self, h, ctx, cache, add_to=None):
         p = self.p
         if cache.writes and not self.own_kv:
             raise ValueError('an attention part without keys and values of its own reads another entry\'s cache')
@@ -233,7 +234,8 @@ class Attention(Mixer):
                 page_size=cache.page_size, block_tables=cache.block_tables, row_seq=ctx.row_seq,
                 max_context=ctx.max_context, scale=self.scale, window=self.window, unmerged=True, plans=ctx.plans,
                 rotate_first=self.norm_after_rotation, softcap=self.softcap, **sizes, **norms)
-            return ops.linear(attended, p['o_proj.weight'], p.get('o_proj.bias'), partials=True)
+            return ops.linear(attended, p['o_proj.weight'], p.get('o_proj.bias'), partials=True,
+                              add_to=add_to if isinstance(attended, ops.Unmerged) else None)
         q = ops.qk_norm_rope_store(
             qkv, rotation=rotation, positions=ctx.positions, slots=cache.slots if cache.writes else None,
             k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size, dtype=self.dtype, norm_dim=self.head_dim,

@@ -174,6 +174,9 @@ class Mixer(Part):
     graph_safe = False
     # True if forward takes ``h`` as an ``ops.Normed`` (a norm not computed yet) as well as a tensor.
     takes_lazy_norm = False
+    # True if forward takes ``add_to=stream`` and may add its result into the float32 residual stream itself; it then returns the
+    # ``ops.Added`` that its last product gave.  (Asked for by blocks whose feed-forward takes an ``ops.Normed``.)
+    adds_to_stream = False
 
     def cache_need(self):
         return None
@@ -188,6 +191,7 @@ class FeedForward(Part):
     A part that sets ``adds_to_stream`` is called as ``forward(h, add_to=stream)`` and may add its result into
     the float32 residual stream itself; it then returns the ``ops.Added`` that its last product gave."""
     adds_to_stream = False
+    takes_lazy_norm = False      # True if forward takes ``h`` as an ``ops.Normed`` as well as a tensor
 
     def forward(self, h):
         raise NotImplementedError

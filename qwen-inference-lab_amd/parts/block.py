@@ -37,10 +37,15 @@ class PreNormBlock(Block):
             pending = None
         if h is None:
             h = self.mixer_norm.forward(stream, pending, self.dtype)
-        mixed = self.mixer.forward(h, ctx, cache)
+        # the mixer's last product may add into the stream where the feed-forward's first one can make the norm in between
+        lazy = self.ffn is not None and self.mixer.adds_to_stream and self.ffn.takes_lazy_norm
+        mixed = self.mixer.forward(h, ctx, cache, add_to=stream) if lazy else self.mixer.forward(h, ctx, cache)
         if self.ffn is None:
             return mixed
-        h = self.ffn_norm.forward(stream, None if isinstance(mixed, ops.Added) else mixed, self.dtype)
+        added = isinstance(mixed, ops.Added)
+        h = self.ffn_norm.forward_lazy(stream, self.dtype, mixed) if lazy and added else None
+        if h is None:
+            h = self.ffn_norm.forward(stream, None if added else mixed, self.dtype)
         return self.ffn.forward(h, add_to=stream) if self.ffn.adds_to_stream else self.ffn.forward(h)
 
     def _forward_scaled(self, stream, pending, ctx, cache):

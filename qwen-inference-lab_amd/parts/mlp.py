@@ -34,6 +34,7 @@ class GatedMLP(FeedForward):
         p['gate_up_proj.weight'] = ops.interleave_gate_up(gate, up) if self.interleaved else torch.cat([gate, up]).contiguous()
 
     adds_to_stream = True
+    takes_lazy_norm = True       # h goes into ops.gated_linear only
 
     def input_matrices(self):
         # silu's product has the activation inside whatever its sizes.  Other functions join the layer's stacked product where there is

@@ -175,3 +175,38 @@ def test_float32_products_of_few_rows(ops, m, n, k, sums, interleaved):
     assert lib.qil_gemm_f32(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, splits, stream) == 0
     want = x.double() @ w.double().t()
     torch.testing.assert_close(out.double().sum(0), want, atol=3e-6 * want.abs().max().item(), rtol=0)
+
+
+# one turn of pieces a thread and more, one to four stages a wave, two parts to four; a window that leaves the first part without keys
+@pytest.mark.parametrize('m', [1, 2, 4])
+@pytest.mark.parametrize('n,heads,d,parts,window', [(1024, 16, 128, 2, 0), (2048, 16, 64, 4, 0), (8, 24, 128, 3, 0), (1024, 32, 128, 4, 40)])
+@pytest.mark.parametrize('inner', [3072, 48])
+def test_second_norm_without_a_kernel(ops, m, n, heads, d, parts, window, inner):
+    """The product behind the merge adds into the stream, the gated product behind it makes the norm: against the same from the
+    kernels that each do one of these (bounds of the tests above)."""
+    lib, part, k = ops.library.load(), 32, heads * d
+    assert lib.qil_gemm_bf16_unmerged_add_takes(m, n, heads, d, parts)
+    positions = torch.tensor([(r * 37 + 5) % (parts * part) for r in range(m - 1)] + [parts * part - 1], dtype=torch.int32).cuda()
+    index, last = torch.arange(parts, device='cuda'), positions // part
+    first = (positions + 1 - window).clamp(min=0) // part if window else torch.zeros_like(last)
+    live = ((index >= first[:, None]) & (index <= last[:, None]))[:, None].expand(m, heads, parts)
+    acc, top, total = rand(m, heads, parts, d), rand(m, heads, parts, seed=1), rand(m, heads, parts, seed=2).abs() + 1
+    workspace = torch.cat([acc.where(live[..., None], torch.nan).flatten(), top.where(live, torch.nan).flatten(), total.where(live, torch.nan).flatten()])
+    w, stream = rand(n, k, dtype=torch.bfloat16, scale=k ** -0.5, seed=3), rand(m, n, seed=4)
+    make = lambda: ops.Unmerged(workspace, positions, torch.empty(m, k, dtype=torch.bfloat16, device='cuda'), heads=heads, head_dim=d, window=window,
+                                part=part, parts=parts)
+    before = stream.clone()
+    want = before.double() + make().merge().double() @ w.double().t()
+    added = ops.linear(make(), w, partials=True, add_to=stream)
+    assert isinstance(added, ops.Added)
+    torch.testing.assert_close(stream.double(), want, atol=3e-6 * want.abs().max().item(), rtol=0)
+    torch.testing.assert_close(added.squares.double(), stream.double().square().reshape(m, n // 8, 8).sum(-1).t(), atol=0, rtol=1e-6)
+    if n % 256:
+        return
+    weight, gate_up = 1 + 0.1 * rand(n, seed=5), rand(2 * inner, n, dtype=torch.bfloat16, scale=n ** -0.5, seed=6)
+    assert lib.qil_gemm_bf16_gated_normed_takes(m, inner, n)
+    lazy = ops.Normed(stream, weight, 1e-6, torch.bfloat16, added)
+    got = ops.gated_linear(lazy, gate_up, torch.bfloat16, interleaved=True)
+    want = ops.gated_linear(lazy.materialize(), gate_up, torch.bfloat16, interleaved=True)
+    # (an operand at a rounding's edge may go either way)
+    torch.testing.assert_close(got.double(), want.double(), atol=2.0 ** -8 * 4 * n ** -0.5 * want.abs().max().item(), rtol=2.0 ** -8)
