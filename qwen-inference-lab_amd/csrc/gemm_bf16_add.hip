@@ -347,13 +347,16 @@ int qil_gemm_bf16_whole(const void* A, const void* W, void* out, int M, int N, i
   return add_launch<false>(A, W, nullptr, out, nullptr, M, N, K, 0, 0, s);
 }
 
-// 1 if qil_gemm_bf16_unmerged_add takes these sizes: up to MERGE_ADD_ROWS rows, at most a block of 8 columns a CU, one to four stages a
-// wave; parts in one turn of loads.
+// 1 if qil_gemm_bf16_unmerged_add takes these sizes: up to four rows and 16 parts in all, at most a block of 8 columns a CU, one to four
+// stages a wave.  Every block merges all rows, which beyond that costs more than the norm's kernel: us a step of 28 layers with partial
+// sums and a norm / so: 1 row of 100 keys 882 / 823, of 3,500 (14 parts) 955 / 893, 4 of 100 936 / 901, but 4 of 2,000 (8 parts each) 1,038 / 1,057,
+// 5 of 100 980 / 1,015, 8 of 300 999 / 1,042.
 #define MERGE_ADD_ROWS 4
+#define MERGE_ADD_PARTS 16
 int qil_gemm_bf16_unmerged_add_takes(int M, int N, int heads, int d, int parts) {
   if (M < 1 || M > MERGE_ADD_ROWS || N < 8 || N % 8 || N > 8 * QIL_CUS || heads < 1 || d < 8 || d % 8 || heads > 65536 || d > 65536) return 0;
   const long K = (long)heads * d;
-  return K % 1024 == 0 && K <= 4096 && parts >= 1 && parts <= 4;
+  return K % 1024 == 0 && K <= 4096 && parts >= 1 && (long)M * parts <= MERGE_ADD_PARTS;
 }
 
 // stream float32 [M, N] += merge(workspace) W^T, the workspace as qil_gemm_bf16_unmerged takes it; squares float32 [N / 8][M]: the rows'
