@@ -372,8 +372,8 @@ attn_tile_kernel(const T* __restrict__ q, int q_stride, const T* __restrict__ k_
     // ---- mask and online softmax (per-lane row statistics).  m holds the running maximum of the RAW
     // scores; the scale (> 0) enters once, in the exponent: p = exp(scale * (s - m)).
     // every key of the tile is visible to every row of the wave unless the tile touches the wave's
-    // first row's future, the window's edge or the rows beyond the sequence
-    const bool all_visible = k0 + BK - 1 <= start + wave_row0 && wave_row0 + 16 * RB <= n &&
+    // first row's future or the window's edge (rows beyond the sequence hold zeros for queries and are not stored)
+    const bool all_visible = k0 + BK - 1 <= start + wave_row0 &&
                              (window <= 0 || k0 > wave_last_pos - window || k0 + BK <= keep);
 #pragma unroll
     for (int b = 0; b < RB; ++b) {

@@ -399,7 +399,8 @@ attn_tile_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* 
   };
   auto attend_tile = [&](int k0, const bf16_t* tile) {
     if (wave_active && k0 <= wave_last_pos) {
-      const bool all_visible = k0 + BK - 1 <= start + wave_row0 && wave_row0 + 16 * RB <= n &&
+      // (rows past the end hold zeros for queries and are not stored: they may see anything)
+      const bool all_visible = k0 + BK - 1 <= start + wave_row0 &&
                                (window <= 0 || k0 > wave_last_pos - window);
       if constexpr (WIDE) {
         if (all_visible) attend_wide(k0, tile, std::false_type());
@@ -542,16 +543,18 @@ extern "C" int qil_attn_tile_bf16(const void* q, int q_stride, const void* k_cac
     const int g128 = heads / kv_heads, gh128 = g128 >= 3 ? 4 : g128;
     const long blocks4 = (long)((max_query + 32 * (4 / gh128) - 1) / (32 * (4 / gh128))) * n_seqs * kv_heads *
                          ((g128 + gh128 - 1) / gh128);
-    // Fewer blocks of 4 waves than CUs (one prompt of up to 1,024 tokens with 8 kv heads): 8 waves in two groups that
-    // split a block's keys, so that every SIMD has two waves (16 : 23 us at 256 tokens, 19 : 20 at 512, 27 : 29 at
-    // 1,024; with more blocks the SIMDs are full anyway and the merge at the end only costs: 66 : 57 at 2,048).
+    // Fewer blocks of 4 waves than CUs (one prompt of up to 1,024 tokens with 8 kv heads), or few more: 8 waves in two groups that
+    // split a block's keys, so that every SIMD has two waves; with many more blocks the SIMDs are full anyway and the merge at
+    // the end only costs, as it does where a block has few tiles of keys.  us in 4 waves / 8, 16 heads in 8 groups: 100 tokens 8.5 / 9.9, 301
+    // 12.3 / 13.4, 500 level, 1,000 25.1 / 22.7, 2,000 42.4 / 36.8, 2,300 (288 blocks) 52.4 / 41.4, 2,900 (368) 62.6 / 60.4; 32 heads: 1,200
+    // (304) 34.4 / 31.5, 1,400 (352) 36.4 / 38.7, 2,048 50.2 / 58.1; two of 600 (304) 20.9 / 24.1; three of 301 and 16 heads 12.8 / 13.7.
     // (Blocks of 8 waves that share a staged tile of keys, 64 rows of 4 heads, were 8 % faster from 8,192 tokens on
     // and are not used: with 64 query heads in 8 groups, two chunks of heads a group, a 2,048-row sequence beside a
     // 64-row one gave, about once in 2,000 calls inside a model, results that differed from one run to the next in a
     // few rows by the rounding of a bfloat16; with 4 waves, or without the placement of blocks by XCD, never in as
     // many calls; nor with the model's large products on this library's own kernels instead of the GPU BLAS, so the
     // difference is probably made in a BLAS product under that timing.  The shape gains nothing any more and stays out.)
-    int waves = blocks4 <= QIL_CUS && window <= 0 ? 16 : 4;
+    int waves = window <= 0 && max_query >= 512 && blocks4 <= (max_query >= 1024 ? QIL_CUS + 64 : QIL_CUS) ? 16 : 4;
     if (tile_waves_override) waves = tile_waves_override;   // 4 or 16 (the two groups)
     if (waves == 16 && window > 0) waves = 4;
     return qil_attn_prompt(q, q_stride, k_cache, v_cache, block_tables, table_stride, cu_seqlens, seq_starts, out, n_seqs,
