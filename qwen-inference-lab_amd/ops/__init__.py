@@ -349,13 +349,14 @@ def _code(dtype):
 
 
 _raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+_current_device = getattr(torch._C, '_cuda_getDevice', torch.cuda.current_device)     # (a launch's operands are on the GPU: it is initialised)
 
 
 def _stream():
     """The current stream's handle.  (torch's direct accessor where it has one: building a Stream object for
     every launch cost a quarter of a small model's step on the host.)"""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -376,7 +377,7 @@ def _require(tensor, name, dtype=None, shape=None):
         raise ValueError(f'{name} must be contiguous')
     if dtype is not None and tensor.dtype != dtype:
         raise ValueError(f'{name} must be {dtype}, is {tensor.dtype}')
-    if shape is not None and tuple(tensor.shape) != tuple(shape):
+    if shape is not None and tensor.shape != tuple(shape):
         raise ValueError(f'{name} must have shape {tuple(shape)}, has {tuple(tensor.shape)}')
 
 
