@@ -213,3 +213,26 @@ def test_second_norm_without_a_kernel(ops, m, n, heads, d, parts, window, inner)
     want = ops.gated_linear(lazy.materialize(), gate_up, torch.bfloat16, interleaved=True)
     # (an operand at a rounding's edge may go either way)
     torch.testing.assert_close(got.double(), want.double(), atol=2.0 ** -8 * 4 * n ** -0.5 * want.abs().max().item(), rtol=2.0 ** -8)
+
+
+# one row more and less than a tile of 32 (64 with groups of two heads), blocks of four waves and of two groups of them, more blocks than
+# CUs, two sequences of which one is short, a history ahead of the rows, a window; sinks
+@pytest.mark.parametrize('heads,kv_heads,d', [(16, 8, 128), (16, 4, 128), (8, 2, 64), (6, 2, 96)])
+@pytest.mark.parametrize('rows,starts,window', [([543], [0], None), ([1057], [0], None), ([65, 33], [40, 0], None), ([1057], [0], 100), ([31], [300], None)])
+@pytest.mark.parametrize('sink', [False, True])
+def test_prompt_attention_of_odd_lengths(ops, heads, kv_heads, d, rows, starts, window, sink):
+    """Tiles of keys that a not quite full tile of rows sees whole are not masked: against the float32 reference, one rounding to
+    bfloat16 and its neighbour."""
+    lengths = [r + s for r, s in zip(rows, starts)]
+    k_cache, v_cache, table, _ = build_cache(lengths, 16, kv_heads, d, torch.bfloat16)
+    q = rand(sum(rows), heads * d, dtype=torch.bfloat16, seed=7)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=16, block_tables=table, scale=d ** -0.5, window=window,
+                row_seq=ints([i for i, r in enumerate(rows) for _ in range(r)]),
+                positions=ints([s + j for r, s in zip(rows, starts) for j in range(r)]), max_context=max(lengths),
+                cu_seqlens=ints([sum(rows[:i]) for i in range(len(rows) + 1)]), seq_starts=ints(starts),
+                single_rows=torch.empty(0, dtype=torch.int32).cuda(), n_seqs=len(rows), max_query=max(rows),
+                sinks=rand(heads, seed=8) if sink else None)
+    got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    torch.testing.assert_close(got.float(), want.float(), atol=2.0 ** -8, rtol=2.0 ** -7)
