@@ -550,8 +550,8 @@ static int launch_tile(const void* q, int q_stride, const void* k_cache, const v
 extern "C" int qil_attn_tile_bf16_takes(int d, int page_size, int table_stride);
 extern "C" int qil_attn_tile_bf16(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                                   const int* block_tables, int table_stride, const int* cu_seqlens,
-                                  const int* seq_starts, void* out, int n_seqs, int max_query, int heads, int kv_heads,
-                                  int d, int page_size, int window, float scale, hipStream_t s);
+                                  const int* seq_starts, void* out, int n_seqs, int max_query, int keys, int heads,
+                                  int kv_heads, int d, int page_size, int window, float scale, hipStream_t s);
 
 extern "C" int qil_attn_prompt_takes(int d, int page_size, int table_stride);
 extern "C" int qil_attn_prompt_capped(const void* q, int q_stride, const void* k_cache, const void* v_cache,
@@ -601,7 +601,8 @@ static int tile_dispatch(const void* q, int q_stride, const void* k_cache, const
                          const int* block_tables, int table_stride, const int* cu_seqlens, const int* seq_starts,
                          void* out, int n_seqs, int max_query, int heads, int kv_heads, int d, int page_size,
                          int window, float scale, int dtype, hipStream_t s, float* workspace, int total_rows, int P,
-                         int parts, float softcap, const float* sinks = nullptr, const float* slopes = nullptr, int keep = 0) {
+                         int parts, float softcap, const float* sinks = nullptr, const float* slopes = nullptr, int keep = 0,
+                         int keys = 0) {
   if (n_seqs == 0 || max_query < 2) return 0;
   if (keep < 0 || (keep > 0 && (window <= 0 || parts > 1))) return -1;
   const bool extended = slopes || keep > 0;
@@ -621,7 +622,7 @@ static int tile_dispatch(const void* q, int q_stride, const void* k_cache, const
                                  n_seqs, max_query, heads, kv_heads, page_size, window, scale, sinks, s);
   if (parts == 1 && softcap <= 0.f && !sinks && !extended && dtype == QIL_BF16 && qil_attn_tile_bf16_takes(d, page_size, table_stride))
     return qil_attn_tile_bf16(q, q_stride, k_cache, v_cache, block_tables, table_stride, cu_seqlens, seq_starts, out,
-                              n_seqs, max_query, heads, kv_heads, d, page_size, window, scale, s);
+                              n_seqs, max_query, keys, heads, kv_heads, d, page_size, window, scale, s);
 #define QIL_TILE_CASE(T, DMAX)                                                                                      \
   return launch_tile<T, DMAX, (sizeof(T) == 2 && DMAX <= 128) ? 2 : 1>(q, q_stride, k_cache, v_cache, block_tables, table_stride, cu_seqlens, seq_starts, out, \
                               n_seqs, max_query, heads, kv_heads, d, page_size, window, scale, s, workspace, total_rows, P, parts, softcap, sinks, slopes, keep)
@@ -636,13 +637,14 @@ static int tile_dispatch(const void* q, int q_stride, const void* k_cache, const
 #undef QIL_TILE_CASE
 }
 
+// keys: of the longest sequence of several rows where the host knows it, else the most rows of one (qil_attn_prompt_waves).
 extern "C" int qil_attn_tile(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                              const int* block_tables, int table_stride, const int* cu_seqlens, const int* seq_starts,
-                             void* out, int n_seqs, int max_query, int heads, int kv_heads, int d, int page_size,
+                             void* out, int n_seqs, int max_query, int keys, int heads, int kv_heads, int d, int page_size,
                              int window, float scale, float softcap, int dtype, const float* sinks, const float* slopes,
                              int keep, hipStream_t s) {
   return tile_dispatch(q, q_stride, k_cache, v_cache, block_tables, table_stride, cu_seqlens, seq_starts, out, n_seqs,
-                       max_query, heads, kv_heads, d, page_size, window, scale, dtype, s, nullptr, 0, 0, 1, softcap, sinks, slopes, keep);
+                       max_query, heads, kv_heads, d, page_size, window, scale, dtype, s, nullptr, 0, 0, 1, softcap, sinks, slopes, keep, keys);
 }
 
 extern "C" int qil_attn_tile_in_parts(const void* q, int q_stride, const void* k_cache, const void* v_cache,

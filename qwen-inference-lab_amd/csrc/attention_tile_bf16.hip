@@ -526,11 +526,29 @@ extern "C" int qil_attn_tile_bf16_takes(int d, int page_size, int table_stride) 
          table_stride >= 1 && table_stride <= FAST_TABLE_MAX;
 }
 
-// The arguments of qil_attn_tile (attention_tile.hip), which calls this when the sizes are taken.
+// Waves a block of the head-128 kernel: 4, or 16 for 8 waves in two groups that split a block's keys, so that every SIMD has two waves.
+// The groups pay where blocks of 4 waves are fewer than CUs, or few more, and a block passes ten tiles of keys or more (``keys``: of the
+// longest sequence, as far as the host knows); with many more blocks the SIMDs are full anyway and the merge at the end only costs, as it
+// does where the tiles are few.  us in 4 waves / 8, whole prompts, 16 heads in 8 groups: 100 tokens 8.5 / 9.9, 301 12.3 / 13.4, 600
+// 18.5 / 19.0, 700 19.5 / 19.1, 1,000 25.1 / 22.7, 2,000 42.4 / 36.8, 2,300 (288 blocks) 52.4 / 41.4, 2,900 (368) 62.6 / 60.4; 32 heads:
+// 1,200 (304) 34.4 / 31.5, 1,400 (352) 36.4 / 38.7, 2,048 50.2 / 58.1; two of 600 (304) 20.9 / 24.1; three of 301 and 16 heads 12.5 / 13.5.
+// Portions behind a history, 16 / 32 heads: 64 rows behind 400 keys 15.9 / 16.7 and 16.8 / 16.8, 128 behind 500 18.7 / 18.2 and 19.2 / 18.7,
+// 256 behind 500 21.1 / 20.1 and 21.6 / 20.6, 33 behind 700 20.2 / 18.9 and 21.2 / 20.3, 64 behind 900 25.1 / 23.9 and 26.0 / 23.9.
+// (From 1,024 keys on fewer blocks than CUs have their keys cut into parts before they come here.  A step that a graph may replay knows
+// its keys only as a bucket that ends beyond that: such a portion stays in 4 waves where its blocks do fill the CUs.)
+extern "C" int qil_attn_prompt_waves(int n_seqs, int max_query, int keys, int heads, int kv_heads, int window) {
+  const int g = heads / kv_heads, gh = g >= 3 ? 4 : g, rows = 32 * (4 / gh);
+  const long blocks = (long)((max_query + rows - 1) / rows) * n_seqs * kv_heads * ((g + gh - 1) / gh);
+  if (window > 0 || keys <= 9 * FAST_BK || (max_query < 512 && keys >= 1024)) return 4;
+  return blocks <= (max_query >= 1024 ? QIL_CUS + 64 : QIL_CUS) ? 16 : 4;
+}
+
+// The arguments of qil_attn_tile (attention_tile.hip), which calls this when the sizes are taken.  keys: of the longest
+// sequence of several rows, where the host knows it, else the most rows of one.
 extern "C" int qil_attn_tile_bf16(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                                   const int* block_tables, int table_stride, const int* cu_seqlens,
-                                  const int* seq_starts, void* out, int n_seqs, int max_query, int heads, int kv_heads,
-                                  int d, int page_size, int window, float scale, hipStream_t s) {
+                                  const int* seq_starts, void* out, int n_seqs, int max_query, int keys, int heads,
+                                  int kv_heads, int d, int page_size, int window, float scale, hipStream_t s) {
   if (n_seqs == 0 || max_query < 2) return 0;
   if (!qil_attn_tile_bf16_takes(d, page_size, table_stride) || heads % kv_heads || n_seqs > 65535 ||
       kv_heads * 2 > 65535)
@@ -540,21 +558,13 @@ extern "C" int qil_attn_tile_bf16(const void* q, int q_stride, const void* k_cac
                                  n_seqs, max_query, heads, kv_heads, page_size, window, scale, s);
   // Head size 128 has a kernel of its own (attention_prompt.hip), in blocks of 4 waves (32 rows of 4 heads).
   if (d == 128) {
-    const int g128 = heads / kv_heads, gh128 = g128 >= 3 ? 4 : g128;
-    const long blocks4 = (long)((max_query + 32 * (4 / gh128) - 1) / (32 * (4 / gh128))) * n_seqs * kv_heads *
-                         ((g128 + gh128 - 1) / gh128);
-    // Fewer blocks of 4 waves than CUs (one prompt of up to 1,024 tokens with 8 kv heads), or few more: 8 waves in two groups that
-    // split a block's keys, so that every SIMD has two waves; with many more blocks the SIMDs are full anyway and the merge at
-    // the end only costs, as it does where a block has few tiles of keys.  us in 4 waves / 8, 16 heads in 8 groups: 100 tokens 8.5 / 9.9, 301
-    // 12.3 / 13.4, 500 level, 1,000 25.1 / 22.7, 2,000 42.4 / 36.8, 2,300 (288 blocks) 52.4 / 41.4, 2,900 (368) 62.6 / 60.4; 32 heads: 1,200
-    // (304) 34.4 / 31.5, 1,400 (352) 36.4 / 38.7, 2,048 50.2 / 58.1; two of 600 (304) 20.9 / 24.1; three of 301 and 16 heads 12.8 / 13.7.
     // (Blocks of 8 waves that share a staged tile of keys, 64 rows of 4 heads, were 8 % faster from 8,192 tokens on
     // and are not used: with 64 query heads in 8 groups, two chunks of heads a group, a 2,048-row sequence beside a
     // 64-row one gave, about once in 2,000 calls inside a model, results that differed from one run to the next in a
     // few rows by the rounding of a bfloat16; with 4 waves, or without the placement of blocks by XCD, never in as
     // many calls; nor with the model's large products on this library's own kernels instead of the GPU BLAS, so the
     // difference is probably made in a BLAS product under that timing.  The shape gains nothing any more and stays out.)
-    int waves = window <= 0 && max_query >= 512 && blocks4 <= (max_query >= 1024 ? QIL_CUS + 64 : QIL_CUS) ? 16 : 4;
+    int waves = qil_attn_prompt_waves(n_seqs, max_query, keys, heads, kv_heads, window);
     if (tile_waves_override) waves = tile_waves_override;   // 4 or 16 (the two groups)
     if (waves == 16 && window > 0) waves = 4;
     return qil_attn_prompt(q, q_stride, k_cache, v_cache, block_tables, table_stride, cu_seqlens, seq_starts, out, n_seqs,

@@ -1274,9 +1274,11 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
                                       int(window or 0), part, parts, _code(qkv.dtype), _ptr(sinks), 0, *_NO_GATE,
                                       _stream()), 'attn_merge')
         else:
+            # (the longest context may be that of a row alone: then a portion is only known to pass its own rows)
+            keys = max_query if single_rows.shape[0] else max_context
             _check(lib.qil_attn_tile(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
                                      block_tables.shape[1], _ptr(cu_seqlens), _ptr(seq_starts), _ptr(out), n_seqs,
-                                     max_query, heads, kv_heads, head_dim, page_size, int(window or 0), float(scale),
+                                     max_query, keys, heads, kv_heads, head_dim, page_size, int(window or 0), float(scale),
                                      cap, _code(qkv.dtype), _ptr(sinks), _ptr(slopes), keep, _stream()), 'attn_tile')
         rows = single_rows.shape[0]
     else:

@@ -245,7 +245,7 @@ def _declare(lib):
     lib.qil_attn_decode_f32.argtypes = [p, i, p, p, p, i, p, p, p, p, p, i, i, i, i, i, i, f, i, i, f, p, p, i, p]
     lib.qil_attn_decode_f32_fused.argtypes = [p, i, p, p, f, p, p, i, i, p, p, p, i, p, p, p, p, i, i, i, i, i, i, f, i, i, i, f, i, i, p, f, i, p, i, p, i, p]
     lib.qil_attn_plan.argtypes = [p, p, i, i, i, p, p]
-    lib.qil_attn_tile.argtypes = [p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, f, f, i, p, p, i, p]
+    lib.qil_attn_tile.argtypes = [p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, i, f, f, i, p, p, i, p]
     lib.qil_gemm_f32.argtypes = [p, p, p, p, i, i, i, i, p]
     lib.qil_gemm_f32_splits.argtypes = [i, i, i]
     lib.qil_gemm_f32_waves.argtypes = [i, i, i, i]
@@ -271,6 +271,8 @@ def _declare(lib):
     lib.qil_gemm_bf16_splits.restype = i
     lib.qil_attn_tile_bf16_takes.argtypes = [i, i, i]
     lib.qil_attn_tile_bf16_takes.restype = i
+    lib.qil_attn_prompt_waves.argtypes = [i, i, i, i, i, i]
+    lib.qil_attn_prompt_waves.restype = i
     lib.qil_attn_tile_parts.argtypes = [i, i, i, i, i, i, i, i, ctypes.POINTER(ctypes.c_int)]
     lib.qil_attn_tile_parts.restype = i
     lib.qil_attn_tile_bf16_parts.argtypes = [p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, i, f, i, i, p]

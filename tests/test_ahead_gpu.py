@@ -236,3 +236,26 @@ def test_prompt_attention_of_odd_lengths(ops, heads, kv_heads, d, rows, starts, 
     got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
     want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
     torch.testing.assert_close(got.float(), want.float(), atol=2.0 ** -8, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize('rows,starts,waves', [([64], [700], 16), ([300, 300], [600, 600], 16), ([64], [100], 4), ([64, 1], [700, 900], 4)])
+def test_block_shape_of_portions_behind_a_history(ops, rows, starts, waves):
+    """By the keys the portion passes, where they are known (a row alone may be the one with the longest context)."""
+    lib, heads, kv_heads, d = ops.library.load(), 16, 8, 128
+    lengths = [r + s for r, s in zip(rows, starts)]
+    k_cache, v_cache, table, _ = build_cache(lengths, 16, kv_heads, d, torch.bfloat16)
+    q = rand(sum(rows), heads * d, dtype=torch.bfloat16, seed=7)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=16, block_tables=table, scale=d ** -0.5, window=None,
+                row_seq=ints([i for i, r in enumerate(rows) for _ in range(r)]),
+                positions=ints([s + j for r, s in zip(rows, starts) for j in range(r)]), max_context=max(lengths),
+                cu_seqlens=ints([sum(rows[:i]) for i in range(len(rows) + 1)]), seq_starts=ints(starts),
+                single_rows=ints([sum(rows[:i]) for i, r in enumerate(rows) if r == 1]), n_seqs=len(rows), max_query=max(rows))
+    got = {}
+    for shape in (0, 4, 16):
+        lib.qil_attn_tile_waves(shape)
+        try:
+            got[shape] = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+        finally:
+            lib.qil_attn_tile_waves(0)
+    assert torch.equal(got[0], got[waves]) and not torch.equal(got[0], got[20 - waves])       # (sums in another order)

@@ -212,3 +212,16 @@ def test_float32_decode_parts_and_kernels():
     assert ops._matrix_attention_wanted(33, 2, 2, 128, 300) and ops._matrix_attention_wanted(48, 16, 16, 128, 1000)
     assert not ops._matrix_attention_wanted(33, 16, 16, 128, 20) and not ops._matrix_attention_wanted(16, 16, 16, 128, 300) and not ops._matrix_attention_wanted(33, 16, 16, 128, 520)
     assert not ops._matrix_attention_wanted(33, 4, 4, 64, 2048) and ops._matrix_attention_wanted(24, 4, 4, 64, 2048)
+
+
+def test_prompt_attention_in_two_groups_of_waves_by_the_keys_a_block_passes(lib):
+    """Not by the rows that come in: a portion behind a history passes all of its keys."""
+    waves = lambda seqs, rows, keys, heads=16, window=0: lib.qil_attn_prompt_waves(seqs, rows, keys, heads, 8, window)
+    for heads in (16, 32):
+        for rows, keys in ((33, 633), (64, 764), (64, 964), (128, 628), (256, 756), (400, 900)):
+            assert waves(1, rows, keys, heads) == 16 and waves(1, rows, keys, heads, 100) == 4
+        for rows, keys in ((33, 33), (64, 64), (64, 264), (128, 428), (256, 456), (400, 400)):
+            assert waves(1, rows, keys, heads) == 4
+    assert waves(3, 300, 900, 32) == 16 and waves(3, 301, 301) == 4 and waves(2, 900, 900) == 16 and waves(2, 600, 600, 32) == 4
+    assert waves(1, 1000, 1000, 32) == 16 and waves(1, 2300, 2300) == 16 and waves(1, 2900, 2900) == 4 and waves(1, 2048, 2048, 32) == 4
+    assert waves(32, 16, 2048, 32) == 4                               # (a graph's bucket of keys)
