@@ -533,13 +533,14 @@ extern "C" int qil_attn_tile_bf16_takes(int d, int page_size, int table_stride) 
 // 18.5 / 19.0, 700 19.5 / 19.1, 1,000 25.1 / 22.7, 2,000 42.4 / 36.8, 2,300 (288 blocks) 52.4 / 41.4, 2,900 (368) 62.6 / 60.4; 32 heads:
 // 1,200 (304) 34.4 / 31.5, 1,400 (352) 36.4 / 38.7, 2,048 50.2 / 58.1; two of 600 (304) 20.9 / 24.1; three of 301 and 16 heads 12.5 / 13.5.
 // Portions behind a history, 16 / 32 heads: 64 rows behind 400 keys 15.9 / 16.7 and 16.8 / 16.8, 128 behind 500 18.7 / 18.2 and 19.2 / 18.7,
-// 256 behind 500 21.1 / 20.1 and 21.6 / 20.6, 33 behind 700 20.2 / 18.9 and 21.2 / 20.3, 64 behind 900 25.1 / 23.9 and 26.0 / 23.9.
-// (From 1,024 keys on fewer blocks than CUs have their keys cut into parts before they come here.  A step that a graph may replay knows
-// its keys only as a bucket that ends beyond that: such a portion stays in 4 waves where its blocks do fill the CUs.)
+// 256 behind 500 21.1 / 20.1 and 21.6 / 20.6, 33 behind 700 20.2 / 18.9 and 21.2 / 20.3, 64 behind 900 25.1 / 23.9 and 26.0 / 23.9; beside rows
+// alone (their kernel included) 64 behind 700 and one row 30.1 / 28.9, 64 behind 300 and one of 900 23.5 / 24.8, two of 300 behind 600 34.0 / 32.7.
+// From 1,024 keys on fewer blocks than CUs have their keys cut into parts before they come here (qil_attn_tile_parts), so that the groups
+// get as many blocks as CUs and up to 64 more: 32 heads, four of 256 behind 1,500 44.6 / 40.0, eight of 128 behind 1,000 33.0 / 31.3.
 extern "C" int qil_attn_prompt_waves(int n_seqs, int max_query, int keys, int heads, int kv_heads, int window) {
   const int g = heads / kv_heads, gh = g >= 3 ? 4 : g, rows = 32 * (4 / gh);
   const long blocks = (long)((max_query + rows - 1) / rows) * n_seqs * kv_heads * ((g + gh - 1) / gh);
-  if (window > 0 || keys <= 9 * FAST_BK || (max_query < 512 && keys >= 1024)) return 4;
+  if (window > 0 || keys <= 9 * FAST_BK) return 4;
   return blocks <= (max_query >= 1024 ? QIL_CUS + 64 : QIL_CUS) ? 16 : 4;
 }
 

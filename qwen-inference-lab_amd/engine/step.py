@@ -129,7 +129,8 @@ class ModelRunner:
             pieces.add(f'token_slots{index}', token_slots)
         facts = dict(n=n, s=s, starts=starts, counts=counts, slots=slots, cu=cu.tolist(), widths=widths,
                      max_context=int(max(st + c for st, c in zip(starts, counts))), n_logit_rows=len(logit_rows),
-                     tile_seqs=sum(c > 1 for c in counts), real=real)
+                     tile_seqs=sum(c > 1 for c in counts),
+                     tile_context=int(max((st + c for st, c in zip(starts, counts) if c > 1), default=0)), real=real)
         return entries, pieces, facts
 
     def _inert(self, pieces, facts):
@@ -171,6 +172,7 @@ class ModelRunner:
             single_rows=part('single_rows') if max(counts) > 1 else None, max_query=max(counts),
             max_context=max_context or facts['max_context'], host_cu_seqlens=facts['cu'], host_starts=facts['starts'],
             host_slots=facts['slots'], requests=[e.request for e in entries], tile_seqs=facts['tile_seqs'],
+            tile_context=None if max_context else facts['tile_context'],
             previous_tokens=part('previous') if self.previous_tokens else None)
         for view in (one for view in self.views for one in (view if isinstance(view, tuple) else (view,))):
             if view is not None and hasattr(view, 'block_tables'):

@@ -1180,7 +1180,8 @@ def tile_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, pag
 
 def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size, block_tables, row_seq, positions,
                     cu_seqlens, seq_starts, single_rows, n_seqs, max_query, max_context, scale, window,
-                    unmerged=False, tile_seqs=None, softcap=None, sinks=None, slopes=None, keep_first=0, plans=None):
+                    unmerged=False, tile_seqs=None, softcap=None, sinks=None, slopes=None, keep_first=0, plans=None,
+                    tile_context=None):
     """Attention of every row of the step over its request's cached keys.
 
     ``q`` [N, heads * head_dim] (head h at columns [h d, (h + 1) d)).  Row n belongs to sequence ``row_seq[n]`` (a row of ``block_tables``) and sees keys j with
@@ -1193,6 +1194,8 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
     (every row alone, context in several parts) for ``linear`` to merge.
     ``tile_seqs``: the caller has put the sequences of two or more rows first and there are this many; the tile
     kernel then gets blocks for these only (None: for every sequence; those of one row leave at once).
+    ``tile_context``: the longest context of the sequences of two or more rows, where the caller knows it; the shape of the prompt
+    kernel's blocks goes by it.
     ``softcap`` c: scores are scaled, then capped softly, c * tanh(score / c), before the softmax.  The kernels
     specialised for bfloat16 heads of 64 and 128 have no cap; capped steps run on the general tile kernel.
     ``sinks`` float32 [heads]: exp(sinks[h]) joins the divisor of head h's softmax once (no key, no value, not
@@ -1274,8 +1277,8 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
                                       int(window or 0), part, parts, _code(qkv.dtype), _ptr(sinks), 0, *_NO_GATE,
                                       _stream()), 'attn_merge')
         else:
-            # (the longest context may be that of a row alone: then a portion is only known to pass its own rows)
-            keys = max_query if single_rows.shape[0] else max_context
+            # (without tile_context the longest context may be that of a row alone: then a portion is only known to pass its own rows)
+            keys = tile_context if tile_context is not None else max_query if single_rows.shape[0] else max_context
             _check(lib.qil_attn_tile(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
                                      block_tables.shape[1], _ptr(cu_seqlens), _ptr(seq_starts), _ptr(out), n_seqs,
                                      max_query, keys, heads, kv_heads, head_dim, page_size, int(window or 0), float(scale),

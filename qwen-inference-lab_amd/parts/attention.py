@@ -240,7 +240,7 @@ class Attention(Mixer):
             qkv, rotation=rotation, positions=ctx.positions, slots=cache.slots if cache.writes else None,
             k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size, dtype=self.dtype, norm_dim=self.head_dim,
             rotate_first=self.norm_after_rotation, **sizes, **norms)
-        planned = dict(plans=ctx.plans) if q.is_cuda else {}
+        planned = dict(plans=ctx.plans, tile_context=ctx.tile_context) if q.is_cuda else {}
         attended = ops.paged_attention(
             q, k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size,
             block_tables=cache.block_tables, row_seq=ctx.row_seq, positions=ctx.positions,
@@ -283,7 +283,7 @@ class Attention(Mixer):
         else:
             q = ops.qk_norm_rope_store(qkv, norm_dim=self.head_dim, rotate_first=self.norm_after_rotation,
                                        q_temperature=self.q_temperature, bias=self.b_qkv_own, **store)
-        planned = dict(plans=ctx.plans) if q.is_cuda else {}
+        planned = dict(plans=ctx.plans, tile_context=ctx.tile_context) if q.is_cuda else {}
         attended = ops.paged_attention(
             q, k_cache=cache.k, v_cache=cache.v, page_size=cache.page_size,
             block_tables=cache.block_tables, row_seq=ctx.row_seq, positions=ctx.positions,

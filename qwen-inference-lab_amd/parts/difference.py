@@ -76,7 +76,7 @@ class DifferenceAttention(Mixer):
             page_size=cache.page_size, block_tables=cache.block_tables, row_seq=ctx.row_seq, positions=ctx.positions,
             cu_seqlens=ctx.cu_seqlens, seq_starts=ctx.seq_starts, single_rows=ctx.single_rows, n_seqs=ctx.n_seqs,
             max_query=ctx.max_query, max_context=ctx.max_context, tile_seqs=ctx.tile_seqs, scale=self.scale, window=None,
-            unmerged=True)
+            unmerged=True, **({'tile_context': ctx.tile_context} if q.is_cuda else {}))
         out = ops.difference_combine(maps, ops.columns(proj, self.gate_offset, self.heads), heads=self.heads, vdim=self.value_dim,
                                      padded=self.padded_dim, factor=self.factor, post=1.0 - self.diff, eps=self.eps, dtype=self.dtype)
         return ops.linear(out, self.p['o_proj.weight'], None, partials=True)

@@ -238,9 +238,12 @@ def test_prompt_attention_of_odd_lengths(ops, heads, kv_heads, d, rows, starts, 
     torch.testing.assert_close(got.float(), want.float(), atol=2.0 ** -8, rtol=2.0 ** -7)
 
 
-@pytest.mark.parametrize('rows,starts,waves', [([64], [700], 16), ([300, 300], [600, 600], 16), ([64], [100], 4), ([64, 1], [700, 900], 4)])
-def test_block_shape_of_portions_behind_a_history(ops, rows, starts, waves):
-    """By the keys the portion passes, where they are known (a row alone may be the one with the longest context)."""
+@pytest.mark.parametrize('rows,starts,told,waves', [([64], [700], None, 16), ([300, 300], [600, 600], None, 16), ([64], [100], None, 4),
+                                                    ([64, 1], [700, 900], None, 4), ([64, 1], [700, 900], 764, 16), ([64, 1], [100, 900], 164, 4),
+                                                    ([256] * 8, [800] * 8, None, 16)])
+def test_block_shape_of_portions_behind_a_history(ops, rows, starts, told, waves):
+    """By the keys the portion passes, where they are known (without ``tile_context`` a row alone may be the one with the longest
+    context)."""
     lib, heads, kv_heads, d = ops.library.load(), 16, 8, 128
     lengths = [r + s for r, s in zip(rows, starts)]
     k_cache, v_cache, table, _ = build_cache(lengths, 16, kv_heads, d, torch.bfloat16)
@@ -250,7 +253,7 @@ def test_block_shape_of_portions_behind_a_history(ops, rows, starts, waves):
                 row_seq=ints([i for i, r in enumerate(rows) for _ in range(r)]),
                 positions=ints([s + j for r, s in zip(rows, starts) for j in range(r)]), max_context=max(lengths),
                 cu_seqlens=ints([sum(rows[:i]) for i in range(len(rows) + 1)]), seq_starts=ints(starts),
-                single_rows=ints([sum(rows[:i]) for i, r in enumerate(rows) if r == 1]), n_seqs=len(rows), max_query=max(rows))
+                single_rows=ints([sum(rows[:i]) for i, r in enumerate(rows) if r == 1]), n_seqs=len(rows), max_query=max(rows), tile_context=told)
     got = {}
     for shape in (0, 4, 16):
         lib.qil_attn_tile_waves(shape)

@@ -224,4 +224,4 @@ def test_prompt_attention_in_two_groups_of_waves_by_the_keys_a_block_passes(lib)
             assert waves(1, rows, keys, heads) == 4
     assert waves(3, 300, 900, 32) == 16 and waves(3, 301, 301) == 4 and waves(2, 900, 900) == 16 and waves(2, 600, 600, 32) == 4
     assert waves(1, 1000, 1000, 32) == 16 and waves(1, 2300, 2300) == 16 and waves(1, 2900, 2900) == 4 and waves(1, 2048, 2048, 32) == 4
-    assert waves(32, 16, 2048, 32) == 4                               # (a graph's bucket of keys)
+    assert waves(8, 128, 1128, 32) == 16 and waves(4, 256, 1756, 32) == 16        # as many blocks as CUs, too many to cut the keys
