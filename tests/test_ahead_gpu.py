@@ -215,8 +215,8 @@ def test_second_norm_without_a_kernel(ops, m, n, heads, d, parts, window, inner)
     torch.testing.assert_close(got.double(), want.double(), atol=2.0 ** -8 * 4 * n ** -0.5 * want.abs().max().item(), rtol=2.0 ** -8)
 
 
-# one row more and less than a tile of 32 (64 with groups of two heads), blocks of four waves and of two groups of them, more blocks than
-# CUs, two sequences of which one is short, a history ahead of the rows, a window; sinks
+# one row more and less than a tile of 32 (64 with groups of two heads), keys in one piece (543 rows) and in parts (1,057 without a
+# window or sinks: fewer blocks than CUs), two sequences of which one is short, a history ahead of the rows, a window; sinks
 @pytest.mark.parametrize('heads,kv_heads,d', [(16, 8, 128), (16, 4, 128), (8, 2, 64), (6, 2, 96)])
 @pytest.mark.parametrize('rows,starts,window', [([543], [0], None), ([1057], [0], None), ([65, 33], [40, 0], None), ([1057], [0], 100), ([31], [300], None)])
 @pytest.mark.parametrize('sink', [False, True])
@@ -233,6 +233,24 @@ def test_prompt_attention_of_odd_lengths(ops, heads, kv_heads, d, rows, starts, 
                 cu_seqlens=ints([sum(rows[:i]) for i in range(len(rows) + 1)]), seq_starts=ints(starts),
                 single_rows=torch.empty(0, dtype=torch.int32).cuda(), n_seqs=len(rows), max_query=max(rows),
                 sinks=rand(heads, seed=8) if sink else None)
+    got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    torch.testing.assert_close(got.float(), want.float(), atol=2.0 ** -8, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize('heads,rows,waves', [(16, 2273, 16), (32, 1505, 4), (16, 607, 16)])
+def test_prompt_attention_of_many_blocks(ops, heads, rows, waves):
+    """Keys in one piece behind a last tile of rows that is not full: 288 blocks of two groups of waves, 384 of four waves, and 80 of
+    two groups.  As above."""
+    lib, kv_heads, d = ops.library.load(), 8, 128
+    k_cache, v_cache, table, _ = build_cache([rows], 16, kv_heads, d, torch.bfloat16)
+    q = rand(rows, heads * d, dtype=torch.bfloat16, seed=7)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    assert ops.tile_key_parts(lib, q.dtype, 1, rows, heads, kv_heads, d, 16, table.shape[1], rows)[1] == 1
+    assert lib.qil_attn_prompt_waves(1, rows, rows, heads, kv_heads, 0) == waves
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=16, block_tables=table, scale=d ** -0.5, window=None,
+                row_seq=ints([0] * rows), positions=ints(range(rows)), max_context=rows, cu_seqlens=ints([0, rows]), seq_starts=ints([0]),
+                single_rows=ints([]), n_seqs=1, max_query=rows)
     got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
     want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
     torch.testing.assert_close(got.float(), want.float(), atol=2.0 ** -8, rtol=2.0 ** -7)
