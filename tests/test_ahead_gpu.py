@@ -177,42 +177,84 @@ def test_float32_products_of_few_rows(ops, m, n, k, sums, interleaved):
     torch.testing.assert_close(out.double().sum(0), want, atol=3e-6 * want.abs().max().item(), rtol=0)
 
 
-# one turn of pieces a thread and more, one to four stages a wave, two parts to four; a window that leaves the first part without keys
-@pytest.mark.parametrize('m', [1, 2, 4])
-@pytest.mark.parametrize('n,heads,d,parts,window', [(1024, 16, 128, 2, 0), (2048, 16, 64, 4, 0), (8, 24, 128, 3, 0), (1024, 32, 128, 4, 40),
-                                                     (1024, 16, 128, 16, 0)])
-@pytest.mark.parametrize('inner', [3072, 48])
-def test_second_norm_without_a_kernel(ops, m, n, heads, d, parts, window, inner):
-    """The product behind the merge adds into the stream, the gated product behind it makes the norm: against the same from the
-    kernels that each do one of these (bounds of the tests above)."""
-    lib, part, k = ops.library.load(), 32, heads * d
-    assert lib.qil_gemm_bf16_unmerged_add_takes(m, n, heads, d, parts) == (m * parts <= 16)
-    if m * parts > 16:
-        return
+def behind_parts(ops, m, n, heads, d, parts, window):
+    """(an unmerged operand, its merged rows in float64, the product's weights); the parts past a row's keys hold NaN."""
+    part, k = 32, heads * d
     positions = torch.tensor([(r * 37 + 5) % (parts * part) for r in range(m - 1)] + [parts * part - 1], dtype=torch.int32).cuda()
     index, last = torch.arange(parts, device='cuda'), positions // part
     first = (positions + 1 - window).clamp(min=0) // part if window else torch.zeros_like(last)
     live = ((index >= first[:, None]) & (index <= last[:, None]))[:, None].expand(m, heads, parts)
     acc, top, total = rand(m, heads, parts, d), rand(m, heads, parts, seed=1), rand(m, heads, parts, seed=2).abs() + 1
     workspace = torch.cat([acc.where(live[..., None], torch.nan).flatten(), top.where(live, torch.nan).flatten(), total.where(live, torch.nan).flatten()])
-    w, stream = rand(n, k, dtype=torch.bfloat16, scale=k ** -0.5, seed=3), rand(m, n, seed=4)
+    w = rand(n, k, dtype=torch.bfloat16, scale=k ** -0.5, seed=3)
     make = lambda: ops.Unmerged(workspace, positions, torch.empty(m, k, dtype=torch.bfloat16, device='cuda'), heads=heads, head_dim=d, window=window,
                                 part=part, parts=parts)
-    before = stream.clone()
-    want = before.double() + make().merge().double() @ w.double().t()
-    added = ops.linear(make(), w, partials=True, add_to=stream)
-    assert isinstance(added, ops.Added)
-    torch.testing.assert_close(stream.double(), want, atol=3e-6 * want.abs().max().item(), rtol=0)
-    torch.testing.assert_close(added.squares.double(), stream.double().square().reshape(m, n // 8, 8).sum(-1).t(), atol=0, rtol=1e-6)
-    if n % 256:
-        return
+    return make(), make().merge().double(), w
+
+
+# one turn of pieces a thread and more, one to four stages a wave, two parts to four; a window that leaves the first part without keys
+SECOND_NORM = [(1024, 16, 128, 2, 0), (2048, 16, 64, 4, 0), (1024, 32, 128, 4, 40), (1024, 16, 128, 16, 0)]
+
+
+# ... one block of 8 columns; more rows, parts and columns than the kernel takes, and heads * d that is no multiple of 1,024
+@pytest.mark.parametrize('m', [1, 2, 3, 4, 5])
+@pytest.mark.parametrize('n,heads,d,parts,window', SECOND_NORM + [(8, 24, 128, 3, 0), (1024, 16, 128, 5, 0), (4096, 32, 128, 2, 0), (1024, 6, 128, 2, 0)])
+def test_products_behind_the_merge_that_add_into_the_stream(ops, m, n, heads, d, parts, window):
+    """Where the rule refuses, partial sums come back and the stream is as it was.  Float32 sums of k products."""
+    lib = ops.library.load()
+    taken = m <= 4 and m * parts <= 16 and n <= 2048 and heads * d % 1024 == 0
+    assert lib.qil_gemm_bf16_unmerged_add_takes(m, n, heads, d, parts) == taken
+    operand, merged, w = behind_parts(ops, m, n, heads, d, parts, window)
+    stream = rand(m, n, seed=4)
+    before, want = stream.clone(), stream.double() + merged @ w.double().t()
+    added = ops.linear(operand, w, partials=True, add_to=stream)
+    if taken:
+        assert isinstance(added, ops.Added)
+        torch.testing.assert_close(added.squares.double(), stream.double().square().reshape(m, n // 8, 8).sum(-1).t(), atol=0, rtol=1e-6)
+        got = stream.double()
+    else:
+        assert isinstance(added, ops.Partials) and torch.equal(stream, before)
+        got = before.double() + added.tensor.double().sum(0)
+    torch.testing.assert_close(got, want, atol=3e-6 * want.abs().max().item(), rtol=0)
+
+
+@pytest.mark.parametrize('m', [1, 2, 3, 4])
+@pytest.mark.parametrize('n,heads,d,parts,window', [case for case in SECOND_NORM if case[3] <= 4])
+@pytest.mark.parametrize('inner', [3072, 48])
+def test_second_norm_without_a_kernel(ops, m, n, heads, d, parts, window, inner):
+    """The product behind the merge adds into the stream, the gated product behind it makes the norm: against the norm's kernel."""
+    operand, _, w = behind_parts(ops, m, n, heads, d, parts, window)
+    stream = rand(m, n, seed=4)
+    added = ops.linear(operand, w, partials=True, add_to=stream)
     weight, gate_up = 1 + 0.1 * rand(n, seed=5), rand(2 * inner, n, dtype=torch.bfloat16, scale=n ** -0.5, seed=6)
-    assert lib.qil_gemm_bf16_gated_normed_takes(m, inner, n)
+    assert ops.library.load().qil_gemm_bf16_gated_normed_takes(m, inner, n)
     lazy = ops.Normed(stream, weight, 1e-6, torch.bfloat16, added)
     got = ops.gated_linear(lazy, gate_up, torch.bfloat16, interleaved=True)
     want = ops.gated_linear(lazy.materialize(), gate_up, torch.bfloat16, interleaved=True)
     # (an operand at a rounding's edge may go either way)
     torch.testing.assert_close(got.double(), want.double(), atol=2.0 ** -8 * 4 * n ** -0.5 * want.abs().max().item(), rtol=2.0 ** -8)
+
+
+# one and two rows a wave in blocks of one wave, of two and of four; blocks of several pairs of tiles, of which the last has too few
+@pytest.mark.parametrize('inner,k,most', [(48, 1152, 2), (48, 1280, 4), (48, 1024, 8), (6160, 2048, 16)])
+def test_gated_products_behind_the_norm(ops, inner, k, most):
+    """silu(gate) * up of the norm of a stream whose rows' squares are there in pieces of 8 columns; the operand as the norm rounds it."""
+    lib = ops.library.load()
+    assert not lib.qil_gemm_bf16_gated_normed_takes(most + 1, inner, k)
+    w, weight = rand(2 * inner, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5), 1 + 0.1 * rand(k, seed=2)
+    interleaved = ops.interleave_gate_up(w[:inner].contiguous(), w[inner:].contiguous())
+    for m in sorted({1, most // 2, most // 2 + 1, most}):
+        assert lib.qil_gemm_bf16_gated_normed_takes(m, inner, k)
+        stream = rand(m, k, scale=3.0)
+        squares = stream.square().reshape(m, k // 8, 8).sum(-1).t().contiguous()
+        out = torch.empty(m, inner, dtype=torch.bfloat16, device='cuda')
+        assert lib.qil_gemm_bf16_gated_normed(stream.data_ptr(), weight.data_ptr(), squares.data_ptr(), k // 8, 1e-6, interleaved.data_ptr(),
+                                              out.data_ptr(), m, inner, k, torch.cuda.current_stream().cuda_stream) == 0
+        normed = (stream.double() / torch.sqrt(stream.double().square().mean(-1, keepdim=True) + 1e-6)).float().bfloat16().float() * weight
+        y = normed.bfloat16().double() @ w.double().t()
+        want = torch.nn.functional.silu(y[:, :inner]) * y[:, inner:]
+        # (an operand at a rounding's edge may go either way)
+        torch.testing.assert_close(out.double(), want, atol=2.0 ** -8 * 4 * k ** -0.5 * want.abs().max().item(), rtol=2.0 ** -8)
 
 
 # one row more and less than a tile of 32 (64 with groups of two heads), keys in one piece (543 rows) and in parts (1,057 without a
