@@ -48,8 +48,9 @@ __device__ __forceinline__ uint4 pack8(const float* v) {
 // What the first loads need stands in the first 56 bytes of the arguments, which arrive in registers; the rest and the row's
 // position and sequence are asked for in batches (a dozen reads of arguments, each waited for by itself, and 10 KB of sines to fetch
 // past stood before the first load of data: 8 rows of 2,000 keys 18.8 -> 17.9 us).
-// FUSED: fused_qkv.h; FREQUENCIES: its rotation is made from frequencies, not read from tables.  WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
-template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false, bool FREQUENCIES = false>
+// FUSED: fused_qkv.h; FREQUENCIES: its rotation is made from frequencies, not read from tables; ANY_PAGE: pages whose size is no power of
+// two.  WHOLE: d == DMAX (always so when FUSED).  PAIRS (not FUSED): a wave has the keys and values of two of its steps in flight.
+template <int DMAX, bool FUSED, bool WHOLE = FUSED, bool PAIRS = false, bool FREQUENCIES = false, bool ANY_PAGE = !FUSED>
 __global__ void __launch_bounds__(DEC_MAX_WAVES * QIL_WAVE)
 attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positions, const int* __restrict__ row_seq,
                    const int* __restrict__ block_tables, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -107,10 +108,14 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
 #pragma unroll
   for (int t = 0; t < DTILES; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  // The page of a key and its place there (a division by a number that is not known takes forty instructions a lane).
-  const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
-  auto page_of = [&](int key) __attribute__((always_inline)) { return __builtin_expect(page_shift >= 0, 1) ? key >> page_shift : key / page_size; };
-  auto place_in = [&](int key) __attribute__((always_inline)) { return __builtin_expect(page_shift >= 0, 1) ? key & (page_size - 1) : key % page_size; };
+  // The page of a key and its place there.  A division by a number that is not known takes forty instructions a lane; a choice at run
+  // time is a branch at each of the first loads' addresses (FUSED: by template; with the new key's page no longer waited for ahead of a
+  // wave's sums, us a call: 16 heads of 128 in 8 groups, 1 row of 100 keys 7.9 -> 7.4, 8 of 2,048 15.9 -> 14.9; 14 heads of 64 in 2, 1 row of
+  // 8,000 7.8 -> 7.2; pages of 24 keys, 4 rows of 300 9.5 -> 8.9).
+  const bool shifts = !ANY_PAGE || (!FUSED && (page_size & (page_size - 1)) == 0);
+  const int page_shift = __builtin_ctz(page_size);
+  auto page_of = [&](int key) __attribute__((always_inline)) { return __builtin_expect(shifts, 1) ? key >> page_shift : key / page_size; };
+  auto place_in = [&](int key) __attribute__((always_inline)) { return __builtin_expect(shifts, 1) ? key & (page_size - 1) : key % page_size; };
 
   // What one 32-key step needs from memory: the K rows of both 16-key sub-tiles and the V^T fragments
   // of every dim tile, found through three entries of the block table.
@@ -405,13 +410,13 @@ attn_decode_kernel(const int* __restrict__ plan, const int* __restrict__ positio
       // (every wave looks up and asks: one without a step of its own for the block's last; conditions would cost the waits' counts)
       look_up(min(step, last_step), page);
       if (new_here) new_page = table[page_of(pos)];
-      asm volatile("" : "+v"(new_page));
       __builtin_amdgcn_sched_barrier(0);
       if (makes_q || makes_new) {
         ask(makes_q, wave * HPP + sub);
         __builtin_amdgcn_sched_barrier(0);
         request(min(step, last_step), page, here);
         __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(new_page));                   // (needed late: held here only so that it is not asked for late)
         arrived();
       } else {
         request(min(step, last_step), page, here);
@@ -651,24 +656,31 @@ extern "C" int qil_attn_decode_fused(const float* qkv, int splits, const float* 
   const void* q = nullptr;
   const int q_stride = 0;
   const int* row_index = nullptr;
-#define QIL_DEC_FUSED(DMAX, FREQUENCIES)                                                                                          \
+#define QIL_DEC_FUSED(DMAX, FREQUENCIES, ANY_PAGE)                                                                                \
   do {                                                                                                                             \
     static bool granted = false;                           /* per instantiation: more LDS than a kernel has without asking */      \
     if (lds > 64 * 1024 && !granted) {                                                                                             \
-      const hipError_t e = hipFuncSetAttribute((const void*)attn_decode_kernel<DMAX, true, true, false, FREQUENCIES>,              \
+      const hipError_t e = hipFuncSetAttribute((const void*)attn_decode_kernel<DMAX, true, true, false, FREQUENCIES, ANY_PAGE>,    \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);                             \
       if (e != hipSuccess) return (int)e;                                                                                          \
       granted = true;                                                                                                              \
     }                                                                                                                              \
-    QIL_DEC_LAUNCH(DMAX, true, true, false, fused, FREQUENCIES);                                                                   \
+    QIL_DEC_LAUNCH(DMAX, true, true, false, fused, FREQUENCIES, ANY_PAGE);                                                         \
   } while (0)
-  if (cos_table && !sin_table) {
-    if (d == 64) QIL_DEC_FUSED(64, true);
-    else QIL_DEC_FUSED(128, true);
+#define QIL_DEC_FUSED_D(FREQUENCIES, ANY_PAGE)                                                                                    \
+  do {                                                                                                                             \
+    if (d == 64) QIL_DEC_FUSED(64, FREQUENCIES, ANY_PAGE);                                                                         \
+    else QIL_DEC_FUSED(128, FREQUENCIES, ANY_PAGE);                                                                                \
+  } while (0)
+  const bool frequencies = cos_table && !sin_table, any_page = (page_size & (page_size - 1)) != 0;
+  if (frequencies) {
+    if (any_page) QIL_DEC_FUSED_D(true, true);
+    else QIL_DEC_FUSED_D(true, false);
   } else {
-    if (d == 64) QIL_DEC_FUSED(64, false);
-    else QIL_DEC_FUSED(128, false);
+    if (any_page) QIL_DEC_FUSED_D(false, true);
+    else QIL_DEC_FUSED_D(false, false);
   }
+#undef QIL_DEC_FUSED_D
 #undef QIL_DEC_FUSED
 #undef QIL_DEC_LAUNCH
   QIL_RETURN_LAUNCH_STATUS();

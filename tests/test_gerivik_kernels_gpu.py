@@ -149,6 +149,8 @@ def test_capped_scores_in_decoding_and_in_prompts(dtype, lengths, page_size, d, 
     ([1, 2, 31, 32, 33, 64, 65, 96], 8, 64, 6, 2, 32, 3, 0.5),
     ([2100, 1, 700, 1290, 64, 2047, 300, 33], 16, 128, 16, 4, 64, 8, 30.0),
     ([257, 512, 513], 32, 128, 8, 1, 128, 1, 5.0),
+    ([1, 23, 24, 25, 96, 257, 300], 24, 64, 7, 1, 64, 2, 5.0),            # pages whose size is no power of two
+    ([1, 39, 40, 41, 96, 257, 300], 40, 128, 16, 2, 128, 5, 5.0),
 ])
 def test_decoding_with_queries_made_inside_is_the_two_kernels(lengths, page_size, d, heads, kv_heads, rot, splits, cap):
     """The decode kernel that makes queries, the new key and the new value itself, with the rotation from frequencies
