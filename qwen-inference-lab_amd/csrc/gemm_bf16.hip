@@ -252,9 +252,10 @@ struct NormedStage {
   }
 };
 
-// ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA).  AHEAD (ASRC 1): W's first requests
-// go out ahead of the parts' arrival (launch_lines).
-template <typename OUT, int ASRC, int WAVES = LINES_WAVES, bool AHEAD = true>
+// ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA).  HOW, behind the merge (launch_lines):
+// W's first requests go out ahead of the parts' arrival, or behind it, with a piece's loads all at once or its row's position first.
+enum { AHEAD, AT_ONCE, POSITION_FIRST };
+template <typename OUT, int ASRC, int WAVES = LINES_WAVES, int HOW = AHEAD>
 __global__ void __launch_bounds__(WAVES * QIL_WAVE)
 gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N, int K,
                        int cols_per_split, UnmergedA unmerged, NormedA normed) {
@@ -316,16 +317,28 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
       c = (of - m * pieces) * 8;
       merge_ask(unmerged, P, m, k_begin + c, parts);
     };
-    auto put = [&]() {
-      float v[8];
-      merge_finish(unmerged, P, m, k_begin + c, parts, v);
+    auto store = [&](const float (&v)[8]) {
       *reinterpret_cast<uint4*>(a_lds + m * row_width + c) =
           make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
     };
-    if constexpr (!AHEAD) {
+    auto put = [&]() {
+      float v[8];
+      merge_finish(unmerged, P, m, k_begin + c, parts, v);
+      store(v);
+    };
+    if constexpr (HOW == AT_ONCE) {
       for (; idx < all; idx += THREADS) {
         ask(idx);
         put();
+      }
+      request_first();
+    } else if constexpr (HOW == POSITION_FIRST) {
+      for (; idx < all; idx += THREADS) {
+        m = idx / pieces;
+        c = (idx - m * pieces) * 8;
+        float v[8];
+        merged_values<8>(unmerged, m, k_begin + c, v);
+        store(v);
       }
       request_first();
     } else if constexpr (WAVES < LINES_WAVES) {
@@ -424,11 +437,11 @@ static bool lines_takes(const void* A, const void* W, const float* bias, int M, 
   return lines_lds(M, K, splits) <= LINES_LDS_LIMIT;
 }
 
-template <typename OUT, int ASRC, int WAVES, bool AHEAD = true>
+template <typename OUT, int ASRC, int WAVES, int HOW = AHEAD>
 static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
                               UnmergedA unmerged, NormedA normed) {
   const size_t lds = lines_lds(M, K, splits, WAVES);
-  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC, WAVES, AHEAD>;
+  auto kernel = gemm_bf16_lines_kernel<OUT, ASRC, WAVES, HOW>;
   static size_t granted = 0;                              // per instantiation
   if (lds > 64 * 1024 && lds > granted) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -447,9 +460,13 @@ static int launch_lines_waves(const bf16_t* A, const bf16_t* W, OUT* C, int M, i
 // the blocks of half the threads take longer for that than they gain (8 rows and 63 parts 16.7 us with 8 waves, 22.5 with 4; 6 rows
 // and 2 parts 5.5 / 5.9; 4 rows 4 is ahead at any number of parts).
 // Behind the merge W's first stages are asked for ahead of the parts' arrival (AHEAD) where all parts come in one turn: up to four of
-// them for blocks of 4 waves, a piece of A a thread for those of 8; a second turn's loads would come back behind W.  us without / with:
-// 1 row of 1,024 x 2,048, 2 parts 4.5 / 4.4 alone and 5.7 / 5.3 inside a step, 9 parts 5.9 / 5.9; 8 rows of 4,096 x 4,096, 4 parts
-// 8.7 / 8.1; 16 rows of 1,024 x 2,048, 2 parts (two pieces a thread) 6.8 / 7.2.
+// them for blocks of 4 waves, a piece of A a thread for those of 8; a second turn's loads would come back behind W, which pays only where
+// a quarter of the threads have none and W is much.  us without / with: 1 row of 1,024 x 2,048, 2 parts 4.5 / 4.4 alone and 5.7 / 5.3 inside a
+// step, 9 parts 5.9 / 5.9; 8 rows of 4,096 x 4,096, 4 parts 8.7 / 8.1, 8 level, 6 rows and 8 parts 10.3 / 9.6, of 1,024 x 2,048 6.9 / 7.5; 16
+// rows of 1,024 x 2,048, 2 parts (two pieces a thread) 6.8 / 7.2.
+// Where they are not, blocks of 8 waves with up to two pieces a thread ask for the row's position first, others for all of a piece at
+// once (us position first / at once: 16 rows of 1,024 x 2,048, 2 parts 6.8 / 7.2, 8 of 896 x 896 8.3 / 8.7, but 16 of 896 x 896 (3.5 pieces) 10.2 / 9.8,
+// 12 of 5,120 x 8,192 24.3 / 23.7, and 2 of 1,024 x 2,048, 16 parts in blocks of 4 waves 6.5 / 6.2).
 #define LINES_FEW_WAVES 4
 template <typename OUT, int ASRC = 0>
 static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, int K, int splits, hipStream_t s,
@@ -457,10 +474,12 @@ static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, 
   const long blocks = (long)((N + 16 * LINES_WAVES - 1) / (16 * LINES_WAVES)) * splits;
   const bool few = M <= (ASRC == 1 ? 4 : 8) && blocks <= QIL_CUS / 2;
   if constexpr (ASRC == 1) {
-    const bool ahead = few ? unmerged.parts <= 4 : (long)M * (K / splits / 8) <= LINES_WAVES * QIL_WAVE;
-    if (!ahead)
-      return few ? launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES, false>(A, W, C, M, N, K, splits, s, unmerged, normed)
-                 : launch_lines_waves<OUT, ASRC, LINES_WAVES, false>(A, W, C, M, N, K, splits, s, unmerged, normed);
+    constexpr int THREADS = LINES_WAVES * QIL_WAVE;
+    const long pieces = (long)M * (K / splits / 8);
+    if (few && unmerged.parts > 4) return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES, AT_ONCE>(A, W, C, M, N, K, splits, s, unmerged, normed);
+    if (!few && pieces > 2 * THREADS) return launch_lines_waves<OUT, ASRC, LINES_WAVES, AT_ONCE>(A, W, C, M, N, K, splits, s, unmerged, normed);
+    if (!few && pieces > (unmerged.parts <= 4 ? THREADS : blocks > QIL_CUS / 2 ? THREADS * 3 / 4 : 0))
+      return launch_lines_waves<OUT, ASRC, LINES_WAVES, POSITION_FIRST>(A, W, C, M, N, K, splits, s, unmerged, normed);
   }
   if (few) return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
   return launch_lines_waves<OUT, ASRC, LINES_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);

@@ -271,8 +271,8 @@ gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, 
     __builtin_amdgcn_s_waitcnt(0x07C);                      // vmcnt(12) lgkmcnt(0): see the whole-line kernel in gemm_bf16.hip
     __builtin_amdgcn_s_barrier();
   } else {
-    MergeParts<4, WAVES == FL_WIDE_WAVES ? 8 : 16> parts;     // (ASRC 1; sixteen parts do not fit the registers of 16 waves)
-    const int P = ASRC == 1 ? merge_part_keys(unmerged) : 0;
+    MergeParts<4, 16> parts;                                // (ASRC 1, AHEAD)
+    const int P = ASRC == 1 && AHEAD ? merge_part_keys(unmerged) : 0;
     float4 gs[4], us[4];                                    // (ASRC 2: four splits of gate and up)
     const size_t stride = (size_t)M * 2 * K;
     int m, c;
@@ -289,14 +289,15 @@ gemm_f32_lines_kernel(const float* __restrict__ A, const float* __restrict__ W, 
     auto ask = [&](int idx) __attribute__((always_inline)) {
       m = idx / pieces;
       c = (idx - m * pieces) * 4;
-      if constexpr (ASRC == 1) merge_ask(unmerged, P, m, k_begin + c, parts);
-      else ask_sums(0);
+      if constexpr (ASRC == 2) ask_sums(0);
+      else if constexpr (AHEAD) merge_ask(unmerged, P, m, k_begin + c, parts);
     };
     auto put = [&]() __attribute__((always_inline)) {
       float4 v;
       if constexpr (ASRC == 1) {
         float merged[4];
-        merge_finish(unmerged, P, m, k_begin + c, parts, merged);
+        if constexpr (AHEAD) merge_finish(unmerged, P, m, k_begin + c, parts, merged);
+        else merged_values<4, WAVES == FL_WIDE_WAVES ? 8 : 16>(unmerged, m, k_begin + c, merged);      // (sixteen parts do not fit the registers of 16 waves)
         v = make_float4(merged[0], merged[1], merged[2], merged[3]);
       } else {
         float4 g = make_float4(0.f, 0.f, 0.f, 0.f), u = g;
