@@ -185,14 +185,18 @@ struct NormedA {
 
 // A block's slice of such an operand, columns k_begin .. k_begin + cols, on its way into LDS: ask() sends the first loads, put() waits for
 // them (not for what was asked for in between) and leaves the rows in LDS, to be met behind a barrier.  M at most twice the waves.
-// A wave adds the pieces of two rows' sums of squares; they are asked for together with what a thread's first two pieces of A are
-// made of.  (All are held in place: the compiler otherwise moves loads whose use stands under a condition down to it.)
+// A wave adds the pieces of two rows' sums of squares; up to 512 of them (4,096 columns in pieces of 8, 8,192 in pieces of 16) are asked for
+// together with what a thread's first two pieces of A are made of.  (Those past 256, asked for at their use, came back behind W: us
+// a product, 12 rows of 6,144 x 2,560 in pieces of 8 11.3 -> 10.4, 1 and 16 of 7,168 x 5,120 in pieces of 16 15.4 -> 14.5 and 19.0 -> 18.1.)
+// (All are held in place: the compiler otherwise moves loads whose use stands under a condition down to it.)
+// MANY: more than 256 pieces (a choice at run time cost 0.1 us of 3.5 where they are fewer).
+template <bool MANY>
 struct NormedStage {
   static constexpr int EARLY = 2, SQUARES = 4;
   const NormedA& normed;
   float* rstd;                                             // 16 floats of LDS
   const int M, K, k_begin, pieces, all, threads, lane, wave, waves;
-  float x[EARLY][8], g[EARLY][8], squares[2][SQUARES];
+  float x[EARLY][8], g[EARLY][8], squares[2][SQUARES], more[2][SQUARES];
   __device__ __forceinline__ NormedStage(const NormedA& n, void* scratch, int m, int k, int first, int cols, int w, int ws)
       : normed(n), rstd(reinterpret_cast<float*>(scratch)), M(m), K(k), k_begin(first), pieces(cols / 8), all(m * (cols / 8)),
         threads(ws * QIL_WAVE), lane(threadIdx.x & (QIL_WAVE - 1)), wave(w), waves(ws) {}
@@ -201,13 +205,19 @@ struct NormedStage {
     ld8(normed.stream + (size_t)m * K + k_begin + c, to_x);
     ld8(normed.weight + k_begin + c, to_g);
   }
+  __device__ __forceinline__ void ask_squares(int r2, int first, float (&to)[SQUARES]) {
+#pragma unroll
+    for (int i = 0; i < SQUARES; ++i)
+      to[i] = normed.squares[(size_t)min(first + lane + i * QIL_WAVE, normed.pieces - 1) * M + min(wave + r2 * waves, M - 1)];
+  }
   __device__ __forceinline__ void ask() {
 #pragma unroll
     for (int r2 = 0; r2 < 2; ++r2)
-      if (!r2 || M > waves)
+      if (!r2 || M > waves) ask_squares(r2, 0, squares[r2]);
+    if constexpr (MANY)
 #pragma unroll
-        for (int i = 0; i < SQUARES; ++i)
-          squares[r2][i] = normed.squares[(size_t)min(lane + i * QIL_WAVE, normed.pieces - 1) * M + min(wave + r2 * waves, M - 1)];
+      for (int r2 = 0; r2 < 2; ++r2)
+        if (!r2 || M > waves) ask_squares(r2, SQUARES * QIL_WAVE, more[r2]);
 #pragma unroll
     for (int u = 0; u < EARLY; ++u)
       if (!u || all > threads) ask_piece(min((int)threadIdx.x + u * threads, all - 1), x[u], g[u]);
@@ -232,7 +242,13 @@ struct NormedStage {
         asm volatile("" : "+v"(squares[r2][i]));
         if (lane + i * QIL_WAVE < normed.pieces) sum += squares[r2][i];
       }
-      for (int p = lane + SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
+      if constexpr (MANY)
+#pragma unroll
+        for (int i = 0; i < SQUARES; ++i) {
+          asm volatile("" : "+v"(more[r2][i]));
+          if (lane + (SQUARES + i) * QIL_WAVE < normed.pieces) sum += more[r2][i];
+        }
+      for (int p = lane + (MANY ? 2 : 1) * SQUARES * QIL_WAVE; p < normed.pieces; p += QIL_WAVE) sum += normed.squares[(size_t)p * M + min(m, M - 1)];
       sum = wave_sum(sum);
       if (lane == 0 && m < M) rstd[m] = rsqrtf(sum / (float)K + normed.eps);
     }
@@ -253,8 +269,9 @@ struct NormedStage {
 };
 
 // ASRC: 0 = A as it is, 1 = merged attention parts (UnmergedA), 2 = normalised stream (NormedA).  HOW, behind the merge (launch_lines):
-// W's first requests go out ahead of the parts' arrival, or behind it, with a piece's loads all at once or its row's position first.
-enum { AHEAD, AT_ONCE, POSITION_FIRST };
+// W's first requests go out ahead of the parts' arrival, or behind it, with a piece's loads all at once or its row's position first;
+// behind the norm: NormedStage's MANY.
+enum { AHEAD, AT_ONCE, POSITION_FIRST, MANY_SQUARES };
 template <typename OUT, int ASRC, int WAVES = LINES_WAVES, int HOW = AHEAD>
 __global__ void __launch_bounds__(WAVES * QIL_WAVE)
 gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, OUT* __restrict__ C, int M, int N, int K,
@@ -302,7 +319,7 @@ gemm_bf16_lines_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
   constexpr int THREADS = WAVES * QIL_WAVE;
   const int pieces = cols_per_split / 8, all = M * pieces;  // (rows past M stay as they are in LDS: their products are never stored)
   if (ASRC == 2) {
-    NormedStage stage(normed, lds + a_rows * row_width + WAVES * (16 * 128), M, K, k_begin, cols_per_split, wave, WAVES);
+    NormedStage<HOW == MANY_SQUARES> stage(normed, lds + a_rows * row_width + WAVES * (16 * 128), M, K, k_begin, cols_per_split, wave, WAVES);
     stage.ask();
     __builtin_amdgcn_sched_barrier(0);
     request_first();
@@ -481,6 +498,10 @@ static int launch_lines(const bf16_t* A, const bf16_t* W, OUT* C, int M, int N, 
     if (!few && pieces > (unmerged.parts <= 4 ? THREADS : blocks > QIL_CUS / 2 ? THREADS * 3 / 4 : 0))
       return launch_lines_waves<OUT, ASRC, LINES_WAVES, POSITION_FIRST>(A, W, C, M, N, K, splits, s, unmerged, normed);
   }
+  if constexpr (ASRC == 2)
+    if (normed.pieces > 256)
+      return few ? launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES, MANY_SQUARES>(A, W, C, M, N, K, splits, s, unmerged, normed)
+                 : launch_lines_waves<OUT, ASRC, LINES_WAVES, MANY_SQUARES>(A, W, C, M, N, K, splits, s, unmerged, normed);
   if (few) return launch_lines_waves<OUT, ASRC, LINES_FEW_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
   return launch_lines_waves<OUT, ASRC, LINES_WAVES>(A, W, C, M, N, K, splits, s, unmerged, normed);
 }
@@ -754,7 +775,7 @@ gemm_bf16_gated_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ 
     request(g1, 0, 1); request(u1, up_offset, 1);
   };
   if constexpr (NORMED) {
-    NormedStage stage(normed, lds + a_rows * row_width + waves * (16 * 128), M, K, 0, K, wave, waves);
+    NormedStage<false> stage(normed, lds + a_rows * row_width + waves * (16 * 128), M, K, 0, K, wave, waves);
     stage.ask();
     __builtin_amdgcn_sched_barrier(0);
     request_first();

@@ -51,9 +51,11 @@ def test_products_behind_the_merge(ops, m, parts, n, heads, d, window):
     torch.testing.assert_close(out.double().sum(0), rounded @ w.double().t(), atol=2.0 ** -8 * 4 * k ** -0.5 * want.abs().max().item(), rtol=1e-5)
 
 
-# a thread's first and second piece of A and more; one and two rows a wave; pieces of 8 and of 16 columns, more than 256 of them
+# a thread's first and second piece of A and more; one and two rows a wave; pieces of 8 and of 16 columns, more than 256 of them in blocks
+# of four and of eight waves, more than 512
 @pytest.mark.parametrize('m', [1, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize('n,k,columns', [(4096, 1024, 8), (64, 384, 16), (6144, 4096, 16), (512, 4608, 16)])
+@pytest.mark.parametrize('n,k,columns', [(4096, 1024, 8), (64, 384, 16), (6144, 4096, 16), (512, 4608, 16), (512, 2560, 8), (6144, 2560, 8),
+                                         (7168, 5120, 16), (512, 5120, 8)])
 def test_products_behind_the_norm(ops, m, n, k, columns):
     """As above, with the operand as the norm rounds it: the row over its root mean square, then the weight."""
     lib = ops.library.load()
