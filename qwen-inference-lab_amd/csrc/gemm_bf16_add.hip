@@ -349,8 +349,10 @@ int qil_gemm_bf16_whole(const void* A, const void* W, void* out, int M, int N, i
 
 // 1 if qil_gemm_bf16_unmerged_add takes these sizes: up to four rows and 16 parts in all, at most a block of 8 columns a CU, one to four
 // stages a wave.  Every block merges all rows, which beyond that costs more than the norm's kernel: us a step of 28 layers with partial
-// sums and a norm / so: 1 row of 100 keys 882 / 823, of 3,500 (14 parts) 955 / 893, 4 of 100 936 / 901, but 4 of 2,000 (8 parts each) 1,038 / 1,057,
-// 5 of 100 980 / 1,015, 8 of 300 999 / 1,042.
+// sums and a norm / so: 1 row of 100 keys 879 / 810, of 3,600 (16 parts) 968 / 903; 2 rows of 100 900 / 840, of 512 (4 parts each) 897 / 853, of
+// 1,600 (8 parts) 939 / 897; 3 rows of 300 930 / 917, of 600 (4 parts) 932 / 917; 4 rows of 100 928 / 917, of 512 (4 parts) 951 / 937; but 4 of 2,000
+// (8 parts) 1,038 / 1,057, 5 of 100 980 / 1,015, 8 of 300 999 / 1,042.  4,096 columns, two blocks a CU, 12 layers: 1 row of 100 keys 1,184 / 1,204, of
+// 2,048 1,252 / 1,315, 4 of 100 1,260 / 1,371.
 #define MERGE_ADD_ROWS 4
 #define MERGE_ADD_PARTS 16
 int qil_gemm_bf16_unmerged_add_takes(int M, int N, int heads, int d, int parts) {
