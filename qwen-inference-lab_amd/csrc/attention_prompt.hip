@@ -7,8 +7,8 @@
 //
 // A wave issues one instruction every four cycles and a product keeps the matrix core for 32, so what a tile costs
 // is the number of instructions it takes and how many of them stand between two products.  Hence:
-//  * global_load_lds_dwordx4: a wave's load puts 1 KB from memory into LDS without passing registers, no LDS write
-//    instruction and no staging registers.  The 64 lanes' 16-byte pieces land side by side, so the layout in LDS is
+//  * buffer_load_dwordx4 into LDS: a wave's load puts 1 KB from memory into LDS without passing registers, no LDS write
+//    instruction and no staging registers (as a buffer load: load_to_lds says why).  The 64 lanes' 16-byte pieces land side by side, so the layout in LDS is
 //    made by the choice of what each lane loads:
 //      K tile  [64 rows][16 pieces]: a load is 4 consecutive keys (1 KB of a page), piece p of row r holds the
 //              dims 8 (p ^ (r & 15)) ..: the fragment reads of 32 rows at one dim offset then spread over all banks;
@@ -17,6 +17,12 @@
 //  * everything of a load's address that changes from tile to tile is the same for the whole wave (the page, found
 //    one tile ahead by one lane per load, and the place in it) and is computed on the scalar unit;
 //  * the next tile's loads are issued between the score products (none after a block's last tile);
+//  * the exponentials of the next 16 keys and the reads of their values stand between the value products of 16 keys; the first
+//    values are asked for ahead of the statistics.  With this and the buffer loads (before, every wait for a fragment was one for all
+//    of a wave's reads, and the exponentials stood ahead of all value products), us, 32 heads in 8 groups: 8,192 tokens 656 -> 618,
+//    2,048 52.9 -> 50.1, 500 16.6 -> 16.0; 16 heads in 4 groups 2,048 44.4 -> 42.0, in two groups of waves 38.6 -> 36.8.  The matrix
+//    cores are then busy for 52 % and the vector units for 49 % of the cycles (8,192 tokens), at a clock that the power limit holds
+//    near 1.6 GHz: what is left are instructions, not waits;
 //  * two tiles in LDS, one barrier a tile: after it every wave's loads of this tile have landed and every wave has
 //    finished with the tile before, whose place the next loads take;
 //  * the reference of a row's exponents is only moved (to the maximum) when a score exceeds it by 2^8 in the
@@ -44,10 +50,17 @@ __device__ __forceinline__ int prompt_row(int kl) {
   return (kl & ~15) + ((kl >> 2) & 1) * 8 + ((kl >> 3) & 1) * 4 + (kl & 3);
 }
 
+// The larger of a lane's value and that of the lane 32 further, without a trip through LDS.
+__device__ __forceinline__ float max_over_halves(float v) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(both.x), __uint_as_float(both.y));
+}
+
 // SPLIT (8 waves, no window, keys in one part): the block's waves are two groups of four that take the same rows and
 // heads and each one half of the block's tiles of keys, with two tiles in LDS of its own; at the end the second
 // group hands its sums over in LDS and the first adds them to its own.  For prompts so short that blocks of 4 waves
-// are fewer than the CUs: every SIMD then has two waves.  (It does not help longer prompts: a wave-tile takes 1.75 us
+// are fewer than the CUs: every SIMD then has two waves.  (It does not help longer prompts: a wave-tile takes 1.5 us
 // of its SIMD's issue slots whether the wave is alone there or not, and 2,048 tokens are 33 wave-tiles a SIMD.)
 // CAP: scores are scaled and capped softly (softcap * tanh(score / softcap)) as they leave the matrix cores; the
 // exponent then scales nothing.
@@ -186,15 +199,13 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* __r
     const int key = (it * GW + wave) * 4;
     const size_t page_at = (size_t)(uint32_t)__builtin_amdgcn_readlane(held, it) << 8;
     const uint32_t in = (uint32_t)(in_page + (key & (page_size - 1))) * (D * 2);
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(k_head + page_at + in + k_lane),
-                                     (__attribute__((address_space(3))) void*)(to + prompt_row(key) * (D * 2)), 16, 0, 0);
+    load_to_lds(k_head + page_at + in, k_lane, to + prompt_row(key) * (D * 2));
   };
   auto load_v = [&](int in_page, int it, unsigned char* to) __attribute__((always_inline)) {
     const int j = it * GW + wave;
     const size_t page_at = (size_t)(uint32_t)__builtin_amdgcn_readlane(held, it) << 8;
     const uint32_t in = (uint32_t)(in_page + ((j >> 1) * 8 & (page_size - 1))) * 2;
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(v_head + page_at + in + v_lane),
-                                     (__attribute__((address_space(3))) void*)(to + BK * D * 2 + j * 1024), 16, 0, 0);
+    load_to_lds(v_head + page_at + in, v_lane, to + BK * D * 2 + j * 1024);
   };
   // any k0: the pages are kept inside the needed ones
   auto load_tile = [&](int k0, int k1, unsigned char* to) __attribute__((always_inline)) {
@@ -284,12 +295,25 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* __r
           s[kt][i] = visible ? s[kt][i] : -INFINITY;
         }
     }
-    float mx = -INFINITY;
+    // the first values are on their way while the statistics are made
+    auto v_fragment = [&](int u, int t) __attribute__((always_inline)) {
+      return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(Vt + u * (2 * D * 16) + t * (32 * 16)));
+    };
+    bf16x8 va[4][WTILES];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int t = 0; t < WTILES; ++t) va[0][t] = v_fragment(0, t);
+    __builtin_amdgcn_sched_barrier(0);
+    float mx = fmaxf(s[0][0], s[1][0]);
+    {
+      float other = fmaxf(s[0][1], s[1][1]);               // two chains
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kt][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, QIL_WAVE));
+      for (int i = 2; i < 16; i += 2) {
+        mx = fmaxf(fmaxf(mx, s[0][i]), s[1][i]);
+        other = fmaxf(fmaxf(other, s[0][i + 1]), s[1][i + 1]);
+      }
+      mx = fmaxf(mx, other);
+    }
+    mx = max_over_halves(mx);
     // the reference of the exponents moves (to the maximum) only if the maximum is 2^8 beyond it, or there was none
     const bool moves = (mx - row_m) * c > 8.f || (row_m == -INFINITY && mx != -INFINITY);
     const float m_new = moves ? mx : row_m;
@@ -304,43 +328,36 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* __r
         for (int i = 0; i < 16; ++i) ow[t][i] *= alpha;
     }
     row_m = m_new;
-    // probabilities, 16 keys at a time (scores 8 (u % 2) .. of 32-key tile u / 2), packed as the B operands of the value
-    // products right away: the float32 values are not kept
+    // Probabilities, 16 keys at a time (scores 8 (u % 2) .. of 32-key tile u / 2), packed as the B operands of the value
+    // products right away: the float32 values are not kept.  Between two value products of 16 keys stand the exponentials of four
+    // scores of the next 16 (two of a lane's eight pairs), and a read of its values: the products take 32 cycles of the
+    // matrix core each and these instructions as many of the vector unit, so neither waits for the other.
     float psum = 0.f;
-    bf16x8 pb[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    uint32_t packed[2][4];
+    auto probabilities = [&](int u, int e) __attribute__((always_inline)) {
       const int kt = u >> 1, st = u & 1;
-      uint32_t packed[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kt][8 * st + 2 * e], c, shift));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[kt][8 * st + 2 * e + 1], c, shift));
-        psum += p0;
-        psum += p1;
-        packed[e] = pack_bf16(p0, p1);
-      }
-      pb[u] = __builtin_bit_cast(bf16x8, make_uint4(packed[0], packed[1], packed[2], packed[3]));
-    }
-    row_l = row_l * alpha + psum;
-    asm volatile("" : "+v"(row_l));                        // summed here, not after the products below
-    auto v_fragment = [&](int u, int t) __attribute__((always_inline)) {
-      return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(Vt + u * (2 * D * 16) + t * (32 * 16)));
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kt][8 * st + 2 * e], c, shift));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(s[kt][8 * st + 2 * e + 1], c, shift));
+      psum += p0;
+      psum += p1;
+      asm volatile("" : "+v"(psum));                       // summed here, not behind the products
+      packed[u & 1][e] = pack_bf16(p0, p1);
     };
-    bf16x8 va[4][WTILES];
 #pragma unroll
-    for (int t = 0; t < WTILES; ++t) va[0][t] = v_fragment(0, t);
+    for (int e = 0; e < 4; ++e) probabilities(0, e);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      if (u + 1 < 4) {
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, make_uint4(packed[u & 1][0], packed[u & 1][1], packed[u & 1][2], packed[u & 1][3]));
 #pragma unroll
-        for (int t = 0; t < WTILES; ++t) va[u + 1][t] = v_fragment(u + 1, t);
+      for (int t = 0; t < WTILES; ++t) {
+        if (u + 1 < 4) va[u + 1][t] = v_fragment(u + 1, t);
+        ow[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[u][t], pb, ow[t], 0, 0, 0);
+        if (u + 1 < 4) probabilities(u + 1, t);
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int t = 0; t < WTILES; ++t) ow[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[u][t], pb[u], ow[t], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
     }
+    row_l = row_l * alpha + psum;
   };
 
   __syncthreads();                                         // the table entries are in place
