@@ -44,7 +44,7 @@ class StepContext:
     fresh: bool = False            # every sequence of the step begins with it, and the step is not described for a graph
     plans: dict = field(default_factory=dict)    # how the step's attention kernels share out their keys, kept from its first layer on
     tile_seqs: int = None          # sequences 0 .. tile_seqs - 1 are those of two or more rows; None: any may be
-    tile_context: int = None       # largest position + 1 of those; None: not known (a step described for a graph)
+    tile_context: int = None       # largest position + 1 of those; None: not known (a step described for a graph of any)
 
 
 class StepPieces:

@@ -18,7 +18,7 @@ temperatures travel in the same array), and a step costs one upload, one replay 
 Steps with prompt portions have recurring shapes too (a portion of the chunk size beside so many single
 tokens, step after step while a long prompt comes in), and for small models their launches cost more than
 their kernels.  A shape that has been seen before (the same numbers of tokens and of wanted places per request,
-largest first, and the same, wider bucket) is captured the second time and replayed from then on; the
+largest first, the same, wider bucket, and beside single tokens portions that all begin their requests or not) is captured the second time and replayed from then on; the
 requests are put into the graph's order and the logits back into the caller's.  The draw stays outside.
 
 A new graph warms up (one run launch by launch, which loads the kernels and sizes the allocator) on inert
@@ -60,7 +60,7 @@ def row_bucket(rows):
 
 
 class _Graph:
-    def __init__(self, runner, entries, pieces, facts, bucket, sampler=None):
+    def __init__(self, runner, entries, pieces, facts, bucket, sampler=None, tile_context=None):
         self.sizes = pieces.sizes()
         self.spans = pieces.spans()
         rows = facts['s']                                   # with the inert rows that fill a decode batch
@@ -79,7 +79,7 @@ class _Graph:
             self.drawn_host = torch.zeros((2, rows), dtype=torch.int32).pin_memory()
         zeros = None if sampler is None else np.zeros((3, rows), dtype=np.int32)
         self.load(runner._inert(pieces, facts), zeros)     # the warm-up's inputs: nobody's pages, nobody's state
-        ctx = runner._context(entries, pieces, facts, self.meta, max_context=bucket)
+        ctx = runner._context(entries, pieces, facts, self.meta, max_context=bucket, tile_context=tile_context)
         side = torch.cuda.Stream(device=device)
         side.wait_stream(torch.cuda.current_stream(device))
         with torch.cuda.stream(side):                       # launch by launch once: loads the library, sizes the allocator
@@ -229,7 +229,12 @@ class DecodeGraphs:
         if limit is not None:
             bucket = min(bucket, -(-limit // ps) * ps)
         width = -(-bucket // ps)
-        key = (tuple(len(e.tokens) for e in ordered), tuple(len(e.want) for e in ordered), bucket)
+        # Steps whose portions are all their requests' first, beside requests that decode, have graphs of their own: the portions'
+        # attention is planned for the keys they bring and not for the longest context of those requests.
+        first_portions = len(ordered[-1].tokens) == 1 and \
+            all(runner.cache.computed[e.request] == 0 for e in ordered if len(e.tokens) > 1)
+        tile_context = len(ordered[0].tokens) if first_portions else None
+        key = (tuple(len(e.tokens) for e in ordered), tuple(len(e.want) for e in ordered), bucket, tile_context)
         graph = self.mixed.get(key)
         described, pieces, facts = runner._describe(ordered, table_width=width, validate=False)
         if graph is None:
@@ -243,7 +248,7 @@ class DecodeGraphs:
             if sightings >= (MIXED_REPLACE_AT if full else MIXED_CAPTURE_AT):
                 if full:
                     self.mixed.pop(next(iter(self.mixed)))          # the least recently replayed
-                graph = self.mixed[key] = _Graph(runner, described, pieces, facts, bucket)
+                graph = self.mixed[key] = _Graph(runner, described, pieces, facts, bucket, tile_context=tile_context)
                 self.mixed_captures += 1
                 del self.seen[key]
         else:
@@ -254,7 +259,7 @@ class DecodeGraphs:
             # of requests, table width and context bucket), so that the kernels, their splits of the keys and the
             # order of their sums are the same whether the step is launched or replayed.
             flat = torch.from_numpy(pieces.flat()).to(runner.model.device)
-            ctx = runner._context(described, pieces, facts, flat, max_context=bucket)
+            ctx = runner._context(described, pieces, facts, flat, max_context=bucket, tile_context=tile_context)
             logits = runner.model.forward(ctx, runner.views)
         else:
             logits = graph.run()

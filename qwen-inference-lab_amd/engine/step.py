@@ -160,8 +160,9 @@ class ModelRunner:
             inert.add(name, values)
         return inert
 
-    def _context(self, entries, pieces, facts, device_flat, max_context=None):
-        """StepContext and cache views over a device int32 array holding the pieces back to back."""
+    def _context(self, entries, pieces, facts, device_flat, max_context=None, tile_context=None):
+        """StepContext and cache views over a device int32 array holding the pieces back to back.  ``max_context``: a graph's
+        bucket instead of the step's own longest context, ``tile_context`` then the portions' (None: any up to the bucket)."""
         spans = pieces.spans()
         part = lambda name: device_flat[spans[name][0]:spans[name][1]]
         s, counts = facts['s'], facts['counts']
@@ -172,7 +173,7 @@ class ModelRunner:
             single_rows=part('single_rows') if max(counts) > 1 else None, max_query=max(counts),
             max_context=max_context or facts['max_context'], host_cu_seqlens=facts['cu'], host_starts=facts['starts'],
             host_slots=facts['slots'], requests=[e.request for e in entries], tile_seqs=facts['tile_seqs'],
-            tile_context=None if max_context else facts['tile_context'],
+            tile_context=tile_context if max_context else facts['tile_context'],
             previous_tokens=part('previous') if self.previous_tokens else None)
         for view in (one for view in self.views for one in (view if isinstance(view, tuple) else (view,))):
             if view is not None and hasattr(view, 'block_tables'):

@@ -245,6 +245,37 @@ def test_a_recurring_shape_gives_the_same_bits_launched_and_replayed(model_folde
         assert torch.equal(first, seen[0][0]) and torch.equal(second, seen[0][1])
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_first_portions_have_graphs_of_their_own(model_folder, dtype):
+    """A portion of 40 tokens beside a decoding row of 300, from its request's start, right behind its first token and deep in
+    it: the same sizes and bucket, two plans of the portion's attention.  Three times over each, so launched,
+    captured and replayed; every logit against the plain model."""
+    from qil_amd.engine import ModelRunner, StepEntry
+    from qil_amd.weights import load_model
+    config = plain.TINY_B
+    folder, weights = model_folder(config, 13)
+    model = load_model(folder, dtype=dtype, device='cuda')
+    row, prompt = random_tokens(config, 312, 5), random_tokens(config, 400, 6)
+    want_row, want = plain.logits(row, weights, config), plain.logits(prompt, weights, config)
+    runner = ModelRunner(model, num_pages=120, page_size=8, max_requests=2)
+    for group in runner.cache.kv_groups:
+        group['k'].fill_(float('nan')), group['v'].fill_(float('nan'))
+    runner.admit('row')
+    runner.step([StepEntry('row', tuple(row[:300]), ())])
+    fed = 300
+    for occurrence in range(3):
+        for start in (0, 1, 24, 300):
+            runner.admit('new')
+            if start:
+                runner.step([StepEntry('new', tuple(prompt[:start]), ())])
+            logits = runner.step([StepEntry('row', (row[fed],), (0,)), StepEntry('new', tuple(prompt[start:start + 40]), (0, 39))]).cpu()
+            torch.testing.assert_close(logits, torch.stack((want_row[fed], want[start], want[start + 39])), **TOLERANCE[dtype])
+            runner.release('new')
+            fed += 1
+    kinds = {key[3] for key in runner.graphs.mixed if key[0] == (40, 1)}
+    assert kinds == {40, None}, runner.graphs.mixed.keys()
+
+
 def test_more_recurring_shapes_than_the_store_holds(model_folder, monkeypatch):
     """Three shapes of mixed steps in turns with room for two graphs: the first two are captured at their second
     coming and replayed from then on; the third is launched kernel by kernel until it has come four times, then takes
