@@ -1194,8 +1194,8 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
     (every row alone, context in several parts) for ``linear`` to merge.
     ``tile_seqs``: the caller has put the sequences of two or more rows first and there are this many; the tile
     kernel then gets blocks for these only (None: for every sequence; those of one row leave at once).
-    ``tile_context``: the longest context of the sequences of two or more rows (or more than it), where the caller knows it; the
-    parts of their keys and the shape of the prompt kernel's blocks go by it.
+    ``tile_context``: the longest context of the sequences of two or more rows, or more than it, never less (keys beyond it are not
+    read), where the caller knows it; the parts of their keys and the shape of the prompt kernel's blocks go by it.
     ``softcap`` c: scores are scaled, then capped softly, c * tanh(score / c), before the softmax.  The kernels
     specialised for bfloat16 heads of 64 and 128 have no cap; capped steps run on the general tile kernel.
     ``sinks`` float32 [heads]: exp(sinks[h]) joins the divisor of head h's softmax once (no key, no value, not
@@ -1250,7 +1250,10 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
             n_seqs = tile_seqs
         # A first portion of 128 rows beside rows of 2,048 tokens: planned for its own 128 keys one kernel of 10.5 us a layer, planned
         # for 2,048 the keys in 16 parts, 14 us, and their merge, 5.
-        reach = max_context if tile_context is None else min(tile_context, max_context)
+        # (Without ``tile_seqs`` the merge takes the rows alone too, by their positions: the parts have to reach as far as they do.)
+        reach = max_context
+        if tile_context is not None and (tile_seqs is not None or not single_rows.shape[0]):
+            reach = min(tile_context, max_context)
         part, parts = tile_key_parts(lib, qkv.dtype, several, max_query, heads, kv_heads,
                                      head_dim, page_size, block_tables.shape[1], reach, general=cap > 0 or slopes is not None)
         if keep:

@@ -324,3 +324,26 @@ def test_block_shape_of_portions_behind_a_history(ops, rows, starts, told, waves
         finally:
             lib.qil_attn_tile_waves(0)
     assert torch.equal(got[0], got[waves]) and not torch.equal(got[0], got[20 - waves])       # (sums in another order)
+
+
+@pytest.mark.parametrize('heads,kv_heads,d,dtype', [(16, 8, 128, torch.bfloat16), (32, 8, 128, torch.bfloat16), (8, 2, 64, torch.bfloat16),
+                                                    (6, 2, 96, torch.bfloat16), (4, 2, 128, torch.float32)])
+@pytest.mark.parametrize('told', [None, 1030])
+@pytest.mark.parametrize('first', [None, 1])
+def test_parts_of_a_portion_beside_a_row_of_a_longer_context(ops, heads, kv_heads, d, dtype, told, first):
+    """40 rows behind 990 keys beside a row alone behind 2,600: whether the keys' parts are made for the portion's own context or
+    for the row's, and whether the merge takes the row too or the portion's rows only."""
+    rows, starts = [40, 1], [990, 2600]
+    lengths = [r + s for r, s in zip(rows, starts)]
+    k_cache, v_cache, table, _ = build_cache(lengths, 16, kv_heads, d, dtype)
+    q = rand(sum(rows), heads * d, dtype=dtype, seed=7)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    step = dict(heads=heads, kv_heads=kv_heads, head_dim=d, page_size=16, block_tables=table, scale=d ** -0.5, window=None,
+                row_seq=ints([i for i, r in enumerate(rows) for _ in range(r)]),
+                positions=ints([s + j for r, s in zip(rows, starts) for j in range(r)]), max_context=max(lengths),
+                cu_seqlens=ints([sum(rows[:i]) for i in range(len(rows) + 1)]), seq_starts=ints(starts),
+                single_rows=ints([rows[0]]), n_seqs=len(rows), max_query=max(rows))
+    got = ops.paged_attention(q, k_cache=k_cache, v_cache=v_cache, tile_context=told, tile_seqs=first, **step)
+    want = refs.paged_attention(q, k_cache=k_cache, v_cache=v_cache, **step)
+    tolerance = dict(atol=2.0 ** -8, rtol=2.0 ** -7) if dtype == torch.bfloat16 else dict(atol=2e-6, rtol=2e-5)
+    torch.testing.assert_close(got.float(), want.float(), **tolerance)
