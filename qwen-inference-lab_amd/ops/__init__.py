@@ -1178,6 +1178,33 @@ def tile_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, pag
     return part.value, parts
 
 
+def portion_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, page_size, table_stride, max_context,
+                      tile_context, general=False, portions_only=False):
+    """``tile_key_parts`` of a step whose portions are known to reach no further than ``tile_context`` (None: max_context), less
+    far than the rows alone beside them.  ``portions_only``: the parts are merged for the portions' rows only.
+
+    Keys that all lie in the first part of the step's plan are not cut at all: every other part would be empty, and the
+    first one's results written in float32, read again and merged.  (us a layer, 32 heads in 8 groups, a first portion of 128
+    rows beside rows of 2,048 tokens: 16 parts 14 and their merge 5, one piece 10.5.  Not so the general bfloat16 kernel, whose one
+    piece gains nothing: 64 rows of 16 heads of 96 in 4 groups, with the row of 2,048 beside them, 23.1 in parts, 24.4 in one
+    piece.)  The bfloat16 kernels for heads of 64 and 128 otherwise plan for the portions' own context (16 heads in 8 groups beside
+    2,048: 600 rows 32.1 -> 26.2, 1,000 rows 45.2 -> 30.4; 300 behind 1,200 beside 16,384 58.3 -> 43.6; at worst level, 600 behind
+    1,000 beside 6,144 43.7 -> 44.8), but for portions behind a history whose context is too short to be cut by itself (64 behind 500
+    beside 2,048: 24.9 in the step's parts, 27.5 in one piece).  The
+    general kernels and the capped form keep the step's plan: parts for a short context of its own are fewer or smaller than what is
+    best there (float32, 8 heads of 256, 400 rows beside 2,048: 79 and 151; 16 heads of 96 in 4 groups, 300 rows: 31 and 39;
+    capped, 16 heads in 4 groups, 600 behind 1,000 beside 6,144: 46 and 58)."""
+    part, parts = tile_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, page_size, table_stride, max_context, general=general)
+    if parts == 1 or tile_context is None or TILE_KEY_PARTS is not None:
+        return part, parts
+    special = dtype == torch.bfloat16 and lib.qil_attn_tile_bf16_takes(head_dim, page_size, table_stride)
+    if tile_context <= part and (special or dtype != torch.bfloat16):
+        return 0, 1
+    if special and head_dim in (64, 128) and not general and portions_only and not max_query < tile_context < 1024:
+        return tile_key_parts(lib, dtype, n_seqs, max_query, heads, kv_heads, head_dim, page_size, table_stride, min(tile_context, max_context))
+    return part, parts
+
+
 def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size, block_tables, row_seq, positions,
                     cu_seqlens, seq_starts, single_rows, n_seqs, max_query, max_context, scale, window,
                     unmerged=False, tile_seqs=None, softcap=None, sinks=None, slopes=None, keep_first=0, plans=None,
@@ -1248,14 +1275,10 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
             if tile_seqs != n_seqs - single_rows.shape[0]:
                 raise ValueError('tile_seqs must count the sequences of two or more rows')
             n_seqs = tile_seqs
-        # A first portion of 128 rows beside rows of 2,048 tokens: planned for its own 128 keys one kernel of 10.5 us a layer, planned
-        # for 2,048 the keys in 16 parts, 14 us, and their merge, 5.
         # (Without ``tile_seqs`` the merge takes the rows alone too, by their positions: the parts have to reach as far as they do.)
-        reach = max_context
-        if tile_context is not None and (tile_seqs is not None or not single_rows.shape[0]):
-            reach = min(tile_context, max_context)
-        part, parts = tile_key_parts(lib, qkv.dtype, several, max_query, heads, kv_heads,
-                                     head_dim, page_size, block_tables.shape[1], reach, general=cap > 0 or slopes is not None)
+        part, parts = portion_key_parts(lib, qkv.dtype, several, max_query, heads, kv_heads, head_dim, page_size, block_tables.shape[1],
+                                        max_context, tile_context, general=cap > 0 or slopes is not None,
+                                        portions_only=tile_seqs is not None or not single_rows.shape[0])
         if keep:
             part, parts = 0, 1
         if parts > 1:

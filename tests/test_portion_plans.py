@@ -80,3 +80,60 @@ def test_every_row_that_is_merged_has_all_its_parts(recorded, portions, alone, t
         if parts > 1 and call[2] is None:                   # no row index: the step's first rows
             assert rows in (sum(n for n, _ in portions), len(got.positions))
             assert max(got.positions[:rows]) // part < parts, (part, parts)
+
+
+def plan_of(recorder):
+    """(keys a part, parts) of the portions' kernel."""
+    if 'qil_attn_tile_bf16_parts' in recorder.calls:
+        return recorder.calls['qil_attn_tile_bf16_parts'][0][-3:-1]
+    if 'qil_attn_tile_in_parts' in recorder.calls:
+        return recorder.calls['qil_attn_tile_in_parts'][0][-5:-3]
+    assert 'qil_attn_tile' in recorder.calls
+    return 0, 1
+
+
+PORTIONS = [[(16, 0)], [(64, 0)], [(128, 0)], [(300, 0)], [(400, 0), (100, 0)], [(512, 0)], [(700, 0)], [(1000, 0)], [(64, 150)], [(64, 500)],
+            [(128, 900)], [(300, 1200)], [(600, 1000)], [(128, 3000)]]
+
+
+@pytest.mark.parametrize('sizes', [dict(dtype=FLOAT32), dict(heads=8, d=256, dtype=FLOAT32), dict(heads=14, kv_heads=2, d=64, dtype=FLOAT32), dict(kv_heads=4, softcap=30.0),
+                                   dict(kv_heads=4, slopes=torch.zeros(16)), dict(kv_heads=4, d=96), dict(d=256), dict(page=24)])
+def test_kernels_with_parts_of_other_sizes_keep_the_steps_plan(recorded, sizes):
+    """... unless all keys of the portions lie in its first part, which the general kernel for bfloat16 cuts all the same."""
+    for portions in PORTIONS:
+        for context in (1100, 2048, 6144, 16384):
+            longest = max(n + s for n, s in portions)
+            if longest >= context:
+                continue
+            part, parts = plan_of(recorded(portions, [context], told=False, **sizes))
+            general = sizes.get('dtype', BFLOAT16) == BFLOAT16 and (sizes.get('d') == 96 or 'page' in sizes)
+            want = (0, 1) if longest <= part and not general else (part, parts)
+            assert plan_of(recorded(portions, [context], **sizes)) == want, (portions, context)
+
+
+@pytest.mark.parametrize('sizes', [dict(), dict(heads=32), dict(heads=64), dict(kv_heads=4, d=64), dict(heads=14, kv_heads=2, d=64), dict(window=700),
+                                   dict(sinks=torch.zeros(16))])
+def test_portions_on_the_kernels_for_heads_of_64_and_128(recorded, sizes):
+    """In one piece where the step's first part holds all their keys; planned for their own context where they bring most of it
+    themselves or it is long enough to be cut, and the merge keeps to them; else as the step."""
+    for portions in PORTIONS:
+        for context in (1100, 2048, 6144, 16384):
+            longest, rows = max(n + s for n, s in portions), max(n for n, _ in portions)
+            if longest >= context:
+                continue
+            step = plan_of(recorded(portions, [context], told=False, **sizes))
+            own = plan_of(recorded(portions, [], told=False, **sizes))
+            got = plan_of(recorded(portions, [context], **sizes))
+            if step[1] > 1 and longest <= step[0]:
+                assert got == (0, 1)
+            elif step[1] > 1 and (longest == rows or longest >= 1024):
+                assert got == own
+            else:
+                assert got == step
+            behind = plan_of(recorded(portions, [context], first=False, **sizes))
+            assert behind == (got if got == (0, 1) and step[0] >= longest else step)
+
+
+def test_a_kept_first_range_stays_in_one_part(recorded):
+    for told in (False, True):
+        assert plan_of(recorded([(128, 900)], [6144], kv_heads=4, window=512, keep_first=64, told=told)) == (0, 1)
