@@ -18,8 +18,8 @@ temperatures travel in the same array), and a step costs one upload, one replay 
 Steps with prompt portions have recurring shapes too (a portion of the chunk size beside so many single
 tokens, step after step while a long prompt comes in), and for small models their launches cost more than
 their kernels.  A shape that has been seen before (the same numbers of tokens and of wanted places per request,
-largest first, the same, wider bucket, and beside single tokens portions that all begin their requests or not) is captured the second time and replayed from then on; the
-requests are put into the graph's order and the logits back into the caller's.  The draw stays outside.
+largest first, the same, wider bucket, and beside single tokens whole prompts or other portions) is captured the second time and
+replayed from then on; the requests are put into the graph's order and the logits back into the caller's.  The draw stays outside.
 
 A new graph warms up (one run launch by launch, which loads the kernels and sizes the allocator) on inert
 inputs of the step's shape, written to the spare page and slot, and is then captured; the step it was made for
@@ -229,11 +229,16 @@ class DecodeGraphs:
         if limit is not None:
             bucket = min(bucket, -(-limit // ps) * ps)
         width = -(-bucket // ps)
-        # Steps whose portions are all their requests' first, beside requests that decode, have graphs of their own: the portions'
-        # attention is planned for the keys they bring and not for the longest context of those requests.
-        first_portions = len(ordered[-1].tokens) == 1 and \
-            all(runner.cache.computed[e.request] == 0 for e in ordered if len(e.tokens) > 1)
-        tile_context = len(ordered[0].tokens) if first_portions else None
+        # Whole prompts (they begin their requests and want logits) beside requests that decode have graphs of their own: their
+        # attention is planned for the keys they bring and not for the longest context of those requests.  The portions of longer
+        # prompts share a graph, the first with those that follow it: one more of every shape costs captures and launched steps
+        # (prompts of 512 tokens in portions of 128, one every 6 steps, 600 such steps: 45 captures and 89 launched with one graph,
+        # 55 and 149 with two; 0.6B sizes 2.07 s and 2.23, 8B sizes of 12 layers 1.77 and 1.84), more than the first portions gain.
+        # Whole prompts gain (100 tokens, 0.6B sizes 100 steps 333 -> 316 ms) and seldom are as long as another prompt's last portion
+        # (where they are, prompts of 128 or 512 tokens in portions of 128: 28 captures and 46 launched -> 33 and 59, 1.13 -> 1.17 s).
+        whole_prompts = len(ordered[-1].tokens) == 1 and \
+            all(e.want and runner.cache.computed[e.request] == 0 for e in ordered if len(e.tokens) > 1)
+        tile_context = len(ordered[0].tokens) if whole_prompts else None
         key = (tuple(len(e.tokens) for e in ordered), tuple(len(e.want) for e in ordered), bucket, tile_context)
         graph = self.mixed.get(key)
         described, pieces, facts = runner._describe(ordered, table_width=width, validate=False)

@@ -258,6 +258,65 @@ def test_which_steps_a_decode_graph_takes(model_folder, cpu_kernels):
     assert not graphs.takes([])
 
 
+def test_which_portions_share_a_graph(model_folder, cpu_kernels, monkeypatch):
+    """Beside a decoding row: the portions of a prompt that comes in in several, its first one too, one graph of their sizes,
+    captured at their second coming; a whole prompt and another one's last portion of as many tokens one each, planned for the
+    prompt's tokens and for any context; every logit against the plain model.  (A graph here is its step, launched again.)"""
+    from qil_amd.engine import graphs as graph_module
+    planned = []
+
+    class Launched:
+        def __init__(self, runner, entries, pieces, facts, bucket, sampler=None, tile_context=None):
+            self.runner, self.meta = runner, torch.from_numpy(pieces.flat()).clone()
+            self.context = runner._context(entries, pieces, facts, self.meta, max_context=bucket, tile_context=tile_context)
+            self.tables = [view.block_tables for view in runner.views], [view.slots for view in runner.views]
+            planned.append((tuple(len(e.tokens) for e in entries), tile_context))
+
+        def load(self, pieces):
+            self.meta.copy_(torch.from_numpy(pieces.flat()))
+
+        def run(self):
+            for view, table, slots in zip(self.runner.views, *self.tables):
+                view.block_tables, view.slots = table, slots
+            return self.runner.model.forward(self.context, self.runner.views)
+
+    monkeypatch.setattr(graph_module, '_Graph', Launched)
+    config = plain.TINY_A
+    folder, weights = model_folder(config, 3)
+    runner = ModelRunner(load_model(folder, dtype=torch.float32, device='cpu'), num_pages=40, page_size=4)
+    poison(runner)
+    runner.graphs = graph_module.DecodeGraphs(runner)
+    runner.graphs.takes = lambda entries: False
+    row, prompt = tokens_for(config, 60, 5), tokens_for(config, 40, 6)
+    want_row, want = plain.logits(row, weights, config), plain.logits(prompt, weights, config)
+    runner.admit('row')
+    runner.step([StepEntry('row', tuple(row[:30]), ())])
+    fed, captures = 30, []
+
+    def beside(request, start, count, wanted):
+        nonlocal fed
+        places = (count - 1,) if wanted else ()
+        logits = runner.step([StepEntry(request, tuple(prompt[start:start + count]), places), StepEntry('row', (row[fed],), (0,))])
+        rows = [want[start + count - 1]] * wanted + [want_row[fed]]
+        torch.testing.assert_close(logits, torch.stack(rows), **TOLERANCE[torch.float32])
+        fed += 1
+        captures.append(runner.graphs.mixed_captures)
+
+    for request in 'ab':                                    # three portions of 8 and a last one of 8 that wants logits
+        runner.admit(request)
+        for start in (0, 8, 16):
+            beside(request, start, 8, False)
+        beside(request, 24, 8, True)
+        runner.release(request)
+    assert captures == [0, 1, 1, 1, 1, 1, 1, 2] and planned == [((8, 1), None)] * 2
+    for request in 'cde':                                   # whole prompts of as many tokens as those last portions
+        runner.admit(request)
+        beside(request, 0, 8, True)
+        runner.release(request)
+    assert captures[8:] == [2, 3, 3] and planned[2:] == [((8, 1), 8)] and runner.graphs.mixed_replays == 8
+    runner.cache.check()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 def test_graph_replays_equal_eager_launches(model_folder, dtype):
