@@ -245,35 +245,65 @@ def test_a_recurring_shape_gives_the_same_bits_launched_and_replayed(model_folde
         assert torch.equal(first, seen[0][0]) and torch.equal(second, seen[0][1])
 
 
+# heads of 32 (the general kernel), and of 128 behind a context bucket of 2,048
+LONG_HEADS = dict(plain.TINY_B, head_dim=128, num_attention_heads=4, max_position_embeddings=4096)
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
-def test_first_portions_have_graphs_of_their_own(model_folder, dtype):
-    """A portion of 40 tokens beside a decoding row of 300, from its request's start, right behind its first token and deep in
-    it: the same sizes and bucket, two plans of the portion's attention.  Three times over each, so launched,
-    captured and replayed; every logit against the plain model."""
+@pytest.mark.parametrize('config', [plain.TINY_B, LONG_HEADS], ids=['heads-of-32', 'heads-of-128'])
+def test_whole_prompts_have_graphs_of_their_own(model_folder, monkeypatch, config, dtype):
+    """Two prompts of 40 and 23 tokens whole beside a decoding row of 300, and portions of as many tokens of longer prompts, from
+    their start (without a wanted place), right behind their first token and deep in them: the same sizes and bucket, two
+    plans of the portions' attention.  Three times over, so launched, captured and replayed; every logit against the plain model."""
+    from qil_amd import ops
     from qil_amd.engine import ModelRunner, StepEntry
     from qil_amd.weights import load_model
-    config = plain.TINY_B
     folder, weights = model_folder(config, 13)
     model = load_model(folder, dtype=dtype, device='cuda')
-    row, prompt = random_tokens(config, 312, 5), random_tokens(config, 400, 6)
-    want_row, want = plain.logits(row, weights, config), plain.logits(prompt, weights, config)
-    runner = ModelRunner(model, num_pages=120, page_size=8, max_requests=2)
+    row, prompts = random_tokens(config, 318, 5), [random_tokens(config, 400, 6), random_tokens(config, 400, 7)]
+    want_row, want = plain.logits(row, weights, config), [plain.logits(tokens, weights, config) for tokens in prompts]
+    runner = ModelRunner(model, num_pages=200, page_size=8, max_requests=3)
     for group in runner.cache.kv_groups:
         group['k'].fill_(float('nan')), group['v'].fill_(float('nan'))
+    plans, plan = [], ops.portion_key_parts
+
+    def recorded(*arguments, **forms):
+        result = plan(*arguments, **forms)
+        plans.append((arguments[10], result))               # what the portions are known to reach, what is made of it
+        return result
+
     runner.admit('row')
     runner.step([StepEntry('row', tuple(row[:300]), ())])
-    fed = 300
+    monkeypatch.setattr(ops, 'portion_key_parts', recorded)
+    fed, seen = 300, {True: set(), False: set()}
     for occurrence in range(3):
-        for start in (0, 1, 24, 300):
-            runner.admit('new')
-            if start:
-                runner.step([StepEntry('new', tuple(prompt[:start]), ())])
-            logits = runner.step([StepEntry('row', (row[fed],), (0,)), StepEntry('new', tuple(prompt[start:start + 40]), (0, 39))]).cpu()
-            torch.testing.assert_close(logits, torch.stack((want_row[fed], want[start], want[start + 39])), **TOLERANCE[dtype])
-            runner.release('new')
+        for start, wanted in ((0, True), (0, False), (1, True), (24, True), (300, True)):
+            for name, tokens in zip('ab', prompts):
+                runner.admit(name)
+                if start:
+                    runner.step([StepEntry(name, tuple(tokens[:start]), ())])
+            plans.clear()
+            entries = [StepEntry(name, tuple(tokens[start:start + count]), (0, count - 1) if wanted else ())
+                       for name, tokens, count in zip('ab', prompts, (40, 23))]
+            logits = runner.step([StepEntry('row', (row[fed],), (0,))] + entries[::-1]).cpu()
+            rows = [want_row[fed]] + ([want[1][start], want[1][start + 22], want[0][start], want[0][start + 39]] if wanted else [])
+            torch.testing.assert_close(logits, torch.stack(rows), **TOLERANCE[dtype])
+            seen[start == 0 and wanted].update(plans)
+            runner.release('a'), runner.release('b')
             fed += 1
-    kinds = {key[3] for key in runner.graphs.mixed if key[0] == (40, 1)}
-    assert kinds == {40, None}, runner.graphs.mixed.keys()
+    shapes = [key for key in runner.graphs.mixed if key[0] == (40, 23, 1)]
+    assert sorted(shapes, key=str) == sorted([((40, 23, 1), (2, 2, 1), longest_of(config), 40), ((40, 23, 1), (2, 2, 1), longest_of(config), None),
+                                              ((40, 23, 1), (0, 0, 1), longest_of(config), None)], key=str)
+    assert runner.graphs.mixed_replays >= 2 * 3, runner.graphs.mixed_replays
+    (told, whole), = seen[True]
+    (not_told, other), = seen[False]
+    assert (told, not_told) == (40, None) and other[1] > 1
+    general = dtype == torch.bfloat16 and config['head_dim'] == 32
+    assert whole == (other if general else (0, 1))
+
+
+def longest_of(config):
+    return min(2048, config['max_position_embeddings'])
 
 
 def test_more_recurring_shapes_than_the_store_holds(model_folder, monkeypatch):

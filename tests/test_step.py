@@ -181,7 +181,8 @@ def test_requests_with_several_tokens_come_first_and_logits_keep_the_callers_ord
 
 
 def test_longest_context_of_the_portions(case):
-    """Not that of the rows alone beside them; a graph's description is for any context of its bucket."""
+    """Not that of the rows alone beside them; a graph's description is for any context of its bucket, or for the portions' that it
+    is made for."""
     config, weights, model, page_size = case
     runner = ModelRunner(model, num_pages=64, page_size=page_size)
     tokens = {r: tokens_for(config, n, seed) for seed, (r, n) in enumerate({'long': 24, 'b': 11, 'c': 7}.items())}
@@ -191,9 +192,10 @@ def test_longest_context_of_the_portions(case):
     entries = [StepEntry('long', tuple(tokens['long'][-1:]), (0,)), StepEntry('b', tuple(tokens['b'][5:]), ()), StepEntry('c', tuple(tokens['c']), ())]
     described, pieces, facts = runner._describe(entries)
     flat = torch.from_numpy(pieces.flat()).to(model.device)
-    context = lambda bucket: runner._context(described, pieces, facts, flat, max_context=bucket)
+    context = lambda bucket, portions=None: runner._context(described, pieces, facts, flat, max_context=bucket, tile_context=portions)
     assert (context(None).max_context, context(None).tile_context) == (24, 11)
     assert (context(32).max_context, context(32).tile_context) == (32, None)
+    assert (context(32, 7).max_context, context(32, 7).tile_context) == (32, 7)
 
 
 def test_step_validation(case):
