@@ -18,11 +18,13 @@
 //    one tile ahead by one lane per load, and the place in it) and is computed on the scalar unit;
 //  * the next tile's loads are issued between the score products (none after a block's last tile);
 //  * the exponentials of the next 16 keys and the reads of their values stand between the value products of 16 keys; the first
-//    values are asked for ahead of the statistics.  With this and the buffer loads (before, every wait for a fragment was one for all
-//    of a wave's reads, and the exponentials stood ahead of all value products), us, 32 heads in 8 groups: 8,192 tokens 656 -> 618,
-//    2,048 52.9 -> 50.1, 500 16.6 -> 16.0; 16 heads in 4 groups 2,048 44.4 -> 42.0, in two groups of waves 38.6 -> 36.8.  The matrix
-//    cores are then busy for 52 % and the vector units for 49 % of the cycles (8,192 tokens), at a clock that the power limit holds
-//    near 1.6 GHz: what is left are instructions, not waits;
+//    values are asked for ahead of the statistics, whose maximum over a row's two lanes is a swap between registers.  us, calls one behind
+//    the other, without all of this (exponentials ahead of all value products, global loads into LDS, a shuffle) and with it, 32 heads
+//    in 8 groups: 8,192 tokens 561 -> 531, 2,048 50.1 -> 48.3, 500 16.2 -> 15.6; 16 heads in 4 groups 2,048 43.4 -> 40.6, in 8 groups and two
+//    groups of waves 36.9 -> 34.6.  With all but one of them (8,192 tokens; 2,048; 2,048 in two groups of waves): exponentials ahead
+//    550, 48.7, 34.7; global loads 538, 47.7, 36.3; a shuffle 536, 49.3, 34.7; first values behind the statistics 534, 48.7, 34.6.
+//    The matrix cores are then busy for 52 % and the vector units for 49 % of the cycles (8,192 tokens), at a clock that the power limit
+//    holds near 1.6 GHz: what is left are instructions, not waits.  (In a model a layer of 8,192 tokens took 615 -> 553 us in a trace.)
 //  * two tiles in LDS, one barrier a tile: after it every wave's loads of this tile have landed and every wave has
 //    finished with the tile before, whose place the next loads take;
 //  * the reference of a row's exponents is only moved (to the maximum) when a score exceeds it by 2^8 in the
@@ -329,11 +331,11 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* __r
     }
     row_m = m_new;
     // Probabilities, 16 keys at a time (scores 8 (u % 2) .. of 32-key tile u / 2), packed as the B operands of the value
-    // products right away: the float32 values are not kept.  Between two value products of 16 keys stand the exponentials of four
-    // scores of the next 16 (two of a lane's eight pairs), and a read of its values: the products take 32 cycles of the
-    // matrix core each and these instructions as many of the vector unit, so neither waits for the other.
+    // products right away: the float32 values are not kept.  Beside each value product of 16 keys stand the exponentials of two
+    // scores of the next 16 (one of a lane's four pairs) and a read of its values, for the vector unit while the matrix core is busy.
     float psum = 0.f;
     uint32_t packed[2][4];
+    static_assert(WTILES == 4, "one pair of the next scores a value product");
     auto probabilities = [&](int u, int e) __attribute__((always_inline)) {
       const int kt = u >> 1, st = u & 1;
       const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kt][8 * st + 2 * e], c, shift));

@@ -529,14 +529,16 @@ extern "C" int qil_attn_tile_bf16_takes(int d, int page_size, int table_stride) 
 // Waves a block of the head-128 kernel: 4, or 16 for 8 waves in two groups that split a block's keys, so that every SIMD has two waves.
 // The groups pay where blocks of 4 waves are fewer than CUs, or few more, and a block passes ten tiles of keys or more (``keys``: of the
 // longest sequence, as far as the host knows); with many more blocks the SIMDs are full anyway and the merge at the end only costs, as it
-// does where the tiles are few.  us in 4 waves / 8, whole prompts, 16 heads in 8 groups: 100 tokens 8.5 / 9.9, 301 12.3 / 13.4, 600
-// 18.5 / 19.0, 700 19.5 / 19.1, 1,000 25.1 / 22.7, 2,000 42.4 / 36.8, 2,300 (288 blocks) 52.4 / 41.4, 2,900 (368) 62.6 / 60.4; 32 heads:
-// 1,200 (304) 34.4 / 31.5, 1,400 (352) 36.4 / 38.7, 2,048 50.2 / 58.1; two of 600 (304) 20.9 / 24.1; three of 301 and 16 heads 12.5 / 13.5.
-// Portions behind a history, 16 / 32 heads: 64 rows behind 400 keys 15.9 / 16.7 and 16.8 / 16.8, 128 behind 500 18.7 / 18.2 and 19.2 / 18.7,
-// 256 behind 500 21.1 / 20.1 and 21.6 / 20.6, 33 behind 700 20.2 / 18.9 and 21.2 / 20.3, 64 behind 900 25.1 / 23.9 and 26.0 / 23.9; beside rows
-// alone (their kernel included) 64 behind 700 and one row 30.1 / 28.9, 64 behind 300 and one of 900 23.5 / 24.8, two of 300 behind 600 34.0 / 32.7.
+// does where the tiles are few.  us in 4 waves / 8, whole prompts, 16 heads in 8 groups: 100 tokens 8.2 / 9.6, 301 11.7 / 12.7, 577
+// 16.5 / 16.3, 600 16.8 / 16.4, 700 18.5 / 18.2, 1,000 23.3 / 21.3, 2,000 40.7 / 34.6, 2,560 (320 blocks) 51.8 / 42.8, 2,900 (368)
+// 58.5 / 57.7; two of 1,300 (336) 31.1 / 34.0; 32 heads: 900 (232) 22.3 / 21.1, 1,280 (320) 30.6 / 29.0, 1,400 (352) 32.6 / 36.3, 2,048 48.5 / 57.5;
+// two of 600 (304) 19.7 / 23.6; three of 301 and 16 heads 12.0 / 13.0.
+// Portions behind a history, 16 / 32 heads: 64 rows behind 400 keys 15.4 / 16.3 and 16.2 / 16.3, 128 behind 500 18.0 / 17.6 and 18.4 / 17.9,
+// 256 behind 500 20.2 / 19.3 and 20.6 / 19.7, 33 behind 700 19.4 / 18.1 and 20.3 / 19.4, 64 behind 900 23.6 / 22.6 and 24.5 / 22.7; beside rows
+// alone (their kernel included) 64 behind 700 and a row of 800 29.0 / 28.1, 64 behind 300 and one of 900 23.2 / 23.7, two of 300 behind 600 and
+// one of 950 32.1 / 31.3.
 // From 1,024 keys on fewer blocks than CUs have their keys cut into parts before they come here (qil_attn_tile_parts), so that the groups
-// get as many blocks as CUs and up to 64 more: 32 heads, four of 256 behind 1,500 44.6 / 40.0, eight of 128 behind 1,000 33.0 / 31.3.
+// get as many blocks as CUs and up to 64 more: 32 heads, four of 256 behind 1,500 40.6 / 37.7, eight of 128 behind 1,000 29.4 / 28.5.
 extern "C" int qil_attn_prompt_waves(int n_seqs, int max_query, int keys, int heads, int kv_heads, int window) {
   const int g = heads / kv_heads, gh = g >= 3 ? 4 : g, rows = 32 * (4 / gh);
   const long blocks = (long)((max_query + rows - 1) / rows) * n_seqs * kv_heads * ((g + gh - 1) / gh);

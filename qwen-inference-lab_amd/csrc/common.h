@@ -37,10 +37,9 @@ __device__ __forceinline__ qil_u32x4 load_once(const void* p) {
 // 16 bytes a lane from `from` (the same for the whole wave) + `lane_offset` bytes straight into LDS at `to` + 16 * lane.  A buffer
 // load, for loops that read LDS meanwhile: the global form is a flat instruction to the compiler, and with a flat one in flight it
 // waits for ALL of a wave's reads of LDS (lgkmcnt(0)) where the oldest are what it needs.
-template <int POLICY = 0>
 __device__ __forceinline__ void load_to_lds(const void* from, uint32_t lane_offset, void* to) {
   const __amdgpu_buffer_rsrc_t source = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(from), 0, (int)0xffffffffu, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(source, (__attribute__((address_space(3))) void*)to, 16, lane_offset, 0, 0, POLICY);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(source, (__attribute__((address_space(3))) void*)to, 16, lane_offset, 0, 0, 0);
 }
 
 __device__ __forceinline__ float ld(const float* p) { return *p; }
