@@ -24,7 +24,7 @@
 //    groups of waves 36.9 -> 34.6.  With all but one of them (8,192 tokens; 2,048; 2,048 in two groups of waves): exponentials ahead
 //    550, 48.7, 34.7; global loads 538, 47.7, 36.3; a shuffle 536, 49.3, 34.7; first values behind the statistics 534, 48.7, 34.6.
 //    The matrix cores are then busy for 52 % and the vector units for 49 % of the cycles (8,192 tokens), at a clock that the power limit
-//    holds near 1.6 GHz: what is left are instructions, not waits.  (In a model a layer of 8,192 tokens took 615 -> 553 us in a trace.)
+//    holds near 1.6 GHz: what is left are instructions, not waits.  (In a model a layer of 8,192 tokens took 619 -> 559 us in a trace.)
 //  * two tiles in LDS, one barrier a tile: after it every wave's loads of this tile have landed and every wave has
 //    finished with the tile before, whose place the next loads take;
 //  * the reference of a row's exponents is only moved (to the maximum) when a score exceeds it by 2^8 in the
