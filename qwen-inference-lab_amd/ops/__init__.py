@@ -1221,8 +1221,8 @@ def paged_attention(q, *, heads, kv_heads, head_dim, k_cache, v_cache, page_size
     (every row alone, context in several parts) for ``linear`` to merge.
     ``tile_seqs``: the caller has put the sequences of two or more rows first and there are this many; the tile
     kernel then gets blocks for these only (None: for every sequence; those of one row leave at once).
-    ``tile_context``: the longest context of the sequences of two or more rows, or more than it, never less (keys beyond it are not
-    read), where the caller knows it; the parts of their keys and the shape of the prompt kernel's blocks go by it.
+    ``tile_context``: the longest context of the sequences of two or more rows, or more than it, never less (keys beyond it may not be
+    read), where the caller knows it; the parts of their keys (``portion_key_parts``) and the shape of the prompt kernel's blocks go by it.
     ``softcap`` c: scores are scaled, then capped softly, c * tanh(score / c), before the softmax.  The kernels
     specialised for bfloat16 heads of 64 and 128 have no cap; capped steps run on the general tile kernel.
     ``sinks`` float32 [heads]: exp(sinks[h]) joins the divisor of head h's softmax once (no key, no value, not

@@ -332,7 +332,8 @@ def test_block_shape_of_portions_behind_a_history(ops, rows, starts, told, waves
 @pytest.mark.parametrize('first', [None, 1])
 def test_parts_of_a_portion_beside_a_row_of_a_longer_context(ops, heads, kv_heads, d, dtype, told, first):
     """40 rows behind 990 keys beside a row alone behind 2,600: whether the keys' parts are made for the portion's own context or
-    for the row's, and whether the merge takes the row too or the portion's rows only."""
+    for the row's, and whether the merge takes the row too or the portion's rows only.  Against the float32 reference: bfloat16 one
+    rounding and its neighbour, float32 sums of a thousand weighted values of size one in another order."""
     rows, starts = [40, 1], [990, 2600]
     lengths = [r + s for r, s in zip(rows, starts)]
     k_cache, v_cache, table, _ = build_cache(lengths, 16, kv_heads, d, dtype)
